@@ -344,3 +344,29 @@ def test_full_log_softmax_fp32_split_rows_merge_inside_the_second_pass(dev):
         np.testing.assert_allclose(out.cpu().numpy(), want, atol=TOL_F32, rtol=0)
         lse = tome_amd.token_logprobs(x, torch.zeros(rows, dtype=torch.int32, device=dev), 0.8, want_lse=True).lse
         np.testing.assert_allclose((x[:, 0] / 0.8 - out[:, 0]).cpu().numpy(), lse.cpu().numpy(), atol=2e-5, rtol=0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,V,stride", [(9, 1, 3), (9, 3, 3), (17, 7, 9), (17, 9, 9), (17, 15, 17), (9, 23, 25), (9, 4099, 4101),
+                                           (9, 50257, 50257), (260, 32771, 32773), (530, 2051, 2053)])
+def test_row_kernel_at_every_phase(dev, dtype, rows, V, stride):
+    """Rows that start at every element phase of a 16-byte unit (odd strides), split over workgroups and not: rows shorter
+    than their head, without a whole unit, with head, units and tail.  The maximum and the target sit at the row's ends
+    and at the first and last unit's borders in turn, with a second equal maximum further right (first one wins)."""
+    rng = np.random.default_rng(rows + V)
+    kvec = 4 if dtype == torch.float32 else 8
+    buf = torch.from_numpy(rng.standard_normal(rows * stride + 8).astype(np.float32)).to(dev).to(dtype)
+    x = torch.as_strided(buf, (rows, V), (stride, 1), 1)              # base off by one element as well
+    t = np.zeros(rows, np.int32)
+    for r in range(rows):
+        head = -(1 + r * stride) % kvec
+        spots = [0, V - 1, head, head - 1, head + kvec - 1, head + (V - head) // kvec * kvec, head + (V - head) // kvec * kvec - 1]
+        spot = min(max(spots[r % len(spots)], 0), V - 1)
+        x[r, spot] = 11.0
+        x[r, min(spot + 1 + r % 9, V - 1)] = 11.0
+        t[r] = spot
+    got, src = _check(x, t, 0.9)
+    np.testing.assert_allclose(got.lp.cpu().numpy(), oracle.logprob_rows(src, t, 0.9), atol=TOL_F32, rtol=0)
+    np.testing.assert_allclose(got.lse.cpu().numpy(), oracle.lse_rows(src, 0.9), atol=TOL_F32, rtol=0)
+    np.testing.assert_allclose(got.entropy.cpu().numpy(), oracle.entropy_rows(src, 0.9), atol=TOL_F32, rtol=0)
+    np.testing.assert_array_equal(got.argmax.cpu().numpy(), oracle.argmax_rows(src))

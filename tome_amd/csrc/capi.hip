@@ -100,11 +100,9 @@ const char* tome_strerror(int code) {
 
 size_t tome_row_logprob_workspace(int64_t rows, int64_t V) {
   if (rows <= 0 || V <= 0) return 0;
-  // Worst case over the vector and the element-wise path; 16 bytes per (row, split).
-  const int s_vec = tome::row_splits_for(rows, V, 8), s_one = tome::row_splits_for(rows, V, 1);
-  const int s4 = tome::row_splits_for(rows, V, 4);
-  int s = s_vec > s_one ? s_vec : s_one;
-  if (s4 > s) s = s4;
+  // The larger of the two element types' split counts; 16 bytes per (row, split).
+  const int s8 = tome::row_splits_for(rows, V, 8), s4 = tome::row_splits_for(rows, V, 4);
+  const int s = s8 > s4 ? s8 : s4;
   return s <= 1 ? 0 : align256((size_t)rows * (size_t)s * 16);
 }
 

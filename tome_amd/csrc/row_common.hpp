@@ -41,6 +41,32 @@ struct Elem<uint16_t> {  // bf16 bit patterns
   }
 };
 
+// A row of V elements as 16-byte load units: `head` single elements up to the first 16-byte boundary, n_units whole units
+// from `p` on, `tail` single elements after them.  The edges (fewer than a unit each) are taken by as many lanes, one
+// element per lane.  Rows of a vocabulary that is no multiple of a unit start anywhere, each row at another phase.
+// Units are numbered in row order, the single elements of the edges being units of their own: element e of the head is
+// unit e, whole unit u is unit head + u, element e of the tail is unit head + n_units + e.
+// Every launch takes this form: rows off a 16-byte boundary went through element-wise loads before (2 or 4 bytes per lane
+// and instruction, bound by the number of loads in flight), 1024 rows of 128258: fp32 271 -> 90 us, bf16 249 -> 51 us, and
+// aligned rows are unchanged (128256: 82.9 / 48.2 -> 82.7 / 48.3 us; their head is empty).
+template <typename T>
+struct RowSpan {
+  static constexpr int kVec = Elem<T>::kVec;
+  const T* row;
+  const u32x4* p;
+  int64_t n_units;
+  int head, tail;
+  __device__ __forceinline__ RowSpan(const T* r, int64_t V) : row(r) {
+    const int off = (int)(reinterpret_cast<uintptr_t>(r) % 16) / (int)sizeof(T);
+    const int to_boundary = (kVec - off) % kVec;
+    head = V < to_boundary ? (int)V : to_boundary;
+    n_units = (V - head) / kVec;
+    tail = (int)(V - head - n_units * kVec);
+    p = reinterpret_cast<const u32x4*>(r + head);
+  }
+  __device__ __forceinline__ int64_t tail_start() const { return head + n_units * kVec; }
+};
+
 template <int N>
 __device__ __forceinline__ float max_of(const float (&x)[N]) {
   float m = x[0];

@@ -6,7 +6,7 @@
 // element is read from HBM once with 16-byte loads and only per-row scalars are written.
 //
 // Grid: rows * splits workgroups of 256 lanes (4 wave64).  A workgroup owns a contiguous
-// range of 16-byte load units of one row, every lane keeps an online (max, sum 2^(y-m))
+// range of 16-byte load units of one row (RowSpan: units start at the row's first 16-byte boundary), every lane keeps an online (max, sum 2^(y-m))
 // pair over the units it reads, lanes are merged by DPP / LDS-crossbar exchanges, the four
 // waves through LDS.  splits == 1 finishes in the same launch; otherwise per-split
 // partials go to the workspace and row_combine_kernel merges them (no float atomics, so
@@ -37,17 +37,17 @@ struct RowArgs {
   float scale;  // log2(e) / temperature
 };
 
-// Unit index -> first element and element count.  Units below n_units are full vectors;
-// units at or above it are the single trailing elements of a row whose V % kVec != 0.
-template <typename T, bool VECTOR>
+// First element of unit `unit` (RowSpan's numbering) that holds the row's maximum.
+template <typename T>
 __device__ __forceinline__ int argmax_in_unit(const T* row, int64_t V, int unit, float mx) {
-  constexpr int kVec = VECTOR ? Elem<T>::kVec : 1;
-  const int64_t n_units = V / kVec;
+  constexpr int kVec = Elem<T>::kVec;
+  const RowSpan<T> sp(row, V);
   // No element above the floor was seen (all -inf / NaN row): report index 0, as a first-max scan would.
-  if (unit < 0 || unit >= n_units + (V - n_units * kVec)) return 0;
-  int64_t first = (unit < n_units) ? (int64_t)unit * kVec : n_units * kVec + (unit - n_units);
-  const int count = (unit < n_units) ? kVec : 1;
-  for (int i = 0; i < count; ++i)
+  if (unit < 0 || unit >= sp.head + sp.n_units + sp.tail) return 0;
+  if (unit < sp.head) return unit;
+  if (unit >= sp.head + sp.n_units) return (int)(sp.tail_start() + (unit - sp.head - sp.n_units));
+  const int64_t first = sp.head + (int64_t)(unit - sp.head) * kVec;
+  for (int i = 0; i < kVec; ++i)
     if (Elem<T>::load1(row + first + i) == mx) return (int)(first + i);
   return (int)first;
 }
@@ -71,14 +71,14 @@ __device__ __forceinline__ void finish_row(const RowArgs& a, const T* row, int64
   if (a.out_lp) a.out_lp[r] = (fmaf(x_t, a.scale, -m) - log2s) * kLn2;  // NaN in, NaN out
   if (a.out_lse) a.out_lse[r] = (m + log2s) * kLn2;
   if constexpr (ENT) a.out_entropy[r] = (log2s - st.w / st.s) * kLn2;  // w is relative to the maximum: no m here
-  if constexpr (AMAX) a.out_argmax[r] = argmax_in_unit<T, true>(row, a.V, st.bi, st.mx);
+  if constexpr (AMAX) a.out_argmax[r] = argmax_in_unit<T>(row, a.V, st.bi, st.mx);
 }
 
 // KEEP: the caller reads the rows again right away (the second pass of the full log-softmax matrix), so they are
 // loaded with ordinary loads and stay in the caches; everyone else streams them past the caches.
-template <typename T, bool VECTOR, bool ENT, bool AMAX, bool KEEP = false>
+template <typename T, bool ENT, bool AMAX, bool KEEP = false>
 __global__ __launch_bounds__(kRowWG) void row_logprob_kernel(RowArgs a) {
-  constexpr int kVec = VECTOR ? Elem<T>::kVec : 1;
+  constexpr int kVec = Elem<T>::kVec;
   __shared__ RowLds lds;
   const int64_t r = blockIdx.x / a.splits;  // problem index
   const int split = blockIdx.x % a.splits;
@@ -105,74 +105,58 @@ __global__ __launch_bounds__(kRowWG) void row_logprob_kernel(RowArgs a) {
   }
 
   const T* row = static_cast<const T*>(a.logits) + src * a.row_stride;
-  const int64_t n_units = a.V / kVec;
-  const int64_t per_split = (n_units + a.splits - 1) / a.splits;
+  const RowSpan<T> sp(row, a.V);
+  const int64_t per_split = (sp.n_units + a.splits - 1) / a.splits;
   const int64_t u0 = per_split * split;
-  const int64_t u1 = (u0 + per_split < n_units) ? u0 + per_split : n_units;
+  const int64_t u1 = (u0 + per_split < sp.n_units) ? u0 + per_split : sp.n_units;
 
   float x_t = 0.f;
   if (tid == 0 && a.splits == 1) x_t = load_target_logit<T>(a, row, r);
   RowStat st = stat_identity();
-  if constexpr (VECTOR) {
-    const u32x4* p = reinterpret_cast<const u32x4*>(row);
-    int64_t u = u0 + tid;
-    for (; u + (kRowUnroll - 1) * kRowWG < u1; u += kRowUnroll * kRowWG) {  // several 16-byte loads in flight per lane
-      u32x4 v[kRowUnroll];
+  if (split == 0 && tid < sp.head) {  // single elements in front of the first whole unit, one per lane
+    float x[1] = {Elem<T>::load1(row + tid)};
+    absorb<1, ENT, AMAX>(st, x, tid, a.scale);
+  }
+  const u32x4* p = sp.p;
+  int64_t u = u0 + tid;
+  for (; u + (kRowUnroll - 1) * kRowWG < u1; u += kRowUnroll * kRowWG) {  // several 16-byte loads in flight per lane
+    u32x4 v[kRowUnroll];
 #pragma unroll
-      for (int k = 0; k < kRowUnroll; ++k) v[k] = KEEP ? p[u + k * kRowWG] : __builtin_nontemporal_load(p + u + k * kRowWG);
+    for (int k = 0; k < kRowUnroll; ++k) v[k] = KEEP ? p[u + k * kRowWG] : __builtin_nontemporal_load(p + u + k * kRowWG);
 #pragma unroll
-      for (int k = 0; k < kRowUnroll; ++k) {
+    for (int k = 0; k < kRowUnroll; ++k) {
+      float x[kVec];
+      Elem<T>::unpack(v[k], x);
+      absorb<kVec, ENT, AMAX>(st, x, sp.head + (int)(u + k * kRowWG), a.scale);
+    }
+  }
+  {  // leftover units of this lane, issued together so their latencies overlap
+    u32x4 v[kRowUnroll - 1];
+#pragma unroll
+    for (int k = 0; k < kRowUnroll - 1; ++k)
+      if (u + k * kRowWG < u1) v[k] = KEEP ? p[u + k * kRowWG] : __builtin_nontemporal_load(p + u + k * kRowWG);
+#pragma unroll
+    for (int k = 0; k < kRowUnroll - 1; ++k)
+      if (u + k * kRowWG < u1) {
         float x[kVec];
         Elem<T>::unpack(v[k], x);
-        absorb<kVec, ENT, AMAX>(st, x, (int)(u + k * kRowWG), a.scale);
+        absorb<kVec, ENT, AMAX>(st, x, sp.head + (int)(u + k * kRowWG), a.scale);
       }
-    }
-    {  // leftover units of this lane, issued together so their latencies overlap
-      u32x4 v[kRowUnroll - 1];
-#pragma unroll
-      for (int k = 0; k < kRowUnroll - 1; ++k)
-        if (u + k * kRowWG < u1) v[k] = KEEP ? p[u + k * kRowWG] : __builtin_nontemporal_load(p + u + k * kRowWG);
-#pragma unroll
-      for (int k = 0; k < kRowUnroll - 1; ++k)
-        if (u + k * kRowWG < u1) {
-          float x[kVec];
-          Elem<T>::unpack(v[k], x);
-          absorb<kVec, ENT, AMAX>(st, x, (int)(u + k * kRowWG), a.scale);
-        }
-    }
-    // Trailing V % kVec elements: one unit each, taken by lane 0 of the last split.
-    if (split == a.splits - 1 && tid == 0) {
-      for (int64_t e = n_units * kVec; e < a.V; ++e) {
-        float x[1] = {Elem<T>::load1(row + e)};
-        absorb<1, ENT, AMAX>(st, x, (int)(n_units + (e - n_units * kVec)), a.scale);
-      }
-    }
-  } else {
-    for (int64_t u = u0 + tid; u < u1; u += kRowWG) {
-      float x[1] = {Elem<T>::load1(row + u)};
-      absorb<1, ENT, AMAX>(st, x, (int)u, a.scale);
-    }
+  }
+  if (split == a.splits - 1 && tid < sp.tail) {  // ... and after the last one
+    const int64_t e = sp.tail_start() + tid;
+    float x[1] = {Elem<T>::load1(row + e)};
+    absorb<1, ENT, AMAX>(st, x, sp.head + (int)sp.n_units + tid, a.scale);
   }
 
   const RowStat tot = block_reduce(st, a.scale, lds);
   if (tid != 0) return;
-  if (a.splits == 1) {
-    if constexpr (VECTOR) {
-      finish_row<T, ENT, AMAX>(a, row, r, tot, x_t);
-    } else {
-      // Scalar path: unit index == element index.
-      RowArgs b = a;
-      b.out_argmax = nullptr;
-      finish_row<T, ENT, false>(b, row, r, tot, x_t);
-      if constexpr (AMAX) a.out_argmax[r] = tot.bi < a.V ? tot.bi : 0;
-    }
-  } else {
-    a.partials[r * a.splits + split] = RowPartial{tot.mx, tot.s, tot.w, tot.bi};
-  }
+  if (a.splits == 1) finish_row<T, ENT, AMAX>(a, row, r, tot, x_t);
+  else a.partials[r * a.splits + split] = RowPartial{tot.mx, tot.s, tot.w, tot.bi};
 }
 
 // One wave per row merges the per-split partials (splits <= 64).
-template <typename T, bool VECTOR, bool ENT, bool AMAX>
+template <typename T, bool ENT, bool AMAX>
 __global__ __launch_bounds__(64) void row_combine_kernel(RowArgs a) {
   const int64_t r = blockIdx.x;
   if (a.row_valid && a.row_valid[r] == 0) return;  // outputs already zeroed by the main kernel
@@ -189,34 +173,27 @@ __global__ __launch_bounds__(64) void row_combine_kernel(RowArgs a) {
   }
   stat_wave_reduce(st, a.scale);
   if (lane != 0) return;
-  if constexpr (VECTOR) {
-    finish_row<T, ENT, AMAX>(a, row, r, st, x_t);
-  } else {
-    RowArgs b = a;
-    b.out_argmax = nullptr;
-    finish_row<T, ENT, false>(b, row, r, st, x_t);
-    if constexpr (AMAX) a.out_argmax[r] = st.bi < a.V ? st.bi : 0;
-  }
+  finish_row<T, ENT, AMAX>(a, row, r, st, x_t);
 }
 
-template <typename T, bool VECTOR, bool ENT, bool AMAX, bool KEEP = false>
+template <typename T, bool ENT, bool AMAX, bool KEEP = false>
 static hipError_t launch_row(const RowArgs& a, int64_t rows, hipStream_t stream, bool skip_combine = false) {
-  hipLaunchKernelGGL((row_logprob_kernel<T, VECTOR, ENT, AMAX, KEEP>), dim3((unsigned)(rows * a.splits)),
+  hipLaunchKernelGGL((row_logprob_kernel<T, ENT, AMAX, KEEP>), dim3((unsigned)(rows * a.splits)),
                      dim3(kRowWG), 0, stream, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.splits == 1 || skip_combine) return e;
-  hipLaunchKernelGGL((row_combine_kernel<T, VECTOR, ENT, AMAX>), dim3((unsigned)rows), dim3(64), 0,
+  hipLaunchKernelGGL((row_combine_kernel<T, ENT, AMAX>), dim3((unsigned)rows), dim3(64), 0,
                      stream, a);
   return hipGetLastError();
 }
 
-template <typename T, bool VECTOR>
+template <typename T>
 static hipError_t dispatch_flags(const RowArgs& a, int64_t rows, hipStream_t stream) {
   const bool ent = a.out_entropy != nullptr, amax = a.out_argmax != nullptr;
-  if (ent && amax) return launch_row<T, VECTOR, true, true>(a, rows, stream);
-  if (ent) return launch_row<T, VECTOR, true, false>(a, rows, stream);
-  if (amax) return launch_row<T, VECTOR, false, true>(a, rows, stream);
-  return launch_row<T, VECTOR, false, false>(a, rows, stream);
+  if (ent && amax) return launch_row<T, true, true>(a, rows, stream);
+  if (ent) return launch_row<T, true, false>(a, rows, stream);
+  if (amax) return launch_row<T, false, true>(a, rows, stream);
+  return launch_row<T, false, false>(a, rows, stream);
 }
 
 // How many workgroups share a row.  From 512 rows on one workgroup per row; smaller batches (decode steps,
@@ -228,7 +205,7 @@ int row_splits_for(int64_t rows, int64_t V, int vec) {
   const int64_t units = V / vec;
   // Short rows (up to 128 KB) in batches of 256 and more: one workgroup per CU is there already, and the combine launch
   // costs more than the second half of the chip brings (256 rows of 32000: fp32 10.6 against 12.0 us, bf16 7.8 against 9.9).
-  if (rows >= 256 && vec > 1 && units <= 8192) return 1;
+  if (rows >= 256 && units <= 8192) return 1;
   const int64_t want_wgs = 512;
   int64_t s = (want_wgs + rows - 1) / rows;
   const int64_t max_by_work = units / (2 * kRowWG);  // >= 2 loads per lane per split
@@ -246,7 +223,6 @@ hipError_t row_logprob_launch_rows(const void* logits, int dtype, int64_t n_rows
                                    int32_t* out_argmax, void* workspace, hipStream_t stream) {
   const int esize = dtype == 0 ? 4 : 2;
   const int vec = 16 / esize;
-  const bool vector_ok = (reinterpret_cast<uintptr_t>(logits) % 16 == 0) && (row_stride % vec == 0);
   RowArgs a;
   a.logits = logits;
   a.row_index = row_index;
@@ -260,13 +236,9 @@ hipError_t row_logprob_launch_rows(const void* logits, int dtype, int64_t n_rows
   a.partials = static_cast<RowPartial*>(workspace);
   a.V = V;
   a.row_stride = row_stride;
-  a.splits = row_splits_for(rows, V, vector_ok ? vec : 1);
+  a.splits = row_splits_for(rows, V, vec);
   a.scale = kLog2e / temperature;
-  if (dtype == 0) {
-    return vector_ok ? dispatch_flags<float, true>(a, rows, stream) : dispatch_flags<float, false>(a, rows, stream);
-  }
-  return vector_ok ? dispatch_flags<uint16_t, true>(a, rows, stream)
-                   : dispatch_flags<uint16_t, false>(a, rows, stream);
+  return dtype == 0 ? dispatch_flags<float>(a, rows, stream) : dispatch_flags<uint16_t>(a, rows, stream);
 }
 
 // The rows' logsumexp for a caller that merges split rows itself: only the main kernel is launched.  With
@@ -276,7 +248,6 @@ hipError_t row_lse_partials_launch(const void* logits, int dtype, int64_t rows, 
                                    float temperature, float* out_lse, void* workspace, int* splits, hipStream_t stream) {
   const int esize = dtype == 0 ? 4 : 2;
   const int vec = 16 / esize;
-  const bool vector_ok = (reinterpret_cast<uintptr_t>(logits) % 16 == 0) && (row_stride % vec == 0);
   RowArgs a{};
   a.logits = logits;
   a.n_rows = rows;
@@ -284,20 +255,15 @@ hipError_t row_lse_partials_launch(const void* logits, int dtype, int64_t rows, 
   a.partials = static_cast<RowPartial*>(workspace);
   a.V = V;
   a.row_stride = row_stride;
-  a.splits = row_splits_for(rows, V, vector_ok ? vec : 1);
+  a.splits = row_splits_for(rows, V, vec);
   a.scale = kLog2e / temperature;
   *splits = a.splits;
   // The caller's second pass reads the matrix again: up to ~3/4 GB it pays to leave the rows in the caches (measured, both
   // passes, fp32 rows of 151936: 64 rows 25.9 -> 24.4 us, 512 rows 155 -> 145, 1024 rows 312 -> 294; 2048 rows 628 -> 648).
-  const bool keep = vector_ok && (double)rows * (double)V * esize <= 768.0 * 1024 * 1024;
-  if (dtype == 0) {
-    if (keep) return launch_row<float, true, false, false, true>(a, rows, stream, true);
-    return vector_ok ? launch_row<float, true, false, false>(a, rows, stream, true)
-                     : launch_row<float, false, false, false>(a, rows, stream, true);
-  }
-  if (keep) return launch_row<uint16_t, true, false, false, true>(a, rows, stream, true);
-  return vector_ok ? launch_row<uint16_t, true, false, false>(a, rows, stream, true)
-                   : launch_row<uint16_t, false, false, false>(a, rows, stream, true);
+  const bool keep = (double)rows * (double)V * esize <= 768.0 * 1024 * 1024;
+  if (dtype == 0)
+    return keep ? launch_row<float, false, false, true>(a, rows, stream, true) : launch_row<float, false, false>(a, rows, stream, true);
+  return keep ? launch_row<uint16_t, false, false, true>(a, rows, stream, true) : launch_row<uint16_t, false, false>(a, rows, stream, true);
 }
 
 hipError_t row_logprob_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
@@ -356,10 +322,9 @@ static hipError_t row_scratch_for_current_device(void** out) {
 }
 
 // Bytes of partials a call with these shapes writes (0 when every row is one workgroup).
-size_t row_partials_bytes(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride) {
+size_t row_partials_bytes(int dtype, int64_t rows, int64_t V) {
   const int vec = 16 / (dtype == 0 ? 4 : 2);
-  const bool vector_ok = (reinterpret_cast<uintptr_t>(logits) % 16 == 0) && (row_stride % vec == 0);
-  const int splits = row_splits_for(rows, V, vector_ok ? vec : 1);
+  const int splits = row_splits_for(rows, V, vec);
   return splits <= 1 ? 0 : (size_t)rows * (size_t)splits * sizeof(RowPartial);
 }
 
@@ -369,7 +334,7 @@ hipError_t row_logprob_noalloc_launch(const void* logits, int dtype, int64_t row
                                       const int32_t* targets, const int32_t* row_valid, float temperature,
                                       float* out_lp, float* out_lse, float* out_entropy, int32_t* out_argmax,
                                       bool* too_big, hipStream_t stream) {
-  *too_big = row_partials_bytes(logits, dtype, rows, V, row_stride) > g_scratch_limit.load(std::memory_order_relaxed);
+  *too_big = row_partials_bytes(dtype, rows, V) > g_scratch_limit.load(std::memory_order_relaxed);
   if (*too_big) return hipSuccess;
   void* ptr = nullptr;
   const hipError_t e = row_scratch_for_current_device(&ptr);
