@@ -196,3 +196,31 @@ def test_decode_step_graph_replays_match_eager(dev):
         (x @ x[:8].T).sum().item()
     x64 = x.cpu().numpy().astype(np.float64)
     np.testing.assert_array_equal(amax.cpu().numpy(), np.argmax(x64, -1))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,V,stride", [(9, 5, 7), (17, 15, 17), (9, 1031, 1033), (17, 4099, 4101), (9, 50257, 50257), (520, 16389, 16391)])
+def test_sampler_at_every_phase(dev, dtype, rows, V, stride):
+    """Rows that start at every element of a 16-byte unit (odd strides, base off by one element): rows without a whole
+    unit, one range and several, register-resident and streaming ranges.  Likely ids sit at the single elements of the
+    row's edges and around the first and last unit."""
+    rng = np.random.default_rng(rows + V)
+    kvec = 4 if dtype == torch.float32 else 8
+    buf = torch.from_numpy((rng.standard_normal(rows * stride + 9) * 2).astype(np.float32)).to(dev).to(dtype)
+    x = torch.as_strided(buf, (rows, V), (stride, 1), 1)
+    for r in range(rows):
+        head = -(1 + r * stride) % kvec
+        for i, spot in enumerate([0, V - 1, head, head - 1, head + (V - head) // kvec * kvec, head + (V - head) // kvec * kvec - 1]):
+            if 0 <= spot < V:
+                x[r, spot] = 9.0 - 0.25 * ((i + r) % 6)
+    x64 = x.float().cpu().numpy().astype(np.float64)
+    k = 20
+    us = _safe_uniforms(x64, 1.0, k, rng)
+    got = tome_amd.sample_tokens(x, 1.0, k, uniforms=torch.from_numpy(us).to(dev), want_topk=True)
+    want_idx, want_val = oracle.top_k_rows(x64, k)
+    want_tok, want_lp = oracle.sample_top_k(x64, us, 1.0, k)
+    np.testing.assert_array_equal(got.topk_idx.cpu().numpy(), want_idx)
+    np.testing.assert_array_equal(got.topk_logit.cpu().numpy()[want_idx >= 0], want_val[want_idx >= 0].astype(np.float32))
+    np.testing.assert_array_equal(got.token.cpu().numpy(), want_tok)
+    np.testing.assert_allclose(got.lp.cpu().numpy(), want_lp, atol=1e-4, rtol=0)
+    np.testing.assert_array_equal(got.argmax.cpu().numpy(), np.argmax(x64, axis=-1))

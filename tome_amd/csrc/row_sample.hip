@@ -11,6 +11,8 @@
 // kernel takes the inverse CDF of softmax(top-k logits / T), the k candidates ordered by logit
 // (descending; equal logits by ascending token id).  MLX's own random stream cannot be matched.
 //
+// Rows may start at any element (RowSpan): 1024 rows of 128258 fp32 / bf16 303 / 445 us on element-wise loads, 94 / 72 us here.
+//
 // A row is shared by `splits` workgroups (decode batches are a few dozen rows: one workgroup per row
 // would leave most of the chip idle).  Each computes, over its range of the row,
 //   * the online (max, sum 2^(y-m)) for the full-vocabulary lse and every lane's own largest element;
@@ -259,10 +261,9 @@ __device__ __forceinline__ void finish_sample(const SampleArgs& a, uint64_t key,
 
 // CACHED: the host promises that a lane owns at most kSampCached load units (short ranges: decode
 // batches split over many workgroups); they are loaded once and both passes run from registers.
-template <typename T, bool VECTOR, bool CACHED>
+template <typename T, bool CACHED>
 __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) void row_sample_kernel(SampleArgs a) {
-  static_assert(VECTOR || !CACHED, "the cached variant is for 16-byte units");
-  constexpr int kVec = VECTOR ? Elem<T>::kVec : 1;
+  constexpr int kVec = Elem<T>::kVec;
   __shared__ SampleLds<kSampCap> sh;
   const int64_t r = blockIdx.x / a.splits;
   const int split = blockIdx.x % a.splits;
@@ -285,14 +286,15 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
   }
 
   const T* row = static_cast<const T*>(a.logits) + r * a.row_stride;
-  const int64_t n_units = a.V / kVec;
-  const int64_t per_split = (n_units + a.splits - 1) / a.splits;
+  const RowSpan<T> sp(row, a.V);
+  const int64_t per_split = (sp.n_units + a.splits - 1) / a.splits;
   const int64_t u0 = per_split * split;
-  const int64_t u1 = (u0 + per_split < n_units) ? u0 + per_split : n_units;
-  // single elements after the last whole unit: lane 0 of the last split
-  const int n_tail = split == a.splits - 1 ? (int)(a.V - n_units * kVec) : 0;
+  const int64_t u1 = (u0 + per_split < sp.n_units) ? u0 + per_split : sp.n_units;
+  // single elements in front of the first whole unit (first split) and after the last one (last split), one per lane
+  const int n_head = split == 0 ? sp.head : 0;
+  const int n_tail = split == a.splits - 1 ? sp.tail : 0;
 
-  const bool big_range = (u1 - u0) * kVec + n_tail > kSampCap;
+  const bool big_range = (u1 - u0) * kVec + n_head + n_tail > kSampCap;
   if (tid == 0) sh.cnt = 0;  // published by the first barrier below, before any candidate is offered
   // A candidate: a logit above -inf (a -inf logit has probability zero and is never drawn; NaN fails every
   // compare) at or above the bound (value first, then the whole key).
@@ -305,7 +307,6 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
       }
     }
   };
-  bool collected = false;  // the streaming variant gathers its candidates during pass 1
 
   // ---- pass 1: full-vocabulary statistics and this lane's own maximum --------------------------
   RowStat st = stat_identity();
@@ -313,18 +314,18 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
   float lane_max = -INFINITY;  // this lane's largest element, or -inf when it saw nothing above -inf
   RowStat tot = stat_identity();
   uint64_t theta = 0;
-  float tail[Elem<T>::kVec - 1];  // cached variant: the single elements after the last whole unit (lane 0 of the last split)
+  const u32x4* p = sp.p;
+  const int64_t tail_e = sp.tail_start() + tid;
+  const float x_head = tid < n_head ? Elem<T>::load1(row + tid) : -INFINITY;  // -inf: adds nothing, is no candidate
+  const float x_tail = tid < n_tail ? Elem<T>::load1(row + tail_e) : -INFINITY;
   if constexpr (CACHED) {
     // Everything a lane owns is in registers, so the statistics take two sweeps over them instead of an online
     // update: the maxima first, then the sum of 2^(y - m) against one reference per wave (no rescaling chain).
-    const u32x4* p = reinterpret_cast<const u32x4*>(row);
 #pragma unroll
     for (int q = 0; q < kSampCached; ++q) {  // unconditional (clamped) loads: all eight in flight together
       const int64_t u = u0 + tid + q * kRowWG;
       cached[q] = __builtin_nontemporal_load(p + (u < u1 ? u : 0));  // unit 0 exists (checked on the host)
     }
-#pragma unroll
-    for (int e = 0; e < kVec - 1; ++e) tail[e] = (tid == 0 && e < n_tail) ? Elem<T>::load1(row + n_units * kVec + e) : -INFINITY;
 #pragma unroll
     for (int q = 0; q < kSampCached; ++q)
       if (u0 + tid + q * kRowWG < u1) {
@@ -332,8 +333,7 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
         Elem<T>::unpack(cached[q], x);
         lane_max = fmaxf(lane_max, max_of_raw<kVec>(x));
       }
-#pragma unroll
-    for (int e = 0; e < kVec - 1; ++e) lane_max = fmaxf(lane_max, tail[e]);
+    lane_max = fmaxf(lane_max, fmaxf(x_head, x_tail));
     float wmax = lane_max;  // maximum of the wave
     wmax = fmaxf(wmax, wave_exchange<0>(wmax));
     wmax = fmaxf(wmax, wave_exchange<1>(wmax));
@@ -355,8 +355,7 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
           s1 += fast_exp2(fmaf(x[i + 1], a.scale, -mm));
         }
       }
-#pragma unroll
-    for (int e = 0; e < kVec - 1; ++e) s0 += fast_exp2(fmaf(tail[e], a.scale, -mm));  // -inf adds nothing
+    s0 += fast_exp2(fmaf(x_head, a.scale, -mm)) + fast_exp2(fmaf(x_tail, a.scale, -mm));
     float ws = s0 + s1;
     ws += wave_exchange<0>(ws);
     ws += wave_exchange<1>(ws);
@@ -373,13 +372,12 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
     for (int w = 0; w < kRowWaves; ++w) stat_merge(tot, RowStat{sh.red.mx[w], sh.red.s[w], 0.f, 0x7fffffff}, a.scale);
     // theta: k-th largest lane maximum (ranges that fit the buffer skip the bound)
     if (big_range) theta = bound_from_lane_maxima(sh, lane_max, k);
-  } else if constexpr (VECTOR) {
+  } else {
     // Streaming variant: candidates are collected during this one pass.  The k-th largest of the
     // lanes' maxima over their FIRST units is already a lower bound of the row's k-th largest, so
     // everything at or above it goes to the buffer as it streams by; after a quarter of the range
     // the bound is renewed from the maxima so far, which lets far less through (a few hundred
     // candidates per row in all).
-    const u32x4* p = reinterpret_cast<const u32x4*>(row);
     constexpr int kGroup = kRowUnroll * kRowWG;                    // units per workgroup and iteration
     const int64_t n_groups = (u1 > u0 ? u1 - u0 : 0) / kGroup;     // iterations in which every lane has all its units
     uint64_t early = 0;  // ranges that fit the buffer are collected whole
@@ -389,7 +387,7 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
       Elem<T>::unpack(v, x);
       if (absorb<kVec, false, true>(st, x, (int)unit, a.scale) >= early_val) {
 #pragma unroll
-        for (int i = 0; i < kVec; ++i) offer(x[i], unit * kVec + i, early, early_val);
+        for (int i = 0; i < kVec; ++i) offer(x[i], sp.head + unit * kVec + i, early, early_val);
       }
     };
     auto renew_bound = [&]() {
@@ -414,7 +412,7 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
         Elem<T>::unpack(first[q], x);
         if (max_of_raw<kVec>(x) >= early_val) {
 #pragma unroll
-          for (int i = 0; i < kVec; ++i) offer(x[i], (u0 + tid + q * kRowWG) * kVec + i, early, early_val);
+          for (int i = 0; i < kVec; ++i) offer(x[i], sp.head + (u0 + tid + q * kRowWG) * kVec + i, early, early_val);
         }
       }
       g0 = 1;
@@ -431,18 +429,15 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
       for (int q = 0; q < kRowUnroll; ++q) consume(v[q], u0 + gi * kGroup + tid + q * kRowWG);
     }
     for (int64_t u = u0 + n_groups * kGroup + tid; u < u1; u += kRowWG) consume(__builtin_nontemporal_load(p + u), u);
-    if (tid == 0) {
-      for (int e = 0; e < n_tail; ++e) {
-        float x[1] = {Elem<T>::load1(row + n_units * kVec + e)};
-        absorb<1, false, true>(st, x, (int)(n_units + e), a.scale);
-        offer(x[0], n_units * kVec + e, early, early_val);
-      }
+    if (tid < n_head) {
+      float x[1] = {x_head};
+      absorb<1, false, true>(st, x, 0, a.scale);
+      offer(x_head, tid, early, early_val);
     }
-    collected = true;
-  } else {
-    for (int64_t u = u0 + tid; u < u1; u += kRowWG) {
-      float x[1] = {Elem<T>::load1(row + u)};
-      absorb<1, false, true>(st, x, (int)u, a.scale);
+    if (tid < n_tail) {
+      float x[1] = {x_tail};
+      absorb<1, false, true>(st, x, 0, a.scale);
+      offer(x_tail, tail_e, early, early_val);
     }
   }
   int m = 0;
@@ -450,19 +445,17 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
   if constexpr (!CACHED) {
     lane_max = st.bi != 0x7fffffff ? st.mx : -INFINITY;  // nothing above the floor seen: -inf
     tot = block_reduce(st, a.scale, sh.red);  // valid in wave 0; its barrier also ends the offers of pass 1
-    if (collected) {
-      const int offered = sh.cnt;
-      if (offered <= kSampCap) {
-        m = offered;
-        scan = false;
-      } else {  // the early bound let too much through: fall back to the bound from the whole range and rescan
-        __syncthreads();
-        if (tid == 0) sh.cnt = 0;
-      }
+    const int offered = sh.cnt;
+    if (offered <= kSampCap) {
+      m = offered;
+      scan = false;
+    } else {  // the early bound let too much through: fall back to the bound from the whole range and rescan
+      __syncthreads();
+      if (tid == 0) sh.cnt = 0;
+      // ---- theta: k-th largest lane maximum (ranges that fit the buffer skip the bound) --------------
+      if (big_range) theta = bound_from_lane_maxima(sh, lane_max, k);
+      else __syncthreads();
     }
-    // ---- theta: k-th largest lane maximum (ranges that fit the buffer skip the bound) --------------
-    if (scan && big_range) theta = bound_from_lane_maxima(sh, lane_max, k);
-    else if (scan && collected) __syncthreads();
   }
 
   // ---- pass 2: collect every element >= theta ---------------------------------------------------
@@ -473,7 +466,7 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
       const float theta_val = theta == 0 ? -INFINITY : key_float((uint32_t)(theta >> 32));
       // Opaque to the optimiser, so that the keys and element indices below are formed where they are
       // used (rarely) instead of being hoisted out of the retry loop into a hundred live registers.
-      uint32_t first_elem = (uint32_t)((u0 + tid) * kVec);
+      uint32_t first_elem = (uint32_t)(sp.head + (u0 + tid) * kVec);
       asm volatile("" : "+v"(first_elem));
 #pragma unroll
       for (int q = 0; q < kSampCached; ++q)
@@ -489,9 +482,8 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
           }
           __builtin_amdgcn_sched_barrier(0);
         }
-      if (tid == 0)
-#pragma unroll
-        for (int e = 0; e < kVec - 1; ++e) offer(tail[e], n_units * kVec + e, theta, theta_val);  // -inf where there is none
+      offer(x_head, tid, theta, theta_val);
+      offer(x_tail, tail_e, theta, theta_val);
       __syncthreads();
       const int offered = sh.cnt;
       if (offered <= kSampCap) {
@@ -517,36 +509,31 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
     while (scan) {
       const float theta_val = theta == 0 ? -INFINITY : key_float((uint32_t)(theta >> 32));
       auto offer2 = [&](float x, int64_t idx) { offer(x, idx, theta, theta_val); };
-      if constexpr (VECTOR) {
-        const u32x4* p = reinterpret_cast<const u32x4*>(row);
-        int64_t u = u0 + tid;
-        for (; u + (kRowUnroll - 1) * kRowWG < u1; u += kRowUnroll * kRowWG) {
-          u32x4 v[kRowUnroll];
+      int64_t u = u0 + tid;
+      for (; u + (kRowUnroll - 1) * kRowWG < u1; u += kRowUnroll * kRowWG) {
+        u32x4 v[kRowUnroll];
 #pragma unroll
-          for (int q = 0; q < kRowUnroll; ++q) v[q] = p[u + q * kRowWG];
+        for (int q = 0; q < kRowUnroll; ++q) v[q] = p[u + q * kRowWG];
 #pragma unroll
-          for (int q = 0; q < kRowUnroll; ++q) {
-            float x[kVec];
-            Elem<T>::unpack(v[q], x);
-            if (max_of_raw<kVec>(x) >= theta_val) {
-#pragma unroll
-              for (int i = 0; i < kVec; ++i) offer2(x[i], (u + q * kRowWG) * kVec + i);
-            }
-          }
-        }
-        for (; u < u1; u += kRowWG) {
+        for (int q = 0; q < kRowUnroll; ++q) {
           float x[kVec];
-          Elem<T>::unpack(p[u], x);
+          Elem<T>::unpack(v[q], x);
           if (max_of_raw<kVec>(x) >= theta_val) {
 #pragma unroll
-            for (int i = 0; i < kVec; ++i) offer2(x[i], u * kVec + i);
+            for (int i = 0; i < kVec; ++i) offer2(x[i], sp.head + (u + q * kRowWG) * kVec + i);
           }
         }
-        if (tid == 0)
-          for (int e = 0; e < n_tail; ++e) offer2(Elem<T>::load1(row + n_units * kVec + e), n_units * kVec + e);
-      } else {
-        for (int64_t u = u0 + tid; u < u1; u += kRowWG) offer2(Elem<T>::load1(row + u), u);
       }
+      for (; u < u1; u += kRowWG) {
+        float x[kVec];
+        Elem<T>::unpack(p[u], x);
+        if (max_of_raw<kVec>(x) >= theta_val) {
+#pragma unroll
+          for (int i = 0; i < kVec; ++i) offer2(x[i], sp.head + u * kVec + i);
+        }
+      }
+      offer2(x_head, tid);
+      offer2(x_tail, tail_e);
       __syncthreads();
       const int offered = sh.cnt;
       if (offered <= kSampCap) {
@@ -686,8 +673,6 @@ hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_
                              int32_t* out_topk_idx, float* out_topk_logit, void* workspace, hipStream_t stream) {
   const int esize = dtype == 0 ? 4 : 2;
   const int vec = 16 / esize;
-  const bool vector_ok = (reinterpret_cast<uintptr_t>(logits) % 16 == 0) && (row_stride % vec == 0);
-  // The workspace is sized for the vector layout; the element-wise instantiation uses the same split count.
   const int splits = sample_splits_for(rows, V, vec);
   char* ws = static_cast<char*>(workspace);
   SampleArgs a{logits, uniforms, row_valid, out_token, out_lp, out_lse, out_argmax, out_topk_idx, out_topk_logit,
@@ -696,15 +681,14 @@ hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_
                V, row_stride, top_k, splits, kLog2e / temperature};
   const dim3 grid((unsigned)(rows * splits)), block(kRowWG);
   const int64_t units_per_split = (V / vec + splits - 1) / splits;
-  const bool cached = vector_ok && V >= vec && units_per_split <= (int64_t)kSampCached * kRowWG;
+  // (two units' worth of elements: every row then holds a whole unit at any phase)
+  const bool cached = V >= 2 * vec && units_per_split <= (int64_t)kSampCached * kRowWG;
   if (dtype == 0) {
-    if (cached) hipLaunchKernelGGL((row_sample_kernel<float, true, true>), grid, block, 0, stream, a);
-    else if (vector_ok) hipLaunchKernelGGL((row_sample_kernel<float, true, false>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((row_sample_kernel<float, false, false>), grid, block, 0, stream, a);
+    if (cached) hipLaunchKernelGGL((row_sample_kernel<float, true>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((row_sample_kernel<float, false>), grid, block, 0, stream, a);
   } else {
-    if (cached) hipLaunchKernelGGL((row_sample_kernel<uint16_t, true, true>), grid, block, 0, stream, a);
-    else if (vector_ok) hipLaunchKernelGGL((row_sample_kernel<uint16_t, true, false>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((row_sample_kernel<uint16_t, false, false>), grid, block, 0, stream, a);
+    if (cached) hipLaunchKernelGGL((row_sample_kernel<uint16_t, true>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((row_sample_kernel<uint16_t, false>), grid, block, 0, stream, a);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || splits == 1) return e;
