@@ -7,9 +7,11 @@
 // workgroups are merged here, by every workgroup of the row for itself (a few partials), which
 // saves the launch of a merge kernel between the two passes.
 //
-// bf16 rows of up to 155648 elements do not need the second read either: a 1024-lane workgroup
+// bf16 rows of 16384 up to 155648 elements do not need the second read either: a 1024-lane workgroup
 // holds such a row in its registers (full_log_softmax_onepass_kernel, below).
 #include "row_common.hpp"
+
+#include <type_traits>
 
 namespace tome {
 
@@ -39,7 +41,16 @@ __device__ __forceinline__ uint32_t sub_pack_bf16(uint32_t u, float inv_temp, fl
   return pack_bf16(__fsub_rn(bf16_lo(z), lse_t), __fsub_rn(bf16_hi(z), lse_t));
 }
 
-template <bool BF16, bool VECTOR, int UNROLL = kFullUnroll>
+// 16-byte units are laid out from the OUTPUT row's first 16-byte boundary: stores are then whole aligned units at any
+// vocabulary size and stride.  Input rows at another phase (a strided view) are read with the same loads at the alignment
+// of their elements.  Against element-wise loads and stores, which every row off a 16-byte boundary took (1024 rows of
+// 128258, both passes): fp32 508 -> 245 us, bf16 (now on the one-pass kernel) 458 -> 107 us.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+__device__ __forceinline__ u32x4 load_unit(const void* row, int64_t byte) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(static_cast<const char*>(row) + byte));
+}
+
+template <bool BF16, int UNROLL = kFullUnroll>
 __global__ __launch_bounds__(kFullWG) void full_log_softmax_kernel(FullArgs a) {
   const int64_t r = blockIdx.x / a.chunks;
   const int chunk = blockIdx.x % a.chunks;
@@ -64,10 +75,11 @@ __global__ __launch_bounds__(kFullWG) void full_log_softmax_kernel(FullArgs a) {
     lse = a.row_lse[r];
   }
   constexpr int kElem = BF16 ? 2 : 4;
-  constexpr int kVec = VECTOR ? 16 / kElem : 1;
-  const char* in_row = static_cast<const char*>(a.in) + r * a.in_stride * kElem;
-  char* out_row = static_cast<char*>(a.out) + r * a.out_stride * kElem;
-  const int64_t n_units = a.V / kVec;
+  typedef typename std::conditional<BF16, uint16_t, float>::type T;
+  const T* in_row = static_cast<const T*>(a.in) + r * a.in_stride;
+  T* out_row = static_cast<T*>(a.out) + r * a.out_stride;
+  const RowSpan<T> sp(out_row, a.V);
+  const int64_t n_units = sp.n_units;
   const int64_t per = (n_units + a.chunks - 1) / a.chunks;
   const int64_t u0 = per * chunk;
   const int64_t u1 = (u0 + per < n_units) ? u0 + per : n_units;
@@ -75,47 +87,42 @@ __global__ __launch_bounds__(kFullWG) void full_log_softmax_kernel(FullArgs a) {
 
   auto scalar_elem = [&](int64_t e) {
     if constexpr (BF16) {
-      const uint16_t b = reinterpret_cast<const uint16_t*>(in_row)[e];
-      reinterpret_cast<uint16_t*>(out_row)[e] =
+      const uint16_t b = in_row[e];
+      out_row[e] =
           f32_to_bf16_bits(__fsub_rn(bf16_rt(__fmul_rn(bf16_bits_to_f32(b), a.inv_temp)), lse_t));
     } else {
-      reinterpret_cast<float*>(out_row)[e] =
-          __fsub_rn(__fmul_rn(reinterpret_cast<const float*>(in_row)[e], a.inv_temp), lse_t);
+      out_row[e] = __fsub_rn(__fmul_rn(in_row[e], a.inv_temp), lse_t);
     }
   };
 
-  if constexpr (VECTOR) {
-    const u32x4* src = reinterpret_cast<const u32x4*>(in_row);
-    u32x4* dst = reinterpret_cast<u32x4*>(out_row);
-    auto convert = [&](const u32x4& v) {
-      u32x4 o;
-      if constexpr (BF16) {
-        o.x = sub_pack_bf16(v.x, a.inv_temp, lse_t);
-        o.y = sub_pack_bf16(v.y, a.inv_temp, lse_t);
-        o.z = sub_pack_bf16(v.z, a.inv_temp, lse_t);
-        o.w = sub_pack_bf16(v.w, a.inv_temp, lse_t);
-      } else {
-        o.x = __float_as_uint(__fsub_rn(__fmul_rn(__uint_as_float(v.x), a.inv_temp), lse_t));
-        o.y = __float_as_uint(__fsub_rn(__fmul_rn(__uint_as_float(v.y), a.inv_temp), lse_t));
-        o.z = __float_as_uint(__fsub_rn(__fmul_rn(__uint_as_float(v.z), a.inv_temp), lse_t));
-        o.w = __float_as_uint(__fsub_rn(__fmul_rn(__uint_as_float(v.w), a.inv_temp), lse_t));
-      }
-      return o;
-    };
-    int64_t u = u0 + threadIdx.x;
-    for (; u + (UNROLL - 1) * kFullWG < u1; u += UNROLL * kFullWG) {  // several 16-byte loads in flight per lane
-      u32x4 v[UNROLL];
-#pragma unroll
-      for (int q = 0; q < UNROLL; ++q) v[q] = __builtin_nontemporal_load(src + u + q * kFullWG);
-#pragma unroll
-      for (int q = 0; q < UNROLL; ++q) __builtin_nontemporal_store(convert(v[q]), dst + u + q * kFullWG);
+  const T* src = in_row + sp.head;
+  u32x4* dst = reinterpret_cast<u32x4*>(out_row + sp.head);
+  auto convert = [&](const u32x4& v) {
+    u32x4 o;
+    if constexpr (BF16) {
+      o.x = sub_pack_bf16(v.x, a.inv_temp, lse_t);
+      o.y = sub_pack_bf16(v.y, a.inv_temp, lse_t);
+      o.z = sub_pack_bf16(v.z, a.inv_temp, lse_t);
+      o.w = sub_pack_bf16(v.w, a.inv_temp, lse_t);
+    } else {
+      o.x = __float_as_uint(__fsub_rn(__fmul_rn(__uint_as_float(v.x), a.inv_temp), lse_t));
+      o.y = __float_as_uint(__fsub_rn(__fmul_rn(__uint_as_float(v.y), a.inv_temp), lse_t));
+      o.z = __float_as_uint(__fsub_rn(__fmul_rn(__uint_as_float(v.z), a.inv_temp), lse_t));
+      o.w = __float_as_uint(__fsub_rn(__fmul_rn(__uint_as_float(v.w), a.inv_temp), lse_t));
     }
-    for (; u < u1; u += kFullWG) __builtin_nontemporal_store(convert(__builtin_nontemporal_load(src + u)), dst + u);
-    if (chunk == a.chunks - 1 && threadIdx.x == 0)
-      for (int64_t e = n_units * kVec; e < a.V; ++e) scalar_elem(e);
-  } else {
-    for (int64_t u = u0 + threadIdx.x; u < u1; u += kFullWG) scalar_elem(u);
+    return o;
+  };
+  int64_t u = u0 + threadIdx.x;
+  for (; u + (UNROLL - 1) * kFullWG < u1; u += UNROLL * kFullWG) {  // several 16-byte loads in flight per lane
+    u32x4 v[UNROLL];
+#pragma unroll
+    for (int q = 0; q < UNROLL; ++q) v[q] = load_unit(src, (u + q * kFullWG) * 16);
+#pragma unroll
+    for (int q = 0; q < UNROLL; ++q) __builtin_nontemporal_store(convert(v[q]), dst + u + q * kFullWG);
   }
+  for (; u < u1; u += kFullWG) __builtin_nontemporal_store(convert(load_unit(src, u * 16)), dst + u);
+  if (chunk == 0 && (int)threadIdx.x < sp.head) scalar_elem(threadIdx.x);
+  if (chunk == a.chunks - 1 && (int)threadIdx.x < sp.tail) scalar_elem(sp.tail_start() + threadIdx.x);
 }
 
 // ---- one pass for bf16 rows that fit a workgroup's registers ----------------------------------------
@@ -132,16 +139,19 @@ __global__ __launch_bounds__(1024) void full_log_softmax_onepass_kernel(FullArgs
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint16_t* in_row = static_cast<const uint16_t*>(a.in) + r * a.in_stride;
   uint16_t* out_row = static_cast<uint16_t*>(a.out) + r * a.out_stride;
-  const u32x4* src = reinterpret_cast<const u32x4*>(in_row);
-  u32x4* dst = reinterpret_cast<u32x4*>(out_row);
-  const int n_units = (int)(a.V / 8);
-  const int n_tail = (int)(a.V - (int64_t)n_units * 8);  // single elements after the last whole unit: lane 0
+  const RowSpan<uint16_t> sp(out_row, a.V);
+  const uint16_t* src = in_row + sp.head;
+  u32x4* dst = reinterpret_cast<u32x4*>(out_row + sp.head);
+  const int n_units = (int)sp.n_units;
+  // single elements in front of the first whole unit and after the last one: one per lane of the first wave
+  const int n_edge = sp.head + sp.tail;
+  const int edge = tid < sp.head ? tid : (int)sp.tail_start() + tid - sp.head;
   const float scale = a.scale;
   u32x4 v[CH];
 #pragma unroll
   for (int q = 0; q < CH; ++q) {  // unconditional (clamped) loads; unit 0 exists (checked on the host)
     const int u = tid + q * 1024;
-    v[q] = __builtin_nontemporal_load(src + (u < n_units ? u : 0));
+    v[q] = load_unit(src, (int64_t)(u < n_units ? u : 0) * 16);
   }
   // the lane's running maximum (floored like every kernel of this path) and sum of 2^((x - maximum) * scale)
   float lm = kMaxFloor, ls = 0.f;
@@ -161,13 +171,11 @@ __global__ __launch_bounds__(1024) void full_log_softmax_onepass_kernel(FullArgs
       ls = s0 + s1;
       lm = nm;
     }
-  if (n_tail != 0 && tid == 0) {  // rare (V not a multiple of 8): fetched here, so that no wait stands in front of the sweep
-    for (int e = 0; e < n_tail; ++e) {
-      const float x = bf16_bits_to_f32(in_row[(int64_t)n_units * 8 + e]);
-      const float nm = fmaxf(lm, x);
-      ls = ls * fast_exp2((lm - nm) * scale) + fast_exp2(fmaf(x, scale, -nm * scale));
-      lm = nm;
-    }
+  if (tid < n_edge) {  // (V not a multiple of 8) fetched here, so that no wait stands in front of the sweep
+    const float x = bf16_bits_to_f32(in_row[edge]);
+    const float nm = fmaxf(lm, x);
+    ls = ls * fast_exp2((lm - nm) * scale) + fast_exp2(fmaf(x, scale, -nm * scale));
+    lm = nm;
   }
   auto merge = [&](float om, float os) {
     const float nm = fmaxf(lm, om);
@@ -221,16 +229,15 @@ __global__ __launch_bounds__(1024) void full_log_softmax_onepass_kernel(FullArgs
       }
     }
   }
-  if (n_tail != 0 && tid == 0)
-    for (int e = 0; e < n_tail; ++e) {
-      const float x = bf16_bits_to_f32(in_row[(int64_t)n_units * 8 + e]);
-      out_row[(int64_t)n_units * 8 + e] = f32_to_bf16_bits(__fsub_rn(bf16_rt(__fmul_rn(x, a.inv_temp)), lse_t));
-    }
+  if (tid < n_edge) {
+    const float x = bf16_bits_to_f32(in_row[edge]);
+    out_row[edge] = f32_to_bf16_bits(__fsub_rn(bf16_rt(__fmul_rn(x, a.inv_temp)), lse_t));
+  }
 }
 
 constexpr int kOnePassUnits = 19;  // 16-byte units per lane: 1024 lanes hold 155648 bf16 elements
 
-// Whether the one-pass kernel takes this call: bf16, 16-byte aligned rows, a row that fits the registers of one
+// Whether the one-pass kernel takes this call: bf16, a row that fits the registers of one
 // workgroup and is long enough to keep most of its 1024 lanes busy.
 // One workgroup per row leaves most of the chip idle on a decode-sized batch, but it is ONE launch where the two-pass form
 // is two: rows of up to 40960 elements always come here (16 rows of 16384 / 32000: 4.3 / 5.4 us against 6.8 / 7.9), longer
@@ -238,11 +245,9 @@ constexpr int kOnePassUnits = 19;  // 16-byte units per lane: 1024 lanes hold 15
 // against 8.0), 131072 ~60 rows (32 rows 12.1 against 8.7, 64 rows 12.4 against 12.8), 151936 ~44 rows (32 / 48 / 64 rows:
 // 13.2 / 13.3 / 13.4 against 11.6 / 14.3 / 16.5); larger batches of 151936: 128 / 512 / 2048 rows 16.9 / 58.4 / 227 against
 // 25.4 / 77.5 / 291.
-bool full_log_softmax_one_pass(const void* in, const void* out, int dtype, int64_t rows, int64_t V, int64_t in_stride, int64_t out_stride) {
-  const bool aligned = reinterpret_cast<uintptr_t>(in) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-                       in_stride % 8 == 0 && out_stride % 8 == 0;
+bool full_log_softmax_one_pass(int dtype, int64_t rows, int64_t V) {
   const bool enough_rows = V <= 40960 || rows * 3000 >= V;
-  return dtype == 1 && aligned && enough_rows && V >= 16384 && V / 8 <= (int64_t)kOnePassUnits * 1024;
+  return dtype == 1 && enough_rows && V >= 16384 && V / 8 <= (int64_t)kOnePassUnits * 1024;
 }
 
 hipError_t full_log_softmax_onepass_launch(const void* in, void* out, int64_t rows, int64_t V, int64_t in_stride,
@@ -271,8 +276,6 @@ hipError_t full_log_softmax_launch(const void* in, void* out, int dtype, int64_t
                                    float* row_lse, const void* partials, int splits, hipStream_t stream) {
   const int esize = dtype == 0 ? 4 : 2;
   const int vec = 16 / esize;
-  const bool vector_ok = reinterpret_cast<uintptr_t>(in) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-                         in_stride % vec == 0 && out_stride % vec == 0;
   FullArgs a;
   a.in = in;
   a.out = out;
@@ -284,7 +287,7 @@ hipError_t full_log_softmax_launch(const void* in, void* out, int dtype, int64_t
   a.in_stride = in_stride;
   a.out_stride = out_stride;
   a.inv_temp = 1.0f / temperature;  // the reference multiplies by 1/temp (model.py:27)
-  const int64_t units = V / (vector_ok ? vec : 1);
+  const int64_t units = V / vec;
   // Many short workgroups stream a read + write mix best, as long as each still issues a few loads per lane.  bf16
   // rows (a batch too small or rows too long for the one-pass kernel): four loads per lane and pass, aiming at 65536
   // workgroups (against 4096: 4096 x 151936 bf16 655 -> 633 us, both passes included).  fp32 rows: workgroups of ONE pass
@@ -295,21 +298,16 @@ hipError_t full_log_softmax_launch(const void* in, void* out, int dtype, int64_t
   int64_t chunks = (65536 + rows - 1) / rows;
   int64_t by_work = units / (kFullUnroll * kFullWG);
   const int f32_unroll = (double)rows * (double)V * 4.0 > 768.0 * 1024 * 1024 ? 1 : 2;
-  if (dtype == 0 && vector_ok) {
+  if (dtype == 0) {
     chunks = by_work = units / (f32_unroll * kFullWG);
   }
   if (chunks > by_work) chunks = by_work;
   if (chunks < 1) chunks = 1;
   a.chunks = (int)chunks;
   const dim3 grid((unsigned)(rows * chunks)), block(kFullWG);
-  if (dtype == 0) {
-    if (!vector_ok) hipLaunchKernelGGL((full_log_softmax_kernel<false, false>), grid, block, 0, stream, a);
-    else if (f32_unroll == 1) hipLaunchKernelGGL((full_log_softmax_kernel<false, true, 1>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((full_log_softmax_kernel<false, true, 2>), grid, block, 0, stream, a);
-  } else {
-    if (vector_ok) hipLaunchKernelGGL((full_log_softmax_kernel<true, true>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((full_log_softmax_kernel<true, false>), grid, block, 0, stream, a);
-  }
+  if (dtype != 0) hipLaunchKernelGGL(full_log_softmax_kernel<true>, grid, block, 0, stream, a);
+  else if (f32_unroll == 1) hipLaunchKernelGGL((full_log_softmax_kernel<false, 1>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((full_log_softmax_kernel<false, 2>), grid, block, 0, stream, a);
   return hipGetLastError();
 }
 
