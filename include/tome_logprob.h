@@ -59,6 +59,24 @@ enum {
   TOME_E_SCRATCH = -8      /* tome_row_logprob_noalloc: the call needs more than the fixed scratch buffer */
 };
 
+/* Which rows of a call count, and the id each is scored against, in the element types their owner keeps
+ * them in (the *_sel entry points; the others take int32 ids and an int32 mask).  Reading them as they are
+ * spares the caller a conversion launch per array.
+ *   targets     ids, int32 or int64 (target_bytes 4 or 8; of an int64 id the low 32 bits count)
+ *   row_valid   nullable mask of 1, 4 or 8 bytes per row (valid_bytes; of 8 the low 4 count), nonzero = valid
+ *   lengths     nullable, instead of row_valid: row r is valid when r % seq_len < lengths[r / seq_len]
+ *               (int32 or int64, length_bytes); the number of rows must be a multiple of seq_len
+ */
+typedef struct TomeRowSel {
+  const void* targets;
+  const void* row_valid;
+  const void* lengths;
+  int64_t seq_len;
+  int32_t target_bytes;
+  int32_t valid_bytes;
+  int32_t length_bytes;
+} TomeRowSel;
+
 int tome_abi_version(void);
 const char* tome_strerror(int code);
 /* hipError_t of the last failing HIP call made by this thread inside the library (0 if none). */
@@ -79,6 +97,12 @@ int tome_row_logprob(const void* logits, int dtype, int64_t rows, int64_t V, int
                      const int32_t* targets, const int32_t* row_valid, float temperature,
                      float* out_lp, float* out_lse, float* out_entropy, int32_t* out_argmax,
                      void* workspace, size_t workspace_bytes, void* stream);
+
+/* tome_row_logprob with the ids and the mask described by `sel`. */
+int tome_row_logprob_sel(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
+                         const TomeRowSel* sel, float temperature, float* out_lp, float* out_lse,
+                         float* out_entropy, int32_t* out_argmax, void* workspace, size_t workspace_bytes,
+                         void* stream);
 
 /* ---- Row kernel over a list of rows -----------------------------------------------
  * The same kernel for the rows a caller names: problem i reads row row_index[i] of `logits`
@@ -208,6 +232,19 @@ int tome_norm_lmhead_logprob(const void* hidden, const void* norm_weight, float 
                              float* out_lse, float* out_entropy, int32_t* out_argmax,
                              void* workspace, size_t workspace_bytes, void* stream);
 
+/* tome_fused_lmhead_logprob (norm_weight == NULL) or tome_norm_lmhead_logprob with the ids and the mask
+ * described by `sel`, optionally over a list of rows: with `hidden_rows` (int32, one entry per token,
+ * no mask then) token p is row hidden_rows[p] of the [n_rows, H] hidden matrix and ids and outputs are
+ * packed in list order - the completion rows of a padded chunk (mlx-impl/node.py:449) without a gather.
+ * An entry outside [0, n_rows) scores NaN (argmax -1).  Workspace: as of the function it stands for.
+ */
+int tome_lmhead_logprob_sel(const void* hidden, const int32_t* hidden_rows, int64_t n_rows,
+                            const void* norm_weight, float norm_eps, const void* weight, int64_t n_tokens,
+                            int64_t H, int64_t V, int64_t hidden_stride, int64_t weight_stride,
+                            const TomeRowSel* sel, float temperature, float* out_lp, float* out_lse,
+                            float* out_entropy, int32_t* out_argmax, void* workspace,
+                            size_t workspace_bytes, void* stream);
+
 /* ---- GRPO policy + reference dual pass --------------------------------------------
  * Two lm_head weight sets over the same hidden states (policy = reference + LoRA merge,
  * mlx-impl/node.py:102-164).  Emits per token
@@ -241,6 +278,13 @@ int tome_grpo_pair(const void* hidden_policy, const void* hidden_ref, const void
                    const int32_t* targets, const int32_t* row_valid, float temperature,
                    float* out_lp, float* out_ref_lp, float* out_k3, float* out_entropy,
                    void* workspace, size_t workspace_bytes, void* stream);
+
+/* tome_grpo_pair with the ids and the mask described by `sel`. */
+int tome_grpo_pair_sel(const void* hidden_policy, const void* hidden_ref, const void* norm_weight,
+                       float norm_eps, const void* w_policy, const void* w_ref, int64_t n_tokens, int64_t H,
+                       int64_t V, int64_t hidden_stride, int64_t weight_stride, const TomeRowSel* sel,
+                       float temperature, float* out_lp, float* out_ref_lp, float* out_k3,
+                       float* out_entropy, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- LoRA merge: the arithmetic of UpdateWeights -----------------------------------
  * Replaces `delta_W = scale * (lora_B @ lora_A)` (mlx-impl/node.py:128) and

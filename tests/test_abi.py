@@ -174,3 +174,31 @@ def test_header_is_plain_c():
     r = subprocess.run(["gcc", "-std=c99", "-Wall", "-Wextra", "-Werror", "-pedantic", "-fsyntax-only", "-x", "c", "-"],
                        input=src, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+def test_row_selection_is_checked_on_the_host():
+    """TomeRowSel: element sizes, mask and lengths together, a row count that is no multiple of the sequence length, and a
+    row list together with a mask are refused before any GPU work."""
+    lib = tome_amd.load_library()
+    P = 0x1000
+
+    def call(sel, rows=6, fn="row", list_=None, n_rows=6):
+        p = None if sel is None else ctypes.addressof(sel)
+        if fn == "row":
+            return lib.tome_row_logprob_sel(P, 1, rows, 64, 64, p, 1.0, P, None, None, None, None, 0, None)
+        if fn == "pair":
+            return lib.tome_grpo_pair_sel(P, P, None, 0.0, P, P, rows, 64, 100, 64, 64, p, 1.0, P, P, P, P, None, 0, None)
+        return lib.tome_lmhead_logprob_sel(P, list_, n_rows, None, 0.0, P, rows, 64, 100, 64, 64, p, 1.0, P, None, None, None, None, 0, None)
+    S = _lib.TomeRowSel
+    for fn in ("row", "pair", "lmhead"):
+        assert call(None, fn=fn) == -1
+        assert call(S(), fn=fn) == -1                                                          # no ids
+        assert call(S(targets=P, target_bytes=2), fn=fn) == -3
+        assert call(S(targets=P, target_bytes=8, row_valid=P, valid_bytes=2), fn=fn) == -3
+        assert call(S(targets=P, target_bytes=8, row_valid=P, valid_bytes=1, lengths=P, length_bytes=8, seq_len=3), fn=fn) == -3
+        for seq, size in ((0, 8), (-1, 8), (4, 8), (1 << 32, 8), (3, 2)):
+            assert call(S(targets=P, target_bytes=8, lengths=P, length_bytes=size, seq_len=seq), fn=fn) == -3
+    assert call(S(targets=P, target_bytes=8, lengths=P, length_bytes=4, seq_len=3), fn="lmhead") == -4   # accepted: workspace missing
+    assert call(S(targets=P, target_bytes=4), fn="lmhead", list_=P, n_rows=0) == -3
+    assert call(S(targets=P, target_bytes=4, row_valid=P, valid_bytes=4), fn="lmhead", list_=P) == -3
+    assert call(S(targets=P, target_bytes=4), fn="lmhead", list_=P) == -4

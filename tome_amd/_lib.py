@@ -20,6 +20,14 @@ SIGNATURES = {
     "tome_row_logprob_workspace": (c_size_t, [c_int64, c_int64]),
     "tome_row_logprob": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_float,
                                  c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
+    "tome_row_logprob_sel": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_float, c_void_p, c_void_p,
+                                     c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
+    "tome_lmhead_logprob_sel": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_float, c_void_p, c_int64, c_int64, c_int64,
+                                        c_int64, c_int64, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_void_p,
+                                        c_void_p, c_size_t, c_void_p]),
+    "tome_grpo_pair_sel": (c_int, [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_int64, c_int64, c_int64,
+                                   c_int64, c_int64, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_void_p,
+                                   c_void_p, c_size_t, c_void_p]),
     "tome_row_logprob_rows": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_float,
                                       c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "tome_row_logprob_noalloc": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_float,
@@ -59,6 +67,12 @@ class TomeLoraJob(ctypes.Structure):
     _fields_ = [("base", c_void_p), ("out", c_void_p), ("lora_a", c_void_p), ("lora_b", c_void_p),
                 ("rows", c_int64), ("cols", c_int64), ("rank", c_int64), ("base_stride", c_int64),
                 ("out_stride", c_int64), ("scale", c_float), ("reserved", ctypes.c_int32)]
+
+
+class TomeRowSel(ctypes.Structure):
+    """``TomeRowSel`` of include/tome_logprob.h."""
+    _fields_ = [("targets", c_void_p), ("row_valid", c_void_p), ("lengths", c_void_p), ("seq_len", c_int64),
+                ("target_bytes", ctypes.c_int32), ("valid_bytes", ctypes.c_int32), ("length_bytes", ctypes.c_int32)]
 
 
 class TomeError(RuntimeError):

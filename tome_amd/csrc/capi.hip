@@ -5,22 +5,20 @@
 #include <stdint.h>
 
 #include "../../include/tome_logprob.h"
+#include "common.hpp"
 
 namespace tome {
 hipError_t row_logprob_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
-                              const int32_t* targets, const int32_t* row_valid, float temperature,
-                              float* out_lp, float* out_lse, float* out_entropy, int32_t* out_argmax,
-                              void* workspace, hipStream_t stream);
+                              const RowSel& sel, float temperature, float* out_lp, float* out_lse, float* out_entropy,
+                              int32_t* out_argmax, void* workspace, hipStream_t stream);
 hipError_t row_logprob_launch_rows(const void* logits, int dtype, int64_t n_rows, const int32_t* row_index, int64_t rows,
-                                   int64_t V, int64_t row_stride, const int32_t* targets, const int32_t* row_valid,
-                                   float temperature, float* out_lp, float* out_lse, float* out_entropy,
-                                   int32_t* out_argmax, void* workspace, hipStream_t stream);
+                                   int64_t V, int64_t row_stride, const RowSel& sel, float temperature, float* out_lp,
+                                   float* out_lse, float* out_entropy, int32_t* out_argmax, void* workspace, hipStream_t stream);
 int row_splits_for(int64_t rows, int64_t V, int vec);
 size_t row_scratch_set_limit(size_t bytes);
 hipError_t row_logprob_noalloc_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
-                                      const int32_t* targets, const int32_t* row_valid, float temperature,
-                                      float* out_lp, float* out_lse, float* out_entropy, int32_t* out_argmax,
-                                      bool* too_big, hipStream_t stream);
+                                      const RowSel& sel, float temperature, float* out_lp, float* out_lse, float* out_entropy,
+                                      int32_t* out_argmax, bool* too_big, hipStream_t stream);
 hipError_t row_lse_partials_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
                                    float temperature, float* out_lse, void* workspace, int* splits, hipStream_t stream);
 hipError_t full_log_softmax_launch(const void* in, void* out, int dtype, int64_t rows, int64_t V,
@@ -30,24 +28,22 @@ bool full_log_softmax_one_pass(int dtype, int64_t rows, int64_t V);
 hipError_t full_log_softmax_onepass_launch(const void* in, void* out, int64_t rows, int64_t V, int64_t in_stride,
                                            int64_t out_stride, float temperature, float* row_lse, hipStream_t stream);
 hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
-                             const float* uniforms, const int32_t* row_valid, float temperature, int top_k,
+                             const float* uniforms, const RowSel& sel, float temperature, int top_k,
                              int32_t* out_token, float* out_lp, float* out_lse, int32_t* out_argmax,
                              int32_t* out_topk_idx, float* out_topk_logit, void* workspace, hipStream_t stream);
 size_t row_sample_workspace_bytes(int64_t rows, int64_t V, int dtype_vec, int top_k);
 size_t fused_workspace_bytes(int64_t n_tokens, int64_t H, int64_t V, int n_weights, bool with_norm);
 bool fused_needs_32bit_extents(int64_t n_tokens, int64_t H, int64_t V);
 void fused_force_kernel(int kind);
-hipError_t fused_lmhead_launch(const void* hidden, const void* norm_weight, float norm_eps, const void* w0,
-                               const void* w1, int64_t n_tokens, int64_t H, int64_t V, int64_t hidden_stride,
-                               int64_t weight_stride, const int32_t* targets,
-                               const int32_t* row_valid, float temperature, float* out_lp, float* out_lse,
+hipError_t fused_lmhead_launch(const void* hidden, const int32_t* hidden_rows, int64_t n_rows, const void* norm_weight, float norm_eps,
+                               const void* w0, const void* w1, int64_t n_tokens, int64_t H, int64_t V, int64_t hidden_stride,
+                               int64_t weight_stride, const RowSel& sel, float temperature, float* out_lp, float* out_lse,
                                float* out_entropy, int32_t* out_argmax, float* out_ref_lp, float* out_k3,
                                void* workspace, hipStream_t stream);
 hipError_t fused_pair_launch(const void* hidden, const void* hidden_ref, const void* norm_weight, float norm_eps,
                              const void* w0, const void* w1, int64_t n_tokens, int64_t H, int64_t V,
-                             int64_t hidden_stride, int64_t weight_stride, const int32_t* targets,
-                             const int32_t* row_valid, float temperature, float* out_lp, float* out_entropy,
-                             float* out_ref_lp, float* out_k3, void* workspace, hipStream_t stream);
+                             int64_t hidden_stride, int64_t weight_stride, const RowSel& sel, float temperature, float* out_lp,
+                             float* out_entropy, float* out_ref_lp, float* out_k3, void* workspace, hipStream_t stream);
 hipError_t mfma_probe_launch(const void* operands, int n_workgroups, int steps, int flags, float* sink, hipStream_t stream);
 struct LoraJobHost;
 hipError_t lora_merge_launch(const LoraJobHost* jobs, int n_jobs, void* workspace, hipStream_t stream);
@@ -75,6 +71,71 @@ bool bad_matrix(int64_t rows, int64_t V, int64_t stride) {
 }
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+tome::RowSel plain_sel(const int32_t* targets, const int32_t* row_valid) {
+  tome::RowSel s;
+  s.targets = targets;
+  s.row_valid = row_valid;
+  return s;
+}
+
+// TomeRowSel of a call over `rows` rows -> what the kernels take.
+int make_sel(const TomeRowSel* in, int64_t rows, tome::RowSel& s) {
+  if (!in) return TOME_E_NULL;
+  if (in->targets && in->target_bytes != 4 && in->target_bytes != 8) return TOME_E_SHAPE;
+  if (in->row_valid && in->valid_bytes != 1 && in->valid_bytes != 4 && in->valid_bytes != 8) return TOME_E_SHAPE;
+  if (in->row_valid && in->lengths) return TOME_E_SHAPE;
+  if (in->lengths) {
+    if (in->length_bytes != 4 && in->length_bytes != 8) return TOME_E_SHAPE;
+    if (in->seq_len <= 0 || in->seq_len > 0x7fffffff || rows > 0x7fffffff || rows % in->seq_len != 0) return TOME_E_SHAPE;
+    s.seq_len = (uint32_t)in->seq_len;
+    s.length_bytes = in->length_bytes;
+  }
+  s.targets = static_cast<const int32_t*>(in->targets);
+  s.row_valid = in->row_valid;
+  s.lengths = in->lengths;
+  if (in->targets) s.target_words = in->target_bytes / 4;
+  if (in->row_valid) s.valid_bytes = in->valid_bytes;
+  return TOME_OK;
+}
+
+// `n_rows`: rows of the hidden matrix (n_tokens unless a row list picks the tokens from more).
+int check_fused(const void* hidden, const void* w, int64_t n_rows, int64_t n_tokens, int64_t H, int64_t V,
+                       int64_t hidden_stride, int64_t weight_stride, const int32_t* targets,
+                float temperature) {
+  if (n_tokens < 0 || H <= 0 || V <= 0 || hidden_stride < H || weight_stride < H) return TOME_E_SHAPE;
+  if (V > (int64_t)0x7fffffff || n_rows > (int64_t)0x7fffffff || n_tokens > (int64_t)0x7fffffff || H > (int64_t)1 << 20) return TOME_E_SHAPE;
+  // Row strides travel as 32-bit byte counts (checked before anything is multiplied by them).
+  if (hidden_stride > (int64_t)0x7fffffff || weight_stride > (int64_t)0x7fffffff) return TOME_E_SHAPE;
+  // The generic kernel (H % 64 != 0) also addresses both matrices with 32-bit byte offsets: each must stay
+  // below 4 GiB there.  The other kernels use 64-bit addresses.
+  if (tome::fused_needs_32bit_extents(n_tokens, H, V) &&
+      (n_rows * hidden_stride * 2 >= ((int64_t)1 << 32) || V * weight_stride * 2 >= ((int64_t)1 << 32)))
+    return TOME_E_SHAPE;
+  if (bad_temperature(temperature)) return TOME_E_TEMPERATURE;
+  if (n_tokens == 0) return TOME_OK;
+  if (!hidden || !w || !targets) return TOME_E_NULL;
+  if (H % 8 != 0 || hidden_stride % 8 != 0 || weight_stride % 8 != 0 ||
+      reinterpret_cast<uintptr_t>(hidden) % 16 != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0)
+    return TOME_E_ALIGN;
+  return TOME_OK;
+}
+
+int row_logprob_checked(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride, const tome::RowSel& sel,
+                        float temperature, float* out_lp, float* out_lse, float* out_entropy, int32_t* out_argmax,
+                        void* workspace, size_t workspace_bytes, void* stream);
+int fused_checked(const void* hidden, const int32_t* hidden_rows, int64_t n_rows, const void* norm_weight, float norm_eps,
+                  const void* weight, int64_t n_tokens, int64_t H, int64_t V, int64_t hidden_stride, int64_t weight_stride,
+                  const tome::RowSel& sel, float temperature, float* out_lp, float* out_lse, float* out_entropy,
+                  int32_t* out_argmax, void* workspace, size_t workspace_bytes, void* stream);
+int pair_checked(const void* hidden_policy, const void* hidden_ref, const void* norm_weight, float norm_eps,
+                 const void* w_policy, const void* w_ref, int64_t n_tokens, int64_t H, int64_t V,
+                 int64_t hidden_stride, int64_t weight_stride, const tome::RowSel& sel, float temperature, float* out_lp,
+                 float* out_ref_lp, float* out_k3, float* out_entropy, void* workspace, size_t workspace_bytes, void* stream);
+int sample_checked(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride, const float* uniforms,
+                   const tome::RowSel& sel, float temperature, int top_k, int32_t* out_token, float* out_lp, float* out_lse,
+                   int32_t* out_argmax, int32_t* out_topk_idx, float* out_topk_logit, void* workspace, size_t workspace_bytes,
+                   void* stream);
 }  // namespace
 
 extern "C" {
@@ -110,19 +171,18 @@ int tome_row_logprob(const void* logits, int dtype, int64_t rows, int64_t V, int
                      const int32_t* targets, const int32_t* row_valid, float temperature, float* out_lp,
                      float* out_lse, float* out_entropy, int32_t* out_argmax, void* workspace,
                      size_t workspace_bytes, void* stream) {
-  if (dtype != TOME_F32 && dtype != TOME_BF16) return TOME_E_DTYPE;
-  if (bad_matrix(rows, V, row_stride)) return TOME_E_SHAPE;
-  if (bad_temperature(temperature)) return TOME_E_TEMPERATURE;
-  if (rows == 0) return TOME_OK;
-  if (!logits) return TOME_E_NULL;
-  if (out_lp && !targets) return TOME_E_NULL;
-  if (!out_lp && !out_lse && !out_entropy && !out_argmax) return TOME_E_NULL;
-  const size_t need = tome_row_logprob_workspace(rows, V);
-  if (need > 0 && (!workspace || workspace_bytes < need)) return TOME_E_WORKSPACE;
-  if (reinterpret_cast<uintptr_t>(logits) % (dtype == TOME_F32 ? 4 : 2) != 0) return TOME_E_ALIGN;
-  return hip_result(tome::row_logprob_launch(logits, dtype, rows, V, row_stride, targets, row_valid, temperature,
-                                             out_lp, out_lse, out_entropy, out_argmax, workspace,
-                                             static_cast<hipStream_t>(stream)));
+  return row_logprob_checked(logits, dtype, rows, V, row_stride, plain_sel(targets, row_valid), temperature, out_lp, out_lse,
+                             out_entropy, out_argmax, workspace, workspace_bytes, stream);
+}
+
+int tome_row_logprob_sel(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride, const TomeRowSel* sel,
+                         float temperature, float* out_lp, float* out_lse, float* out_entropy, int32_t* out_argmax,
+                         void* workspace, size_t workspace_bytes, void* stream) {
+  tome::RowSel s;
+  const int rc = make_sel(sel, rows, s);
+  if (rc != TOME_OK) return rc;
+  return row_logprob_checked(logits, dtype, rows, V, row_stride, s, temperature, out_lp, out_lse, out_entropy, out_argmax,
+                             workspace, workspace_bytes, stream);
 }
 
 int tome_row_logprob_rows(const void* logits, int dtype, int64_t n_rows, int64_t V, int64_t row_stride,
@@ -139,8 +199,8 @@ int tome_row_logprob_rows(const void* logits, int dtype, int64_t n_rows, int64_t
   const size_t need = tome_row_logprob_workspace(n_index, V);
   if (need > 0 && (!workspace || workspace_bytes < need)) return TOME_E_WORKSPACE;
   if (reinterpret_cast<uintptr_t>(logits) % (dtype == TOME_F32 ? 4 : 2) != 0) return TOME_E_ALIGN;
-  return hip_result(tome::row_logprob_launch_rows(logits, dtype, n_rows, row_index, n_index, V, row_stride, targets,
-                                                  nullptr, temperature, out_lp, out_lse, out_entropy, out_argmax,
+  return hip_result(tome::row_logprob_launch_rows(logits, dtype, n_rows, row_index, n_index, V, row_stride,
+                                                  plain_sel(targets, nullptr), temperature, out_lp, out_lse, out_entropy, out_argmax,
                                                   workspace, static_cast<hipStream_t>(stream)));
 }
 
@@ -156,8 +216,8 @@ int tome_row_logprob_noalloc(const void* logits, int dtype, int64_t rows, int64_
   if (!out_lp && !out_lse && !out_entropy && !out_argmax) return TOME_E_NULL;
   if (reinterpret_cast<uintptr_t>(logits) % (dtype == TOME_F32 ? 4 : 2) != 0) return TOME_E_ALIGN;
   bool too_big = false;
-  const hipError_t e = tome::row_logprob_noalloc_launch(logits, dtype, rows, V, row_stride, targets, row_valid,
-                                                        temperature, out_lp, out_lse, out_entropy, out_argmax,
+  const hipError_t e = tome::row_logprob_noalloc_launch(logits, dtype, rows, V, row_stride,
+                                                        plain_sel(targets, row_valid), temperature, out_lp, out_lse, out_entropy, out_argmax,
                                                         &too_big, static_cast<hipStream_t>(stream));
   if (too_big) return TOME_E_SCRATCH;
   return hip_result(e);
@@ -175,17 +235,8 @@ int tome_row_sample(const void* logits, int dtype, int64_t rows, int64_t V, int6
                     int32_t* out_token, float* out_lp, float* out_lse, int32_t* out_argmax,
                     int32_t* out_topk_idx, float* out_topk_logit, void* workspace, size_t workspace_bytes,
                     void* stream) {
-  if (dtype != TOME_F32 && dtype != TOME_BF16) return TOME_E_DTYPE;
-  if (bad_matrix(rows, V, row_stride) || top_k < 1 || top_k > 32) return TOME_E_SHAPE;
-  if (bad_temperature(temperature)) return TOME_E_TEMPERATURE;
-  if (rows == 0) return TOME_OK;
-  if (!logits || !out_token) return TOME_E_NULL;
-  const size_t need = tome_row_sample_workspace(dtype, rows, V, top_k);
-  if (need > 0 && (!workspace || workspace_bytes < need)) return TOME_E_WORKSPACE;
-  if (reinterpret_cast<uintptr_t>(logits) % (dtype == TOME_F32 ? 4 : 2) != 0) return TOME_E_ALIGN;
-  return hip_result(tome::row_sample_launch(logits, dtype, rows, V, row_stride, uniforms, row_valid, temperature,
-                                            top_k, out_token, out_lp, out_lse, out_argmax, out_topk_idx,
-                                            out_topk_logit, workspace, static_cast<hipStream_t>(stream)));
+  return sample_checked(logits, dtype, rows, V, row_stride, uniforms, plain_sel(nullptr, row_valid), temperature, top_k,
+                        out_token, out_lp, out_lse, out_argmax, out_topk_idx, out_topk_logit, workspace, workspace_bytes, stream);
 }
 
 int tome_full_log_softmax(const void* logits, void* out, int dtype, int64_t rows, int64_t V,
@@ -214,26 +265,6 @@ int tome_full_log_softmax(const void* logits, void* out, int dtype, int64_t rows
                                                   row_lse, workspace, splits, s));
 }
 
-static int check_fused(const void* hidden, const void* w, int64_t n_tokens, int64_t H, int64_t V,
-                       int64_t hidden_stride, int64_t weight_stride, const int32_t* targets, float temperature) {
-  if (n_tokens < 0 || H <= 0 || V <= 0 || hidden_stride < H || weight_stride < H) return TOME_E_SHAPE;
-  if (V > (int64_t)0x7fffffff || n_tokens > (int64_t)0x7fffffff || H > (int64_t)1 << 20) return TOME_E_SHAPE;
-  // Row strides travel as 32-bit byte counts (checked before anything is multiplied by them).
-  if (hidden_stride > (int64_t)0x7fffffff || weight_stride > (int64_t)0x7fffffff) return TOME_E_SHAPE;
-  // The generic kernel (H % 64 != 0) also addresses both matrices with 32-bit byte offsets: each must stay
-  // below 4 GiB there.  The other kernels use 64-bit addresses.
-  if (tome::fused_needs_32bit_extents(n_tokens, H, V) &&
-      (n_tokens * hidden_stride * 2 >= ((int64_t)1 << 32) || V * weight_stride * 2 >= ((int64_t)1 << 32)))
-    return TOME_E_SHAPE;
-  if (bad_temperature(temperature)) return TOME_E_TEMPERATURE;
-  if (n_tokens == 0) return TOME_OK;
-  if (!hidden || !w || !targets) return TOME_E_NULL;
-  if (H % 8 != 0 || hidden_stride % 8 != 0 || weight_stride % 8 != 0 ||
-      reinterpret_cast<uintptr_t>(hidden) % 16 != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0)
-    return TOME_E_ALIGN;
-  return TOME_OK;
-}
-
 void tome_select_fused_kernel(int kind) {
   tome::fused_force_kernel(kind == 0 || kind == 1 || (kind >= 3 && kind <= 5) ? kind : -1);
 }
@@ -248,15 +279,22 @@ int tome_fused_lmhead_logprob(const void* hidden, const void* weight, int64_t n_
                               const int32_t* row_valid, float temperature, float* out_lp, float* out_lse,
                               float* out_entropy, int32_t* out_argmax, void* workspace, size_t workspace_bytes,
                               void* stream) {
-  const int rc = check_fused(hidden, weight, n_tokens, H, V, hidden_stride, weight_stride, targets, temperature);
-  if (rc != TOME_OK || n_tokens == 0) return rc;
-  if (!out_lp) return TOME_E_NULL;
-  const size_t need = tome_fused_lmhead_logprob_workspace(n_tokens, H, V);
-  if (!workspace || workspace_bytes < need) return TOME_E_WORKSPACE;
-  return hip_result(tome::fused_lmhead_launch(hidden, nullptr, 0.f, weight, nullptr, n_tokens, H, V, hidden_stride, weight_stride,
-                                              targets, row_valid, temperature, out_lp, out_lse, out_entropy,
-                                              out_argmax, nullptr, nullptr, workspace,
-                                              static_cast<hipStream_t>(stream)));
+  return fused_checked(hidden, nullptr, n_tokens, nullptr, 0.f, weight, n_tokens, H, V, hidden_stride, weight_stride,
+                       plain_sel(targets, row_valid), temperature, out_lp, out_lse, out_entropy, out_argmax, workspace,
+                       workspace_bytes, stream);
+}
+
+int tome_lmhead_logprob_sel(const void* hidden, const int32_t* hidden_rows, int64_t n_rows, const void* norm_weight,
+                            float norm_eps, const void* weight, int64_t n_tokens, int64_t H, int64_t V, int64_t hidden_stride,
+                            int64_t weight_stride, const TomeRowSel* sel, float temperature, float* out_lp, float* out_lse,
+                            float* out_entropy, int32_t* out_argmax, void* workspace, size_t workspace_bytes, void* stream) {
+  tome::RowSel s;
+  const int rc = make_sel(sel, n_tokens, s);
+  if (rc != TOME_OK) return rc;
+  if (hidden_rows && s.masked()) return TOME_E_SHAPE;  // a list names the rows: there is nothing to mask
+  return fused_checked(hidden, hidden_rows, hidden_rows ? n_rows : n_tokens, norm_weight, norm_eps, weight, n_tokens, H, V,
+                       hidden_stride, weight_stride, s, temperature, out_lp, out_lse, out_entropy, out_argmax, workspace,
+                       workspace_bytes, stream);
 }
 
 size_t tome_norm_lmhead_logprob_workspace(int64_t n_tokens, int64_t H, int64_t V) {
@@ -269,17 +307,10 @@ int tome_norm_lmhead_logprob(const void* hidden, const void* norm_weight, float 
                              const int32_t* targets, const int32_t* row_valid, float temperature, float* out_lp,
                              float* out_lse, float* out_entropy, int32_t* out_argmax, void* workspace,
                              size_t workspace_bytes, void* stream) {
-  const int rc = check_fused(hidden, weight, n_tokens, H, V, hidden_stride, weight_stride, targets, temperature);
-  if (rc != TOME_OK || n_tokens == 0) return rc;
-  if (!out_lp || !norm_weight) return TOME_E_NULL;
-  if (reinterpret_cast<uintptr_t>(norm_weight) % 16 != 0) return TOME_E_ALIGN;
-  if (!(norm_eps >= 0.f) || !isfinite(norm_eps)) return TOME_E_SHAPE;
-  const size_t need = tome_norm_lmhead_logprob_workspace(n_tokens, H, V);
-  if (!workspace || workspace_bytes < need) return TOME_E_WORKSPACE;
-  return hip_result(tome::fused_lmhead_launch(hidden, norm_weight, norm_eps, weight, nullptr, n_tokens, H, V,
-                                              hidden_stride, weight_stride, targets, row_valid, temperature, out_lp,
-                                              out_lse, out_entropy, out_argmax, nullptr, nullptr, workspace,
-                                              static_cast<hipStream_t>(stream)));
+  if (n_tokens > 0 && hidden && weight && targets && out_lp && !norm_weight) return TOME_E_NULL;
+  return fused_checked(hidden, nullptr, n_tokens, norm_weight, norm_eps, weight, n_tokens, H, V, hidden_stride, weight_stride,
+                       plain_sel(targets, row_valid), temperature, out_lp, out_lse, out_entropy, out_argmax, workspace,
+                       workspace_bytes, stream);
 }
 
 size_t tome_grpo_dual_workspace(int64_t n_tokens, int64_t H, int64_t V) {
@@ -291,14 +322,14 @@ int tome_grpo_dual(const void* hidden, const void* w_policy, const void* w_ref, 
                    int64_t V, int64_t hidden_stride, int64_t weight_stride, const int32_t* targets,
                    const int32_t* row_valid, float temperature, float* out_lp, float* out_ref_lp, float* out_k3,
                    float* out_entropy, void* workspace, size_t workspace_bytes, void* stream) {
-  const int rc = check_fused(hidden, w_policy, n_tokens, H, V, hidden_stride, weight_stride, targets, temperature);
+  const int rc = check_fused(hidden, w_policy, n_tokens, n_tokens, H, V, hidden_stride, weight_stride, targets, temperature);
   if (rc != TOME_OK || n_tokens == 0) return rc;
   if (!w_ref || !out_lp || !out_ref_lp) return TOME_E_NULL;
   if (reinterpret_cast<uintptr_t>(w_ref) % 16 != 0) return TOME_E_ALIGN;
   const size_t need = tome_grpo_dual_workspace(n_tokens, H, V);
   if (!workspace || workspace_bytes < need) return TOME_E_WORKSPACE;
-  return hip_result(tome::fused_lmhead_launch(hidden, nullptr, 0.f, w_policy, w_ref, n_tokens, H, V, hidden_stride, weight_stride,
-                                              targets, row_valid, temperature, out_lp, nullptr, out_entropy,
+  return hip_result(tome::fused_lmhead_launch(hidden, nullptr, n_tokens, nullptr, 0.f, w_policy, w_ref, n_tokens, H, V,
+                                              hidden_stride, weight_stride, plain_sel(targets, row_valid), temperature, out_lp, nullptr, out_entropy,
                                               nullptr, out_ref_lp, out_k3, workspace,
                                               static_cast<hipStream_t>(stream)));
 }
@@ -315,19 +346,21 @@ int tome_grpo_pair(const void* hidden_policy, const void* hidden_ref, const void
                    int64_t hidden_stride, int64_t weight_stride, const int32_t* targets, const int32_t* row_valid,
                    float temperature, float* out_lp, float* out_ref_lp, float* out_k3, float* out_entropy,
                    void* workspace, size_t workspace_bytes, void* stream) {
-  const int rc = check_fused(hidden_policy, w_policy, n_tokens, H, V, hidden_stride, weight_stride, targets, temperature);
-  if (rc != TOME_OK || n_tokens == 0) return rc;
-  if (!hidden_ref || !w_ref || !out_lp || !out_ref_lp) return TOME_E_NULL;
-  if (reinterpret_cast<uintptr_t>(w_ref) % 16 != 0 || reinterpret_cast<uintptr_t>(hidden_ref) % 16 != 0 ||
-      reinterpret_cast<uintptr_t>(norm_weight) % 16 != 0)
-    return TOME_E_ALIGN;
-  if (norm_weight && (!(norm_eps >= 0.f) || !isfinite(norm_eps))) return TOME_E_SHAPE;
-  const size_t need = tome_grpo_pair_workspace(n_tokens, H, V, norm_weight != nullptr);
-  if (!workspace || workspace_bytes < need) return TOME_E_WORKSPACE;
-  return hip_result(tome::fused_pair_launch(hidden_policy, hidden_ref, norm_weight, norm_eps, w_policy, w_ref, n_tokens,
-                                            H, V, hidden_stride, weight_stride, targets, row_valid, temperature,
-                                            out_lp, out_entropy, out_ref_lp, out_k3, workspace,
-                                            static_cast<hipStream_t>(stream)));
+  return pair_checked(hidden_policy, hidden_ref, norm_weight, norm_eps, w_policy, w_ref, n_tokens, H, V, hidden_stride,
+                      weight_stride, plain_sel(targets, row_valid), temperature, out_lp, out_ref_lp, out_k3, out_entropy,
+                      workspace, workspace_bytes, stream);
+}
+
+int tome_grpo_pair_sel(const void* hidden_policy, const void* hidden_ref, const void* norm_weight, float norm_eps,
+                       const void* w_policy, const void* w_ref, int64_t n_tokens, int64_t H, int64_t V,
+                       int64_t hidden_stride, int64_t weight_stride, const TomeRowSel* sel, float temperature, float* out_lp,
+                       float* out_ref_lp, float* out_k3, float* out_entropy, void* workspace, size_t workspace_bytes,
+                       void* stream) {
+  tome::RowSel s;
+  const int rc = make_sel(sel, n_tokens, s);
+  if (rc != TOME_OK) return rc;
+  return pair_checked(hidden_policy, hidden_ref, norm_weight, norm_eps, w_policy, w_ref, n_tokens, H, V, hidden_stride,
+                      weight_stride, s, temperature, out_lp, out_ref_lp, out_k3, out_entropy, workspace, workspace_bytes, stream);
 }
 
 int tome_probe_mfma_ceiling(const void* operands, size_t operand_bytes, int n_workgroups, int steps, int flags,
@@ -381,3 +414,77 @@ int tome_lora_merge(const TomeLoraJob* jobs, int64_t n_jobs, void* workspace, si
 }
 
 }  // extern "C"
+
+namespace {
+int row_logprob_checked(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride, const tome::RowSel& sel,
+                        float temperature, float* out_lp, float* out_lse, float* out_entropy, int32_t* out_argmax,
+                        void* workspace, size_t workspace_bytes, void* stream) {
+  if (dtype != TOME_F32 && dtype != TOME_BF16) return TOME_E_DTYPE;
+  if (bad_matrix(rows, V, row_stride)) return TOME_E_SHAPE;
+  if (bad_temperature(temperature)) return TOME_E_TEMPERATURE;
+  if (rows == 0) return TOME_OK;
+  if (!logits) return TOME_E_NULL;
+  if (out_lp && !sel.targets) return TOME_E_NULL;
+  if (!out_lp && !out_lse && !out_entropy && !out_argmax) return TOME_E_NULL;
+  const size_t need = tome_row_logprob_workspace(rows, V);
+  if (need > 0 && (!workspace || workspace_bytes < need)) return TOME_E_WORKSPACE;
+  if (reinterpret_cast<uintptr_t>(logits) % (dtype == TOME_F32 ? 4 : 2) != 0) return TOME_E_ALIGN;
+  return hip_result(tome::row_logprob_launch(logits, dtype, rows, V, row_stride, sel, temperature,
+                                             out_lp, out_lse, out_entropy, out_argmax, workspace,
+                                             static_cast<hipStream_t>(stream)));
+}
+
+int sample_checked(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride, const float* uniforms,
+                   const tome::RowSel& sel, float temperature, int top_k, int32_t* out_token, float* out_lp, float* out_lse,
+                   int32_t* out_argmax, int32_t* out_topk_idx, float* out_topk_logit, void* workspace, size_t workspace_bytes,
+                   void* stream) {
+  if (dtype != TOME_F32 && dtype != TOME_BF16) return TOME_E_DTYPE;
+  if (bad_matrix(rows, V, row_stride) || top_k < 1 || top_k > 32) return TOME_E_SHAPE;
+  if (bad_temperature(temperature)) return TOME_E_TEMPERATURE;
+  if (rows == 0) return TOME_OK;
+  if (!logits || !out_token) return TOME_E_NULL;
+  const size_t need = tome_row_sample_workspace(dtype, rows, V, top_k);
+  if (need > 0 && (!workspace || workspace_bytes < need)) return TOME_E_WORKSPACE;
+  if (reinterpret_cast<uintptr_t>(logits) % (dtype == TOME_F32 ? 4 : 2) != 0) return TOME_E_ALIGN;
+  return hip_result(tome::row_sample_launch(logits, dtype, rows, V, row_stride, uniforms, sel, temperature,
+                                            top_k, out_token, out_lp, out_lse, out_argmax, out_topk_idx,
+                                            out_topk_logit, workspace, static_cast<hipStream_t>(stream)));
+}
+
+int fused_checked(const void* hidden, const int32_t* hidden_rows, int64_t n_rows, const void* norm_weight, float norm_eps,
+                  const void* weight, int64_t n_tokens, int64_t H, int64_t V, int64_t hidden_stride, int64_t weight_stride,
+                  const tome::RowSel& sel, float temperature, float* out_lp, float* out_lse, float* out_entropy,
+                  int32_t* out_argmax, void* workspace, size_t workspace_bytes, void* stream) {
+  if (n_rows <= 0 && n_tokens > 0) return TOME_E_SHAPE;
+  const int rc = check_fused(hidden, weight, n_rows > n_tokens ? n_rows : n_tokens, n_tokens, H, V, hidden_stride,
+                             weight_stride, sel.targets, temperature);
+  if (rc != TOME_OK || n_tokens == 0) return rc;
+  if (!out_lp) return TOME_E_NULL;
+  if (reinterpret_cast<uintptr_t>(norm_weight) % 16 != 0) return TOME_E_ALIGN;
+  if (norm_weight && (!(norm_eps >= 0.f) || !isfinite(norm_eps))) return TOME_E_SHAPE;
+  const size_t need = align256(tome::fused_workspace_bytes(n_tokens, H, V, 1, norm_weight != nullptr));
+  if (!workspace || workspace_bytes < need) return TOME_E_WORKSPACE;
+  return hip_result(tome::fused_lmhead_launch(hidden, hidden_rows, n_rows, norm_weight, norm_eps, weight, nullptr, n_tokens, H, V,
+                                              hidden_stride, weight_stride, sel, temperature, out_lp, out_lse, out_entropy,
+                                              out_argmax, nullptr, nullptr, workspace, static_cast<hipStream_t>(stream)));
+}
+
+int pair_checked(const void* hidden_policy, const void* hidden_ref, const void* norm_weight, float norm_eps,
+                 const void* w_policy, const void* w_ref, int64_t n_tokens, int64_t H, int64_t V,
+                 int64_t hidden_stride, int64_t weight_stride, const tome::RowSel& sel, float temperature, float* out_lp,
+                 float* out_ref_lp, float* out_k3, float* out_entropy, void* workspace, size_t workspace_bytes, void* stream) {
+  const int rc = check_fused(hidden_policy, w_policy, n_tokens, n_tokens, H, V, hidden_stride, weight_stride, sel.targets, temperature);
+  if (rc != TOME_OK || n_tokens == 0) return rc;
+  if (!hidden_ref || !w_ref || !out_lp || !out_ref_lp) return TOME_E_NULL;
+  if (reinterpret_cast<uintptr_t>(w_ref) % 16 != 0 || reinterpret_cast<uintptr_t>(hidden_ref) % 16 != 0 ||
+      reinterpret_cast<uintptr_t>(norm_weight) % 16 != 0)
+    return TOME_E_ALIGN;
+  if (norm_weight && (!(norm_eps >= 0.f) || !isfinite(norm_eps))) return TOME_E_SHAPE;
+  const size_t need = tome_grpo_pair_workspace(n_tokens, H, V, norm_weight != nullptr);
+  if (!workspace || workspace_bytes < need) return TOME_E_WORKSPACE;
+  return hip_result(tome::fused_pair_launch(hidden_policy, hidden_ref, norm_weight, norm_eps, w_policy, w_ref, n_tokens,
+                                            H, V, hidden_stride, weight_stride, sel, temperature,
+                                            out_lp, out_entropy, out_ref_lp, out_k3, workspace,
+                                            static_cast<hipStream_t>(stream)));
+}
+}  // namespace

@@ -70,6 +70,36 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_hw{lo, hi}, bf16x2_hw));
 }
 
+// ---- which rows count, and the id each is scored against -------------------------------------
+// Ids, masks and per-sequence lengths are read in the element types their owners keep them in (torch's int64 ids and bool
+// masks among them): converting them first is a launch of its own per array, 2-5 us each on the stream in front of
+// kernels of 5-100 us.
+struct RowSel {
+  const int32_t* targets = nullptr;   // 32-bit words; `target_words` of them per id (2: int64, the low word counts)
+  const void* row_valid = nullptr;    // nullable; `valid_bytes` 1, 4 or 8 (8: the low word counts) per row, nonzero = valid
+  const void* lengths = nullptr;      // nullable; row r is valid when r % seq_len < lengths[r / seq_len]
+  int target_words = 1;
+  int valid_bytes = 4;
+  int length_bytes = 4;               // 4 or 8
+  uint32_t seq_len = 1;
+
+  __host__ __device__ bool masked() const { return row_valid != nullptr || lengths != nullptr; }
+  __device__ __forceinline__ int32_t target(int64_t r) const { return targets[r * target_words]; }
+  __device__ __forceinline__ bool mask_value(int64_t r) const {
+    if (valid_bytes == 1) return static_cast<const uint8_t*>(row_valid)[r] != 0;
+    return static_cast<const int32_t*>(row_valid)[r * (valid_bytes / 4)] != 0;
+  }
+  __device__ __forceinline__ bool inside_length(uint32_t r) const {
+    const uint32_t b = r / seq_len;
+    const int64_t len = length_bytes == 8 ? static_cast<const int64_t*>(lengths)[b] : static_cast<const int32_t*>(lengths)[b];
+    return (int64_t)(r - b * seq_len) < len;
+  }
+  __device__ __forceinline__ bool valid(int64_t r) const {
+    if (row_valid) return mask_value(r);
+    return !lengths || inside_length((uint32_t)r);
+  }
+};
+
 // ---- wave64 lane exchange --------------------------------------------------------------
 // Steps inside a 16-lane row use DPP (no LDS traffic); the two steps that cross rows go
 // through the LDS crossbar (ds_bpermute via __shfl_xor).  After steps 0..3 every lane of a

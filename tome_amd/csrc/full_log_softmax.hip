@@ -74,7 +74,6 @@ __global__ __launch_bounds__(kFullWG) void full_log_softmax_kernel(FullArgs a) {
   } else {
     lse = a.row_lse[r];
   }
-  constexpr int kElem = BF16 ? 2 : 4;
   typedef typename std::conditional<BF16, uint16_t, float>::type T;
   const T* in_row = static_cast<const T*>(a.in) + r * a.in_stride;
   T* out_row = static_cast<T*>(a.out) + r * a.out_stride;

@@ -152,9 +152,10 @@ __device__ __forceinline__ bool fused_locate(const FusedSchedule& s, int bid, in
 struct FusedArgs {
   const char* hidden;
   const char* weight;
-  const int32_t* targets;
+  RowSel sel;                // its targets (the mask went into row_index)
   const int32_t* row_index;  // compacted valid rows (position -> row of targets / outputs), or nullptr = identity
-  const int32_t* hidden_index;  // position -> row of `hidden`: row_index, or nullptr when hidden is already compact
+  const int32_t* hidden_index;  // position -> row of `hidden`: row_index, the caller's row list, or nullptr when hidden is already compact
+  int n_rows;                   // rows of `hidden`; an entry of a caller's list outside them reads a row inside (and scores NaN)
   const int32_t* n_valid;    // device scalar, or nullptr = n_tokens
   const FusedSchedule* sched_dev;  // written by compact_rows_kernel next to n_valid, or nullptr = `sched`
   FusedPartial* partials;
@@ -313,7 +314,7 @@ __global__ __launch_bounds__(kFusedWG, 2) void fused_lmhead_kernel(FusedArgs a) 
   for (int j = 0; j < kBLoads; ++j) {
     int p = t0 + ld_row + 32 * j;
     p = p < n_valid ? p : n_valid - 1;
-    const int tok = a.hidden_index ? a.hidden_index[p] : p;
+    const int tok = a.hidden_index ? min(max(a.hidden_index[p], 0), a.n_rows - 1) : p;
     boff[j] = (uint32_t)tok * a.hidden_stride_b + ld_c * 16;
   }
   uint32_t aoff[kALoads];
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(kFusedWG, 2) void fused_lmhead_kernel(FusedArgs a) 
     tx[bt] = -INFINITY;
     int p = t0 + wave_t * kWaveT + bt * 32 + l32;
     int t = -1;
-    if (p < n_valid) t = a.targets[a.row_index ? a.row_index[p] : p];
+    if (p < n_valid) t = a.sel.target(a.row_index ? a.row_index[p] : p);
     tgt[bt] = (t >= 0 && t < a.V) ? t : -1;
   }
 
@@ -722,7 +723,7 @@ __global__ __launch_bounds__(k2WG) void fused_lmhead_dma_kernel(FusedArgs a) {
   for (int j = 0; j < kBLoads; ++j) {
     int p = t0 + (j * 8 + wave) * 8 + dr;
     p = p < n_valid ? p : n_valid - 1;
-    const int tok = a.hidden_index ? a.hidden_index[p] : p;
+    const int tok = a.hidden_index ? min(max(a.hidden_index[p], 0), a.n_rows - 1) : p;
     pb[j] = a.hidden + (int64_t)tok * a.hidden_stride_b + dc * 16;
   }
 
@@ -736,7 +737,7 @@ __global__ __launch_bounds__(k2WG) void fused_lmhead_dma_kernel(FusedArgs a) {
     tx[bt] = -INFINITY;
     const int p = t0 + wave_t * kWaveTok + bt * 16 + l16;
     int t = -1;
-    if (p < n_valid) t = a.targets[a.row_index ? a.row_index[p] : p];
+    if (p < n_valid) t = a.sel.target(a.row_index ? a.row_index[p] : p);
     tgt[bt] = (t >= 0 && t < a.V) ? t : -1;
   }
 
@@ -986,7 +987,7 @@ __global__ __launch_bounds__(512) void fused_lmhead_small_kernel(FusedArgs a) {
   for (int j = 0; j < NBT; ++j) {
     int p = j * 16 + l16;
     p = p < n_valid ? p : n_valid - 1;
-    const int tok = a.hidden_index ? a.hidden_index[p] : p;
+    const int tok = a.hidden_index ? min(max(a.hidden_index[p], 0), a.n_rows - 1) : p;
     const char* hp = a.hidden + (int64_t)tok * a.hidden_stride_b + kb0;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) fb[ks][j] = *reinterpret_cast<const bf16x8*>(hp + ks * 64);
@@ -998,7 +999,7 @@ __global__ __launch_bounds__(512) void fused_lmhead_small_kernel(FusedArgs a) {
   if (wave < NBT) {
     const int p = wave * 16 + l16;
     int t = -1;
-    if (p < n_valid) t = a.targets[a.row_index ? a.row_index[p] : p];
+    if (p < n_valid) t = a.sel.target(a.row_index ? a.row_index[p] : p);
     tgt[0] = (t >= 0 && t < a.V) ? t : -1;
   }
 
@@ -1081,10 +1082,10 @@ __global__ __launch_bounds__(512) void fused_lmhead_small_kernel(FusedArgs a) {
 }
 
 // ---- compaction of valid rows ----------------------------------------------------------------
-// One workgroup: row_index[0 .. n_valid) = ascending indices of rows with row_valid != 0.
+// One workgroup: row_index[0 .. n_valid) = ascending indices of the valid rows.
 // Outputs of masked rows are zeroed here.
 struct CompactArgs {
-  const int32_t* row_valid;
+  RowSel sel;
   int32_t* row_index;
   int32_t* n_valid;
   float* out0;
@@ -1119,11 +1120,17 @@ __global__ __launch_bounds__(1024) void compact_rows_kernel(CompactArgs a) {
   for (int64_t b0 = 0; b0 < a.n; b0 += batch_rows) {
     const int64_t first = b0 + (int64_t)wave * wave_rows;
     int v[kChunks];
+    // unconditional (clamped) loads: all of them in flight together
+    auto load_mask = [&](auto&& value) {
 #pragma unroll
-    for (int c = 0; c < kChunks; ++c) {  // unconditional (clamped) loads: all of them in flight together
-      const int64_t r = first + c * 64 + lane;
-      v[c] = a.row_valid[r < a.n ? r : a.n - 1];
-    }
+      for (int c = 0; c < kChunks; ++c) {
+        const int64_t r = first + c * 64 + lane;
+        v[c] = value(r < a.n ? r : a.n - 1);
+      }
+    };
+    if (!a.sel.row_valid) load_mask([&](int64_t r) { return a.sel.inside_length((uint32_t)r) ? 1 : 0; });
+    else if (a.sel.valid_bytes == 1) load_mask([&](int64_t r) { return (int)static_cast<const uint8_t*>(a.sel.row_valid)[r]; });
+    else load_mask([&](int64_t r) { return static_cast<const int32_t*>(a.sel.row_valid)[r * (a.sel.valid_bytes / 4)]; });
 #pragma unroll
     for (int c = 0; c < kChunks; ++c) v[c] = (c < n_chunks && first + c * 64 + lane < a.n) ? v[c] : 0;
     int cnt = 0;
@@ -1169,10 +1176,10 @@ struct NormArgs {
   const char* x;             // bf16 [n, H]
   const uint16_t* w;         // bf16 [H]
   char* y;                   // bf16 [n_valid, H], dense
-  const int32_t* row_index;  // or nullptr = identity
+  const int32_t* row_index;  // or nullptr = identity; entries outside [0, n_rows) read a row inside
   const int32_t* n_valid;    // or nullptr = n
   uint32_t x_stride_b;
-  int n, H;
+  int n, n_rows, H;
   float eps;
 };
 
@@ -1181,7 +1188,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(NormArgs a) {
   const int p = blockIdx.x * 4 + (threadIdx.x >> 6);  // one wave per row
   const int n_valid = a.n_valid ? *a.n_valid : a.n;
   if (p >= n_valid) return;
-  const int row = a.row_index ? a.row_index[p] : p;
+  const int row = a.row_index ? min(max(a.row_index[p], 0), a.n_rows - 1) : p;
   const u32x4* x = reinterpret_cast<const u32x4*>(a.x + (int64_t)row * a.x_stride_b);
   const u32x4* w = reinterpret_cast<const u32x4*>(a.w);
   u32x4* y = reinterpret_cast<u32x4*>(a.y + (int64_t)p * a.H * 2);
@@ -1226,6 +1233,8 @@ struct CombineArgs {
   float* out_ref_lp;
   float* out_k3;
   int32_t* out_argmax;
+  const int32_t* hidden_rows;  // the caller's row list, or nullptr: an entry outside [0, n_rows) scores NaN (argmax -1)
+  int n_rows;
   int n_tokens;
   const FusedSchedule* sched_dev;  // as in FusedArgs
   FusedSchedule sched;
@@ -1287,6 +1296,13 @@ __global__ __launch_bounds__(256) void fused_combine_kernel(CombineArgs a) {
     ref_lp = txr == -INFINITY ? __builtin_nanf("") : (fmaf(txr, a.scale, -mr) - fast_log2(sr.s)) * kLn2;
   }
   if (lane != 0) return;
+  if (a.hidden_rows && (uint32_t)a.hidden_rows[p] >= (uint32_t)a.n_rows) {  // (never with a second weight set)
+    if (a.out_argmax) a.out_argmax[tok] = -1;
+    if (a.out_lp) a.out_lp[tok] = __builtin_nanf("");
+    if (a.out_lse) a.out_lse[tok] = __builtin_nanf("");
+    if (a.out_entropy) a.out_entropy[tok] = __builtin_nanf("");
+    return;
+  }
   // The sweep kernels name the element themselves: bi is the vocab row of the first maximum among the fp32
   // logits they accumulated (0 when nothing above the floor was seen, as a first-maximum scan would say).
   if (a.out_argmax) a.out_argmax[tok] = st.bi == 0x7fffffff ? 0 : st.bi;
@@ -1561,10 +1577,11 @@ static int launch_main(const FusedArgs& a, const FusedPlan& plan, bool want_argm
 
 // One sweep per (hidden, weight) pair: the policy pair always, and a reference pair when a second weight
 // set (`w1`) or a second hidden-state matrix (`hidden_ref`) is given; either may repeat the policy's.
-static hipError_t fused_launch_impl(const void* hidden, const void* hidden_ref, const void* norm_weight,
+// `hidden_rows` (nullable): token p is row hidden_rows[p] of a hidden matrix of `n_rows` rows, ids and outputs packed.
+static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_rows, int64_t n_rows, const void* hidden_ref, const void* norm_weight,
                                     float norm_eps, const void* w0, const void* w1, int64_t n_tokens, int64_t H,
-                                    int64_t V, int64_t hidden_stride, int64_t weight_stride, const int32_t* targets,
-                                    const int32_t* row_valid, float temperature, float* out_lp, float* out_lse,
+                                    int64_t V, int64_t hidden_stride, int64_t weight_stride, const RowSel& sel,
+                                    float temperature, float* out_lp, float* out_lse,
                                     float* out_entropy, int32_t* out_argmax, float* out_ref_lp, float* out_k3,
                                     void* workspace, hipStream_t stream) {
   const bool second = w1 != nullptr || hidden_ref != nullptr;
@@ -1574,10 +1591,10 @@ static hipError_t fused_launch_impl(const void* hidden, const void* hidden_ref, 
   const FusedPlan plan = fused_plan(n_tokens, H, V);
   int32_t* n_valid = nullptr;
   int32_t* row_index = nullptr;
-  if (row_valid) {
+  if (sel.masked()) {
     n_valid = reinterpret_cast<int32_t*>(ws);
     row_index = reinterpret_cast<int32_t*>(ws + off_index());
-    CompactArgs c{row_valid, row_index, n_valid, out_lp, out_lse, out_entropy, out_ref_lp, out_k3, out_argmax,
+    CompactArgs c{sel, row_index, n_valid, out_lp, out_lse, out_entropy, out_ref_lp, out_k3, out_argmax,
                   (int)n_tokens, plan.bt, plan.slots, plan.n_vunits, plan.upt};
     hipLaunchKernelGGL(compact_rows_kernel, dim3(1), dim3(1024), 0, stream, c);
     hipError_t e = hipGetLastError();
@@ -1585,18 +1602,19 @@ static hipError_t fused_launch_impl(const void* hidden, const void* hidden_ref, 
   }
   FusedArgs a;
   a.hidden = static_cast<const char*>(hidden);
-  a.targets = targets;
+  a.sel = sel;
   a.row_index = row_index;
-  a.hidden_index = row_index;
+  a.hidden_index = hidden_rows ? hidden_rows : row_index;
+  a.n_rows = (int)n_rows;
   a.n_valid = n_valid;
   a.hidden_stride_b = (uint32_t)(hidden_stride * 2);
   a.weight_stride_b = (uint32_t)(weight_stride * 2);
-  a.hidden_bytes = (uint32_t)(((n_tokens - 1) * hidden_stride + H) * 2);  // read by the generic kernel only (< 4 GiB there)
+  a.hidden_bytes = (uint32_t)(((n_rows - 1) * hidden_stride + H) * 2);  // read by the generic kernel only (< 4 GiB there)
   const char* second_hidden = static_cast<const char*>(hidden_ref);
   if (norm_weight) {  // normalise the valid rows into a dense buffer and multiply that
     char* normed = ws + off_partials(n_tokens) + (second ? 2 : 1) * partial_bytes(n_tokens, H, V);
-    NormArgs na{a.hidden, static_cast<const uint16_t*>(norm_weight), normed, row_index, n_valid,
-                a.hidden_stride_b, (int)n_tokens, (int)H, norm_eps};
+    NormArgs na{a.hidden, static_cast<const uint16_t*>(norm_weight), normed, a.hidden_index, n_valid,
+                a.hidden_stride_b, (int)n_tokens, (int)n_rows, (int)H, norm_eps};
     hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((unsigned)((n_tokens + 3) / 4)), dim3(256), 0, stream, na);
     if (hidden_ref != hidden) {
       na.x = static_cast<const char*>(hidden_ref);
@@ -1618,7 +1636,7 @@ static hipError_t fused_launch_impl(const void* hidden, const void* hidden_ref, 
   a.unit32 = plan.unit32;
   a.slots = plan.slots;
   // Workspace header: [0] n_valid, [16..32) the schedule derived from it on the device.
-  a.sched_dev = row_valid ? reinterpret_cast<const FusedSchedule*>(n_valid + 4) : nullptr;
+  a.sched_dev = sel.masked() ? reinterpret_cast<const FusedSchedule*>(n_valid + 4) : nullptr;
   a.sched = fused_schedule((int)n_tokens, plan.bt, plan.slots, plan.n_vunits, plan.upt);
   a.scale = kLog2e / temperature;
   FusedPartial* p0 = reinterpret_cast<FusedPartial*>(ws + off_partials(n_tokens));
@@ -1654,6 +1672,8 @@ static hipError_t fused_launch_impl(const void* hidden, const void* hidden_ref, 
   c.out_ref_lp = out_ref_lp;
   c.out_k3 = out_k3;
   c.out_argmax = out_argmax;
+  c.hidden_rows = hidden_rows;
+  c.n_rows = (int)n_rows;
   c.n_tokens = (int)n_tokens;
   c.sched_dev = a.sched_dev;
   c.sched = a.sched;
@@ -1662,24 +1682,22 @@ static hipError_t fused_launch_impl(const void* hidden, const void* hidden_ref, 
   return hipGetLastError();
 }
 
-hipError_t fused_lmhead_launch(const void* hidden, const void* norm_weight, float norm_eps, const void* w0,
+hipError_t fused_lmhead_launch(const void* hidden, const int32_t* hidden_rows, int64_t n_rows, const void* norm_weight, float norm_eps, const void* w0,
                                const void* w1, int64_t n_tokens, int64_t H, int64_t V, int64_t hidden_stride,
-                               int64_t weight_stride, const int32_t* targets,
-                               const int32_t* row_valid, float temperature, float* out_lp, float* out_lse,
+                               int64_t weight_stride, const RowSel& sel, float temperature, float* out_lp, float* out_lse,
                                float* out_entropy, int32_t* out_argmax, float* out_ref_lp, float* out_k3,
                                void* workspace, hipStream_t stream) {
-  return fused_launch_impl(hidden, nullptr, norm_weight, norm_eps, w0, w1, n_tokens, H, V, hidden_stride, weight_stride,
-                           targets, row_valid, temperature, out_lp, out_lse, out_entropy, out_argmax, out_ref_lp, out_k3,
+  return fused_launch_impl(hidden, hidden_rows, n_rows, nullptr, norm_weight, norm_eps, w0, w1, n_tokens, H, V, hidden_stride, weight_stride,
+                           sel, temperature, out_lp, out_lse, out_entropy, out_argmax, out_ref_lp, out_k3,
                            workspace, stream);
 }
 
 hipError_t fused_pair_launch(const void* hidden, const void* hidden_ref, const void* norm_weight, float norm_eps,
                              const void* w0, const void* w1, int64_t n_tokens, int64_t H, int64_t V,
-                             int64_t hidden_stride, int64_t weight_stride, const int32_t* targets,
-                             const int32_t* row_valid, float temperature, float* out_lp, float* out_entropy,
+                             int64_t hidden_stride, int64_t weight_stride, const RowSel& sel, float temperature, float* out_lp, float* out_entropy,
                              float* out_ref_lp, float* out_k3, void* workspace, hipStream_t stream) {
-  return fused_launch_impl(hidden, hidden_ref, norm_weight, norm_eps, w0, w1, n_tokens, H, V, hidden_stride,
-                           weight_stride, targets, row_valid, temperature, out_lp, nullptr, out_entropy, nullptr,
+  return fused_launch_impl(hidden, nullptr, n_tokens, hidden_ref, norm_weight, norm_eps, w0, w1, n_tokens, H, V, hidden_stride,
+                           weight_stride, sel, temperature, out_lp, nullptr, out_entropy, nullptr,
                            out_ref_lp, out_k3, workspace, stream);
 }
 

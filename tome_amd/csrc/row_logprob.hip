@@ -19,13 +19,12 @@
 namespace tome {
 
 // A launch scores `problems`: problem i reads row i of the logits - or, with a row list, row row_index[i] - and
-// owns entry i of targets, row_valid, the outputs and the partials.
+// owns entry i of the targets, the mask, the outputs and the partials.
 struct RowArgs {
   const void* logits;
   const int32_t* row_index;  // nullable: problem -> row of `logits` (a row outside [0, n_rows) scores NaN, argmax -1)
   int64_t n_rows;            // rows the logits matrix holds (only read with a row list)
-  const int32_t* targets;
-  const int32_t* row_valid;
+  RowSel sel;
   float* out_lp;
   float* out_lse;
   float* out_entropy;
@@ -57,8 +56,8 @@ __device__ __forceinline__ int argmax_in_unit(const T* row, int64_t V, int unit,
 // when the row has been streamed.
 template <typename T>
 __device__ __forceinline__ float load_target_logit(const RowArgs& a, const T* row, int64_t r) {
-  if (!a.out_lp || !a.targets) return __builtin_nanf("");
-  const int32_t t = a.targets[r];
+  if (!a.out_lp || !a.sel.targets) return __builtin_nanf("");
+  const int32_t t = a.sel.target(r);
   return (t >= 0 && t < a.V) ? Elem<T>::load1(row + t) : __builtin_nanf("");
 }
 
@@ -84,7 +83,7 @@ __global__ __launch_bounds__(kRowWG) void row_logprob_kernel(RowArgs a) {
   const int split = blockIdx.x % a.splits;
   const int tid = threadIdx.x;
 
-  if (a.row_valid && a.row_valid[r] == 0) {  // masked row: not read, outputs zeroed
+  if (!a.sel.valid(r)) {  // masked row: not read, outputs zeroed
     if (split == 0 && tid == 0) {
       if (a.out_lp) a.out_lp[r] = 0.f;
       if (a.out_lse) a.out_lse[r] = 0.f;
@@ -159,7 +158,7 @@ __global__ __launch_bounds__(kRowWG) void row_logprob_kernel(RowArgs a) {
 template <typename T, bool ENT, bool AMAX>
 __global__ __launch_bounds__(64) void row_combine_kernel(RowArgs a) {
   const int64_t r = blockIdx.x;
-  if (a.row_valid && a.row_valid[r] == 0) return;  // outputs already zeroed by the main kernel
+  if (!a.sel.valid(r)) return;  // outputs already zeroed by the main kernel
   const int64_t src = a.row_index ? (int64_t)a.row_index[r] : r;
   if (a.row_index && (uint64_t)src >= (uint64_t)a.n_rows) return;  // outputs already written by the main kernel
   const int lane = threadIdx.x;
@@ -218,8 +217,7 @@ int row_splits_for(int64_t rows, int64_t V, int vec) {
 // `rows` problems.  With `row_index` (device, one entry per problem) problem i reads row row_index[i] of a matrix
 // of `n_rows` rows; without it, row i.
 hipError_t row_logprob_launch_rows(const void* logits, int dtype, int64_t n_rows, const int32_t* row_index, int64_t rows,
-                                   int64_t V, int64_t row_stride, const int32_t* targets, const int32_t* row_valid,
-                                   float temperature, float* out_lp, float* out_lse, float* out_entropy,
+                                   int64_t V, int64_t row_stride, const RowSel& sel, float temperature, float* out_lp, float* out_lse, float* out_entropy,
                                    int32_t* out_argmax, void* workspace, hipStream_t stream) {
   const int esize = dtype == 0 ? 4 : 2;
   const int vec = 16 / esize;
@@ -227,8 +225,7 @@ hipError_t row_logprob_launch_rows(const void* logits, int dtype, int64_t n_rows
   a.logits = logits;
   a.row_index = row_index;
   a.n_rows = n_rows;
-  a.targets = targets;
-  a.row_valid = row_valid;
+  a.sel = sel;
   a.out_lp = out_lp;
   a.out_lse = out_lse;
   a.out_entropy = out_entropy;
@@ -267,10 +264,9 @@ hipError_t row_lse_partials_launch(const void* logits, int dtype, int64_t rows, 
 }
 
 hipError_t row_logprob_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
-                              const int32_t* targets, const int32_t* row_valid, float temperature,
-                              float* out_lp, float* out_lse, float* out_entropy, int32_t* out_argmax,
-                              void* workspace, hipStream_t stream) {
-  return row_logprob_launch_rows(logits, dtype, rows, nullptr, rows, V, row_stride, targets, row_valid, temperature,
+                              const RowSel& sel, float temperature, float* out_lp, float* out_lse, float* out_entropy,
+                              int32_t* out_argmax, void* workspace, hipStream_t stream) {
+  return row_logprob_launch_rows(logits, dtype, rows, nullptr, rows, V, row_stride, sel, temperature,
                                  out_lp, out_lse, out_entropy, out_argmax, workspace, stream);
 }
 
@@ -331,15 +327,14 @@ size_t row_partials_bytes(int dtype, int64_t rows, int64_t V) {
 // row_logprob_launch with the partials in the library's own scratch array.  `too_big` is set (and nothing
 // launched) when the call would need more than the array holds.
 hipError_t row_logprob_noalloc_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
-                                      const int32_t* targets, const int32_t* row_valid, float temperature,
-                                      float* out_lp, float* out_lse, float* out_entropy, int32_t* out_argmax,
+                                      const RowSel& sel, float temperature, float* out_lp, float* out_lse, float* out_entropy, int32_t* out_argmax,
                                       bool* too_big, hipStream_t stream) {
   *too_big = row_partials_bytes(dtype, rows, V) > g_scratch_limit.load(std::memory_order_relaxed);
   if (*too_big) return hipSuccess;
   void* ptr = nullptr;
   const hipError_t e = row_scratch_for_current_device(&ptr);
   if (e != hipSuccess) return e;
-  return row_logprob_launch(logits, dtype, rows, V, row_stride, targets, row_valid, temperature, out_lp, out_lse,
+  return row_logprob_launch(logits, dtype, rows, V, row_stride, sel, temperature, out_lp, out_lse,
                             out_entropy, out_argmax, ptr, stream);
 }
 

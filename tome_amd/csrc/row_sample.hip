@@ -40,7 +40,7 @@ constexpr int kSampMaxK = 32;  // one tightening round is then sure to drop >= 3
 struct SampleArgs {
   const void* logits;
   const float* uniforms;      // one per row, or nullptr = greedy (candidate 0)
-  const int32_t* row_valid;   // nullable
+  RowSel sel;                 // its mask only
   int32_t* out_token;
   float* out_lp;              // nullable
   float* out_lse;             // nullable
@@ -83,7 +83,6 @@ struct SampleLds {
 // Wave-cooperative collection without atomics: every wave owns a quarter of a key buffer and a running count that is
 // the same in all its lanes; the lanes that pass take consecutive slots by their position among the passing lanes.
 // An LDS atomic that returns the slot costs a round trip per candidate, and those trips queue up behind each other.
-constexpr int kSampWaveCap = kSampCap / kRowWaves;
 struct WaveCollector {
   uint64_t* region;
   int cap;
@@ -270,7 +269,7 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int k = a.top_k;
 
-  if (a.row_valid && a.row_valid[r] == 0) {  // masked row: not read
+  if (!a.sel.valid(r)) {  // masked row: not read
     if (split != 0) return;
     if (tid == 0) {
       a.out_token[r] = -1;
@@ -565,7 +564,7 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 __global__ __launch_bounds__(kRowWG) void row_sample_combine_kernel(SampleArgs a) {
   __shared__ SampleLds<kSampMergeCap> sh;
   const int64_t r = blockIdx.x;
-  if (a.row_valid && a.row_valid[r] == 0) return;  // outputs already written by the main kernel
+  if (!a.sel.valid(r)) return;  // outputs already written by the main kernel
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int k = a.top_k, m = a.splits * k;         // <= 64 * 32 = kSampMergeCap
   const uint64_t* keys = a.part_keys + r * m;      // per split: its k keys in descending order, 0 past the end
@@ -668,14 +667,14 @@ size_t row_sample_workspace_bytes(int64_t rows, int64_t V, int dtype_vec, int to
 }
 
 hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
-                             const float* uniforms, const int32_t* row_valid, float temperature, int top_k,
+                             const float* uniforms, const RowSel& sel, float temperature, int top_k,
                              int32_t* out_token, float* out_lp, float* out_lse, int32_t* out_argmax,
                              int32_t* out_topk_idx, float* out_topk_logit, void* workspace, hipStream_t stream) {
   const int esize = dtype == 0 ? 4 : 2;
   const int vec = 16 / esize;
   const int splits = sample_splits_for(rows, V, vec);
   char* ws = static_cast<char*>(workspace);
-  SampleArgs a{logits, uniforms, row_valid, out_token, out_lp, out_lse, out_argmax, out_topk_idx, out_topk_logit,
+  SampleArgs a{logits, uniforms, sel, out_token, out_lp, out_lse, out_argmax, out_topk_idx, out_topk_logit,
                reinterpret_cast<uint64_t*>(ws),
                reinterpret_cast<float2*>(ws + align256s((size_t)rows * splits * top_k * sizeof(uint64_t))),
                V, row_stride, top_k, splits, kLog2e / temperature};
