@@ -107,6 +107,19 @@ def load_library() -> ctypes.CDLL:
     return lib
 
 
+_ops = None
+
+
+def torch_ops():
+    """The native host side of the tensor operators (csrc/torch_binding.cpp); built and loaded with the library."""
+    global _ops
+    if _ops is None:
+        load_library()
+        from . import _torch_ops
+        _ops = _torch_ops
+    return _ops
+
+
 def check(code: int) -> None:
     if code == 0:
         return

@@ -1,0 +1,329 @@
+// Host side of the operators on torch tensors: argument checks, output and workspace allocation and the C-ABI call in
+// native code.  The launches of a decode-sized call take 5-10 us on the GPU; in Python the same work (a dozen torch calls, two
+// ctypes calls) took 15-21 us a call and was what such a call cost (8 x 151936 fp32: 21.6 us a call, the kernels 7.5).
+// Nothing is kept between calls.  The stream is torch's current one, passed by the caller as a raw handle; no HIP headers
+// are needed here.
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <pybind11/pybind11.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <optional>
+#include <string>
+#include <tuple>
+#include <vector>
+
+#include "../../include/tome_logprob.h"
+
+namespace py = pybind11;
+using at::Tensor;
+typedef std::optional<Tensor> MaybeTensor;
+
+namespace {
+
+std::string str(const c10::Device& d) { return d.str(); }
+
+void require_gpu(const Tensor& t) {
+  if (!t.is_cuda())
+    throw std::runtime_error("tome_amd operators run on a ROCm GPU only (there is no CPU fallback); got a tensor on " + str(t.device()));
+}
+void require_same(const Tensor& t, const c10::Device& dev) {
+  require_gpu(t);
+  if (t.device() != dev) throw py::value_error("all tensors must be on the same device");
+}
+
+int dtype_code(const Tensor& t) {
+  if (t.scalar_type() == at::kFloat) return TOME_F32;
+  if (t.scalar_type() == at::kBFloat16) return TOME_BF16;
+  throw py::type_error(std::string("logits must be float32 or bfloat16, got ") + c10::toString(t.scalar_type()));
+}
+
+// Status codes become the exceptions of tome_amd._lib.check.
+void check(int code) {
+  if (code == TOME_OK) return;
+  py::module_::import("tome_amd._lib").attr("check")(code);
+}
+
+// [..., V] -> [rows, V] with unit stride along V, copying only when no such view exists.
+Tensor rows_view(const Tensor& x) {
+  if (x.dim() == 0) throw py::value_error("expected a tensor with a vocabulary axis");
+  const int64_t V = x.size(-1);
+  Tensor y = x.stride(-1) != 1 && V > 1 ? x.contiguous() : x;
+  if (y.dim() == 2) return y;
+  if (y.dim() == 1) return y.unsqueeze(0);
+  int64_t rows = 1;
+  for (int64_t d = 0; d + 1 < y.dim(); ++d) rows *= y.size(d);
+  return y.reshape({rows, V});
+}
+
+// Outputs of `n` rows take the leading shape of the input; `v` is already of that shape for [rows, V] inputs.
+Tensor shaped(const Tensor& v, const Tensor& like) {
+  if (like.dim() == 2) return v;
+  return v.view(like.sizes().slice(0, like.dim() - 1));
+}
+MaybeTensor shaped(const MaybeTensor& v, const Tensor& like) { return v ? MaybeTensor(shaped(*v, like)) : v; }
+
+// Integer ids of `n` entries on `dev`, int32 or int64 as they are, other integer types as int32.
+Tensor ids_of(const Tensor& t, int64_t n, const c10::Device& dev, const char* what) {
+  if (t.device() != dev) throw py::value_error(std::string(what) + " must be on " + str(dev));
+  if (t.numel() != n)
+    throw py::value_error(std::string(what) + " has " + std::to_string(t.numel()) + " entries, expected " + std::to_string(n));
+  const auto st = t.scalar_type();
+  if (!at::isIntegralType(st, /*includeBool=*/false)) throw py::type_error(std::string(what) + " must be an integer tensor");
+  if (st == at::kInt || st == at::kLong) return t.contiguous();
+  return t.to(at::kInt).contiguous();
+}
+
+// TomeRowSel and the tensors it points into.
+struct Sel {
+  TomeRowSel c{};
+  Tensor targets, mask;
+
+  Sel(const MaybeTensor& tg, const MaybeTensor& lengths, const MaybeTensor& row_valid, const Tensor& like, int64_t n,
+      const c10::Device& dev) {
+    if (lengths && row_valid) throw py::value_error("pass lengths or row_valid, not both");
+    if (tg) {
+      targets = ids_of(*tg, n, dev, "targets");
+      c.targets = targets.data_ptr();
+      c.target_bytes = (int32_t)targets.element_size();
+    }
+    if (row_valid) {
+      if (row_valid->numel() != n)
+        throw py::value_error("row_valid has " + std::to_string(row_valid->numel()) + " entries, expected " + std::to_string(n));
+      const auto st = row_valid->scalar_type();
+      const bool as_is = st == at::kBool || st == at::kByte || st == at::kChar || st == at::kInt || st == at::kLong;
+      mask = row_valid->device() == dev && as_is ? row_valid->contiguous() : row_valid->to(dev, at::kInt).contiguous();
+      c.row_valid = mask.data_ptr();
+      c.valid_bytes = (int32_t)mask.element_size();
+    } else if (lengths) {
+      if (like.dim() != 3) throw py::value_error("lengths needs inputs shaped [batch, seq, ...]");
+      if (lengths->numel() != like.size(0))
+        throw py::value_error("lengths has " + std::to_string(lengths->numel()) + " entries, expected " + std::to_string(like.size(0)));
+      const auto st = lengths->scalar_type();
+      mask = lengths->device() == dev && (st == at::kInt || st == at::kLong) ? lengths->contiguous()
+                                                                             : lengths->to(dev, at::kLong).contiguous();
+      c.lengths = mask.data_ptr();
+      c.length_bytes = (int32_t)mask.element_size();
+      c.seq_len = like.size(1) > 0 ? like.size(1) : 1;
+    }
+  }
+};
+
+Tensor workspace(size_t bytes, const at::TensorOptions& o) {
+  return bytes > 0 ? at::empty({(int64_t)bytes}, o.dtype(at::kByte)) : Tensor();
+}
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+template <typename T>
+T* ptr(const MaybeTensor& t) { return t ? static_cast<T*>(t->data_ptr()) : nullptr; }
+MaybeTensor maybe_empty(bool want, int64_t n, const at::TensorOptions& o) {
+  return want ? MaybeTensor(at::empty({n}, o)) : MaybeTensor();
+}
+void* stream_ptr(uintptr_t s) { return reinterpret_cast<void*>(s); }
+
+typedef std::tuple<Tensor, MaybeTensor, MaybeTensor, MaybeTensor> RowOutputs;  // lp, lse, entropy, argmax
+
+RowOutputs token_logprobs(const Tensor& logits, const Tensor& targets, double temperature, const MaybeTensor& lengths,
+                          const MaybeTensor& row_valid, bool want_lse, bool want_entropy, bool want_argmax, uintptr_t stream) {
+  require_gpu(logits);
+  const c10::Device dev = logits.device();
+  const int dtype = dtype_code(logits);
+  const Tensor x = rows_view(logits);
+  const int64_t rows = x.size(0), V = x.size(1);
+  c10::DeviceGuard guard(dev);
+  const Sel sel(targets, lengths, row_valid, logits, rows, dev);
+  const at::TensorOptions f32 = at::TensorOptions().dtype(at::kFloat).device(dev), i32 = f32.dtype(at::kInt);
+  Tensor lp = at::empty({rows}, f32);
+  MaybeTensor lse = maybe_empty(want_lse, rows, f32), ent = maybe_empty(want_entropy, rows, f32), amax = maybe_empty(want_argmax, rows, i32);
+  const size_t bytes = tome_row_logprob_workspace(rows, V);
+  const Tensor ws = workspace(bytes, f32);
+  check(tome_row_logprob_sel(x.data_ptr(), dtype, rows, V, rows > 1 ? x.stride(0) : V, &sel.c, (float)temperature,
+                             lp.data_ptr<float>(), ptr<float>(lse), ptr<float>(ent), ptr<int32_t>(amax), ptr(ws), bytes,
+                             stream_ptr(stream)));
+  return {shaped(lp, logits), shaped(lse, logits), shaped(ent, logits), shaped(amax, logits)};
+}
+
+RowOutputs token_logprobs_rows(const Tensor& logits, const Tensor& row_index, const Tensor& targets, double temperature,
+                               bool want_lse, bool want_entropy, bool want_argmax, uintptr_t stream) {
+  require_gpu(logits);
+  const c10::Device dev = logits.device();
+  const int dtype = dtype_code(logits);
+  const Tensor x = rows_view(logits);
+  const int64_t rows = x.size(0), V = x.size(1), n = row_index.numel();
+  c10::DeviceGuard guard(dev);
+  const Tensor idx = ids_of(row_index, n, dev, "row_index").to(at::kInt), tg = ids_of(targets, n, dev, "targets").to(at::kInt);
+  const at::TensorOptions f32 = at::TensorOptions().dtype(at::kFloat).device(dev), i32 = f32.dtype(at::kInt);
+  Tensor lp = at::empty({n}, f32);
+  MaybeTensor lse = maybe_empty(want_lse, n, f32), ent = maybe_empty(want_entropy, n, f32), amax = maybe_empty(want_argmax, n, i32);
+  const size_t bytes = tome_row_logprob_workspace(n, V);
+  const Tensor ws = workspace(bytes, f32);
+  check(tome_row_logprob_rows(x.data_ptr(), dtype, rows, V, rows > 1 ? x.stride(0) : V, idx.data_ptr<int32_t>(), n,
+                              tg.data_ptr<int32_t>(), (float)temperature, lp.data_ptr<float>(), ptr<float>(lse), ptr<float>(ent),
+                              ptr<int32_t>(amax), ptr(ws), bytes, stream_ptr(stream)));
+  return {lp, lse, ent, amax};
+}
+
+// token, lp, argmax (rows of one allocation, in this order), candidate ids and logits; `mask` int32
+std::tuple<Tensor, Tensor, Tensor, MaybeTensor, MaybeTensor> sample_tokens(const Tensor& logits, double temperature, int64_t top_k,
+                                                                           const MaybeTensor& uniforms, const MaybeTensor& mask,
+                                                                           bool want_topk, uintptr_t stream) {
+  require_gpu(logits);
+  const c10::Device dev = logits.device();
+  const int dtype = dtype_code(logits);
+  const Tensor x = rows_view(logits);
+  const int64_t rows = x.size(0), V = x.size(1);
+  if (top_k < 1 || top_k > 32) throw py::value_error("top_k must be in 1..32");
+  c10::DeviceGuard guard(dev);
+  if (mask) require_same(*mask, dev);
+  Tensor u;
+  if (uniforms) {
+    u = uniforms->to(dev, at::kFloat).contiguous();
+    if (u.numel() != rows)
+      throw py::value_error("uniforms must have one value per row (" + std::to_string(rows) + "), got " + std::to_string(u.numel()));
+  }
+  const at::TensorOptions i32 = at::TensorOptions().dtype(at::kInt).device(dev);
+  const Tensor packed = at::empty({3, rows}, i32);
+  const Tensor tok = packed.select(0, 0), lp = packed.select(0, 1).view(at::kFloat), amax = packed.select(0, 2);
+  MaybeTensor tki, tkl;
+  if (want_topk) {
+    tki = at::empty({rows, top_k}, i32);
+    tkl = at::empty({rows, top_k}, i32.dtype(at::kFloat));
+  }
+  const size_t bytes = tome_row_sample_workspace(dtype, rows, V, (int)top_k);
+  const Tensor ws = workspace(bytes, i32);
+  int32_t* out = packed.data_ptr<int32_t>();
+  check(tome_row_sample(x.data_ptr(), dtype, rows, V, rows > 1 ? x.stride(0) : V, u.defined() ? u.data_ptr<float>() : nullptr,
+                        ptr<const int32_t>(mask), (float)temperature, (int)top_k, out,
+                        reinterpret_cast<float*>(out + rows), nullptr, out + 2 * rows, ptr<int32_t>(tki), ptr<float>(tkl), ptr(ws),
+                        bytes, stream_ptr(stream)));
+  if (want_topk && logits.dim() != 2) {
+    std::vector<int64_t> shape(logits.sizes().begin(), logits.sizes().end());
+    shape.back() = top_k;
+    tki = tki->view(shape);
+    tkl = tkl->view(shape);
+  }
+  return {shaped(tok, logits), shaped(lp, logits), shaped(amax, logits), tki, tkl};
+}
+
+Tensor fused_log_softmax(const Tensor& logits, double temperature, uintptr_t stream) {
+  require_gpu(logits);
+  const c10::Device dev = logits.device();
+  const int dtype = dtype_code(logits);
+  const Tensor x = rows_view(logits);
+  const int64_t rows = x.size(0), V = x.size(1);
+  c10::DeviceGuard guard(dev);
+  const at::TensorOptions f32 = at::TensorOptions().dtype(at::kFloat).device(dev);
+  const Tensor out = at::empty(logits.sizes(), f32.dtype(logits.scalar_type()));
+  // the rows' lse, and behind it the workspace
+  const size_t lse_bytes = ((size_t)rows * 4 + 255) & ~(size_t)255, bytes = tome_row_logprob_workspace(rows, V);
+  const Tensor ws = at::empty({(int64_t)(lse_bytes + bytes)}, f32.dtype(at::kByte));
+  char* base = static_cast<char*>(ws.data_ptr());
+  check(tome_full_log_softmax(x.data_ptr(), out.data_ptr(), dtype, rows, V, rows > 1 ? x.stride(0) : V, V, (float)temperature,
+                              reinterpret_cast<float*>(base), bytes > 0 ? base + lse_bytes : nullptr, bytes, stream_ptr(stream)));
+  return out;
+}
+
+void check_bf16(const Tensor& hidden, const Tensor& weight) {
+  if (hidden.scalar_type() != at::kBFloat16 || weight.scalar_type() != at::kBFloat16)
+    throw py::type_error("hidden and lm_head weights must be bfloat16 (the reference loads bf16 weights, mlx-impl/load_weights.py:20-22)");
+}
+void check_weight(const Tensor& w, int64_t H) {
+  if (w.dim() != 2 || w.size(1) != H)
+    throw py::value_error("weight must be [V, " + std::to_string(H) + "] (rows = vocabulary, as embed_tokens.weight)");
+}
+Tensor unit_columns(const Tensor& w) { return w.stride(1) == 1 ? w : w.contiguous(); }
+Tensor check_norm(const MaybeTensor& norm, int64_t H, const c10::Device& dev) {
+  if (!norm) return Tensor();
+  if (norm->scalar_type() != at::kBFloat16 || norm->dim() != 1 || norm->size(0) != H || norm->device() != dev)
+    throw py::value_error("norm_weight must be a bfloat16 [" + std::to_string(H) + "] tensor on " + str(dev));
+  return norm->contiguous();
+}
+
+// hidden_rows: a list of rows of the flattened hidden states; targets and outputs are then packed in list order.
+RowOutputs lmhead_logprobs(const Tensor& hidden, const Tensor& weight, const Tensor& targets, double temperature,
+                           const MaybeTensor& lengths, const MaybeTensor& row_valid, bool want_lse, bool want_entropy,
+                           bool want_argmax, const MaybeTensor& norm_weight, double norm_eps, const MaybeTensor& hidden_rows,
+                           uintptr_t stream) {
+  require_gpu(hidden);
+  const c10::Device dev = hidden.device();
+  require_same(weight, dev);
+  check_bf16(hidden, weight);
+  const int64_t H = hidden.size(-1);
+  check_weight(weight, H);
+  const Tensor h = rows_view(hidden), w = unit_columns(weight);
+  const int64_t n_rows = h.size(0), V = w.size(0), n = hidden_rows ? hidden_rows->numel() : n_rows;
+  c10::DeviceGuard guard(dev);
+  const Sel sel(targets, lengths, row_valid, hidden, n, dev);
+  const Tensor list = hidden_rows ? ids_of(*hidden_rows, n, dev, "hidden_rows").to(at::kInt) : Tensor();
+  const Tensor nw = check_norm(norm_weight, H, dev);
+  const at::TensorOptions f32 = at::TensorOptions().dtype(at::kFloat).device(dev), i32 = f32.dtype(at::kInt);
+  Tensor lp = at::empty({n}, f32);
+  MaybeTensor lse = maybe_empty(want_lse, n, f32), ent = maybe_empty(want_entropy, n, f32), amax = maybe_empty(want_argmax, n, i32);
+  const size_t bytes = nw.defined() ? tome_norm_lmhead_logprob_workspace(n, H, V) : tome_fused_lmhead_logprob_workspace(n, H, V);
+  const Tensor ws = workspace(bytes, f32);
+  check(tome_lmhead_logprob_sel(h.data_ptr(), static_cast<const int32_t*>(ptr(list)), n_rows, ptr(nw), (float)norm_eps, w.data_ptr(),
+                                n, H, V, n_rows > 1 ? h.stride(0) : H, w.stride(0), &sel.c, (float)temperature,
+                                lp.data_ptr<float>(), ptr<float>(lse), ptr<float>(ent), ptr<int32_t>(amax), ptr(ws), bytes,
+                                stream_ptr(stream)));
+  if (hidden_rows) return {lp, lse, ent, amax};
+  return {shaped(lp, hidden), shaped(lse, hidden), shaped(ent, hidden), shaped(amax, hidden)};
+}
+
+// policy log-prob, reference log-prob, k3, policy entropy
+std::tuple<Tensor, Tensor, Tensor, Tensor> grpo_pair(const Tensor& hidden_policy, const MaybeTensor& hidden_ref, const Tensor& w_policy,
+                                                     const MaybeTensor& w_ref, const Tensor& targets, double temperature,
+                                                     const MaybeTensor& lengths, const MaybeTensor& row_valid,
+                                                     const MaybeTensor& norm_weight, double norm_eps, uintptr_t stream) {
+  require_gpu(hidden_policy);
+  const c10::Device dev = hidden_policy.device();
+  require_same(w_policy, dev);
+  check_bf16(hidden_policy, w_policy);
+  const int64_t H = hidden_policy.size(-1);
+  check_weight(w_policy, H);
+  if (w_ref) {
+    require_same(*w_ref, dev);
+    check_bf16(hidden_policy, *w_ref);
+    check_weight(*w_ref, H);
+    if (w_ref->sizes() != w_policy.sizes()) throw py::value_error("policy and reference weights must have the same shape");
+  }
+  Tensor h = rows_view(hidden_policy), r = h;
+  if (hidden_ref) {
+    require_same(*hidden_ref, dev);
+    if (hidden_ref->scalar_type() != at::kBFloat16 || hidden_ref->sizes() != hidden_policy.sizes())
+      throw py::value_error("hidden_ref must be bfloat16 with hidden_policy's shape");
+    r = rows_view(*hidden_ref);
+  }
+  Tensor wp = unit_columns(w_policy), wr = w_ref ? unit_columns(*w_ref) : wp;
+  c10::DeviceGuard guard(dev);
+  if (wp.stride(0) != wr.stride(0)) {
+    wp = wp.contiguous();
+    wr = wr.contiguous();
+  }
+  const int64_t n = h.size(0), V = wp.size(0);
+  if (n > 1 && h.stride(0) != r.stride(0)) {
+    h = h.contiguous();
+    r = r.contiguous();
+  }
+  const Sel sel(targets, lengths, row_valid, hidden_policy, n, dev);
+  const Tensor nw = check_norm(norm_weight, H, dev);
+  const at::TensorOptions f32 = at::TensorOptions().dtype(at::kFloat).device(dev);
+  const Tensor lp = at::empty({n}, f32), ref_lp = at::empty({n}, f32), k3 = at::empty({n}, f32), ent = at::empty({n}, f32);
+  const size_t bytes = tome_grpo_pair_workspace(n, H, V, nw.defined() ? 1 : 0);
+  const Tensor ws = workspace(bytes, f32);
+  check(tome_grpo_pair_sel(h.data_ptr(), r.data_ptr(), ptr(nw), (float)norm_eps, wp.data_ptr(), wr.data_ptr(), n, H, V,
+                           n > 1 ? h.stride(0) : H, wp.stride(0), &sel.c, (float)temperature, lp.data_ptr<float>(),
+                           ref_lp.data_ptr<float>(), k3.data_ptr<float>(), ent.data_ptr<float>(), ptr(ws), bytes, stream_ptr(stream)));
+  return {shaped(lp, hidden_policy), shaped(ref_lp, hidden_policy), shaped(k3, hidden_policy), shaped(ent, hidden_policy)};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_torch_ops, m) {
+  m.doc() = "Native host side of tome_amd's operators (argument checks, allocation, C-ABI calls)";
+  m.def("rows_view", &rows_view);
+  m.def("token_logprobs", &token_logprobs);
+  m.def("token_logprobs_rows", &token_logprobs_rows);
+  m.def("sample_tokens", &sample_tokens);
+  m.def("fused_log_softmax", &fused_log_softmax);
+  m.def("lmhead_logprobs", &lmhead_logprobs);
+  m.def("grpo_pair", &grpo_pair);
+}

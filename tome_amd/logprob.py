@@ -20,7 +20,6 @@ from typing import NamedTuple, Optional
 import torch
 
 from . import _lib
-from ._lib import TOME_BF16, TOME_F32
 
 
 class TokenLogprobs(NamedTuple):
@@ -45,25 +44,6 @@ class DualLogprobs(NamedTuple):
     entropy: torch.Tensor   # entropy of the policy distribution
 
 
-def _require_gpu(*tensors: torch.Tensor) -> torch.device:
-    dev = tensors[0].device
-    for t in tensors:
-        if not t.is_cuda:
-            raise RuntimeError("tome_amd operators run on a ROCm GPU only (there is no CPU fallback); "
-                               f"got a tensor on {t.device}")
-        if t.device != dev:
-            raise ValueError("all tensors must be on the same device")
-    return dev
-
-
-def _dtype_code(t: torch.Tensor) -> int:
-    if t.dtype == torch.float32:
-        return TOME_F32
-    if t.dtype == torch.bfloat16:
-        return TOME_BF16
-    raise TypeError(f"logits must be float32 or bfloat16, got {t.dtype}")
-
-
 def _check_temperature(temperature: float) -> float:
     temperature = float(temperature)
     if not (temperature > 0.0) or temperature == float("inf"):
@@ -72,66 +52,20 @@ def _check_temperature(temperature: float) -> float:
     return temperature
 
 
+def _tensor(t, like: torch.Tensor, on_device: bool = True):
+    """``t`` as a tensor (ids, masks and lengths may also be given as lists)."""
+    if t is None or isinstance(t, torch.Tensor):
+        return t
+    return torch.as_tensor(t, device=like.device) if on_device else torch.as_tensor(t)
+
+
 def _rows_view(x: torch.Tensor) -> torch.Tensor:
-    """[..., V] -> [rows, V] with unit stride along V, copying only when no such view exists."""
-    if x.dim() == 0:
-        raise ValueError("expected a tensor with a vocabulary axis")
-    V = x.shape[-1]
-    if x.dim() == 1:
-        x = x.unsqueeze(0)
-    if x.stride(-1) != 1 and V > 1:
-        x = x.contiguous()
-    if x.dim() == 2:
-        return x
-    try:
-        return x.view(-1, V)
-    except RuntimeError:
-        return x.reshape(-1, V)
-
-
-def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
-    return None if t is None else t.data_ptr()
-
-
-def _stream(dev: torch.device) -> int:
-    """Raw hipStream_t of torch's current stream on ``dev`` (the launch stream of every call)."""
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)   # a fraction of the cost of the Stream object
-    if raw is not None and dev.index is not None:
-        return raw(dev.index)
-    return torch.cuda.current_stream(dev).cuda_stream
-
-
-class _on_device:
-    """``torch.cuda.device(dev)`` that does nothing when ``dev`` is already current (the usual case):
-    the HIP launches of the library go to the current device, so it has to be the tensors' one."""
-
-    def __init__(self, dev: torch.device):
-        idx = dev.index if dev.index is not None else torch.cuda.current_device()
-        self._guard = None if idx == torch.cuda.current_device() else torch.cuda.device(idx)
-
-    def __enter__(self):
-        if self._guard is not None:
-            self._guard.__enter__()
-
-    def __exit__(self, *exc):
-        if self._guard is not None:
-            return self._guard.__exit__(*exc)
-        return False
-
-
-def _as_i32(t, n: int, dev: torch.device, what: str) -> torch.Tensor:
-    t = torch.as_tensor(t, device=dev) if not isinstance(t, torch.Tensor) else t
-    if t.device != dev:
-        raise ValueError(f"{what} must be on {dev}")
-    if t.numel() != n:
-        raise ValueError(f"{what} has {t.numel()} entries, expected {n}")
-    if t.dtype.is_floating_point or t.dtype == torch.bool:
-        raise TypeError(f"{what} must be an integer tensor")
-    return t.reshape(-1).to(torch.int32).contiguous()
+    """[..., V] -> [rows, V] with unit stride along V, copying only when no such view exists (as every operator does)."""
+    return _lib.torch_ops().rows_view(x)
 
 
 def _row_valid(lead_shape, n_rows: int, lengths, row_valid, dev) -> Optional[torch.Tensor]:
-    """Row mask from either an explicit mask or per-sequence lengths over a [B, L] leading shape."""
+    """int32 row mask from either an explicit mask or per-sequence lengths over a [B, L] leading shape."""
     if lengths is not None and row_valid is not None:
         raise ValueError("pass lengths or row_valid, not both")
     if row_valid is not None:
@@ -151,8 +85,13 @@ def _row_valid(lead_shape, n_rows: int, lengths, row_valid, dev) -> Optional[tor
     return (torch.arange(L, device=dev).reshape(1, L) < ln).to(torch.int32).reshape(-1).contiguous()
 
 
-def _workspace(nbytes: int, dev: torch.device) -> Optional[torch.Tensor]:
-    return torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes > 0 else None
+_current_raw_stream = torch._C._cuda_getCurrentRawStream   # a fraction of the cost of the Stream object
+
+
+def _stream(t: torch.Tensor) -> int:
+    """Raw hipStream_t of torch's current stream on ``t``'s GPU (the launch stream of every call); 0 for a CPU tensor,
+    which the operators refuse."""
+    return _current_raw_stream(t.get_device()) if t.is_cuda else 0
 
 
 def token_logprobs(logits: torch.Tensor, targets, temperature: float = 1.0, lengths=None, *,
@@ -165,29 +104,9 @@ def token_logprobs(logits: torch.Tensor, targets, temperature: float = 1.0, leng
     ``row_valid`` are not read; their outputs are 0 (argmax -1).  Outputs are float32
     with the leading shape.
     """
-    lib = _lib.load_library()
-    dev = _require_gpu(logits)
-    temperature = _check_temperature(temperature)
-    dtype = _dtype_code(logits)
-    lead = tuple(logits.shape[:-1])
-    x = _rows_view(logits)
-    rows, V = x.shape
-    tg = _as_i32(targets, rows, dev, "targets")
-    rv = _row_valid(lead, rows, lengths, row_valid, dev)
-    with _on_device(dev):
-        lp = torch.empty(rows, dtype=torch.float32, device=dev)
-        lse = torch.empty(rows, dtype=torch.float32, device=dev) if want_lse else None
-        ent = torch.empty(rows, dtype=torch.float32, device=dev) if want_entropy else None
-        amax = torch.empty(rows, dtype=torch.int32, device=dev) if want_argmax else None
-        ws_bytes = lib.tome_row_logprob_workspace(rows, V)
-        ws = _workspace(ws_bytes, dev)
-        _lib.check(lib.tome_row_logprob(x.data_ptr(), dtype, rows, V, x.stride(0) if rows > 1 else V,
-                                        tg.data_ptr(), _ptr(rv), temperature, lp.data_ptr(), _ptr(lse),
-                                        _ptr(ent), _ptr(amax), _ptr(ws), ws_bytes, _stream(dev)))
-
-    def _shaped(t):
-        return None if t is None else t.reshape(lead)
-    return TokenLogprobs(_shaped(lp), _shaped(lse), _shaped(ent), _shaped(amax))
+    return TokenLogprobs(*_lib.torch_ops().token_logprobs(
+        logits, _tensor(targets, logits), _check_temperature(temperature), _tensor(lengths, logits, False),
+        _tensor(row_valid, logits), want_lse, want_entropy, want_argmax, _stream(logits)))
 
 
 def token_logprobs_rows(logits: torch.Tensor, row_index, targets, temperature: float = 1.0, *,
@@ -199,27 +118,9 @@ def token_logprobs_rows(logits: torch.Tensor, row_index, targets, temperature: f
     local_compute_logprobs on the slices (node.py:400-404) for the whole chunk in one launch; rows that are not
     listed are neither read nor launched.  An index outside the matrix scores NaN (argmax -1).
     """
-    lib = _lib.load_library()
-    dev = _require_gpu(logits)
-    temperature = _check_temperature(temperature)
-    dtype = _dtype_code(logits)
-    x = _rows_view(logits)
-    rows, V = x.shape
-    idx = torch.as_tensor(row_index, device=dev) if not isinstance(row_index, torch.Tensor) else row_index
-    n = idx.numel()
-    idx = _as_i32(idx, n, dev, "row_index")
-    tg = _as_i32(targets, n, dev, "targets")
-    with _on_device(dev):
-        lp = torch.empty(n, dtype=torch.float32, device=dev)
-        lse = torch.empty(n, dtype=torch.float32, device=dev) if want_lse else None
-        ent = torch.empty(n, dtype=torch.float32, device=dev) if want_entropy else None
-        amax = torch.empty(n, dtype=torch.int32, device=dev) if want_argmax else None
-        ws_bytes = lib.tome_row_logprob_workspace(n, V)
-        ws = _workspace(ws_bytes, dev)
-        _lib.check(lib.tome_row_logprob_rows(x.data_ptr(), dtype, rows, V, x.stride(0) if rows > 1 else V, idx.data_ptr(), n,
-                                             tg.data_ptr(), temperature, lp.data_ptr(), _ptr(lse), _ptr(ent), _ptr(amax),
-                                             _ptr(ws), ws_bytes, _stream(dev)))
-    return TokenLogprobs(lp, lse, ent, amax)
+    return TokenLogprobs(*_lib.torch_ops().token_logprobs_rows(
+        logits, _tensor(row_index, logits), _tensor(targets, logits), _check_temperature(temperature), want_lse, want_entropy,
+        want_argmax, _stream(logits)))
 
 
 def sample_tokens(logits: torch.Tensor, temperature: float, top_k: int = 20, *, uniforms=None,
@@ -235,38 +136,21 @@ def sample_tokens(logits: torch.Tensor, temperature: float, top_k: int = 20, *, 
     row; drawn with ``torch.rand`` from ``generator`` when omitted) - candidates ordered by
     logit descending, equal logits by ascending id.  MLX's random stream is not reproduced.
     """
-    lib = _lib.load_library()
-    dev = _require_gpu(logits)
     greedy = float(temperature) == 0.0
     temperature = _check_temperature(1.0 if greedy else temperature)
-    dtype = _dtype_code(logits)
-    lead = tuple(logits.shape[:-1])
-    x = _rows_view(logits)
-    rows, V = x.shape
-    if not 1 <= int(top_k) <= 32:
-        raise ValueError("top_k must be in 1..32")
-    rv = _row_valid(lead, rows, lengths, row_valid, dev)
-    with _on_device(dev):
-        u = None
-        if not greedy:
-            if uniforms is None:
-                u = torch.rand(rows, dtype=torch.float32, device=dev, generator=generator)
-            else:
-                u = torch.as_tensor(uniforms, dtype=torch.float32, device=dev).reshape(-1).contiguous()
-                if u.numel() != rows:
-                    raise ValueError(f"uniforms must have one value per row ({rows}), got {u.numel()}")
-        packed = torch.empty((3, rows), dtype=torch.int32, device=dev)   # token | lp bits | argmax: one allocation,
-        tok, lp, amax = packed[0], packed[1].view(torch.float32), packed[2]  # and (token, lp) leave in one copy
-        tki = torch.empty((rows, top_k), dtype=torch.int32, device=dev) if want_topk else None
-        tkl = torch.empty((rows, top_k), dtype=torch.float32, device=dev) if want_topk else None
-        ws_bytes = lib.tome_row_sample_workspace(dtype, rows, V, int(top_k))
-        ws = _workspace(ws_bytes, dev)
-        _lib.check(lib.tome_row_sample(x.data_ptr(), dtype, rows, V, x.stride(0) if rows > 1 else V, _ptr(u), _ptr(rv),
-                                       temperature, int(top_k), tok.data_ptr(), lp.data_ptr(), None, amax.data_ptr(),
-                                       _ptr(tki), _ptr(tkl), _ptr(ws), ws_bytes, _stream(dev)))
-    return SampledTokens(tok.reshape(lead), lp.reshape(lead), amax.reshape(lead),
-                         None if tki is None else tki.reshape(*lead, top_k),
-                         None if tkl is None else tkl.reshape(*lead, top_k))
+    if greedy:
+        uniforms = None
+    elif uniforms is None:
+        if not logits.is_cuda:
+            raise RuntimeError("tome_amd operators run on a ROCm GPU only (there is no CPU fallback); "
+                               f"got a tensor on {logits.device}")
+        uniforms = torch.rand(logits.shape[:-1].numel(), dtype=torch.float32, device=logits.device, generator=generator)
+    mask = None
+    if row_valid is not None or lengths is not None:
+        lead = logits.shape[:-1]
+        mask = _row_valid(lead, lead.numel(), lengths, row_valid, logits.device)
+    return SampledTokens(*_lib.torch_ops().sample_tokens(
+        logits, temperature, int(top_k), _tensor(uniforms, logits), mask, want_topk, _stream(logits)))
 
 
 class DecodeStepGraph:
@@ -281,7 +165,10 @@ class DecodeStepGraph:
     """
 
     def __init__(self, logits: torch.Tensor, temperature: float, top_k: int = 20, *, uniforms: Optional[torch.Tensor] = None):
-        dev = _require_gpu(logits)
+        if not logits.is_cuda:
+            raise RuntimeError("tome_amd operators run on a ROCm GPU only (there is no CPU fallback); "
+                               f"got a tensor on {logits.device}")
+        dev = logits.device
         self.logits = logits
         rows = logits.numel() // logits.shape[-1]
         self.uniforms = uniforms if uniforms is not None else torch.rand(rows, dtype=torch.float32, device=dev)
@@ -313,38 +200,7 @@ def local_compute_logprobs(logits: torch.Tensor, ids: torch.Tensor, temp: float)
 
 def fused_log_softmax(logits: torch.Tensor, temperature: float = 1.0) -> torch.Tensor:
     """Drop-in for mlx-impl/model.py:77-89: full log-softmax with temperature, same shape and dtype."""
-    lib = _lib.load_library()
-    dev = _require_gpu(logits)
-    temperature = _check_temperature(temperature)
-    dtype = _dtype_code(logits)
-    x = _rows_view(logits)
-    rows, V = x.shape
-    with _on_device(dev):
-        out = torch.empty((rows, V), dtype=logits.dtype, device=dev)
-        row_lse = torch.empty(rows, dtype=torch.float32, device=dev)
-        ws_bytes = lib.tome_row_logprob_workspace(rows, V)
-        ws = _workspace(ws_bytes, dev)
-        _lib.check(lib.tome_full_log_softmax(x.data_ptr(), out.data_ptr(), dtype, rows, V,
-                                             x.stride(0) if rows > 1 else V, V, temperature,
-                                             row_lse.data_ptr(), _ptr(ws), ws_bytes, _stream(dev)))
-    return out.reshape(logits.shape)
-
-
-def _check_fused_inputs(hidden: torch.Tensor, *weights: torch.Tensor):
-    dev = _require_gpu(hidden, *weights)
-    if hidden.dtype != torch.bfloat16 or any(w.dtype != torch.bfloat16 for w in weights):
-        raise TypeError("hidden and lm_head weights must be bfloat16 "
-                        "(the reference loads bf16 weights, mlx-impl/load_weights.py:20-22)")
-    H = hidden.shape[-1]
-    for w in weights:
-        if w.dim() != 2 or w.shape[1] != H:
-            raise ValueError(f"weight must be [V, {H}] (rows = vocabulary, as embed_tokens.weight), got {tuple(w.shape)}")
-        if w.shape != weights[0].shape:
-            raise ValueError("policy and reference weights must have the same shape")
-    lead = tuple(hidden.shape[:-1])
-    h2 = _rows_view(hidden)
-    ws_ = [w if w.stride(1) == 1 else w.contiguous() for w in weights]
-    return dev, lead, h2, ws_
+    return _lib.torch_ops().fused_log_softmax(logits, _check_temperature(temperature), _stream(logits))
 
 
 def fused_lmhead_logprobs(hidden: torch.Tensor, weight: torch.Tensor, targets, temperature: float = 1.0,
@@ -362,39 +218,9 @@ def fused_lmhead_logprobs(hidden: torch.Tensor, weight: torch.Tensor, targets, t
     RMSNorm (``mx.fast.rms_norm(x, weight, eps)``, model.py:336-343, :536) is applied to the valid
     rows first.
     """
-    lib = _lib.load_library()
-    dev, lead, h2, (w,) = _check_fused_inputs(hidden, weight)
-    temperature = _check_temperature(temperature)
-    n, H = h2.shape
-    V = w.shape[0]
-    tg = _as_i32(targets, n, dev, "targets")
-    rv = _row_valid(lead, n, lengths, row_valid, dev)
-    with _on_device(dev):
-        lp = torch.empty(n, dtype=torch.float32, device=dev)
-        lse = torch.empty(n, dtype=torch.float32, device=dev) if want_lse else None
-        ent = torch.empty(n, dtype=torch.float32, device=dev) if want_entropy else None
-        amax = torch.empty(n, dtype=torch.int32, device=dev) if want_argmax else None
-        if norm_weight is None:
-            ws_bytes = lib.tome_fused_lmhead_logprob_workspace(n, H, V)
-            ws = _workspace(ws_bytes, dev)
-            _lib.check(lib.tome_fused_lmhead_logprob(h2.data_ptr(), w.data_ptr(), n, H, V,
-                                                     h2.stride(0) if n > 1 else H, w.stride(0),
-                                                     tg.data_ptr(), _ptr(rv), temperature, lp.data_ptr(), _ptr(lse),
-                                                     _ptr(ent), _ptr(amax), _ptr(ws), ws_bytes, _stream(dev)))
-        else:
-            if norm_weight.dtype != torch.bfloat16 or norm_weight.shape != (H,) or norm_weight.device != dev:
-                raise ValueError(f"norm_weight must be a bfloat16 [{H}] tensor on {dev}")
-            nw = norm_weight.contiguous()
-            ws_bytes = lib.tome_norm_lmhead_logprob_workspace(n, H, V)
-            ws = _workspace(ws_bytes, dev)
-            _lib.check(lib.tome_norm_lmhead_logprob(h2.data_ptr(), nw.data_ptr(), float(norm_eps), w.data_ptr(), n, H, V,
-                                                    h2.stride(0) if n > 1 else H, w.stride(0),
-                                                    tg.data_ptr(), _ptr(rv), temperature, lp.data_ptr(), _ptr(lse),
-                                                    _ptr(ent), _ptr(amax), _ptr(ws), ws_bytes, _stream(dev)))
-
-    def _shaped(t):
-        return None if t is None else t.reshape(lead)
-    return TokenLogprobs(_shaped(lp), _shaped(lse), _shaped(ent), _shaped(amax))
+    return TokenLogprobs(*_lib.torch_ops().lmhead_logprobs(
+        hidden, weight, _tensor(targets, hidden), _check_temperature(temperature), _tensor(lengths, hidden, False),
+        _tensor(row_valid, hidden), want_lse, want_entropy, want_argmax, norm_weight, float(norm_eps), None, _stream(hidden)))
 
 
 def grpo_dual_logprobs(hidden: torch.Tensor, w_policy: torch.Tensor, w_ref: torch.Tensor, targets,
@@ -405,25 +231,9 @@ def grpo_dual_logprobs(hidden: torch.Tensor, w_policy: torch.Tensor, w_ref: torc
     LoRA delta, mlx-impl/node.py:102-164).  k3 and entropy have no counterpart in the
     reference node; they are defined by their closed forms.
     """
-    lib = _lib.load_library()
-    dev, lead, h2, (wp, wr) = _check_fused_inputs(hidden, w_policy, w_ref)
-    if wp.stride(0) != wr.stride(0):
-        wr = wr.contiguous()
-        wp = wp.contiguous()
-    temperature = _check_temperature(temperature)
-    n, H = h2.shape
-    V = wp.shape[0]
-    tg = _as_i32(targets, n, dev, "targets")
-    rv = _row_valid(lead, n, lengths, row_valid, dev)
-    with _on_device(dev):
-        outs = [torch.empty(n, dtype=torch.float32, device=dev) for _ in range(4)]
-        ws_bytes = lib.tome_grpo_dual_workspace(n, H, V)
-        ws = _workspace(ws_bytes, dev)
-        _lib.check(lib.tome_grpo_dual(h2.data_ptr(), wp.data_ptr(), wr.data_ptr(), n, H, V,
-                                      h2.stride(0) if n > 1 else H, wp.stride(0), tg.data_ptr(), _ptr(rv),
-                                      temperature, outs[0].data_ptr(), outs[1].data_ptr(), outs[2].data_ptr(),
-                                      outs[3].data_ptr(), _ptr(ws), ws_bytes, _stream(dev)))
-    return DualLogprobs(*(o.reshape(lead) for o in outs))
+    return DualLogprobs(*_lib.torch_ops().grpo_pair(
+        hidden, None, w_policy, w_ref, _tensor(targets, hidden), _check_temperature(temperature),
+        _tensor(lengths, hidden, False), _tensor(row_valid, hidden), None, 0.0, _stream(hidden)))
 
 
 def grpo_pair_logprobs(hidden_policy: torch.Tensor, hidden_ref: torch.Tensor, w_policy: torch.Tensor, targets,
@@ -437,36 +247,7 @@ def grpo_pair_logprobs(hidden_policy: torch.Tensor, hidden_ref: torch.Tensor, w_
     states and share the final norm and the lm_head (mlx-impl/model.py:536-538): ``w_ref``
     defaults to ``w_policy``.  ``norm_weight`` as in ``fused_lmhead_logprobs``, applied to both.
     """
-    lib = _lib.load_library()
-    ws_in = (w_policy,) if w_ref is None else (w_policy, w_ref)
-    dev, lead, h2, ws_ = _check_fused_inputs(hidden_policy, *ws_in)
-    _require_gpu(hidden_policy, hidden_ref)
-    if hidden_ref.dtype != torch.bfloat16 or hidden_ref.shape != hidden_policy.shape:
-        raise ValueError("hidden_ref must be bfloat16 with hidden_policy's shape")
-    r2 = _rows_view(hidden_ref)
-    wp = ws_[0]
-    wr = ws_[1] if w_ref is not None else wp
-    if wp.stride(0) != wr.stride(0):
-        wp, wr = wp.contiguous(), wr.contiguous()
-    n, H = h2.shape
-    if n > 1 and h2.stride(0) != r2.stride(0):
-        h2, r2 = h2.contiguous(), r2.contiguous()
-    temperature = _check_temperature(temperature)
-    V = wp.shape[0]
-    tg = _as_i32(targets, n, dev, "targets")
-    rv = _row_valid(lead, n, lengths, row_valid, dev)
-    nw = None
-    if norm_weight is not None:
-        _require_gpu(hidden_policy, norm_weight)
-        if norm_weight.dtype != torch.bfloat16 or norm_weight.shape != (H,):
-            raise ValueError(f"norm_weight must be bfloat16 [{H}]")
-        nw = norm_weight.contiguous()
-    with _on_device(dev):
-        outs = [torch.empty(n, dtype=torch.float32, device=dev) for _ in range(4)]
-        ws_bytes = lib.tome_grpo_pair_workspace(n, H, V, 1 if nw is not None else 0)
-        ws = _workspace(ws_bytes, dev)
-        _lib.check(lib.tome_grpo_pair(h2.data_ptr(), r2.data_ptr(), _ptr(nw), float(norm_eps), wp.data_ptr(),
-                                      wr.data_ptr(), n, H, V, h2.stride(0) if n > 1 else H, wp.stride(0),
-                                      tg.data_ptr(), _ptr(rv), temperature, outs[0].data_ptr(), outs[1].data_ptr(),
-                                      outs[2].data_ptr(), outs[3].data_ptr(), _ptr(ws), ws_bytes, _stream(dev)))
-    return DualLogprobs(*(o.reshape(lead) for o in outs))
+    return DualLogprobs(*_lib.torch_ops().grpo_pair(
+        hidden_policy, hidden_ref, w_policy, w_ref, _tensor(targets, hidden_policy), _check_temperature(temperature),
+        _tensor(lengths, hidden_policy, False), _tensor(row_valid, hidden_policy), norm_weight, float(norm_eps),
+        _stream(hidden_policy)))
