@@ -393,3 +393,29 @@ def test_full_log_softmax_at_every_phase(dev, dtype, rows, V, in_stride):
         assert (diff <= 0.125 + 1e-6).all() and (diff == 0).mean() > 0.99
         for edge in (diff[:, :8], diff[:, -8:]):
             assert (edge == 0).mean() > 0.95
+
+
+@pytest.mark.parametrize("dtype,rows,V", [(torch.float32, r, v) for r, v in (
+    (3, 16384), (3, 16391), (3, 32768), (20, 32772), (20, 53248), (530, 40003), (19, 53253), (28, 81920), (36, 81924), (36, 106496), (36, 106501),
+    (52, 151937), (41, 122880), (90, 262144), (530, 262151))] + [(torch.bfloat16, r, v) for r, v in (
+        (66, 155656), (70, 163841), (90, 212992), (90, 213001), (110, 262150))])
+def test_full_log_softmax_one_launch_at_the_edges_of_its_stores(dev, dtype, rows, V):
+    """Rows that fill exactly, and by one unit more, what a lane keeps in registers (8, 13, 20 or 17 units), in LDS (9 more) and
+    one turn of the second read (3 units), with single elements at either end.  Against float64 on the GPU: fp32 at 1e-4; bf16
+    at one output step (0.125 below 32) with more than 99 % equal to the oracle's rounding steps applied to the float64 lse."""
+    g = torch.Generator(device=dev).manual_seed(rows + V)
+    x = torch.empty((rows, V), dtype=dtype, device=dev).normal_(0.0, 2.0, generator=g)
+    x[rows // 2, V - 1] = 14.0
+    x[rows // 3, 0] = 14.0
+    T = 0.9
+    out = tome_amd.fused_log_softmax(x, T)
+    for r0 in range(0, rows, 32):
+        z = x[r0:r0 + 32].double() / T
+        lse = torch.logsumexp(z, -1, keepdim=True)
+        if dtype == torch.float32:
+            assert float((out[r0:r0 + 32].double() - (z - lse)).abs().max()) < TOL_F32
+        else:
+            zt = (x[r0:r0 + 32].float() * (1.0 / T)).to(dtype).float()
+            want = (zt - lse.to(dtype).float()).to(dtype).float()
+            diff = (out[r0:r0 + 32].float() - want).abs()
+            assert float(diff.max()) <= 0.125 + 1e-6 and float((diff == 0).float().mean()) > 0.99

@@ -25,7 +25,7 @@ hipError_t full_log_softmax_launch(const void* in, void* out, int dtype, int64_t
                                    int64_t in_stride, int64_t out_stride, float temperature,
                                    float* row_lse, const void* partials, int splits, hipStream_t stream);
 bool full_log_softmax_one_pass(int dtype, int64_t rows, int64_t V);
-hipError_t full_log_softmax_onepass_launch(const void* in, void* out, int64_t rows, int64_t V, int64_t in_stride,
+hipError_t full_log_softmax_onepass_launch(const void* in, void* out, int dtype, int64_t rows, int64_t V, int64_t in_stride,
                                            int64_t out_stride, float temperature, float* row_lse, hipStream_t stream);
 hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
                              const float* uniforms, const RowSel& sel, float temperature, int top_k,
@@ -254,7 +254,7 @@ int tome_full_log_softmax(const void* logits, void* out, int dtype, int64_t rows
   hipStream_t s = static_cast<hipStream_t>(stream);
   // bf16 rows that fit one workgroup's registers: read once, written once
   if (tome::full_log_softmax_one_pass(dtype, rows, V))
-    return hip_result(tome::full_log_softmax_onepass_launch(logits, out, rows, V, in_row_stride, out_row_stride, temperature,
+    return hip_result(tome::full_log_softmax_onepass_launch(logits, out, dtype, rows, V, in_row_stride, out_row_stride, temperature,
                                                             row_lse, s));
   // otherwise two passes: the rows' logsumexp (split rows leave their partials in the workspace), then the matrix
   int splits = 1;
