@@ -101,9 +101,9 @@ struct RowSel {
 };
 
 // ---- wave64 lane exchange --------------------------------------------------------------
-// Steps inside a 16-lane row use DPP (no LDS traffic); the two steps that cross rows go
-// through the LDS crossbar (ds_bpermute via __shfl_xor).  After steps 0..3 every lane of a
-// row holds that row's reduction, so the mirror patterns pair the right halves.
+// Steps inside a 16-lane row use DPP; the two steps that cross rows swap rows (halves) between two copies of the value
+// (v_permlane16_swap / v_permlane32_swap), so a reduction never leaves the VALU for the LDS crossbar.  After steps 0..3
+// every lane of a row holds that row's reduction, so the mirror patterns pair the right halves.
 template <int STEP>
 __device__ __forceinline__ float wave_exchange(float v) {
   if constexpr (STEP == 0) {  // quad_perm [1,0,3,2]
@@ -115,9 +115,13 @@ __device__ __forceinline__ float wave_exchange(float v) {
   } else if constexpr (STEP == 3) {  // row_mirror
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, true));
   } else if constexpr (STEP == 4) {
-    return __shfl_xor(v, 16, 64);
+    // rows 1 and 3 of the first copy change places with rows 0 and 2 of the second: [r0 r0 r2 r2], [r1 r1 r3 r3]
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float((threadIdx.x & 16) ? p[0] : p[1]);
   } else {
-    return __shfl_xor(v, 32, 64);
+    // the halves likewise: [lo lo], [hi hi]
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float((threadIdx.x & 32) ? p[0] : p[1]);
   }
 }
 template <int STEP>
