@@ -43,6 +43,31 @@ def test_row_matches_oracle(dev, dtype, rows, V, T):
     assert (r.lp.cpu().numpy() <= 1e-6).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,V", [(1, 24576), (24, 24577), (25, 24577), (9, 4099), (256, 8191), (257, 8200), (257, 33001), (511, 16391),
+                                    (512, 16391), (351, 33000)])
+def test_row_workgroup_sizes(dev, dtype, rows, V):
+    """Either side of every line between split rows and one workgroup of 4, 8 or 16 waves a row: all statistics, special
+    values among them, at the bar of the other fp32 sums; masked rows exit, ties keep the first maximum."""
+    rng = np.random.default_rng(rows * 7 + V)
+    x32 = (rng.standard_normal((rows, V)) * 3.0).astype(np.float32)
+    x32[0, V // 3] = x32[0, V - 1] = 40.0                                       # a tie across waves
+    x32[-1, 5::2] = -np.inf
+    t = rng.integers(0, V, size=rows).astype(np.int32)
+    valid = (rng.random(rows) < 0.8).astype(np.int32)
+    valid[[0, -1]] = 1
+    xt = torch.from_numpy(x32).to(dev).to(dtype)
+    r, x = _check(xt, t, 0.8, row_valid=torch.from_numpy(valid).to(dev))
+    on = valid != 0
+    lp, want = r.lp.cpu().numpy(), oracle.logprob_rows(x, t, 0.8)
+    fin = np.isfinite(want)
+    np.testing.assert_allclose(lp[on & fin], want[on & fin], atol=TOL_F32, rtol=0)
+    assert np.isneginf(lp[on & ~fin]).all() and (lp[~on] == 0).all()
+    np.testing.assert_allclose(r.lse.cpu().numpy()[on], oracle.lse_rows(x, 0.8)[on], atol=TOL_F32, rtol=0)
+    np.testing.assert_allclose(r.entropy.cpu().numpy()[on], oracle.entropy_rows(x, 0.8)[on], atol=TOL_F32, rtol=0)
+    np.testing.assert_array_equal(r.argmax.cpu().numpy(), np.where(on, oracle.argmax_rows(x), -1))
+
+
 def test_row_strided_and_misaligned_views(dev):
     """Row slices of a [B, L, V] tensor (node.py:449) and views that break 16-byte alignment."""
     rng = np.random.default_rng(5)

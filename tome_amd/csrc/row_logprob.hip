@@ -5,9 +5,9 @@
 // reference reads each row three times and writes a full [rows, V] matrix; here each
 // element is read from HBM once with 16-byte loads and only per-row scalars are written.
 //
-// Grid: rows * splits workgroups of 256 lanes (4 wave64).  A workgroup owns a contiguous
+// Grid: rows * splits workgroups of 4 wave64, or rows workgroups of 8 or 16 (row_waves_unsplit).  A workgroup owns a contiguous
 // range of 16-byte load units of one row (RowSpan: units start at the row's first 16-byte boundary), every lane keeps an online (max, sum 2^(y-m))
-// pair over the units it reads, lanes are merged by DPP / LDS-crossbar exchanges, the four
+// pair over the units it reads, lanes are merged by DPP and row swaps, the
 // waves through LDS.  splits == 1 finishes in the same launch; otherwise per-split
 // partials go to the workspace and row_combine_kernel merges them (no float atomics, so
 // results do not depend on scheduling).
@@ -75,10 +75,11 @@ __device__ __forceinline__ void finish_row(const RowArgs& a, const T* row, int64
 
 // KEEP: the caller reads the rows again right away (the second pass of the full log-softmax matrix), so they are
 // loaded with ordinary loads and stay in the caches; everyone else streams them past the caches.
-template <typename T, bool ENT, bool AMAX, bool KEEP = false>
-__global__ __launch_bounds__(kRowWG) void row_logprob_kernel(RowArgs a) {
+template <typename T, bool ENT, bool AMAX, bool KEEP, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void row_logprob_kernel(RowArgs a) {
   constexpr int kVec = Elem<T>::kVec;
-  __shared__ RowLds lds;
+  constexpr int kWG = WAVES * 64;
+  __shared__ RowLdsT<WAVES> lds;
   const int64_t r = blockIdx.x / a.splits;  // problem index
   const int split = blockIdx.x % a.splits;
   const int tid = threadIdx.x;
@@ -118,28 +119,28 @@ __global__ __launch_bounds__(kRowWG) void row_logprob_kernel(RowArgs a) {
   }
   const u32x4* p = sp.p;
   int64_t u = u0 + tid;
-  for (; u + (kRowUnroll - 1) * kRowWG < u1; u += kRowUnroll * kRowWG) {  // several 16-byte loads in flight per lane
+  for (; u + (kRowUnroll - 1) * kWG < u1; u += kRowUnroll * kWG) {  // several 16-byte loads in flight per lane
     u32x4 v[kRowUnroll];
 #pragma unroll
-    for (int k = 0; k < kRowUnroll; ++k) v[k] = KEEP ? p[u + k * kRowWG] : __builtin_nontemporal_load(p + u + k * kRowWG);
+    for (int k = 0; k < kRowUnroll; ++k) v[k] = KEEP ? p[u + k * kWG] : __builtin_nontemporal_load(p + u + k * kWG);
 #pragma unroll
     for (int k = 0; k < kRowUnroll; ++k) {
       float x[kVec];
       Elem<T>::unpack(v[k], x);
-      absorb<kVec, ENT, AMAX>(st, x, sp.head + (int)(u + k * kRowWG), a.scale);
+      absorb<kVec, ENT, AMAX>(st, x, sp.head + (int)(u + k * kWG), a.scale);
     }
   }
   {  // leftover units of this lane, issued together so their latencies overlap
     u32x4 v[kRowUnroll - 1];
 #pragma unroll
     for (int k = 0; k < kRowUnroll - 1; ++k)
-      if (u + k * kRowWG < u1) v[k] = KEEP ? p[u + k * kRowWG] : __builtin_nontemporal_load(p + u + k * kRowWG);
+      if (u + k * kWG < u1) v[k] = KEEP ? p[u + k * kWG] : __builtin_nontemporal_load(p + u + k * kWG);
 #pragma unroll
     for (int k = 0; k < kRowUnroll - 1; ++k)
-      if (u + k * kRowWG < u1) {
+      if (u + k * kWG < u1) {
         float x[kVec];
         Elem<T>::unpack(v[k], x);
-        absorb<kVec, ENT, AMAX>(st, x, sp.head + (int)(u + k * kRowWG), a.scale);
+        absorb<kVec, ENT, AMAX>(st, x, sp.head + (int)(u + k * kWG), a.scale);
       }
   }
   if (split == a.splits - 1 && tid < sp.tail) {  // ... and after the last one
@@ -175,10 +176,10 @@ __global__ __launch_bounds__(64) void row_combine_kernel(RowArgs a) {
   finish_row<T, ENT, AMAX>(a, row, r, st, x_t);
 }
 
-template <typename T, bool ENT, bool AMAX, bool KEEP = false>
+template <typename T, bool ENT, bool AMAX, bool KEEP, int WAVES>
 static hipError_t launch_row(const RowArgs& a, int64_t rows, hipStream_t stream, bool skip_combine = false) {
-  hipLaunchKernelGGL((row_logprob_kernel<T, ENT, AMAX, KEEP>), dim3((unsigned)(rows * a.splits)),
-                     dim3(kRowWG), 0, stream, a);
+  hipLaunchKernelGGL((row_logprob_kernel<T, ENT, AMAX, KEEP, WAVES>), dim3((unsigned)(rows * a.splits)),
+                     dim3(WAVES * 64), 0, stream, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.splits == 1 || skip_combine) return e;
   hipLaunchKernelGGL((row_combine_kernel<T, ENT, AMAX>), dim3((unsigned)rows), dim3(64), 0,
@@ -186,16 +187,23 @@ static hipError_t launch_row(const RowArgs& a, int64_t rows, hipStream_t stream,
   return hipGetLastError();
 }
 
-template <typename T>
-static hipError_t dispatch_flags(const RowArgs& a, int64_t rows, hipStream_t stream) {
-  const bool ent = a.out_entropy != nullptr, amax = a.out_argmax != nullptr;
-  if (ent && amax) return launch_row<T, true, true>(a, rows, stream);
-  if (ent) return launch_row<T, true, false>(a, rows, stream);
-  if (amax) return launch_row<T, false, true>(a, rows, stream);
-  return launch_row<T, false, false>(a, rows, stream);
+template <typename T, bool ENT, bool AMAX>
+static hipError_t launch_waves(const RowArgs& a, int64_t rows, int waves, hipStream_t stream) {
+  if (waves == 16) return launch_row<T, ENT, AMAX, false, 16>(a, rows, stream);
+  if (waves == 8) return launch_row<T, ENT, AMAX, false, 8>(a, rows, stream);
+  return launch_row<T, ENT, AMAX, false, kRowWaves>(a, rows, stream);
 }
 
-// How many workgroups share a row.  From 512 rows on one workgroup per row; smaller batches (decode steps,
+template <typename T>
+static hipError_t dispatch_flags(const RowArgs& a, int64_t rows, int waves, hipStream_t stream) {
+  const bool ent = a.out_entropy != nullptr, amax = a.out_argmax != nullptr;
+  if (ent && amax) return launch_waves<T, true, true>(a, rows, waves, stream);
+  if (ent) return launch_waves<T, true, false>(a, rows, waves, stream);
+  if (amax) return launch_waves<T, false, true>(a, rows, waves, stream);
+  return launch_waves<T, false, false>(a, rows, waves, stream);
+}
+
+// How many workgroups share a row, where rows are split (and the bound the workspace is sized for).  From 512 rows on one workgroup per row; smaller batches (decode steps,
 // the 64-row CPU-comparison case) are split so that ~2 workgroups per CU are in flight, as long as every
 // split keeps a few loads per lane.  Measured: aiming at 512 to 2048 workgroups is equal within 0.5 us for
 // 32-256 rows, and 512 spares the 512- and 1024-row batches the combine launch (27.0 against 30.6 us,
@@ -212,6 +220,26 @@ int row_splits_for(int64_t rows, int64_t V, int vec) {
   if (s > 64) s = 64;
   if (s < 1) s = 1;
   return (int)s;
+}
+
+// Workgroup size for a launch of `rows` rows, 0 = split the rows as above.  Splitting a row costs a second launch (2-3 us,
+// as much as a decode-sized call's loads); a workgroup of 8 or 16 waves keeps enough loads of ONE row in flight that between
+// about a row per thousand elements and 512 rows the single launch is the faster one, and always for rows of up to 24576
+// elements.  Inside a captured graph, split / 16 waves a row (us): 64 x 32000 fp32 8.4 / 6.5, 128 x 32000 9.6 / 6.9, 200 x
+// 100000 18.7 / 15.6, 200 x 151936 bf16 16.5 / 13.8; on the other side of the line 48 x 65536 8.6 / 8.9, 64 x 100000 9.8 /
+// 11.9, 64 x 151936 12.0 / 16.1, 96 x 151936 bf16 11.6 / 12.9.  A little above one row per CU, long rows are dealt out more
+// evenly in halves (300 x 151936: fp32 34.5 / 37.0, bf16 21.1 / 22.0; 393 rows 45.3 / 40.5 and 27.4 / 23.7).
+// Above one row per CU 8 waves are as fast as 16 or faster (393 x 50257 bf16, all statistics: 4 / 8 / 16 waves 14.2 / 12.9 /
+// 13.7); short rows do not fill more waves (4096 elements: 300 rows 4.4 / 5.2 / 6.3, 64 rows 8 / 16 waves 4.0 / 4.4).
+static int row_waves_unsplit(int64_t rows, int64_t V, int vec) {
+  const int64_t units = V / vec;
+  if (rows >= 512 || units < 4 * kRowWG) return row_splits_for(rows, V, vec) == 1 ? kRowWaves : 0;
+  if (rows > 256) {
+    if (rows < 352 && V > 98304) return 0;
+    return units < 16 * kRowWG ? kRowWaves : 8;
+  }
+  if (V > 24576 && rows * 1000 < V) return 0;
+  return units < 12 * kRowWG ? 8 : 16;
 }
 
 // `rows` problems.  With `row_index` (device, one entry per problem) problem i reads row row_index[i] of a matrix
@@ -233,9 +261,10 @@ hipError_t row_logprob_launch_rows(const void* logits, int dtype, int64_t n_rows
   a.partials = static_cast<RowPartial*>(workspace);
   a.V = V;
   a.row_stride = row_stride;
-  a.splits = row_splits_for(rows, V, vec);
+  const int waves = row_waves_unsplit(rows, V, vec);
+  a.splits = waves ? 1 : row_splits_for(rows, V, vec);
   a.scale = kLog2e / temperature;
-  return dtype == 0 ? dispatch_flags<float>(a, rows, stream) : dispatch_flags<uint16_t>(a, rows, stream);
+  return dtype == 0 ? dispatch_flags<float>(a, rows, waves, stream) : dispatch_flags<uint16_t>(a, rows, waves, stream);
 }
 
 // The rows' logsumexp for a caller that merges split rows itself: only the main kernel is launched.  With
@@ -259,8 +288,10 @@ hipError_t row_lse_partials_launch(const void* logits, int dtype, int64_t rows, 
   // passes, fp32 rows of 151936: 64 rows 25.9 -> 24.4 us, 512 rows 155 -> 145, 1024 rows 312 -> 294; 2048 rows 628 -> 648).
   const bool keep = (double)rows * (double)V * esize <= 768.0 * 1024 * 1024;
   if (dtype == 0)
-    return keep ? launch_row<float, false, false, true>(a, rows, stream, true) : launch_row<float, false, false>(a, rows, stream, true);
-  return keep ? launch_row<uint16_t, false, false, true>(a, rows, stream, true) : launch_row<uint16_t, false, false>(a, rows, stream, true);
+    return keep ? launch_row<float, false, false, true, kRowWaves>(a, rows, stream, true)
+                : launch_row<float, false, false, false, kRowWaves>(a, rows, stream, true);
+  return keep ? launch_row<uint16_t, false, false, true, kRowWaves>(a, rows, stream, true)
+              : launch_row<uint16_t, false, false, false, kRowWaves>(a, rows, stream, true);
 }
 
 hipError_t row_logprob_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
