@@ -160,7 +160,8 @@ size_t tome_row_logprob_noalloc_limit(size_t bytes);
  *   out_argmax   first maximum of the row;  out_topk_idx / out_topk_logit  [rows, top_k], the
  *                candidates themselves (-1 / 0 past the end of a row with fewer finite logits)
  * Masked rows give token -1.  Small batches split each row over several workgroups and need
- * the workspace that tome_row_sample_workspace() sizes (0 for large batches).
+ * the workspace that tome_row_sample_workspace() sizes (0 for large fp32 batches; large bf16 batches
+ * run without one too, more slowly).
  */
 size_t tome_row_sample_workspace(int dtype, int64_t rows, int64_t V, int top_k);
 int tome_row_sample(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,

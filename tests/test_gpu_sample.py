@@ -52,6 +52,49 @@ def test_sampler_matches_oracle(dev, rows, V, dtype, T, k):
     np.testing.assert_allclose(got.lp.cpu().numpy(), lp2.cpu().numpy(), atol=2e-6, rtol=0)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,V,k,kind", [
+    (3, 8192, 20, "normal"), (3, 8197, 32, "normal"), (2, 16384, 20, "normal"), (2, 32771, 1, "normal"), (1, 270001, 20, "normal"),
+    (1, 600001, 32, "normal"), (2, 20011, 20, "equal"), (2, 20011, 20, "few_values"), (2, 20011, 32, "one_cell"), (2, 50000, 20, "one_lane"),
+    (2, 20011, 20, "edges"), (2, 20011, 20, "sparse"), (2, 300001, 20, "equal"),
+])
+def test_sampler_cells(dev, dtype, rows, V, k, kind):
+    """The decode form at the sizes and orderings where it can go wrong: rows of one block of cells and one element more, more
+    cells than a lane keeps and more blocks than workgroups a row, many equal logits (the lowest ids win), all large ones in
+    one 128-byte cell or in one lane's cells, in the single elements at a row's ends, and fewer than k above -inf.  Ids and
+    candidates are exact, log-probs to 1e-4 as everywhere."""
+    rng = np.random.default_rng(V + k)
+    x = rng.standard_normal((rows, V)).astype(np.float32)
+    if kind == "equal":
+        x[:] = 1.5
+    elif kind == "few_values":
+        x = np.round(x).astype(np.float32)
+    elif kind == "one_cell":
+        x[:, 6400:6432] += 20.0
+    elif kind == "one_lane":
+        x[:, 32 * 77::32 * 256] += 20.0
+        x[:, 32 * 77 + 5::32 * 256] += 30.0
+    elif kind == "edges":
+        x[:, :6] += 20.0
+        x[:, -6:] += 20.0
+    elif kind == "sparse":
+        keep = x[:, [3, 9000, V - 1]].copy()
+        x[:] = -np.inf
+        x[:, [3, 9000, V - 1]] = keep
+    wide = torch.full((rows, V + 3), 99.0, dtype=dtype, device=dev)               # rows at changing phases, large values around them
+    wide[:, 1:V + 1] = torch.from_numpy(x).to(dev)
+    xt = wide[:, 1:V + 1]
+    x64 = xt.float().cpu().numpy().astype(np.float64)
+    us = _safe_uniforms(x64, 0.9, k, rng) if kind != "sparse" else np.full(rows, 0.01, np.float32)
+    got = tome_amd.sample_tokens(xt, 0.9, k, uniforms=torch.from_numpy(us).to(dev), want_topk=True)
+    want_idx, want_val = oracle.top_k_rows(x64, k)
+    np.testing.assert_array_equal(got.topk_idx.cpu().numpy(), want_idx)
+    np.testing.assert_array_equal(got.topk_logit.cpu().numpy()[want_idx >= 0], want_val[want_idx >= 0].astype(np.float32))
+    want_tok, want_lp = oracle.sample_top_k(x64, us, 0.9, k)
+    np.testing.assert_array_equal(got.token.cpu().numpy(), want_tok)
+    np.testing.assert_allclose(got.lp.cpu().numpy(), want_lp, atol=1e-4, rtol=0)
+
+
 @pytest.mark.parametrize("rows,V,dtype", [(2300, 65536, torch.float32), (1700, 32768, torch.bfloat16)])
 def test_sampler_streams_large_batches(dev, rows, V, dtype):
     """Batches beyond ~950 fp32 / ~340 bf16 rows of 151936 (counted in ranges of 8192 elements) take one streaming

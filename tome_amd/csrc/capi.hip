@@ -32,6 +32,7 @@ hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_
                              int32_t* out_token, float* out_lp, float* out_lse, int32_t* out_argmax,
                              int32_t* out_topk_idx, float* out_topk_logit, void* workspace, hipStream_t stream);
 size_t row_sample_workspace_bytes(int64_t rows, int64_t V, int dtype_vec, int top_k);
+bool row_sample_needs_workspace(int64_t rows, int64_t V, int vec);
 size_t fused_workspace_bytes(int64_t n_tokens, int64_t H, int64_t V, int n_weights, bool with_norm);
 bool fused_needs_32bit_extents(int64_t n_tokens, int64_t H, int64_t V);
 void fused_force_kernel(int kind);
@@ -443,8 +444,8 @@ int sample_checked(const void* logits, int dtype, int64_t rows, int64_t V, int64
   if (bad_temperature(temperature)) return TOME_E_TEMPERATURE;
   if (rows == 0) return TOME_OK;
   if (!logits || !out_token) return TOME_E_NULL;
-  const size_t need = tome_row_sample_workspace(dtype, rows, V, top_k);
-  if (need > 0 && (!workspace || workspace_bytes < need)) return TOME_E_WORKSPACE;
+  if (workspace_bytes < tome_row_sample_workspace(dtype, rows, V, top_k)) workspace = nullptr;
+  if (!workspace && tome::row_sample_needs_workspace(rows, V, dtype == TOME_F32 ? 4 : 8)) return TOME_E_WORKSPACE;
   if (reinterpret_cast<uintptr_t>(logits) % (dtype == TOME_F32 ? 4 : 2) != 0) return TOME_E_ALIGN;
   return hip_result(tome::row_sample_launch(logits, dtype, rows, V, row_stride, uniforms, sel, temperature,
                                             top_k, out_token, out_lp, out_lse, out_argmax, out_topk_idx,

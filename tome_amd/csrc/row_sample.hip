@@ -13,27 +13,43 @@
 //
 // Rows may start at any element (RowSpan): 1024 rows of 128258 fp32 / bf16 303 / 445 us on element-wise loads, 94 / 72 us here.
 //
-// A row is shared by `splits` workgroups (decode batches are a few dozen rows: one workgroup per row
-// would leave most of the chip idle).  Each computes, over its range of the row,
+// Two forms.
+//
+// Decode batches (row_sample_cells_kernel + row_sample_pick_kernel): the first launch streams the rows from as many
+// workgroups as fill the chip and leaves, besides the partial (max, sum 2^(y-m)), the maximum of every CELL of 8 consecutive
+// load units (128 bytes: a cache line).  The second, a workgroup per row, takes the k best cells by (maximum, lower cell
+// first) and reads only those again: as cells lie in the order of the ids, they hold the row's top k - were a top-k element
+// in another cell, each of the k better cells would hold an element that precedes it.  Nothing but a maximum per lane
+// and load unit is then paid per element, and the selection is done once a row instead of once a range (the form before:
+// every workgroup ranked the candidates of its range, a second launch merged splits * k keys).
+// Two launches either way; 64 x 151936 fp32 20.2 -> 15 us (7 streaming, 7 picking), 8 rows 14.6 -> 10, 64 x 50257 25 -> 11; bf16 64 x 151936
+// 20.4 -> 13, 256 rows 40 -> 23, 700 rows 67 -> 47, 1024 x 50257 172 -> 31.  The streaming launch runs at the rate of the
+// memory (38.9 MB in 6.5 us); the other one is a chain of some 12000 cycles: kernel arguments and first loads 1500, cell maxima 1700,
+// the bound 1500, cells collected 1800, partial statistics 1200 (beside the elements' load), elements 1000, ranks 1100, draw 1000.
+//
+// Large batches (row_sample_kernel, one workgroup a row, no workspace): per row,
 //   * the online (max, sum 2^(y-m)) for the full-vocabulary lse and every lane's own largest element;
 //   * a lower bound `theta` of the k-th largest logit: the k-th largest of the lane maxima (four waves,
 //     each extracting its ceil(k/4) largest);
 //   * every element >= theta, as a candidate in an LDS buffer (typically k + a few entries).
-// Short ranges (a lane owns <= 8 load units) are loaded once and kept in registers for the candidate
-// scan.  Long ranges are streamed once: theta comes from the lanes' first units, is renewed after a
-// quarter of the range, and candidates are collected as the row goes by; only when the buffer overflows
-// is the range scanned a second time with the bound from all of it.
+// Short rows (a lane owns <= 8 load units) are loaded once and kept in registers for the candidate
+// scan.  Long rows are streamed once: theta comes from the lanes' first units, is renewed after a
+// quarter of the row, and candidates are collected as the row goes by; only when the buffer overflows
+// is the row scanned a second time with the bound from all of it.
 // Candidates are 64-bit keys (order-preserving image of the float, then ~index), so there are no
-// ties and "the top k" is unique.  A buffer overflow (adversarial orderings only) raises theta to
-// the k-th largest of what was kept - still a lower bound - and rescans.  The final k are ranked by
-// counting.  With splits > 1 every workgroup leaves its k keys and its (max, sum) in the workspace
-// and row_sample_combine_kernel selects among the splits * k keys and draws.
+// ties and the top k is unique.  If a buffer overflows (adversarial orderings), theta is raised to
+// the k-th largest of what was kept - still a lower bound - and the scan is repeated.  The final k are ranked by
+// counting.
 #include "row_common.hpp"
+#include <type_traits>
 
 namespace tome {
 
 constexpr int kSampCap = 1024;      // candidate keys per buffer in the main kernel (2 x 8 KB of LDS: 8 workgroups per CU)
-constexpr int kSampMergeCap = 2048; // in the combine kernel: up to 64 splits x 32 keys
+constexpr int kCellUnits = 8;       // load units per cell: consecutive, one 128-byte line
+constexpr int kCellBlock = kCellUnits * kRowWG;  // load units a workgroup of the cells kernel takes at a time (256 cells)
+// Keys per buffer of the pick kernel: k <= 32 cells of 8 units of up to 8 elements, and the single elements of the edges.
+constexpr int kSampPickCap = 32 * kCellUnits * 8 + 64;
 constexpr int kSampCached = 8;      // a lane keeps up to this many load units in registers between the passes
 constexpr int kSampMaxK = 32;  // one tightening round is then sure to drop >= 32 of the 64 sampled keys
 
@@ -47,12 +63,14 @@ struct SampleArgs {
   int32_t* out_argmax;        // nullable
   int32_t* out_topk_idx;      // nullable, [rows, top_k], -1 past the end of a short row
   float* out_topk_logit;      // nullable, [rows, top_k] raw logits
-  uint64_t* part_keys;        // workspace: [rows, splits, top_k] (splits > 1)
-  float2* part_stat;          // workspace: [rows, splits] (max, sum)
+  float* cells;               // workspace: [rows, n_cells] cell maxima (splits > 0)
+  float2* part_stat;          // workspace: [rows, splits * kRowWaves] (max, sum)
   int64_t V;
   int64_t row_stride;
   int top_k;
-  int splits;
+  int splits;                 // workgroups per row of the cells kernel
+  int blocks_per_split;
+  int64_t n_cells;            // a multiple of 256
   float scale;                // log2(e) / temperature
 };
 
@@ -76,25 +94,9 @@ struct SampleLds {
   uint64_t top[kSampMaxK];
   uint64_t thr4[kRowWaves];
   int cnt;
+  int cnt2;
   int wave_cnt[kRowWaves];
   RowLds red;
-};
-
-// Wave-cooperative collection without atomics: every wave owns a quarter of a key buffer and a running count that is
-// the same in all its lanes; the lanes that pass take consecutive slots by their position among the passing lanes.
-// An LDS atomic that returns the slot costs a round trip per candidate, and those trips queue up behind each other.
-struct WaveCollector {
-  uint64_t* region;
-  int cap;
-  int count;  // wave-uniform; keeps counting past `cap` (overflow is detected from it), nothing is stored there
-  // Must be reached by all lanes of the wave together.
-  __device__ __forceinline__ void offer(bool pass, uint64_t key) {
-    const uint64_t b = __ballot(pass);
-    if (b == 0) return;
-    const int pos = count + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
-    if (pass && pos < cap) region[pos] = key;
-    count += __builtin_popcountll(b);
-  }
 };
 
 // Keys of four wave regions (counts c[w], region w starting at base + w * stride) as one list: entry i.
@@ -114,10 +116,12 @@ __device__ __forceinline__ uint64_t region_entry(const uint64_t* base, int strid
 __device__ __forceinline__ uint64_t wave_sorted_top_k(uint64_t key, int m, int k) {
   const uint32_t lo = (uint32_t)key, hi = (uint32_t)(key >> 32);
   int rank = 0;
-  for (int j = 0; j < m; ++j) {
-    const uint64_t o = ((uint64_t)__builtin_amdgcn_readlane(hi, j) << 32) | (uint32_t)__builtin_amdgcn_readlane(lo, j);
-    rank += o > key ? 1 : 0;
-  }
+  for (int j0 = 0; j0 < m; j0 += 8)  // (lanes from m on hold 0: counted by nobody)
+#pragma unroll
+    for (int j = j0; j < j0 + 8; ++j) {
+      const uint64_t o = ((uint64_t)__builtin_amdgcn_readlane(hi, j) << 32) | (uint32_t)__builtin_amdgcn_readlane(lo, j);
+      rank += o > key ? 1 : 0;
+    }
   const bool keep = key != 0 && rank < k;           // k <= kSampMaxK = 32: lane 63 is never a destination
   const int dst = (keep ? rank : 63) * 4;
   const uint32_t slo = (uint32_t)__builtin_amdgcn_ds_permute(dst, (int)(keep ? lo : 0u));
@@ -188,6 +192,21 @@ __device__ uint64_t select_top_k(Lds& sh, uint64_t* cur, uint64_t* other, int m,
   return sh.top[k - 1];
 }
 
+// Maximum of a value over the wave, as a uniform value: six v_max_f32 with DPP sources towards lane 63 (lanes without a source
+// keep theirs; each DPP read of a register just written waits two slots).  All lanes of the wave must call it.
+__device__ __forceinline__ float wave_max_uniform(float v) {
+  asm volatile(
+      "s_nop 1\n"
+      "v_max_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n s_nop 1\n"
+      "v_max_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n s_nop 1\n"
+      "v_max_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n s_nop 1\n"
+      "v_max_f32_dpp %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n s_nop 1\n"
+      "v_max_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n s_nop 1\n"
+      "v_max_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n s_nop 1"
+      : "+v"(v));
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), 63));
+}
+
 // Lower bound of the k-th largest element of this workgroup's range from the lanes' own maxima (-inf
 // for a lane that saw nothing): each wave extracts its ceil(k/4) largest lane maxima one by one (a
 // wave-wide max, then the first lane that holds it steps aside), and the smallest of the four results
@@ -198,13 +217,7 @@ __device__ uint64_t bound_from_lane_maxima(Lds& sh, float lane_max, int k) {
   const int want = (k + kRowWaves - 1) / kRowWaves;
   float v = lane_max, kth = -INFINITY;
   for (int t = 0; t < want; ++t) {
-    float m = v;  // wave-wide maximum: four DPP steps inside the rows, two exchanges across them
-    m = fmaxf(m, wave_exchange<0>(m));
-    m = fmaxf(m, wave_exchange<1>(m));
-    m = fmaxf(m, wave_exchange<2>(m));
-    m = fmaxf(m, wave_exchange<3>(m));
-    m = fmaxf(m, wave_exchange<4>(m));
-    m = fmaxf(m, wave_exchange<5>(m));
+    const float m = wave_max_uniform(v);
     kth = m;
     const uint64_t holders = __ballot(v == m);
     if (holders == 0) break;  // cannot happen (lane maxima are never NaN); guards the ctz below
@@ -221,26 +234,31 @@ __device__ uint64_t bound_from_lane_maxima(Lds& sh, float lane_max, int k) {
 
 // Wave 0: draw among the sorted candidates (lane i < k holds the (i+1)-th largest key, 0 = none) and write the
 // row's outputs.  `tot` holds the full-vocabulary (max, sum) in every lane.
-__device__ __forceinline__ void finish_sample(const SampleArgs& a, uint64_t key, int64_t r, const RowStat& tot, int lane) {
+__device__ __forceinline__ float read_lane(float v, int i) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), i));
+}
+__device__ __forceinline__ void finish_sample(const SampleArgs& a, uint64_t key, int64_t r, const RowStat& tot, int lane, float uniform) {
   const int k = a.top_k;
   const bool have = key != 0;
   const float x = have ? key_float((uint32_t)(key >> 32)) : -INFINITY;
   const int n_have = __builtin_popcountll(__ballot(have));
-  const float x0 = __shfl(x, 0, 64);
-  float cdf = have ? fast_exp2((x - x0) * a.scale) : 0.f;  // inclusive scan below
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const float up = __shfl_up(cdf, off, 64);
-    if (lane >= off) cdf += up;
-  }
+  const float x0 = read_lane(x, 0);
+  // Inclusive scan over the first 32 lanes (k <= kSampMaxK), without leaving the VALU: inside the 16-lane rows, then the first
+  // row's total to the second.
+  float cdf = have ? fast_exp2((x - x0) * a.scale) : 0.f;
+  cdf += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(cdf), 0x111, 0xF, 0xF, true));  // row_shr:1
+  cdf += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(cdf), 0x112, 0xF, 0xF, true));
+  cdf += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(cdf), 0x114, 0xF, 0xF, true));
+  cdf += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(cdf), 0x118, 0xF, 0xF, true));
+  cdf += lane >= 16 ? read_lane(cdf, 15) : 0.f;
   int chosen = 0;
   if (a.uniforms && n_have > 0) {
-    const float total = __shfl(cdf, n_have - 1, 64);
-    const float target = a.uniforms[r] * total;
+    const float target = uniform * read_lane(cdf, n_have - 1);
     chosen = __builtin_popcountll(__ballot(have && cdf <= target));
     chosen = chosen < n_have ? chosen : n_have - 1;
   }
-  const uint64_t ckey = __shfl(key, chosen, 64);
+  const float cx = read_lane(x, chosen);
+  const int32_t cidx = (int32_t)__builtin_amdgcn_readlane((int)key_index(key), chosen);
   if (a.out_topk_idx && lane < k) a.out_topk_idx[r * k + lane] = have ? (int32_t)key_index(key) : -1;
   if (a.out_topk_logit && lane < k) a.out_topk_logit[r * k + lane] = have ? x : 0.f;
   if (lane != 0) return;
@@ -251,47 +269,48 @@ __device__ __forceinline__ void finish_sample(const SampleArgs& a, uint64_t key,
     if (a.out_lp) a.out_lp[r] = __builtin_nanf("");
     if (a.out_argmax) a.out_argmax[r] = 0;
   } else {
-    a.out_token[r] = (int32_t)key_index(ckey);
-    if (a.out_lp) a.out_lp[r] = (fmaf(key_float((uint32_t)(ckey >> 32)), a.scale, -m2) - log2s) * kLn2;
+    a.out_token[r] = cidx;
+    if (a.out_lp) a.out_lp[r] = (fmaf(cx, a.scale, -m2) - log2s) * kLn2;
     if (a.out_argmax) a.out_argmax[r] = (int32_t)key_index(key);
   }
   if (a.out_lse) a.out_lse[r] = (m2 + log2s) * kLn2;
 }
 
-// CACHED: the host promises that a lane owns at most kSampCached load units (short ranges: decode
-// batches split over many workgroups); they are loaded once and both passes run from registers.
+// A masked row: not read.
+__device__ __forceinline__ void masked_sample(const SampleArgs& a, int64_t r, int tid) {
+  if (tid == 0) {
+    a.out_token[r] = -1;
+    if (a.out_lp) a.out_lp[r] = 0.f;
+    if (a.out_lse) a.out_lse[r] = 0.f;
+    if (a.out_argmax) a.out_argmax[r] = -1;
+  }
+  if (tid < a.top_k) {
+    if (a.out_topk_idx) a.out_topk_idx[r * a.top_k + tid] = -1;
+    if (a.out_topk_logit) a.out_topk_logit[r * a.top_k + tid] = 0.f;
+  }
+}
+
+// CACHED: the host promises that a lane owns at most kSampCached load units (short rows); they are loaded
+// once and both passes run from registers.
 template <typename T, bool CACHED>
 __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) void row_sample_kernel(SampleArgs a) {
   constexpr int kVec = Elem<T>::kVec;
   __shared__ SampleLds<kSampCap> sh;
-  const int64_t r = blockIdx.x / a.splits;
-  const int split = blockIdx.x % a.splits;
+  const int64_t r = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int k = a.top_k;
 
-  if (!a.sel.valid(r)) {  // masked row: not read
-    if (split != 0) return;
-    if (tid == 0) {
-      a.out_token[r] = -1;
-      if (a.out_lp) a.out_lp[r] = 0.f;
-      if (a.out_lse) a.out_lse[r] = 0.f;
-      if (a.out_argmax) a.out_argmax[r] = -1;
-    }
-    if (tid < k) {
-      if (a.out_topk_idx) a.out_topk_idx[r * k + tid] = -1;
-      if (a.out_topk_logit) a.out_topk_logit[r * k + tid] = 0.f;
-    }
+  if (!a.sel.valid(r)) {
+    masked_sample(a, r, tid);
     return;
   }
 
   const T* row = static_cast<const T*>(a.logits) + r * a.row_stride;
   const RowSpan<T> sp(row, a.V);
-  const int64_t per_split = (sp.n_units + a.splits - 1) / a.splits;
-  const int64_t u0 = per_split * split;
-  const int64_t u1 = (u0 + per_split < sp.n_units) ? u0 + per_split : sp.n_units;
-  // single elements in front of the first whole unit (first split) and after the last one (last split), one per lane
-  const int n_head = split == 0 ? sp.head : 0;
-  const int n_tail = split == a.splits - 1 ? sp.tail : 0;
+  const int64_t u0 = 0, u1 = sp.n_units;
+  // single elements in front of the first whole unit and after the last one, one per lane
+  const int n_head = sp.head;
+  const int n_tail = sp.tail;
 
   const bool big_range = (u1 - u0) * kVec + n_head + n_tail > kSampCap;
   if (tid == 0) sh.cnt = 0;  // published by the first barrier below, before any candidate is offered
@@ -550,120 +569,384 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
     sorted = lane < k ? sh.top[lane] : 0;
   }
 
-  // ---- wave 0: the row's outputs, or this range's record for the combine kernel -----------------------
-  if (a.splits == 1) {
-    finish_sample(a, sorted, r, tot, lane);
-  } else {
-    const int64_t slot = r * a.splits + split;
-    if (lane < k) a.part_keys[slot * k + lane] = sorted;
-    if (lane == 0) a.part_stat[slot] = float2{tot.mx, tot.s};
-  }
+  finish_sample(a, sorted, r, tot, lane, a.uniforms ? a.uniforms[r] : 0.f);  // wave 0
 }
 
-// splits > 1: one workgroup per row merges the splits' candidates and statistics and draws.
-__global__ __launch_bounds__(kRowWG) void row_sample_combine_kernel(SampleArgs a) {
-  __shared__ SampleLds<kSampMergeCap> sh;
-  const int64_t r = blockIdx.x;
-  if (!a.sel.valid(r)) return;  // outputs already written by the main kernel
+// First launch of the decode form: partial statistics and cell maxima of one row's blocks [b0, b1).  Edge elements (RowSpan's
+// head and tail) are left to the second launch.
+template <typename T>
+__global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) void row_sample_cells_kernel(SampleArgs a) {
+  constexpr int kVec = Elem<T>::kVec;
+  const int64_t r = blockIdx.x / a.splits;
+  const int split = blockIdx.x % a.splits;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int k = a.top_k, m = a.splits * k;         // <= 64 * 32 = kSampMergeCap
-  const uint64_t* keys = a.part_keys + r * m;      // per split: its k keys in descending order, 0 past the end
-  // Every key is fetched once, up front and together with the statistics and the heads for the bound: the kernel then
-  // waits for global memory one time (the previous launch wrote these bytes on other dies, so each wait is a trip
-  // beyond the L2).
-  constexpr int kPer = kSampMergeCap / kRowWG;
-  constexpr int kWaveCap = kSampMergeCap / kRowWaves;
-  uint64_t mine[kPer];
+  if (!a.sel.valid(r)) return;  // outputs are written by the second launch
+  const T* row = static_cast<const T*>(a.logits) + r * a.row_stride;
+  const RowSpan<T> sp(row, a.V);
+  const int n_blocks = (int)(a.n_cells / kRowWG);
+  const int b0 = split * a.blocks_per_split;
+  const int b1 = b0 + a.blocks_per_split < n_blocks ? b0 + a.blocks_per_split : n_blocks;
+  float* cells = a.cells + r * a.n_cells + wave * 8 + (lane >> 3) + (lane & 7) * (kRowWG / 8);
+  const u32x4 none = sizeof(T) == 4 ? u32x4{0xff800000u, 0xff800000u, 0xff800000u, 0xff800000u}   // -inf
+                                    : u32x4{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
+  float mx = kMaxFloor, s = 0.f;
+  for (int b = b0; b < b1; ++b) {
+    const int64_t u = (int64_t)b * kCellBlock + tid;
+    u32x4 v[kCellUnits];
+    if ((int64_t)(b + 1) * kCellBlock <= sp.n_units) {  // uniform
 #pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const int i = tid + q * kRowWG;
-    mine[q] = i < m ? keys[i] : 0;
-  }
-  RowStat st = stat_identity();
-  uint64_t head = 0;
-  if (wave == 0) {
-    if (lane < a.splits) {
-      const float2 p = a.part_stat[r * a.splits + lane];
-      st.mx = p.x;
-      st.s = p.y;
+      for (int q = 0; q < kCellUnits; ++q) v[q] = __builtin_nontemporal_load(sp.p + u + q * kRowWG);
+    } else {
+#pragma unroll
+      for (int q = 0; q < kCellUnits; ++q) v[q] = u + q * kRowWG < sp.n_units ? __builtin_nontemporal_load(sp.p + u + q * kRowWG) : none;
     }
-    // A lower bound of the k-th largest from the heads of the lists: the largest 64 / splits keys of every
-    // split; where those are k keys or more, their k-th largest keeps a few dozen of the splits * k keys.
-    if (m > 64) {
-      const int per = 64 / a.splits;               // >= 1: splits <= 64
-      const int sp = lane / per, j = lane % per;
-      if (sp < a.splits && j < k) head = keys[sp * k + j];
+    float m[kCellUnits];
+#pragma unroll
+    for (int q = 0; q < kCellUnits; ++q) {
+      float x[kVec];
+      Elem<T>::unpack(v[q], x);
+      m[q] = max_of_raw<kVec>(x);
     }
-    uint64_t thr = 0;
-    if (m > 64) {
-      const int rank = wave_rank(head, 64);
-      const uint64_t at = __ballot(head != 0 && rank == k - 1);  // at most one lane: keys are distinct
-      if (at != 0) {
-        const int src = __builtin_ctzll(at);
-        thr = ((uint64_t)__builtin_amdgcn_readlane((uint32_t)(head >> 32), src) << 32) |
-              (uint32_t)__builtin_amdgcn_readlane((uint32_t)head, src);
+    // Opaque to the optimiser: the second sweep unpacks again instead of keeping every element in a register of its own.
+#pragma unroll
+    for (int q = 0; q < kCellUnits; ++q) asm volatile("" : "+v"(v[q].x), "+v"(v[q].y), "+v"(v[q].z), "+v"(v[q].w));
+    const float mx_new = raw_max3(raw_max3(raw_max3(mx, m[0], m[1]), m[2], m[3]), raw_max3(m[4], m[5], m[6]), m[7]);
+    const float mm = mx_new * a.scale;
+    float s0 = s * fast_exp2((mx - mx_new) * a.scale), s1 = 0.f;
+#pragma unroll
+    for (int q = 0; q < kCellUnits; ++q) {
+      float x[kVec];
+      Elem<T>::unpack(v[q], x);
+#pragma unroll
+      for (int i = 0; i < kVec; i += 2) {
+        s0 += fast_exp2(fmaf(x[i], a.scale, -mm));
+        s1 += fast_exp2(fmaf(x[i + 1], a.scale, -mm));
       }
     }
-    if (lane == 0) sh.thr4[0] = thr;
+    s = s0 + s1;
+    mx = mx_new;
+    // Cell maxima: over groups of eight lanes, all eight units at once (each register is read through DPP eight
+    // instructions after it was written; the s_nop covers the first one).
+    asm volatile(
+        "s_nop 1\n"
+        "v_max_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %1, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %3, %3, %3 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %4, %4, %4 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %5, %5, %5 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %6, %6, %6 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %7, %7, %7 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %1, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %2, %2, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %3, %3, %3 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %4, %4, %4 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %5, %5, %5 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %6, %6, %6 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %7, %7, %7 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %1, %1, %1 row_half_mirror row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %2, %2, %2 row_half_mirror row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %3, %3, %3 row_half_mirror row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %4, %4, %4 row_half_mirror row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %5, %5, %5 row_half_mirror row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %6, %6, %6 row_half_mirror row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %7, %7, %7 row_half_mirror row_mask:0xf bank_mask:0xf\n"
+        "s_nop 1"
+        : "+v"(m[0]), "+v"(m[1]), "+v"(m[2]), "+v"(m[3]), "+v"(m[4]), "+v"(m[5]), "+v"(m[6]), "+v"(m[7]));
+    float mine = m[0];  // lane j of a group keeps unit row j's maximum: every lane stores one cell
+#pragma unroll
+    for (int q = 1; q < kCellUnits; ++q) mine = (lane & 7) == q ? m[q] : mine;
+    cells[(int64_t)b * kRowWG] = mine;
   }
-  __syncthreads();
-  const uint64_t thr = sh.thr4[0];
-  WaveCollector col{sh.a + wave * kWaveCap, kWaveCap, 0};  // a wave offers at most kPer * 64 = kWaveCap keys: no overflow
+  float wm = mx;
+  wm = raw_max(wm, wave_exchange<0>(wm));
+  wm = raw_max(wm, wave_exchange<1>(wm));
+  wm = raw_max(wm, wave_exchange<2>(wm));
+  wm = raw_max(wm, wave_exchange<3>(wm));
+  wm = raw_max(wm, wave_exchange<4>(wm));
+  wm = raw_max(wm, wave_exchange<5>(wm));
+  s *= fast_exp2((mx - wm) * a.scale);
+  s += wave_exchange<0>(s);
+  s += wave_exchange<1>(s);
+  s += wave_exchange<2>(s);
+  s += wave_exchange<3>(s);
+  s += wave_exchange<4>(s);
+  s += wave_exchange<5>(s);
+  if (lane == 0) a.part_stat[(r * a.splits + split) * kRowWaves + wave] = float2{wm, s};
+}
+
+// Second launch: one workgroup per row takes the best cells, reads them, ranks their elements and draws.  Its time is that of
+// one chain of dependent steps run once per workgroup, the code fetched cold: loads come first and unconditionally, the usual
+// path is short and straight, whatever does not follow from the common case sits behind a branch at its end.
+template <typename T>
+__global__ __launch_bounds__(kRowWG) void row_sample_pick_kernel(SampleArgs a) {
+  constexpr int kVec = Elem<T>::kVec;
+  constexpr int kHold = 32;                      // cell maxima a lane keeps: 8192 cells a row
+  constexpr int kStats = 64 * kRowWaves / 64;    // partial statistics per lane of wave 0 (splits <= 64)
+  constexpr int kWaveCap = kSampPickCap / kRowWaves;
+  __shared__ SampleLds<kSampPickCap> sh;
+  const int64_t r = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int k = a.top_k;
+  const float* cells = a.cells + r * a.n_cells;
+  const int per_lane = (int)(a.n_cells / kRowWG);
+  float c[kHold];
 #pragma unroll
-  for (int q = 0; q < kPer; ++q)
-    if (q * kRowWG + wave * 64 < m)  // wave-uniform
-      col.offer(mine[q] != 0 && mine[q] >= thr, mine[q]);
-  if (lane == 0) sh.wave_cnt[wave] = col.count;
-  __syncthreads();
-  int c[kRowWaves];
+  for (int q0 = 0; q0 < kHold; q0 += 8) {  // eight loads at a time: up to 7 past this row's cells (the workspace has room)
+    if (q0 < per_lane) {
 #pragma unroll
-  for (int w = 0; w < kRowWaves; ++w) c[w] = sh.wave_cnt[w];
-  const int kept = c[0] + c[1] + c[2] + c[3];
-  uint64_t sorted;
-  if (kept <= 64) {  // the usual case: wave 0 ranks them in registers
-    if (wave != 0) return;
-    sorted = wave_sorted_top_k(lane < kept ? region_entry(sh.a, kWaveCap, c, lane) : 0, kept, k);
-  } else {
-    for (int i = tid; i < kept; i += kRowWG) sh.b[i] = region_entry(sh.a, kWaveCap, c, i);
+      for (int q = q0; q < q0 + 8; ++q) c[q] = cells[tid + q * kRowWG];
+    } else {
+#pragma unroll
+      for (int q = q0; q < q0 + 8; ++q) c[q] = -INFINITY;
+    }
+  }
+  const int n_part = a.splits * kRowWaves;
+  const float2* stats = a.part_stat + r * n_part;
+  float2 part[kStats];
+#pragma unroll
+  for (int q = 0; q < kStats; ++q) part[q] = stats[lane + q * 64 < n_part ? lane + q * 64 : 0];
+  const float uniform = a.uniforms ? a.uniforms[r] : 0.f;
+  if (!a.sel.valid(r)) {
+    masked_sample(a, r, tid);
+    return;
+  }
+  const T* row = static_cast<const T*>(a.logits) + r * a.row_stride;
+  const RowSpan<T> sp(row, a.V);
+  // The single elements of the edges (at most 7 on either side): lanes 0 .. 7 and 8 .. 15.
+  const bool edge = tid < 8 ? tid < sp.head : tid - 8 < sp.tail;
+  const int64_t edge_e = tid < 8 ? tid : sp.tail_start() + (tid - 8);
+  const float x_edge = edge ? Elem<T>::load1(row + edge_e) : -INFINITY;  // -inf: no candidate
+  if (tid < 64) sh.b[tid] = 0;  // the ranking below reads 64 entries; published by the barriers of the bound
+  if (tid == 0) sh.cnt2 = 0;
+  float lane_max = -INFINITY;  // fmaxf also drops the NaN of a cell that holds nothing else
+#pragma unroll
+  for (int q = 0; q < kHold; ++q) c[q] = q < per_lane ? c[q] : -INFINITY;
+#pragma unroll
+  for (int q = 0; q < kHold; q += 2) lane_max = fmaxf(lane_max, fmaxf(c[q], c[q + 1]));
+  for (int q = kHold; q < per_lane; ++q) lane_max = fmaxf(lane_max, cells[(int64_t)q * kRowWG + tid]);
+
+  // ---- the cells at or above a lower bound of the k-th best ----------------------------------------
+  uint64_t theta = bound_from_lane_maxima(sh, lane_max, k);
+  float least = fmaxf(key_float((uint32_t)(theta >> 32)), -__FLT_MAX__);  // -inf is never a candidate
+  // Every wave owns a quarter of the buffer and a running count that is the same in all its lanes; the lanes that pass take
+  // consecutive slots by their position among the passing lanes (an LDS atomic per candidate would queue up).
+  int count = 0;
+  auto offer_cell = [&](float w, int q) {
+    const uint64_t b = __ballot(w >= least);
+    if (__builtin_expect(b == 0, 1)) return;
+    const int pos = count + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
+    if (w >= least && pos < kWaveCap) sh.a[wave * kWaveCap + pos] = ((uint64_t)__float_as_uint(w) << 32) | (uint32_t)(q * kRowWG + tid);
+    count += __builtin_popcountll(b);
+  };
+#pragma unroll
+  for (int q0 = 0; q0 < kHold; q0 += 8)
+    if (q0 < per_lane) {
+#pragma unroll
+      for (int q = q0; q < q0 + 8; ++q) offer_cell(c[q], q);
+    }
+  for (int q = kHold; q < per_lane; ++q) offer_cell(cells[(int64_t)q * kRowWG + tid], q);
+  if (lane == 0) sh.wave_cnt[wave] = count;
+  __syncthreads();
+  int n_wave[kRowWaves], n_best = 0;
+  bool fits = true;
+#pragma unroll
+  for (int w = 0; w < kRowWaves; ++w) {
+    n_wave[w] = sh.wave_cnt[w];
+    n_best += n_wave[w];
+    fits = fits && n_wave[w] <= kWaveCap;
+  }
+
+  // ---- their elements: eight lanes a cell, one load unit each -----------------------------------------
+  // cells_of(j): the cell of this lane's group in round j (32 groups a round), -1 = none.  Elements at or above `least` go to
+  // sh.b, consecutive slots per wave by position among the passing lanes; sh.cnt2 counts what passed, stored or not.
+  const u32x4 none = sizeof(T) == 4 ? u32x4{0xff800000u, 0xff800000u, 0xff800000u, 0xff800000u}   // -inf
+                                    : u32x4{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
+  const int group = tid >> 3;
+  auto load_unit = [&](int64_t cell) {
+    const int64_t u = cell * kCellUnits + (lane & 7);
+    return cell >= 0 && u < sp.n_units ? sp.p[u] : none;
+  };
+  auto offer_n = [&](const float* e, auto n, auto index_of) {
+    uint64_t pass[decltype(n)::value];
+    int total = 0;
+#pragma unroll
+    for (int i = 0; i < decltype(n)::value; ++i) {
+      pass[i] = __ballot(e[i] >= least);
+      total += __builtin_popcountll(pass[i]);
+    }
+    if (total == 0) return;  // wave-uniform
+    int at = 0;
+    if (lane == 0) at = atomicAdd(&sh.cnt2, total);
+    at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+    for (int i = 0; i < decltype(n)::value; ++i) {
+      if (pass[i] == 0) continue;
+      const int pos = at + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(pass[i] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)pass[i], 0u));
+      if (e[i] >= least && pos < kSampPickCap) sh.b[pos] = make_key(e[i], (uint32_t)index_of(i));
+      at += __builtin_popcountll(pass[i]);
+    }
+  };
+  auto offer_unit = [&](const u32x4& v, int64_t cell) {
+    float x[kVec];
+    Elem<T>::unpack(v, x);
+    offer_n(x, std::integral_constant<int, kVec>(), [&](int i) { return sp.head + (cell * kCellUnits + (lane & 7)) * kVec + i; });
+  };
+  auto offer_edge = [&]() {
+    if (wave == 0 && sp.head + sp.tail > 0) offer_n(&x_edge, std::integral_constant<int, 1>(), [&](int) { return edge_e; });
+  };
+
+  RowStat st = stat_identity();
+  auto merge_stats = [&]() {  // the maximum first, then every partial sum moved to it
+    float mx = fmaxf(x_edge, kMaxFloor);
+#pragma unroll
+    for (int q = 0; q < kStats; ++q) mx = fmaxf(mx, part[q].x);  // (lanes past the end hold a copy of entry 0)
+    mx = fmaxf(mx, wave_exchange<0>(mx));
+    mx = fmaxf(mx, wave_exchange<1>(mx));
+    mx = fmaxf(mx, wave_exchange<2>(mx));
+    mx = fmaxf(mx, wave_exchange<3>(mx));
+    mx = fmaxf(mx, wave_exchange<4>(mx));
+    mx = fmaxf(mx, wave_exchange<5>(mx));
+    float sum = fast_exp2(fmaf(x_edge, a.scale, -mx * a.scale));
+#pragma unroll
+    for (int q = 0; q < kStats; ++q) sum += lane + q * 64 < n_part ? part[q].y * fast_exp2((part[q].x - mx) * a.scale) : 0.f;
+    sum += wave_exchange<0>(sum);
+    sum += wave_exchange<1>(sum);
+    sum += wave_exchange<2>(sum);
+    sum += wave_exchange<3>(sum);
+    sum += wave_exchange<4>(sum);
+    sum += wave_exchange<5>(sum);
+    st.mx = mx;
+    st.s = sum;
+  };
+  int m = kSampPickCap + 1;
+  if (__builtin_expect(n_best <= 64, 1)) {
+    const int64_t c0 = group < n_best ? (int64_t)(uint32_t)region_entry(sh.a, kWaveCap, n_wave, group) : -1;
+    const u32x4 v0 = load_unit(c0);
+    int64_t c1 = -1;
+    u32x4 v1 = none;
+    if (n_best > 32) {
+      if (group + 32 < n_best) c1 = (int64_t)(uint32_t)region_entry(sh.a, kWaveCap, n_wave, group + 32);
+      v1 = load_unit(c1);
+    }
+    if (wave == 0) merge_stats();  // while the loads are under way
+    offer_unit(v0, c0);
+    if (n_best > 32) offer_unit(v1, c1);
+    offer_edge();
     __syncthreads();
-    select_top_k(sh, sh.b, sh.a, kept, k);
-    if (wave != 0) return;
-    sorted = lane < k ? sh.top[lane] : 0;
+    m = sh.cnt2;
   }
-  stat_wave_reduce(st, a.scale);
-  finish_sample(a, sorted, r, st, lane);
+  if (__builtin_expect(m > kSampPickCap, 0)) {
+    // Far more cells or elements than k at or above the bound (many equal ones, or the large ones all in a few lanes): the k
+    // best cells by whole keys, and the elements of those alone, which always fit.
+    if (wave == 0) merge_stats();
+    if (n_best <= 64 || fits) {
+      __syncthreads();
+      for (int i = tid; i < n_best; i += kRowWG) {
+        const uint64_t raw = region_entry(sh.a, kWaveCap, n_wave, i);
+        sh.b[i] = make_key(__uint_as_float((uint32_t)(raw >> 32)), (uint32_t)raw);
+      }
+      __syncthreads();
+    } else {
+      for (;;) {
+        __syncthreads();
+        if (tid == 0) sh.cnt = 0;
+        __syncthreads();
+        for (int q = 0; q < per_lane; ++q) {
+          const float w = cells[(int64_t)q * kRowWG + tid];
+          const uint64_t key = make_key(w, (uint32_t)(q * kRowWG + tid));
+          if (w > -INFINITY && key >= theta) {
+            const int pos = atomicAdd(&sh.cnt, 1);
+            if (pos < kSampPickCap) sh.b[pos] = key;
+          }
+        }
+        __syncthreads();
+        n_best = sh.cnt;
+        if (n_best <= kSampPickCap) break;
+        // Overflow: the k-th largest of the keys that were kept is a strictly higher lower bound.
+        __syncthreads();
+        theta = select_top_k(sh, sh.b, sh.a, kSampPickCap, k);
+      }
+    }
+    select_top_k(sh, sh.b, sh.a, n_best, k);
+    const uint64_t kth = sh.top[k - 1], mine = sh.top[group];  // kSampMaxK = 32 cells, 32 groups
+    if (kth != 0) least = key_float((uint32_t)(kth >> 32));
+    __syncthreads();
+    if (tid < 64) sh.b[tid] = 0;
+    if (tid == 0) sh.cnt2 = 0;
+    __syncthreads();
+    const int64_t cell = mine != 0 ? (int64_t)key_index(mine) : -1;
+    offer_unit(load_unit(cell), cell);
+    offer_edge();
+    __syncthreads();
+    m = sh.cnt2;
+  }
+  uint64_t sorted;
+  if (__builtin_expect(m <= 64, 1)) {
+    // Four lanes a key, each counting the larger ones among 16 entries (0 past the end).
+    const uint64_t key = sh.b[tid >> 2];
+    const int first = (tid & 3) * 16;
+    int rank = 0;
+    if ((tid & 3) * 16 < m)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) rank += sh.b[first + j] > key ? 1 : 0;
+    rank += __builtin_amdgcn_update_dpp(0, rank, 0xB1, 0xF, 0xF, true);
+    rank += __builtin_amdgcn_update_dpp(0, rank, 0x4E, 0xF, 0xF, true);
+    if (tid < kSampMaxK) sh.top[tid] = 0;
+    __syncthreads();
+    if ((tid & 3) == 0 && key != 0 && rank < k) sh.top[rank] = key;
+    __syncthreads();
+  } else {
+    select_top_k(sh, sh.b, sh.a, m, k);
+  }
+  if (wave != 0) return;
+  sorted = lane < k ? sh.top[lane] : 0;
+  finish_sample(a, sorted, r, st, lane, uniform);
 }
 
 int row_splits_for(int64_t rows, int64_t V, int vec);
 
-// Workgroups per row.  Decode-sized batches are cut into ranges of ~8192 elements whatever the batch size: the selection
-// bookkeeping of a workgroup grows with its elements, 8192 fp32 elements are the most a workgroup keeps in
-// registers between its passes, and fewer, fatter workgroups beat filling the chip (64 rows fp32: 19-20
-// splits 23 us, 32 splits 27 us, 12 splits 37 us; 256 rows: 20 splits 47 us, the row kernel's 8 splits
-// 68 us).  Very small batches still get enough workgroups to pull a row from many CUs.  Larger batches follow the
-// row kernel (one workgroup per row from 512 rows on, which streams the row once); where that takes over was measured
-// at V = 151936, ranges against the row kernel's policy: fp32 512 / 768 / 900 / 1024 / 1152 rows 62.5 / 85.4 / 97.4 / 110.5 /
-// 125.2 us against 83.0 / 92.6 / 100.5 / 107.9 / 121.4; bf16 256 / 300 / 340 / 400 rows 41.3 / 46.6 / 50.5 / 56.8 against 47.7 /
-// 50.4 / 50.9 / 53.6 (a bf16 range holds twice the elements per byte, and it is the per-element work that costs).
-static int sample_splits_for(int64_t rows, int64_t V, int vec) {
-  const int base = row_splits_for(rows, V, vec);
+// Batches that need a workspace: those whose rows are worth more than one workgroup.  They always take the decode form.
+bool row_sample_needs_workspace(int64_t rows, int64_t V, int vec) {
   int64_t s = (V + 8191) / 8192;
   const int64_t most_ranges = vec == 4 ? 18000 : 6500;   // rows * ranges: ~950 fp32 rows, ~340 bf16 rows at V = 151936
-  if (rows * s > most_ranges) return base;
+  if (rows * s > most_ranges) return row_splits_for(rows, V, vec) > 1;
   const int64_t fill = (512 + rows - 1) / rows;
   if (s < fill) s = fill;
   const int64_t max_by_work = (V / vec) / (2 * kRowWG);  // >= 2 load units per lane and split
   if (s > max_by_work) s = max_by_work;
-  if (s > 64) s = 64;
-  if (s < 1) s = 1;
-  return (int)s;
+  return s > 1;
+}
+// Batches that take the decode form if they are given its workspace: larger bf16 ones as well, up to the largest measured
+// (rows of 151936: 700 / 1000 / 1500 67 / 76 / 97 us streamed, 47 / 63 / 93 in cells; 2500 x 65536 89 / 74).  fp32 rows stream as fast as they are read either way (1000 x 151936: 114 us in cells, 108 streamed).
+static bool sample_prefers_cells(int64_t rows, int64_t V, int vec) {
+  if (row_sample_needs_workspace(rows, V, vec)) return true;
+  return vec == 8 && V >= 16384 && rows * V <= (int64_t)1 << 28;
+}
+
+// The decode form's work split: one block of 2048 load units (32 KB) per workgroup, more only where a row would take more than
+// 64 workgroups.  Measured with 512 to 4096 workgroups in the launch: equal up to ~128 rows of 151936, from there on one block
+// is the fastest (400 / 1000 rows fp32 51-55 / 122-124 us against 49.8 / 114, 700 rows bf16 50-61 against 46.5), also
+// against a variant that requests the next block before it takes in the present one.
+struct CellPlan {
+  int splits, blocks_per_split;
+  int64_t n_cells;
+};
+static CellPlan cell_plan(int64_t V, int vec) {
+  const int64_t blocks = (V / vec + kCellBlock - 1) / kCellBlock;
+  const int64_t per = (blocks + 63) / 64;
+  return CellPlan{(int)((blocks + per - 1) / per), (int)per, blocks * kRowWG};
 }
 
 static size_t align256s(size_t b) { return (b + 255) & ~(size_t)255; }
 size_t row_sample_workspace_bytes(int64_t rows, int64_t V, int dtype_vec, int top_k) {
-  const int splits = sample_splits_for(rows, V, dtype_vec);
-  if (splits == 1) return 0;
-  return align256s((size_t)rows * splits * top_k * sizeof(uint64_t)) + align256s((size_t)rows * splits * sizeof(float2));
+  (void)top_k;
+  if (!sample_prefers_cells(rows, V, dtype_vec)) return 0;
+  const CellPlan p = cell_plan(V, dtype_vec);
+  // (the second launch reads up to 7 x 256 cells past a row's own)
+  return align256s((size_t)(rows * p.n_cells + 7 * kRowWG) * sizeof(float)) + align256s((size_t)rows * p.splits * kRowWaves * sizeof(float2));
 }
 
 hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
@@ -672,16 +955,40 @@ hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_
                              int32_t* out_topk_idx, float* out_topk_logit, void* workspace, hipStream_t stream) {
   const int esize = dtype == 0 ? 4 : 2;
   const int vec = 16 / esize;
-  const int splits = sample_splits_for(rows, V, vec);
-  char* ws = static_cast<char*>(workspace);
-  SampleArgs a{logits, uniforms, sel, out_token, out_lp, out_lse, out_argmax, out_topk_idx, out_topk_logit,
-               reinterpret_cast<uint64_t*>(ws),
-               reinterpret_cast<float2*>(ws + align256s((size_t)rows * splits * top_k * sizeof(uint64_t))),
-               V, row_stride, top_k, splits, kLog2e / temperature};
-  const dim3 grid((unsigned)(rows * splits)), block(kRowWG);
-  const int64_t units_per_split = (V / vec + splits - 1) / splits;
+  SampleArgs a{};
+  a.logits = logits;
+  a.uniforms = uniforms;
+  a.sel = sel;
+  a.out_token = out_token;
+  a.out_lp = out_lp;
+  a.out_lse = out_lse;
+  a.out_argmax = out_argmax;
+  a.out_topk_idx = out_topk_idx;
+  a.out_topk_logit = out_topk_logit;
+  a.V = V;
+  a.row_stride = row_stride;
+  a.top_k = top_k;
+  a.scale = kLog2e / temperature;
+  const dim3 block(kRowWG);
+  if (workspace && sample_prefers_cells(rows, V, vec)) {
+    const CellPlan p = cell_plan(V, vec);
+    a.cells = static_cast<float*>(workspace);
+    a.part_stat = reinterpret_cast<float2*>(static_cast<char*>(workspace) + align256s((size_t)(rows * p.n_cells + 7 * kRowWG) * sizeof(float)));
+    a.splits = p.splits;
+    a.blocks_per_split = p.blocks_per_split;
+    a.n_cells = p.n_cells;
+    const dim3 grid((unsigned)(rows * p.splits));
+    if (dtype == 0) hipLaunchKernelGGL((row_sample_cells_kernel<float>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((row_sample_cells_kernel<uint16_t>), grid, block, 0, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (dtype == 0) hipLaunchKernelGGL((row_sample_pick_kernel<float>), dim3((unsigned)rows), block, 0, stream, a);
+    else hipLaunchKernelGGL((row_sample_pick_kernel<uint16_t>), dim3((unsigned)rows), block, 0, stream, a);
+    return hipGetLastError();
+  }
+  const dim3 grid((unsigned)rows);
   // (two units' worth of elements: every row then holds a whole unit at any phase)
-  const bool cached = V >= 2 * vec && units_per_split <= (int64_t)kSampCached * kRowWG;
+  const bool cached = V >= 2 * vec && V / vec <= (int64_t)kSampCached * kRowWG;
   if (dtype == 0) {
     if (cached) hipLaunchKernelGGL((row_sample_kernel<float, true>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((row_sample_kernel<float, false>), grid, block, 0, stream, a);
@@ -689,9 +996,6 @@ hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_
     if (cached) hipLaunchKernelGGL((row_sample_kernel<uint16_t, true>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((row_sample_kernel<uint16_t, false>), grid, block, 0, stream, a);
   }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || splits == 1) return e;
-  hipLaunchKernelGGL(row_sample_combine_kernel, dim3((unsigned)rows), block, 0, stream, a);
   return hipGetLastError();
 }
 
