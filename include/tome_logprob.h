@@ -170,6 +170,15 @@ int tome_row_sample(const void* logits, int dtype, int64_t rows, int64_t V, int6
                     int32_t* out_topk_idx, float* out_topk_logit, void* workspace,
                     size_t workspace_bytes, void* stream);
 
+/* One step of a decode loop (node.py:578-608, 346-374): tome_row_sample with the loop's state kept on the
+ * device.  `active` (int32, one per row) is the mask on entry; a row that draws stop_token (-2: none does)
+ * is taken out of it.  out_next gets the next step's input ids: the drawn token, or idle_token for rows that
+ * are no longer active.  out_token and out_lp may lie in page-locked host memory. */
+int tome_row_sample_step(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
+                         const float* uniforms, int32_t* active, float temperature, int top_k,
+                         int32_t stop_token, int64_t idle_token, int32_t* out_token, float* out_lp,
+                         int64_t* out_next, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---- Full log-softmax matrix ------------------------------------------------------
  * fused_log_softmax(logits, temperature) as the reference returns it
  * (mlx-impl/model.py:77-89): out[r, j] = T(x[r, j] * (1/temp)) - T(lse_r), same shape

@@ -78,3 +78,27 @@ def test_judge_decode_matches_oracle(dev, T, eos):
     for g, w in zip(got, want):
         np.testing.assert_allclose(g["log_probs"], w["log_probs"], atol=1e-4, rtol=0)
     assert all(eos not in g["tokens"][1:] for g in got)                # EOS never recorded after the first token (node.py:369-370)
+
+
+@pytest.mark.parametrize("rows,V_step", [(1, 5), (33, 3001), (16, 40000), (9, 50257)])
+@pytest.mark.parametrize("stop", [-1, 2])
+def test_sample_step_keeps_the_loop_state(dev, rows, V_step, stop):
+    """tome_row_sample_step in every kernel form: tokens and log-probs (in page-locked memory) as sample_tokens gives them,
+    rows leave the mask exactly when they draw the stop token, the next ids are the tokens or the idle one."""
+    from tome_amd.logprob import sample_step
+    g = torch.Generator(device=dev).manual_seed(rows + V_step)
+    active = torch.ones(rows, dtype=torch.int32, device=dev)
+    host = torch.empty((2, rows), dtype=torch.int32, pin_memory=True)
+    for _ in range(4):
+        x = torch.randn((rows, V_step), device=dev, generator=g)
+        x[torch.rand(rows, device=dev, generator=g) < 0.4, 2] += 50.0
+        u = torch.rand(rows, device=dev, generator=g)
+        before = active.clone()
+        want = tome_amd.sample_tokens(x, 0.9, 4, uniforms=u, row_valid=before)
+        nxt = sample_step(x, 0.9, 4, u, active, host, stop, 77)
+        torch.cuda.synchronize()
+        tok = want.token.to(torch.int64)
+        assert torch.equal(host[0], want.token.cpu()) and torch.equal(host[1].view(torch.float32), want.lp.cpu())
+        left = (before != 0) & (tok != stop)
+        assert torch.equal(active != 0, left)
+        assert torch.equal(nxt, torch.where(left, tok, torch.full_like(tok, 77)))

@@ -30,7 +30,8 @@ hipError_t full_log_softmax_onepass_launch(const void* in, void* out, int dtype,
 hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
                              const float* uniforms, const RowSel& sel, float temperature, int top_k,
                              int32_t* out_token, float* out_lp, float* out_lse, int32_t* out_argmax,
-                             int32_t* out_topk_idx, float* out_topk_logit, void* workspace, hipStream_t stream);
+                             int32_t* out_topk_idx, float* out_topk_logit, const DecodeState& state, void* workspace,
+                             hipStream_t stream);
 size_t row_sample_workspace_bytes(int64_t rows, int64_t V, int dtype_vec, int top_k);
 bool row_sample_needs_workspace(int64_t rows, int64_t V, int vec);
 size_t fused_workspace_bytes(int64_t n_tokens, int64_t H, int64_t V, int n_weights, bool with_norm);
@@ -135,8 +136,8 @@ int pair_checked(const void* hidden_policy, const void* hidden_ref, const void* 
                  float* out_ref_lp, float* out_k3, float* out_entropy, void* workspace, size_t workspace_bytes, void* stream);
 int sample_checked(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride, const float* uniforms,
                    const tome::RowSel& sel, float temperature, int top_k, int32_t* out_token, float* out_lp, float* out_lse,
-                   int32_t* out_argmax, int32_t* out_topk_idx, float* out_topk_logit, void* workspace, size_t workspace_bytes,
-                   void* stream);
+                   int32_t* out_argmax, int32_t* out_topk_idx, float* out_topk_logit, const tome::DecodeState& state, void* workspace,
+                   size_t workspace_bytes, void* stream);
 }  // namespace
 
 extern "C" {
@@ -237,7 +238,22 @@ int tome_row_sample(const void* logits, int dtype, int64_t rows, int64_t V, int6
                     int32_t* out_topk_idx, float* out_topk_logit, void* workspace, size_t workspace_bytes,
                     void* stream) {
   return sample_checked(logits, dtype, rows, V, row_stride, uniforms, plain_sel(nullptr, row_valid), temperature, top_k,
-                        out_token, out_lp, out_lse, out_argmax, out_topk_idx, out_topk_logit, workspace, workspace_bytes, stream);
+                        out_token, out_lp, out_lse, out_argmax, out_topk_idx, out_topk_logit, tome::DecodeState(), workspace,
+                        workspace_bytes, stream);
+}
+
+int tome_row_sample_step(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
+                         const float* uniforms, int32_t* active, float temperature, int top_k, int32_t stop_token,
+                         int64_t idle_token, int32_t* out_token, float* out_lp, int64_t* out_next, void* workspace,
+                         size_t workspace_bytes, void* stream) {
+  if (rows > 0 && (!active || !out_next)) return TOME_E_NULL;
+  tome::DecodeState state;
+  state.active = active;
+  state.out_next = out_next;
+  state.idle_token = idle_token;
+  state.stop_token = stop_token;
+  return sample_checked(logits, dtype, rows, V, row_stride, uniforms, plain_sel(nullptr, active), temperature, top_k,
+                        out_token, out_lp, nullptr, nullptr, nullptr, nullptr, state, workspace, workspace_bytes, stream);
 }
 
 int tome_full_log_softmax(const void* logits, void* out, int dtype, int64_t rows, int64_t V,
@@ -437,8 +453,8 @@ int row_logprob_checked(const void* logits, int dtype, int64_t rows, int64_t V, 
 
 int sample_checked(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride, const float* uniforms,
                    const tome::RowSel& sel, float temperature, int top_k, int32_t* out_token, float* out_lp, float* out_lse,
-                   int32_t* out_argmax, int32_t* out_topk_idx, float* out_topk_logit, void* workspace, size_t workspace_bytes,
-                   void* stream) {
+                   int32_t* out_argmax, int32_t* out_topk_idx, float* out_topk_logit, const tome::DecodeState& state, void* workspace,
+                   size_t workspace_bytes, void* stream) {
   if (dtype != TOME_F32 && dtype != TOME_BF16) return TOME_E_DTYPE;
   if (bad_matrix(rows, V, row_stride) || top_k < 1 || top_k > 32) return TOME_E_SHAPE;
   if (bad_temperature(temperature)) return TOME_E_TEMPERATURE;
@@ -449,7 +465,7 @@ int sample_checked(const void* logits, int dtype, int64_t rows, int64_t V, int64
   if (reinterpret_cast<uintptr_t>(logits) % (dtype == TOME_F32 ? 4 : 2) != 0) return TOME_E_ALIGN;
   return hip_result(tome::row_sample_launch(logits, dtype, rows, V, row_stride, uniforms, sel, temperature,
                                             top_k, out_token, out_lp, out_lse, out_argmax, out_topk_idx,
-                                            out_topk_logit, workspace, static_cast<hipStream_t>(stream)));
+                                            out_topk_logit, state, workspace, static_cast<hipStream_t>(stream)));
 }
 
 int fused_checked(const void* hidden, const int32_t* hidden_rows, int64_t n_rows, const void* norm_weight, float norm_eps,

@@ -100,6 +100,14 @@ struct RowSel {
   }
 };
 
+// What a decode loop keeps on the device between its sampler calls (all null / zero: a plain call).
+struct DecodeState {
+  int32_t* active = nullptr;     // in / out: rows that still generate
+  int64_t* out_next = nullptr;
+  int64_t idle_token = 0;
+  int32_t stop_token = -2;       // -2: nothing stops a row (-1 is "no token could be drawn")
+};
+
 // ---- wave64 lane exchange --------------------------------------------------------------
 // Steps inside a 16-lane row use DPP; the two steps that cross rows swap rows (halves) between two copies of the value
 // (v_permlane16_swap / v_permlane32_swap), so a reduction never leaves the VALU for the LDS crossbar.  After steps 0..3

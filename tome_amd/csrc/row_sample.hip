@@ -63,6 +63,12 @@ struct SampleArgs {
   int32_t* out_argmax;        // nullable
   int32_t* out_topk_idx;      // nullable, [rows, top_k], -1 past the end of a short row
   float* out_topk_logit;      // nullable, [rows, top_k] raw logits
+  // A decode loop's state (out_next set): `active` is also the mask `sel` reads, and loses the rows that draw stop_token;
+  // out_next is the next step's input id, idle_token for rows that are done.
+  int32_t* active;
+  int64_t* out_next;
+  int64_t idle_token;
+  int32_t stop_token;
   float* cells;               // workspace: [rows, n_cells] cell maxima (splits > 0)
   float2* part_stat;          // workspace: [rows, splits * kRowWaves] (max, sum)
   int64_t V;
@@ -262,6 +268,12 @@ __device__ __forceinline__ void finish_sample(const SampleArgs& a, uint64_t key,
   if (a.out_topk_idx && lane < k) a.out_topk_idx[r * k + lane] = have ? (int32_t)key_index(key) : -1;
   if (a.out_topk_logit && lane < k) a.out_topk_logit[r * k + lane] = have ? x : 0.f;
   if (lane != 0) return;
+  if (a.out_next) {  // every lane of this workgroup has read the row's mask long ago
+    const int32_t token = n_have == 0 ? -1 : cidx;
+    const bool stop = token == a.stop_token;
+    a.out_next[r] = stop ? a.idle_token : token;
+    if (stop) a.active[r] = 0;
+  }
   const float m2 = tot.mx * a.scale;
   const float log2s = fast_log2(tot.s);
   if (n_have == 0) {  // nothing above -inf in the row
@@ -283,6 +295,7 @@ __device__ __forceinline__ void masked_sample(const SampleArgs& a, int64_t r, in
     if (a.out_lp) a.out_lp[r] = 0.f;
     if (a.out_lse) a.out_lse[r] = 0.f;
     if (a.out_argmax) a.out_argmax[r] = -1;
+    if (a.out_next) a.out_next[r] = a.idle_token;
   }
   if (tid < a.top_k) {
     if (a.out_topk_idx) a.out_topk_idx[r * a.top_k + tid] = -1;
@@ -952,7 +965,8 @@ size_t row_sample_workspace_bytes(int64_t rows, int64_t V, int dtype_vec, int to
 hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
                              const float* uniforms, const RowSel& sel, float temperature, int top_k,
                              int32_t* out_token, float* out_lp, float* out_lse, int32_t* out_argmax,
-                             int32_t* out_topk_idx, float* out_topk_logit, void* workspace, hipStream_t stream) {
+                             int32_t* out_topk_idx, float* out_topk_logit, const DecodeState& state, void* workspace,
+                             hipStream_t stream) {
   const int esize = dtype == 0 ? 4 : 2;
   const int vec = 16 / esize;
   SampleArgs a{};
@@ -965,6 +979,10 @@ hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_
   a.out_argmax = out_argmax;
   a.out_topk_idx = out_topk_idx;
   a.out_topk_logit = out_topk_logit;
+  a.active = state.active;
+  a.out_next = state.out_next;
+  a.idle_token = state.idle_token;
+  a.stop_token = state.stop_token;
   a.V = V;
   a.row_stride = row_stride;
   a.top_k = top_k;

@@ -204,6 +204,37 @@ std::tuple<Tensor, Tensor, Tensor, MaybeTensor, MaybeTensor> sample_tokens(const
   return {shaped(tok, logits), shaped(lp, logits), shaped(amax, logits), tki, tkl};
 }
 
+// One step of a decode loop: `active` int32 [rows] on the GPU (updated), `host` int32 [2, rows] in page-locked memory (receives
+// tokens and log-probs once the stream is synchronised).  Returns the next step's int64 input ids.
+Tensor sample_step(const Tensor& logits, double temperature, int64_t top_k, const MaybeTensor& uniforms, const Tensor& active,
+                   const Tensor& host, int64_t stop_token, int64_t idle_token, uintptr_t stream) {
+  require_gpu(logits);
+  const c10::Device dev = logits.device();
+  const int dtype = dtype_code(logits);
+  const Tensor x = rows_view(logits);
+  const int64_t rows = x.size(0), V = x.size(1);
+  if (top_k < 1 || top_k > 32) throw py::value_error("top_k must be in 1..32");
+  c10::DeviceGuard guard(dev);
+  require_same(active, dev);
+  if (active.numel() != rows || host.numel() != 2 * rows)
+    throw py::value_error("logits must have one row per sequence (" + std::to_string(active.numel()) + "), got " + std::to_string(rows));
+  Tensor u;
+  if (uniforms) {
+    u = uniforms->to(dev, at::kFloat).contiguous();
+    if (u.numel() != rows)
+      throw py::value_error("uniforms must have one value per row (" + std::to_string(rows) + "), got " + std::to_string(u.numel()));
+  }
+  const Tensor next = at::empty({rows}, active.options().dtype(at::kLong));
+  const size_t bytes = tome_row_sample_workspace(dtype, rows, V, (int)top_k);
+  const Tensor ws = workspace(bytes, active.options());
+  int32_t* out = host.data_ptr<int32_t>();
+  const int32_t stop = stop_token >= 0 && stop_token <= INT32_MAX ? (int32_t)stop_token : -2;
+  check(tome_row_sample_step(x.data_ptr(), dtype, rows, V, rows > 1 ? x.stride(0) : V, u.defined() ? u.data_ptr<float>() : nullptr,
+                             active.data_ptr<int32_t>(), (float)temperature, (int)top_k, stop, idle_token, out,
+                             reinterpret_cast<float*>(out + rows), next.data_ptr<int64_t>(), ptr(ws), bytes, stream_ptr(stream)));
+  return next;
+}
+
 Tensor fused_log_softmax(const Tensor& logits, double temperature, uintptr_t stream) {
   require_gpu(logits);
   const c10::Device dev = logits.device();
@@ -323,6 +354,7 @@ PYBIND11_MODULE(_torch_ops, m) {
   m.def("token_logprobs", &token_logprobs);
   m.def("token_logprobs_rows", &token_logprobs_rows);
   m.def("sample_tokens", &sample_tokens);
+  m.def("sample_step", &sample_step);
   m.def("fused_log_softmax", &fused_log_softmax);
   m.def("lmhead_logprobs", &lmhead_logprobs);
   m.def("grpo_pair", &grpo_pair);

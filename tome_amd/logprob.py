@@ -153,6 +153,16 @@ def sample_tokens(logits: torch.Tensor, temperature: float, top_k: int = 20, *, 
         logits, temperature, int(top_k), _tensor(uniforms, logits), mask, want_topk, _stream(logits)))
 
 
+def sample_step(logits: torch.Tensor, temperature: float, top_k: int, uniforms, active: torch.Tensor, host: torch.Tensor,
+                stop_token: int, idle_token: int) -> torch.Tensor:
+    """``sample_tokens`` as a step of the decode loops (``tome_amd.decode``): the rows of ``active`` (int32, on the GPU) are
+    sampled and leave it when they draw ``stop_token`` (negative: none does); tokens and log-probs go to ``host`` (int32
+    [2, rows], page-locked); returns the next input ids, int64, ``idle_token`` for rows that are no longer active."""
+    temperature = _check_temperature(1.0 if float(temperature) == 0.0 else temperature)
+    return _lib.torch_ops().sample_step(logits, temperature, int(top_k), _tensor(uniforms, logits), active, host, int(stop_token),
+                                        int(idle_token), _stream(logits))
+
+
 class DecodeStepGraph:
     """``sample_tokens`` for one fixed decode-batch shape, captured once as a HIP graph and replayed.
 
