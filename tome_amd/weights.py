@@ -13,15 +13,14 @@ and the result being non-cumulative: base weights always come from the frozen re
 """
 from __future__ import annotations
 
-import ctypes
 import logging
 from dataclasses import dataclass, field
 from typing import List, Optional, Sequence, Tuple
 
-import numpy as np
 import torch
 
 from . import _lib
+from .logprob import _stream
 
 logger = logging.getLogger(__name__)
 
@@ -56,85 +55,22 @@ def lora_merge(jobs: Sequence[MergeJob]) -> None:
     bf16, the scaling by the bf16-rounded scalar to bf16, the sum to bf16.  ``lora_A`` [rank, cols] and
     ``lora_B`` [rows, rank] may both be None (``out = base + 0``).  ``out`` may be ``base`` itself.
     """
-    if not jobs:
-        return
-    lib = _lib.load_library()
-    arr = (_lib.TomeLoraJob * len(jobs))()
-    keep = []
-    dev = jobs[0][0].device
-    for i, (base, out, a, b, scale) in enumerate(jobs):
-        for t in (base, out, a, b):
-            if t is None:
-                continue
-            if not t.is_cuda:
-                raise RuntimeError("tome_amd operators run on a ROCm GPU only (there is no CPU fallback); "
-                                   f"got a tensor on {t.device}")
-            if t.device != dev:
-                raise ValueError("all tensors of a merge must be on the same device")
-            if t.dtype != torch.bfloat16 or t.dim() != 2:
-                raise TypeError("LoRA merges work on 2-D bfloat16 tensors (inference.proto:71-72)")
-        if out.shape != base.shape or base.stride(1) != 1 or out.stride(1) != 1:
-            raise ValueError("base and out must have the same shape and unit stride along the input dimension")
-        rows, cols = base.shape
-        rank = 0
-        if (a is None) != (b is None):
-            raise ValueError("lora_A and lora_B come together")
-        if a is not None:
-            rank = a.shape[0]
-            if a.shape != (rank, cols) or b.shape != (rows, rank):
-                raise ValueError(f"lora_A must be [rank, {cols}] and lora_B [{rows}, rank]; got {tuple(a.shape)}, {tuple(b.shape)}")
-            a, b = a.contiguous(), b.contiguous()
-            if rank % 8 != 0:                       # zero-pad the rank: extra terms of the product are exact zeros
-                pad = 8 - rank % 8
-                a = torch.cat([a, a.new_zeros(pad, cols)], 0)
-                b = torch.cat([b, b.new_zeros(rows, pad)], 1).contiguous()
-                rank += pad
-            keep += [a, b]
-        j = arr[i]
-        j.base, j.out = base.data_ptr(), out.data_ptr()
-        j.lora_a, j.lora_b = (a.data_ptr(), b.data_ptr()) if a is not None else (None, None)
-        j.rows, j.cols, j.rank = rows, cols, rank
-        j.base_stride = base.stride(0) if rows > 1 else cols
-        j.out_stride = out.stride(0) if rows > 1 else cols
-        j.scale = float(scale)
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
-        jobs_ptr = ctypes.cast(arr, ctypes.c_void_p)
-        ws_bytes = lib.tome_lora_merge_workspace(jobs_ptr, len(jobs))
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-        _lib.check(lib.tome_lora_merge(jobs_ptr, len(jobs), None if ws is None else ws.data_ptr(), ws_bytes, stream))
-    del keep, ws                                   # launches are stream-ordered; torch frees on the same stream
+    if jobs:
+        _lib.torch_ops().lora_merge(list(jobs), _stream(jobs[0][0]))
 
 
 def _upload_lora(entries: Sequence[Tuple[object, float]], dev: torch.device) -> dict:
-    """All adapters of a request in ONE host-to-device copy.
+    """All adapters of a request through one staging buffer.
 
-    Each ``LayerUpdate`` is decoded as the reference does - ``np.frombuffer(raw, uint16).reshape(shape)`` viewed
-    as bf16 (node.py:123-126) - with the rank zero-padded to a multiple of 8 (extra terms of the product are exact
-    zeros) and every matrix starting on a 16-byte boundary of one staging array.  Returns
-    ``{id(update): (lora_A [rank, in], lora_B [out, rank])}`` as views of the uploaded buffer.
+    Each ``LayerUpdate`` is decoded as the reference does - raw ``uint16`` of the stated shape viewed as bf16
+    (node.py:123-126) - with the rank zero-padded to a multiple of 8 and every matrix starting on a 16-byte boundary.
+    Returns ``{id(update): (lora_A [rank, in], lora_B [out, rank])}`` as views of the uploaded buffer.  The copying and the job
+    table of ``lora_merge`` are native (a request of 84 adapters, 7 MB: 1.48 -> 0.74 ms with the merge itself).
     """
-    parts, layout, total = [], {}, 0
-    for up, _ in entries:
-        a = np.frombuffer(up.lora_A, dtype=np.uint16).reshape([int(v) for v in up.shape_A])
-        b = np.frombuffer(up.lora_B, dtype=np.uint16).reshape([int(v) for v in up.shape_B])
-        if a.ndim != 2 or b.ndim != 2 or a.shape[0] != b.shape[1]:
-            raise ValueError(f"lora_A {a.shape} and lora_B {b.shape} do not form a rank decomposition")
-        pad = -a.shape[0] % 8
-        if pad:
-            a = np.concatenate([a, np.zeros((pad, a.shape[1]), np.uint16)], 0)
-            b = np.concatenate([b, np.zeros((b.shape[0], pad), np.uint16)], 1)
-        offs = []
-        for m in (a, b):
-            offs.append((total, m.shape))
-            parts.append((total, m))
-            total += -(-m.size // 8) * 8
-        layout[id(up)] = offs
-    stage = np.zeros(total, dtype=np.uint16)
-    for off, m in parts:
-        stage[off:off + m.size] = m.reshape(-1)
-    buf = torch.from_numpy(stage.view(np.int16)).to(dev).view(torch.bfloat16)
-    return {key: tuple(buf[off:off + sh[0] * sh[1]].view(sh) for off, sh in offs) for key, offs in layout.items()}
+    ups = [up for up, _ in entries]
+    views = _lib.torch_ops().stage_adapters([(up.lora_A, [int(v) for v in up.shape_A], up.lora_B, [int(v) for v in up.shape_B])
+                                             for up in ups], str(dev))
+    return {id(up): v for up, v in zip(ups, views)}
 
 
 def apply_weight_update(policy_layers: Sequence, reference_layers: Sequence, updates: Sequence, *,
