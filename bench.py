@@ -1104,7 +1104,7 @@ def main():
                                    "fp32 logits [64, 151936] (config 1's shape), top_k 20",
                        "rows": t["rows"], "top_k": t["top_k"], "vocab": V},
             "roofline": hbm_roofline(t["bytes"], t["ms"], traffic_of("row_sample_decode_64rows"),
-                                     "row_sample_kernel<f32> + row_sample_combine_kernel")}
+                                     "row_sample_cells_kernel<f32> + row_sample_pick_kernel<f32>")}
         done("decode_sampler")
     if "lora" in only:
         t = bench_lora(dev, K, W)
