@@ -933,10 +933,11 @@ bool row_sample_needs_workspace(int64_t rows, int64_t V, int vec) {
   return s > 1;
 }
 // Batches that take the decode form if they are given its workspace: larger bf16 ones as well, up to the largest measured
-// (rows of 151936: 700 / 1000 / 1500 67 / 76 / 97 us streamed, 47 / 63 / 93 in cells; 2500 x 65536 89 / 74).  fp32 rows stream as fast as they are read either way (1000 x 151936: 114 us in cells, 108 streamed).
+// (rows of 151936: 700 / 1000 / 1500 67 / 76 / 97 us streamed, 47 / 63 / 93 in cells; 2500 x 65536
+// 89 / 72, 8000 x 32000 150 / 131).  Rows shorter than that stream faster (4000 x 16384 39 / 47, 2500 x 20000 42 / 44).  fp32 rows stream as fast as they are read either way (1000 x 151936: 114 us in cells, 108 streamed).
 static bool sample_prefers_cells(int64_t rows, int64_t V, int vec) {
   if (row_sample_needs_workspace(rows, V, vec)) return true;
-  return vec == 8 && V >= 16384 && rows * V <= (int64_t)1 << 28;
+  return vec == 8 && V >= 32000 && rows * V <= (int64_t)1 << 28;
 }
 
 // The decode form's work split: one block of 2048 load units (32 KB) per workgroup, more only where a row would take more than
