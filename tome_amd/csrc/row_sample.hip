@@ -705,12 +705,15 @@ __global__ __launch_bounds__(kRowWG) void row_sample_pick_kernel(SampleArgs a) {
   const int k = a.top_k;
   const float* cells = a.cells + r * a.n_cells;
   const int per_lane = (int)(a.n_cells / kRowWG);
+  // A lane's cells: `slot` of every block.  In a row of a single block, which may be half empty, waves are dealt every fourth
+  // cell, so that all four have maxima (the bound needs some in each): bf16 rows of 12000 19.6 -> 10.1 us.
+  const int slot = per_lane > 1 ? tid : lane * kRowWaves + wave;
   float c[kHold];
 #pragma unroll
   for (int q0 = 0; q0 < kHold; q0 += 8) {  // eight loads at a time: up to 7 past this row's cells (the workspace has room)
     if (q0 < per_lane) {
 #pragma unroll
-      for (int q = q0; q < q0 + 8; ++q) c[q] = cells[tid + q * kRowWG];
+      for (int q = q0; q < q0 + 8; ++q) c[q] = cells[slot + q * kRowWG];
     } else {
 #pragma unroll
       for (int q = q0; q < q0 + 8; ++q) c[q] = -INFINITY;
@@ -739,7 +742,7 @@ __global__ __launch_bounds__(kRowWG) void row_sample_pick_kernel(SampleArgs a) {
   for (int q = 0; q < kHold; ++q) c[q] = q < per_lane ? c[q] : -INFINITY;
 #pragma unroll
   for (int q = 0; q < kHold; q += 2) lane_max = fmaxf(lane_max, fmaxf(c[q], c[q + 1]));
-  for (int q = kHold; q < per_lane; ++q) lane_max = fmaxf(lane_max, cells[(int64_t)q * kRowWG + tid]);
+  for (int q = kHold; q < per_lane; ++q) lane_max = fmaxf(lane_max, cells[(int64_t)q * kRowWG + slot]);
 
   // ---- the cells at or above a lower bound of the k-th best ----------------------------------------
   uint64_t theta = bound_from_lane_maxima(sh, lane_max, k);
@@ -751,7 +754,7 @@ __global__ __launch_bounds__(kRowWG) void row_sample_pick_kernel(SampleArgs a) {
     const uint64_t b = __ballot(w >= least);
     if (__builtin_expect(b == 0, 1)) return;
     const int pos = count + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
-    if (w >= least && pos < kWaveCap) sh.a[wave * kWaveCap + pos] = ((uint64_t)__float_as_uint(w) << 32) | (uint32_t)(q * kRowWG + tid);
+    if (w >= least && pos < kWaveCap) sh.a[wave * kWaveCap + pos] = ((uint64_t)__float_as_uint(w) << 32) | (uint32_t)(q * kRowWG + slot);
     count += __builtin_popcountll(b);
   };
 #pragma unroll
@@ -760,7 +763,7 @@ __global__ __launch_bounds__(kRowWG) void row_sample_pick_kernel(SampleArgs a) {
 #pragma unroll
       for (int q = q0; q < q0 + 8; ++q) offer_cell(c[q], q);
     }
-  for (int q = kHold; q < per_lane; ++q) offer_cell(cells[(int64_t)q * kRowWG + tid], q);
+  for (int q = kHold; q < per_lane; ++q) offer_cell(cells[(int64_t)q * kRowWG + slot], q);
   if (lane == 0) sh.wave_cnt[wave] = count;
   __syncthreads();
   int n_wave[kRowWaves], n_best = 0;
@@ -868,8 +871,8 @@ __global__ __launch_bounds__(kRowWG) void row_sample_pick_kernel(SampleArgs a) {
         if (tid == 0) sh.cnt = 0;
         __syncthreads();
         for (int q = 0; q < per_lane; ++q) {
-          const float w = cells[(int64_t)q * kRowWG + tid];
-          const uint64_t key = make_key(w, (uint32_t)(q * kRowWG + tid));
+          const float w = cells[(int64_t)q * kRowWG + slot];
+          const uint64_t key = make_key(w, (uint32_t)(q * kRowWG + slot));
           if (w > -INFINITY && key >= theta) {
             const int pos = atomicAdd(&sh.cnt, 1);
             if (pos < kSampPickCap) sh.b[pos] = key;
