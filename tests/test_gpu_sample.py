@@ -95,6 +95,60 @@ def test_sampler_cells(dev, dtype, rows, V, k, kind):
     np.testing.assert_allclose(got.lp.cpu().numpy(), want_lp, atol=1e-4, rtol=0)
 
 
+def _stepped_orderings(V, cell, kind):
+    """Rows of V elements whose candidates exceed the sampler's buffers at its first bound."""
+    rng = np.random.default_rng(V)
+    x = rng.standard_normal(V).astype(np.float32)
+    if kind == "equal":
+        x[:] = 1.5
+    elif kind == "ascending":                      # steps of 1/64 up to 0: exact in fp32, ties in bf16
+        x = (np.arange(V, dtype=np.float32) - (V - 1)) / 64
+    elif kind == "plateau":                        # 700 equal maxima: they fit the buffer, but not one count
+        x[rng.choice(V, 700, replace=False)] = 20.0
+    elif kind == "one_wave":                       # 600 equal cell maxima in the cells of one wave, five in the others'
+        cells = np.arange(V // cell)               # (cell c belongs to lane c % 256)
+        mine = cells[cells % 256 // 64 == 1][:600]
+        others = np.concatenate([64 * w + np.arange(9) for w in (0, 2, 3)])
+        x[np.concatenate([mine, others]) * cell + cell // 2] = 20.0
+    return x
+
+
+@pytest.mark.parametrize("dtype,rows,V,kinds", [
+    # cells: between 529 and 2112 cells at or above the bound, more than 528 of them in one wave's quarter of the buffer
+    (torch.float32, 3, 151936, ["one_wave", "equal", "ascending"]),
+    (torch.bfloat16, 3, 303872, ["one_wave", "equal", "ascending"]),
+    # one workgroup a row, the row in registers
+    (torch.float32, 9, 3001, ["equal", "ascending", "plateau"]),
+    (torch.bfloat16, 9, 6001, ["equal", "ascending", "plateau"]),
+    # one workgroup a row, streamed
+    (torch.float32, 6100, 16421, ["normal", "equal", "ascending", "plateau"]),
+    (torch.bfloat16, 2300, 20011, ["normal", "equal", "ascending", "plateau"]),
+])
+def test_sampler_buffers_overflow(dev, dtype, rows, V, kinds):
+    """Every kernel form on orderings that overflow its candidate buffer (the bound is tightened and the row scanned again) or
+    fill it beyond what one count ranks, at every phase of the rows.  Each ordering is one row repeated through the batch, so
+    that the oracle ranks it once: candidates exact, drawn ids among them, log-probs to 1e-4."""
+    k, T = 20, 1.0
+    cell = 8 * (4 if dtype == torch.float32 else 8)
+    pats = torch.from_numpy(np.stack([_stepped_orderings(V, cell, kind) for kind in kinds])).to(dev).to(dtype)
+    stride = V + (2 if V % 2 else 3)                                                   # odd: every phase of a 16-byte unit
+    buf = torch.full((rows * stride + 1,), 99.0, dtype=dtype, device=dev)              # large values between the rows
+    x = torch.as_strided(buf, (rows, V), (stride, 1), 1)
+    which = torch.arange(rows, device=dev) % len(kinds)
+    for i in range(len(kinds)):
+        x[i::len(kinds)] = pats[i]
+    us = torch.rand(rows, device=dev, generator=torch.Generator(device=dev).manual_seed(3))
+    got = tome_amd.sample_tokens(x, T, k, uniforms=us, want_topk=True)
+    p64 = pats.float().cpu().numpy().astype(np.float64)
+    want_idx, _ = oracle.top_k_rows(p64, k)
+    w = which.cpu().numpy()
+    np.testing.assert_array_equal(got.topk_idx.cpu().numpy(), want_idx[w])
+    tok = got.token.cpu().numpy()
+    assert (want_idx[w] == tok[:, None]).any(axis=1).all()
+    lse = np.array([oracle.logprob_rows(p64[i:i + 1], [0], T)[0] - p64[i, 0] / T for i in range(len(kinds))])   # -lse
+    np.testing.assert_allclose(got.lp.cpu().numpy(), p64[w, tok] / T + lse[w], atol=1e-4, rtol=0)
+
+
 @pytest.mark.parametrize("rows,V,dtype", [(2300, 65536, torch.float32), (1700, 32768, torch.bfloat16)])
 def test_sampler_streams_large_batches(dev, rows, V, dtype):
     """Batches beyond ~950 fp32 / ~340 bf16 rows of 151936 (counted in ranges of 8192 elements) take one streaming

@@ -162,6 +162,9 @@ template <class Lds>
 __device__ uint64_t select_top_k(Lds& sh, uint64_t* cur, uint64_t* other, int m, int k) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   while (m > kRowWG) {
+    // Callers pass an `m` that every wave has just read from sh.cnt or sh.cnt2, and the round clears sh.cnt below: without this
+    // barrier a wave that is late at its read would see 0, take another path and leave the others' barriers unpaired.
+    __syncthreads();
     const uint64_t key = cur[(int)(((int64_t)tid * m) >> 8)];
     const int rank = wave_rank(key, 64);
     const int want = (k + kRowWaves - 1) / kRowWaves;
