@@ -102,3 +102,34 @@ def test_sample_step_keeps_the_loop_state(dev, rows, V_step, stop):
         left = (before != 0) & (tok != stop)
         assert torch.equal(active != 0, left)
         assert torch.equal(nxt, torch.where(left, tok, torch.full_like(tok, 77)))
+
+
+def test_sample_step_checks_where_the_gpu_writes(dev):
+    """`host` and `active` reach the kernel as addresses: memory the GPU must not write, strided tensors, other types and
+    sizes are refused before anything is launched, each with a message of its own."""
+    from tome_amd.logprob import sample_step
+    rows = 4
+    x = torch.zeros((rows, 300), device=dev)
+    active = torch.ones(rows, dtype=torch.int32, device=dev)
+    pinned = torch.empty((2, rows), dtype=torch.int32, pin_memory=True)
+    step = lambda a, h: sample_step(x, 0.0, 4, None, a, h, -1, 0)
+    with pytest.raises(ValueError, match="page-locked"):
+        step(active, torch.empty((2, rows), dtype=torch.int32))
+    with pytest.raises(ValueError, match="host must hold"):
+        step(active, pinned[:1])
+    with pytest.raises(ValueError, match="one row per sequence"):
+        step(active[:2], pinned)
+    with pytest.raises(ValueError, match="contiguous"):
+        step(active, torch.empty((rows, 2), dtype=torch.int32, pin_memory=True).t())
+    with pytest.raises(ValueError, match="contiguous"):
+        step(torch.ones(2 * rows, dtype=torch.int32, device=dev)[::2], pinned)
+    with pytest.raises(TypeError, match="int32"):
+        step(active.long(), pinned)
+    with pytest.raises(TypeError, match="int32"):
+        step(active, torch.empty((2, rows), dtype=torch.float32, pin_memory=True))
+    with pytest.raises(RuntimeError, match="CPU fallback"):
+        step(active.cpu(), pinned)
+    on_gpu = torch.empty((2, rows), dtype=torch.int32, device=dev)                # ... and what may be written still is
+    assert torch.equal(step(active, on_gpu), step(active, pinned))
+    torch.cuda.synchronize()
+    assert torch.equal(on_gpu.cpu(), pinned)

@@ -205,8 +205,9 @@ std::tuple<Tensor, Tensor, Tensor, MaybeTensor, MaybeTensor> sample_tokens(const
   return {shaped(tok, logits), shaped(lp, logits), shaped(amax, logits), tki, tkl};
 }
 
-// One step of a decode loop: `active` int32 [rows] on the GPU (updated), `host` int32 [2, rows] in page-locked memory (receives
-// tokens and log-probs once the stream is synchronised).  Returns the next step's int64 input ids.
+// One step of a decode loop: `active` int32 [rows] on the GPU (updated), `host` int32 [2, rows] in page-locked memory or on the GPU
+// (receives tokens and log-probs once the stream is synchronised); both dense: the kernel is given their addresses.  Returns the
+// next step's int64 input ids.
 Tensor sample_step(const Tensor& logits, double temperature, int64_t top_k, const MaybeTensor& uniforms, const Tensor& active,
                    const Tensor& host, int64_t stop_token, int64_t idle_token, uintptr_t stream) {
   require_gpu(logits);
@@ -217,8 +218,14 @@ Tensor sample_step(const Tensor& logits, double temperature, int64_t top_k, cons
   if (top_k < 1 || top_k > 32) throw py::value_error("top_k must be in 1..32");
   c10::DeviceGuard guard(dev);
   require_same(active, dev);
-  if (active.numel() != rows || host.numel() != 2 * rows)
+  if (active.scalar_type() != at::kInt || host.scalar_type() != at::kInt) throw py::type_error("active and host must be int32 tensors");
+  if (active.numel() != rows)
     throw py::value_error("logits must have one row per sequence (" + std::to_string(active.numel()) + "), got " + std::to_string(rows));
+  if (host.numel() != 2 * rows)
+    throw py::value_error("host must hold two values per sequence (" + std::to_string(2 * rows) + "), got " + std::to_string(host.numel()));
+  if (!active.is_contiguous() || !host.is_contiguous()) throw py::value_error("active and host must be contiguous");
+  if (rows > 0 && host.device() != dev && !(host.is_cpu() && host.is_pinned()))
+    throw py::value_error("host must be page-locked memory or on " + str(dev) + ": the GPU writes to it");
   Tensor u;
   if (uniforms) {
     u = uniforms->to(dev, at::kFloat).contiguous();
