@@ -133,3 +133,20 @@ def test_sample_step_checks_where_the_gpu_writes(dev):
     assert torch.equal(step(active, on_gpu), step(active, pinned))
     torch.cuda.synchronize()
     assert torch.equal(on_gpu.cpu(), pinned)
+
+
+def test_sample_step_draws_as_sample_tokens_does(dev):
+    """Temperature 0 is greedy whatever the uniforms; without uniforms they are drawn, from torch's generator of the GPU."""
+    from tome_amd.logprob import sample_step
+    rows = 512
+    x = torch.zeros((rows, 4), device=dev)                             # four equal logits: greedy is always id 0
+    active = torch.ones(rows, dtype=torch.int32, device=dev)
+    host = torch.empty((2, rows), dtype=torch.int32, pin_memory=True)
+    assert not sample_step(x, 0.0, 4, torch.full((rows,), 0.9, device=dev), active, host, -1, 0).any()
+    torch.manual_seed(11)
+    want = tome_amd.sample_tokens(x, 1.0, 4).token
+    torch.manual_seed(11)
+    got = sample_step(x, 1.0, 4, None, active, host, -1, 0)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want.long()) and torch.equal(host[0], want.cpu())
+    assert len(got.unique()) == 4

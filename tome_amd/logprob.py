@@ -123,6 +123,19 @@ def token_logprobs_rows(logits: torch.Tensor, row_index, targets, temperature: f
         want_argmax, _stream(logits)))
 
 
+def _draw(logits: torch.Tensor, temperature: float, uniforms, generator: Optional[torch.Generator]):
+    """(temperature, uniforms) of a sampler call: greedy (no uniforms) at temperature 0, else one uniform per row."""
+    if float(temperature) == 0.0:
+        return 1.0, None
+    temperature = _check_temperature(temperature)
+    if uniforms is None:
+        if not logits.is_cuda:
+            raise RuntimeError("tome_amd operators run on a ROCm GPU only (there is no CPU fallback); "
+                               f"got a tensor on {logits.device}")
+        uniforms = torch.rand(logits.shape[:-1].numel(), dtype=torch.float32, device=logits.device, generator=generator)
+    return temperature, uniforms
+
+
 def sample_tokens(logits: torch.Tensor, temperature: float, top_k: int = 20, *, uniforms=None,
                   generator: Optional[torch.Generator] = None, row_valid=None, lengths=None,
                   want_topk: bool = False) -> SampledTokens:
@@ -136,15 +149,7 @@ def sample_tokens(logits: torch.Tensor, temperature: float, top_k: int = 20, *, 
     row; drawn with ``torch.rand`` from ``generator`` when omitted) - candidates ordered by
     logit descending, equal logits by ascending id.  MLX's random stream is not reproduced.
     """
-    greedy = float(temperature) == 0.0
-    temperature = _check_temperature(1.0 if greedy else temperature)
-    if greedy:
-        uniforms = None
-    elif uniforms is None:
-        if not logits.is_cuda:
-            raise RuntimeError("tome_amd operators run on a ROCm GPU only (there is no CPU fallback); "
-                               f"got a tensor on {logits.device}")
-        uniforms = torch.rand(logits.shape[:-1].numel(), dtype=torch.float32, device=logits.device, generator=generator)
+    temperature, uniforms = _draw(logits, temperature, uniforms, generator)
     mask = None
     if row_valid is not None or lengths is not None:
         lead = logits.shape[:-1]
@@ -157,8 +162,9 @@ def sample_step(logits: torch.Tensor, temperature: float, top_k: int, uniforms, 
                 stop_token: int, idle_token: int) -> torch.Tensor:
     """``sample_tokens`` as a step of the decode loops (``tome_amd.decode``): the rows of ``active`` (int32, on the GPU) are
     sampled and leave it when they draw ``stop_token`` (negative: none does); tokens and log-probs go to ``host`` (int32
-    [2, rows], page-locked); returns the next input ids, int64, ``idle_token`` for rows that are no longer active."""
-    temperature = _check_temperature(1.0 if float(temperature) == 0.0 else temperature)
+    [2, rows], page-locked); returns the next input ids, int64, ``idle_token`` for rows that are no longer active.
+    ``temperature`` and ``uniforms`` as in ``sample_tokens``: 0 is greedy, uniforms are drawn when omitted."""
+    temperature, uniforms = _draw(logits, temperature, uniforms, None)
     return _lib.torch_ops().sample_step(logits, temperature, int(top_k), _tensor(uniforms, logits), active, host, int(stop_token),
                                         int(idle_token), _stream(logits))
 
