@@ -3,6 +3,8 @@
 // ctypes calls) took 15-21 us a call and was what such a call cost (8 x 151936 fp32: 21.6 us a call, the kernels 7.5).
 // Nothing is kept between calls.  The stream is torch's current one, passed by the caller as a raw handle; no HIP headers
 // are needed here.
+// The operators run without the GIL: a mask, lengths or uniforms in host memory are copied to the GPU in the call, and such a
+// copy waits for all work queued on the stream before it.
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <pybind11/pybind11.h>
@@ -42,6 +44,7 @@ int dtype_code(const Tensor& t) {
 // Status codes become the exceptions of tome_amd._lib.check.
 void check(int code) {
   if (code == TOME_OK) return;
+  py::gil_scoped_acquire gil;
   py::module_::import("tome_amd._lib").attr("check")(code);
 }
 
@@ -437,12 +440,13 @@ std::vector<std::pair<Tensor, Tensor>> stage_adapters(const py::list& entries, c
       total += (parts.back().size() + 7) / 8 * 8;
     }
   }
-  c10::OptionalDeviceGuard guard;
-  if (dev.is_cuda()) guard.reset_device(dev);
-  const Tensor host = at::empty({total}, at::TensorOptions().dtype(at::kShort).pinned_memory(dev.is_cuda()));
-  const Tensor buf = dev.is_cuda() ? at::empty({total}, at::TensorOptions().dtype(at::kShort).device(dev)) : host;
+  Tensor buf;
   {
     py::gil_scoped_release nogil;
+    c10::OptionalDeviceGuard guard;
+    if (dev.is_cuda()) guard.reset_device(dev);
+    const Tensor host = at::empty({total}, at::TensorOptions().dtype(at::kShort).pinned_memory(dev.is_cuda()));
+    buf = dev.is_cuda() ? at::empty({total}, at::TensorOptions().dtype(at::kShort).device(dev)) : host;
     uint16_t* stage = reinterpret_cast<uint16_t*>(host.data_ptr<int16_t>());
     size_t begin = 0;
     for (size_t i = 0; i < parts.size(); ++i) {
@@ -520,6 +524,7 @@ void lora_merge(const py::list& jobs, uintptr_t stream) {
     table.push_back(j);
   }
   if (table.empty()) return;
+  py::gil_scoped_release nogil;
   c10::DeviceGuard guard(dev);
   const size_t bytes = tome_lora_merge_workspace(table.data(), (int64_t)table.size());
   const Tensor ws = workspace(bytes, at::TensorOptions().dtype(at::kByte).device(dev));
@@ -530,14 +535,15 @@ void lora_merge(const py::list& jobs, uintptr_t stream) {
 
 PYBIND11_MODULE(_torch_ops, m) {
   m.doc() = "Native host side of tome_amd's operators (argument checks, allocation, C-ABI calls)";
-  m.def("rows_view", &rows_view);
-  m.def("token_logprobs", &token_logprobs);
-  m.def("token_logprobs_rows", &token_logprobs_rows);
-  m.def("sample_tokens", &sample_tokens);
-  m.def("sample_step", &sample_step);
-  m.def("fused_log_softmax", &fused_log_softmax);
-  m.def("lmhead_logprobs", &lmhead_logprobs);
-  m.def("grpo_pair", &grpo_pair);
+  typedef py::call_guard<py::gil_scoped_release> NoGil;
+  m.def("rows_view", &rows_view, NoGil());
+  m.def("token_logprobs", &token_logprobs, NoGil());
+  m.def("token_logprobs_rows", &token_logprobs_rows, NoGil());
+  m.def("sample_tokens", &sample_tokens, NoGil());
+  m.def("sample_step", &sample_step, NoGil());
+  m.def("fused_log_softmax", &fused_log_softmax, NoGil());
+  m.def("lmhead_logprobs", &lmhead_logprobs, NoGil());
+  m.def("grpo_pair", &grpo_pair, NoGil());
   m.def("stage_adapters", &stage_adapters);
   m.def("lora_merge", &lora_merge);
 }
