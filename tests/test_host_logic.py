@@ -210,3 +210,15 @@ def test_decode_loops_refuse_a_row_without_a_token(monkeypatch, loop):
     done = dec.rollout_decode(lambda t: model_step(t), first, 1, 0.0, 6, 5) if loop == "rollout" else \
         dec.judge_decode(lambda t: model_step(t), first, 0.0, 6, 5)
     assert [d["tokens"] for d in done] == ([[4, 5]] * B if loop == "rollout" else [[4]] * B)
+
+
+def test_grpo_calls_need_a_reference():
+    """A missing reference (w_ref of the dual, hidden_ref of the pair) is an error: scored against the policy itself, the KL
+    of a training step would silently be 0."""
+    h, w, t = torch.zeros(2, 8, dtype=torch.bfloat16), torch.zeros(16, 8, dtype=torch.bfloat16), torch.zeros(2, dtype=torch.int64)
+    with pytest.raises(TypeError, match="w_ref"):
+        tome_amd.grpo_dual_logprobs(h, w, None, t)
+    with pytest.raises(TypeError, match="hidden_ref"):
+        tome_amd.grpo_pair_logprobs(h, None, w, t)
+    with pytest.raises(RuntimeError, match="CPU fallback"):            # ... and w_ref of the pair does default to the policy's
+        tome_amd.grpo_pair_logprobs(h, h, w, t)

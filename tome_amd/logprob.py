@@ -59,6 +59,12 @@ def _tensor(t, like: torch.Tensor, on_device: bool = True):
     return torch.as_tensor(t, device=like.device) if on_device else torch.as_tensor(t)
 
 
+def _require_tensor(t, what: str) -> None:
+    """For arguments that the native call also takes as None, with another meaning."""
+    if not isinstance(t, torch.Tensor):
+        raise TypeError(f"{what} must be a tensor, got {type(t).__name__}")
+
+
 def _rows_view(x: torch.Tensor) -> torch.Tensor:
     """[..., V] -> [rows, V] with unit stride along V, copying only when no such view exists (as every operator does)."""
     return _lib.torch_ops().rows_view(x)
@@ -247,6 +253,7 @@ def grpo_dual_logprobs(hidden: torch.Tensor, w_policy: torch.Tensor, w_ref: torc
     LoRA delta, mlx-impl/node.py:102-164).  k3 and entropy have no counterpart in the
     reference node; they are defined by their closed forms.
     """
+    _require_tensor(w_ref, "w_ref")
     return DualLogprobs(*_lib.torch_ops().grpo_pair(
         hidden, None, w_policy, w_ref, _tensor(targets, hidden), _check_temperature(temperature),
         _tensor(lengths, hidden, False), _tensor(row_valid, hidden), None, 0.0, _stream(hidden)))
@@ -263,6 +270,7 @@ def grpo_pair_logprobs(hidden_policy: torch.Tensor, hidden_ref: torch.Tensor, w_
     states and share the final norm and the lm_head (mlx-impl/model.py:536-538): ``w_ref``
     defaults to ``w_policy``.  ``norm_weight`` as in ``fused_lmhead_logprobs``, applied to both.
     """
+    _require_tensor(hidden_ref, "hidden_ref")
     return DualLogprobs(*_lib.torch_ops().grpo_pair(
         hidden_policy, hidden_ref, w_policy, w_ref, _tensor(targets, hidden_policy), _check_temperature(temperature),
         _tensor(lengths, hidden_policy, False), _tensor(row_valid, hidden_policy), norm_weight, float(norm_eps),
