@@ -222,3 +222,18 @@ def test_grpo_calls_need_a_reference():
         tome_amd.grpo_pair_logprobs(h, None, w, t)
     with pytest.raises(RuntimeError, match="CPU fallback"):            # ... and w_ref of the pair does default to the policy's
         tome_amd.grpo_pair_logprobs(h, h, w, t)
+
+
+def test_judge_decode_without_an_eos_token(monkeypatch):
+    """eos_token_id None (a model without one): every item runs to max_tokens.  Sampler stubbed as above."""
+    from tome_amd import decode as dec
+    from tome_amd.logprob import SampledTokens
+
+    def stub_sampler(logits, temperature, top_k, *, uniforms=None, row_valid=None):
+        tok = logits.argmax(dim=-1).to(torch.int32)
+        return SampledTokens(tok, torch.zeros(tok.shape), tok, None, None)
+
+    monkeypatch.setattr(dec, "sample_tokens", stub_sampler)
+    logits = torch.eye(4)[[2, 0, 3]]
+    got = dec.judge_decode(lambda tokens: logits, logits, 0.0, 3, None)
+    assert [g["tokens"] for g in got] == [[2] * 3, [0] * 3, [3] * 3]

@@ -141,7 +141,8 @@ def judge_decode(model_step: Callable[[torch.Tensor], torch.Tensor], first_logit
     """
     dev = first_logits.device
     B = first_logits.shape[0]
-    loop = _Loop(B, dev, eos_token_id, 0)                                      # an inactive item is fed token 0 (node.py:350)
+    # an inactive item is fed token 0 (node.py:350); without an EOS token (None) nothing ends one
+    loop = _Loop(B, dev, -1 if eos_token_id is None else eos_token_id, 0)
     tok, lp = loop.step(first_logits, temperature, top_k, _uniforms(uniform_source, 0, B, dev, generator))
     width = max(int(max_tokens), 1)
     toks = np.zeros((B, width), dtype=np.int64)
@@ -154,7 +155,7 @@ def judge_decode(model_step: Callable[[torch.Tensor], torch.Tensor], first_logit
             break
         logits = model_step(loop.next)
         tok, lp = loop.step(logits, temperature, top_k, _uniforms(uniform_source, step + 1, B, dev, generator), active)
-        ended = active & (tok == eos_token_id)                                 # node.py:369-370: EOS is not recorded
+        ended = active & (tok == loop.stop)                                    # node.py:369-370: EOS is not recorded
         rows = np.nonzero(active & ~ended)[0]
         toks[rows, lens[rows]] = tok[rows]                                     # node.py:371-373
         lps[rows, lens[rows]] = lp[rows]
