@@ -2,6 +2,9 @@
 and the entry-point bookkeeping (restated in the oracle, node.py:391-461) on a stub model."""
 import asyncio
 import inspect
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -237,3 +240,12 @@ def test_judge_decode_without_an_eos_token(monkeypatch):
     logits = torch.eye(4)[[2, 0, 3]]
     got = dec.judge_decode(lambda tokens: logits, logits, 0.0, 3, None)
     assert [g["tokens"] for g in got] == [[2] * 3, [0] * 3, [3] * 3]
+
+
+def test_package_imports_without_a_gpu_build_of_torch():
+    """The parts that use no GPU (the wire format, the messages) need no GPU runtime in torch: its raw-stream getter may be
+    missing.  In a process of its own, as the package binds the getter at import."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(tome_amd.__file__)))
+    code = ("import torch\nif hasattr(torch._C, '_cuda_getCurrentRawStream'): del torch._C._cuda_getCurrentRawStream\n"
+            "import tome_amd\nassert tome_amd.Prompt('a', [1]).tokens == [1]\n")
+    subprocess.run([sys.executable, "-c", code], cwd=root, check=True, timeout=120)

@@ -91,13 +91,17 @@ def _row_valid(lead_shape, n_rows: int, lengths, row_valid, dev) -> Optional[tor
     return (torch.arange(L, device=dev).reshape(1, L) < ln).to(torch.int32).reshape(-1).contiguous()
 
 
-_current_raw_stream = torch._C._cuda_getCurrentRawStream   # a fraction of the cost of the Stream object
+# A fraction of the cost of the Stream object; a torch built without a GPU runtime does not have it, and imports this package for
+# the parts that need none.
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(t: torch.Tensor) -> int:
     """Raw hipStream_t of torch's current stream on ``t``'s GPU (the launch stream of every call); 0 for a CPU tensor,
     which the operators refuse."""
-    return _current_raw_stream(t.get_device()) if t.is_cuda else 0
+    if not t.is_cuda:
+        return 0
+    return _current_raw_stream(t.get_device()) if _current_raw_stream else torch.cuda.current_stream(t.device).cuda_stream
 
 
 def token_logprobs(logits: torch.Tensor, targets, temperature: float = 1.0, lengths=None, *,
