@@ -121,6 +121,7 @@ def _stepped_orderings(V, cell, kind):
     (torch.float32, 9, 3001, ["equal", "ascending", "plateau"]),
     (torch.bfloat16, 9, 6001, ["equal", "ascending", "plateau"]),
     # one workgroup a row, streamed
+    (torch.float32, 1500, 14335, ["normal", "equal", "ascending", "plateau"]),
     (torch.float32, 6100, 16421, ["normal", "equal", "ascending", "plateau"]),
     (torch.bfloat16, 2300, 20011, ["normal", "equal", "ascending", "plateau"]),
 ])

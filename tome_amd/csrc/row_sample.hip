@@ -932,6 +932,13 @@ bool row_sample_needs_workspace(int64_t rows, int64_t V, int vec) {
   int64_t s = (V + 8191) / 8192;
   const int64_t most_ranges = vec == 4 ? 18000 : 6500;   // rows * ranges: ~950 fp32 rows, ~340 bf16 rows at V = 151936
   if (rows * s > most_ranges) return row_splits_for(rows, V, vec) > 1;
+  // fp32 rows of a block of cells and part of a second one, by the thousand: two launches and a nearly empty workgroup a row cost
+  // more than one workgroup that streams the row.  Cells / streamed, us: 8200 elements 1500 rows 26.6 / 19.5, 12000 elements
+  // 1000 / 1500 / 4000 / 8000 rows 22.6 / 23.8, 31.3 / 27.9, 62.7 / 53.1, 115.1 / 90.5, 14000 elements 1000 / 1500 / 4000 rows 24.6 / 25.5,
+  // 33.7 / 31.7, 68.4 / 58.7; 15001 elements 2000 / 4000 rows 39.0 / 41.0, 65.6 / 62.9; 16384 elements 3000 / 4000 / 8000 rows
+  // 50.6 / 51.1, 65.3 / 63.2, 124.4 / 110.1.  (Ranges of 8192 elements kept in registers, the form before the cells, took 12000
+  // elements 21.2, 28.5, 58.6, 109.0.)
+  if (vec == 4 && V <= 16384 && rows >= (V <= 14336 ? 1500 : 3500)) return false;
   const int64_t fill = (512 + rows - 1) / rows;
   if (s < fill) s = fill;
   const int64_t max_by_work = (V / vec) / (2 * kRowWG);  // >= 2 load units per lane and split
