@@ -101,6 +101,7 @@ struct SampleLds {
   uint64_t thr4[kRowWaves];
   int cnt;
   int cnt2;
+  int kept;       // select_top_k's own count
   int wave_cnt[kRowWaves];
   RowLds red;
 };
@@ -158,30 +159,31 @@ __device__ __forceinline__ int wave_rank(uint64_t key, int m) {
 // largest from a sample: every wave ranks 64 keys of its own (256 distinct positions spread over the
 // buffer), and the smallest of the four ceil(k/4)-th largest has >= k sampled keys at or above it;
 // at least 32 sampled keys fall below it, so every round makes progress.
+//
+// The rounds count in sh.kept and leave sh.cnt alone: callers pass an `m` that every wave has just read from sh.cnt, with no barrier
+// in between, and a wave late at that read would see a cleared count, take another path and leave the others' barriers unpaired.
+// (A barrier at the head of the round is as safe, but costs the pick kernel's usual path, which never gets here, 0.27 us.)
 template <class Lds>
 __device__ uint64_t select_top_k(Lds& sh, uint64_t* cur, uint64_t* other, int m, int k) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   while (m > kRowWG) {
-    // Callers pass an `m` that every wave has just read from sh.cnt or sh.cnt2, and the round clears sh.cnt below: without this
-    // barrier a wave that is late at its read would see 0, take another path and leave the others' barriers unpaired.
-    __syncthreads();
     const uint64_t key = cur[(int)(((int64_t)tid * m) >> 8)];
     const int rank = wave_rank(key, 64);
     const int want = (k + kRowWaves - 1) / kRowWaves;
     if (lane == 0) sh.thr4[wave] = 0;  // stays 0 (no bound) when fewer than `want` sampled keys are real
     __builtin_amdgcn_wave_barrier();
     if (key != 0 && rank == want - 1) sh.thr4[wave] = key;
-    if (tid == 0) sh.cnt = 0;
+    if (tid == 0) sh.kept = 0;
     __syncthreads();
     uint64_t thr = sh.thr4[0];
 #pragma unroll
     for (int w = 1; w < kRowWaves; ++w) thr = sh.thr4[w] < thr ? sh.thr4[w] : thr;
     for (int i = tid; i < m; i += kRowWG) {
       const uint64_t key2 = cur[i];
-      if (key2 >= thr && key2 != 0) other[atomicAdd(&sh.cnt, 1)] = key2;
+      if (key2 >= thr && key2 != 0) other[atomicAdd(&sh.kept, 1)] = key2;
     }
     __syncthreads();
-    const int kept = sh.cnt;
+    const int kept = sh.kept;
     __syncthreads();
     if (kept == m) break;  // cannot happen for k <= 32 (see kSampMaxK); guards against an endless loop
     m = kept;
