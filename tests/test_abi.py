@@ -117,10 +117,9 @@ def test_argument_checks_run_on_host():
     assert samp(logits=None) == -1 and samp(tok=None) == -1 and samp(logits=P + 2) == -6
     assert samp(V=151936) == -4                                      # a small batch splits its rows: workspace needed
     assert lib.tome_row_sample_workspace(0, 4096, 151936, 20) == 0 and lib.tome_row_sample_workspace(0, 64, 151936, 20) > 0
-    # fp32 rows of up to 16384 elements stream (no workspace) in batches of 1500 and 3500 rows, by their length
-    for V, most in ((14336, 1499), (14337, 3499), (16384, 3499)):
-        assert lib.tome_row_sample_workspace(0, most, V, 20) > 0 and lib.tome_row_sample_workspace(0, most + 1, V, 20) == 0
-    assert lib.tome_row_sample_workspace(0, 4000, 16385, 20) > 0 and lib.tome_row_sample_workspace(1, 2000, 14336, 20) > 0
+    # fp32 rows of up to 13312 elements stream (no workspace) from 1500 rows on
+    assert lib.tome_row_sample_workspace(0, 1499, 13312, 20) > 0 and lib.tome_row_sample_workspace(0, 1500, 13312, 20) == 0
+    assert lib.tome_row_sample_workspace(0, 4000, 13313, 20) > 0 and lib.tome_row_sample_workspace(1, 2000, 13312, 20) > 0
     dual = lib.tome_grpo_dual(P, P, None, 8, 64, 100, 64, 64, P, None, 1.0, P, P, P, P, None, 0, None)
     assert dual == -1
     pair = lambda **k: lib.tome_grpo_pair(P, k.get("href", P), k.get("nw", None), k.get("eps", 1e-6), P, k.get("wref", P), 8, 64,

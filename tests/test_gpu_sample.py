@@ -105,7 +105,7 @@ def _stepped_orderings(V, cell, kind):
         x = (np.arange(V, dtype=np.float32) - (V - 1)) / 64
     elif kind == "plateau":                        # 700 equal maxima: they fit the buffer, but not one count
         x[rng.choice(V, 700, replace=False)] = 20.0
-    elif kind == "one_wave":                       # 600 equal cell maxima in the cells of one wave, five in the others'
+    elif kind == "one_wave":                       # up to 600 equal cell maxima in one wave's cells, nine in each of the others'
         cells = np.arange(V // cell)               # (cell c belongs to lane c % 256)
         mine = cells[cells % 256 // 64 == 1][:600]
         others = np.concatenate([64 * w + np.arange(9) for w in (0, 2, 3)])
@@ -114,14 +114,19 @@ def _stepped_orderings(V, cell, kind):
 
 
 @pytest.mark.parametrize("dtype,rows,V,kinds", [
-    # cells: between 529 and 2112 cells at or above the bound, more than 528 of them in one wave's quarter of the buffer
+    # cells: more of them at or above the bound in one wave than its quarter of the buffer holds, but not than all of it
     (torch.float32, 3, 151936, ["one_wave", "equal", "ascending"]),
     (torch.bfloat16, 3, 303872, ["one_wave", "equal", "ascending"]),
+    # ... at the most blocks of cells (8) that the small instantiation of the second launch takes, and one more
+    (torch.float32, 4, 65536, ["normal", "one_wave", "equal", "ascending"]),
+    (torch.float32, 4, 65541, ["normal", "one_wave", "equal", "ascending"]),
+    (torch.bfloat16, 4, 131072, ["normal", "one_wave", "equal", "ascending"]),
+    (torch.bfloat16, 4, 131081, ["normal", "one_wave", "equal", "ascending"]),
     # one workgroup a row, the row in registers
     (torch.float32, 9, 3001, ["equal", "ascending", "plateau"]),
     (torch.bfloat16, 9, 6001, ["equal", "ascending", "plateau"]),
     # one workgroup a row, streamed
-    (torch.float32, 1500, 14335, ["normal", "equal", "ascending", "plateau"]),
+    (torch.float32, 1500, 13311, ["normal", "equal", "ascending", "plateau"]),
     (torch.float32, 6100, 16421, ["normal", "equal", "ascending", "plateau"]),
     (torch.bfloat16, 2300, 20011, ["normal", "equal", "ascending", "plateau"]),
 ])

@@ -48,8 +48,9 @@ namespace tome {
 constexpr int kSampCap = 1024;      // candidate keys per buffer in the main kernel (2 x 8 KB of LDS: 8 workgroups per CU)
 constexpr int kCellUnits = 8;       // load units per cell: consecutive, one 128-byte line
 constexpr int kCellBlock = kCellUnits * kRowWG;  // load units a workgroup of the cells kernel takes at a time (256 cells)
-// Keys per buffer of the pick kernel: k <= 32 cells of 8 units of up to 8 elements, and the single elements of the edges.
-constexpr int kSampPickCap = 32 * kCellUnits * 8 + 64;
+// Keys per buffer of the pick kernel: k <= 32 cells of 8 units, and the single elements of the edges.
+template <typename T>
+constexpr int kSampPickCap = 32 * kCellUnits * Elem<T>::kVec + 64;
 constexpr int kSampCached = 8;      // a lane keeps up to this many load units in registers between the passes
 constexpr int kSampMaxK = 32;  // one tightening round is then sure to drop >= 32 of the 64 sampled keys
 
@@ -698,13 +699,18 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 // Second launch: one workgroup per row takes the best cells, reads them, ranks their elements and draws.  Its time is that of
 // one chain of dependent steps run once per workgroup, the code fetched cold: loads come first and unconditionally, the usual
 // path is short and straight, whatever does not follow from the common case sits behind a branch at its end.
-template <typename T>
+// In batches of 1000 rows and more it is bound by how many rows are in flight: rows of up to 8 blocks of cells take an
+// instantiation that holds 8 maxima a lane instead of 32 (53 VGPRs instead of 90), and the candidate buffers have the size the
+// element type needs (fp32 18 KB of LDS instead of 34): 8 workgroups a CU instead of 4 in fp32.  Both launches, us: fp32 65536
+// elements x 1400 / 2000 rows 74.9 -> 71.8, 103.7 -> 99.8, 24000 x 6000 132.9 -> 121.3, 12000 x 1000 22.2 -> 21.3; bf16 24000 x 1000
+// 24.0 -> 22.8, 65536 x 700 23.9 -> 23.0; rows above 8 blocks unchanged.
+template <typename T, int kHold>                 // kHold: cell maxima a lane keeps (a multiple of 8)
 __global__ __launch_bounds__(kRowWG) void row_sample_pick_kernel(SampleArgs a) {
   constexpr int kVec = Elem<T>::kVec;
-  constexpr int kHold = 32;                      // cell maxima a lane keeps: 8192 cells a row
+  constexpr int kCap = kSampPickCap<T>;
   constexpr int kStats = 64 * kRowWaves / 64;    // partial statistics per lane of wave 0 (splits <= 64)
-  constexpr int kWaveCap = kSampPickCap / kRowWaves;
-  __shared__ SampleLds<kSampPickCap> sh;
+  constexpr int kWaveCap = kCap / kRowWaves;
+  __shared__ SampleLds<kCap> sh;
   const int64_t r = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int k = a.top_k;
@@ -806,7 +812,7 @@ __global__ __launch_bounds__(kRowWG) void row_sample_pick_kernel(SampleArgs a) {
     for (int i = 0; i < decltype(n)::value; ++i) {
       if (pass[i] == 0) continue;
       const int pos = at + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(pass[i] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)pass[i], 0u));
-      if (e[i] >= least && pos < kSampPickCap) sh.b[pos] = make_key(e[i], (uint32_t)index_of(i));
+      if (e[i] >= least && pos < kCap) sh.b[pos] = make_key(e[i], (uint32_t)index_of(i));
       at += __builtin_popcountll(pass[i]);
     }
   };
@@ -842,7 +848,7 @@ __global__ __launch_bounds__(kRowWG) void row_sample_pick_kernel(SampleArgs a) {
     st.mx = mx;
     st.s = sum;
   };
-  int m = kSampPickCap + 1;
+  int m = kCap + 1;
   if (__builtin_expect(n_best <= 64, 1)) {
     const int64_t c0 = group < n_best ? (int64_t)(uint32_t)region_entry(sh.a, kWaveCap, n_wave, group) : -1;
     const u32x4 v0 = load_unit(c0);
@@ -859,7 +865,7 @@ __global__ __launch_bounds__(kRowWG) void row_sample_pick_kernel(SampleArgs a) {
     __syncthreads();
     m = sh.cnt2;
   }
-  if (__builtin_expect(m > kSampPickCap, 0)) {
+  if (__builtin_expect(m > kCap, 0)) {
     // Far more cells or elements than k at or above the bound (many equal ones, or the large ones all in a few lanes): the k
     // best cells by whole keys, and the elements of those alone, which always fit.
     if (wave == 0) merge_stats();
@@ -880,15 +886,15 @@ __global__ __launch_bounds__(kRowWG) void row_sample_pick_kernel(SampleArgs a) {
           const uint64_t key = make_key(w, (uint32_t)(q * kRowWG + slot));
           if (w > -INFINITY && key >= theta) {
             const int pos = atomicAdd(&sh.cnt, 1);
-            if (pos < kSampPickCap) sh.b[pos] = key;
+            if (pos < kCap) sh.b[pos] = key;
           }
         }
         __syncthreads();
         n_best = sh.cnt;
-        if (n_best <= kSampPickCap) break;
+        if (n_best <= kCap) break;
         // Overflow: the k-th largest of the keys that were kept is a strictly higher lower bound.
         __syncthreads();
-        theta = select_top_k(sh, sh.b, sh.a, kSampPickCap, k);
+        theta = select_top_k(sh, sh.b, sh.a, kCap, k);
       }
     }
     select_top_k(sh, sh.b, sh.a, n_best, k);
@@ -935,12 +941,11 @@ bool row_sample_needs_workspace(int64_t rows, int64_t V, int vec) {
   const int64_t most_ranges = vec == 4 ? 18000 : 6500;   // rows * ranges: ~950 fp32 rows, ~340 bf16 rows at V = 151936
   if (rows * s > most_ranges) return row_splits_for(rows, V, vec) > 1;
   // fp32 rows of a block of cells and part of a second one, by the thousand: two launches and a nearly empty workgroup a row cost
-  // more than one workgroup that streams the row.  Cells / streamed, us: 8200 elements 1500 rows 26.6 / 19.5, 12000 elements
-  // 1000 / 1500 / 4000 / 8000 rows 22.6 / 23.8, 31.3 / 27.9, 62.7 / 53.1, 115.1 / 90.5, 14000 elements 1000 / 1500 / 4000 rows 24.6 / 25.5,
-  // 33.7 / 31.7, 68.4 / 58.7; 15001 elements 2000 / 4000 rows 39.0 / 41.0, 65.6 / 62.9; 16384 elements 3000 / 4000 / 8000 rows
-  // 50.6 / 51.1, 65.3 / 63.2, 124.4 / 110.1.  (Ranges of 8192 elements kept in registers, the form before the cells, took 12000
-  // elements 21.2, 28.5, 58.6, 109.0.)
-  if (vec == 4 && V <= 16384 && rows >= (V <= 14336 ? 1500 : 3500)) return false;
+  // more than one workgroup that streams the row.  Cells / streamed, us: 8200 elements 1500 rows 24.3 / 20.0, 12000 elements
+  // 1000 / 1500 / 2000 / 4000 / 6000 rows 21.3 / 23.8, 27.7 / 27.5, 35.2 / 36.4, 56.4 / 53.0, 79.4 / 72.6, 13000 elements 1500 / 4000
+  // rows 28.8 / 28.6, 59.8 / 53.8; 14000 elements 2000 / 4000 rows 36.6 / 38.2, 60.4 / 58.3; 16384 elements 4000 rows 58.8 / 63.2.
+  // (Ranges of 8192 elements kept in registers, the form before the cells, took 12000 elements 21.8, 28.8, 33.3, 58.5, 84.0.)
+  if (vec == 4 && V <= 13312 && rows >= 1500) return false;
   const int64_t fill = (512 + rows - 1) / rows;
   if (s < fill) s = fill;
   const int64_t max_by_work = (V / vec) / (2 * kRowWG);  // >= 2 load units per lane and split
@@ -1016,8 +1021,12 @@ hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_
     else hipLaunchKernelGGL((row_sample_cells_kernel<uint16_t>), grid, block, 0, stream, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (dtype == 0) hipLaunchKernelGGL((row_sample_pick_kernel<float>), dim3((unsigned)rows), block, 0, stream, a);
-    else hipLaunchKernelGGL((row_sample_pick_kernel<uint16_t>), dim3((unsigned)rows), block, 0, stream, a);
+    const bool few = p.n_cells <= 8 * kRowWG;
+    const dim3 pick_grid((unsigned)rows);
+    if (dtype == 0 && few) hipLaunchKernelGGL((row_sample_pick_kernel<float, 8>), pick_grid, block, 0, stream, a);
+    else if (dtype == 0) hipLaunchKernelGGL((row_sample_pick_kernel<float, 32>), pick_grid, block, 0, stream, a);
+    else if (few) hipLaunchKernelGGL((row_sample_pick_kernel<uint16_t, 8>), pick_grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((row_sample_pick_kernel<uint16_t, 32>), pick_grid, block, 0, stream, a);
     return hipGetLastError();
   }
   const dim3 grid((unsigned)rows);
