@@ -444,3 +444,20 @@ def test_full_log_softmax_one_launch_at_the_edges_of_its_stores(dev, dtype, rows
             want = (zt - lse.to(dtype).float()).to(dtype).float()
             diff = (out[r0:r0 + 32].float() - want).abs()
             assert float(diff.max()) <= 0.125 + 1e-6 and float((diff == 0).float().mean()) > 0.99
+
+
+@pytest.mark.parametrize("rows", [1, 256, 257, 515])
+@pytest.mark.parametrize("V", [16384, 16391, 40001, 65535, 65536])
+def test_full_log_softmax_bf16_rows_of_two_workgroups_a_cu(dev, rows, V):
+    """bf16 rows of up to 65536 elements on either side of the batch size from which two workgroups share a CU, from the
+    shortest row of the one-launch form to the longest, with and without single elements at the ends.  As above."""
+    g = torch.Generator(device=dev).manual_seed(rows + V)
+    x = torch.empty((rows, V), dtype=torch.bfloat16, device=dev).normal_(0.0, 2.0, generator=g)
+    x[rows // 2, V - 1] = 14.0
+    x[rows // 3, 0] = 14.0
+    for T in (1.0, 0.9):
+        z = x.double() / T
+        zt = (x.float() * (1.0 / T)).to(torch.bfloat16).float()
+        want = (zt - torch.logsumexp(z, -1, keepdim=True).to(torch.bfloat16).float()).to(torch.bfloat16).float()
+        diff = (tome_amd.fused_log_softmax(x, T).float() - want).abs()
+        assert float(diff.max()) <= 0.125 + 1e-6 and float((diff == 0).float().mean()) > 0.99

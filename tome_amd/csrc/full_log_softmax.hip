@@ -126,8 +126,13 @@ __global__ __launch_bounds__(kFullWG) void full_log_softmax_kernel(FullArgs a) {
 // With a single workgroup on the CU nothing else covers its arithmetic, so every lane keeps a running (maximum, sum) of
 // its own and takes in each unit as it arrives (the row kernel's online update) instead of a sweep for the maximum, a
 // barrier and a sweep for the sum after the last byte has landed; the lanes' states are merged through one barrier.
-template <int CH>
-__global__ __launch_bounds__(1024) void full_log_softmax_onepass_kernel(FullArgs a) {
+//
+// Rows of up to 65536 elements need 64 registers a lane, so that two workgroups share a CU and one's loads run under the
+// other's arithmetic: batches of more than 256 rows take an instantiation held to that (at 69 registers, one workgroup a CU:
+// 512 / 1024 / 2048 rows of 32000 13.4 -> 11.1, 26.3 -> 23.9, 51.7 -> 44.9 us, 4096 x 16384 65.4 -> 51.2, 512 x 65536 25.2 -> 22.2).
+// Smaller batches have a CU per row and are 0.1 us faster without the limit.
+template <int CH, int WAVES>  // WAVES per SIMD: 4, or 8 for two workgroups on a CU
+__global__ __launch_bounds__(1024, WAVES) void full_log_softmax_onepass_kernel(FullArgs a) {
   constexpr int kWaves = 16;
   __shared__ float red_m[kWaves], red_s[kWaves];
   const int64_t r = blockIdx.x;
@@ -144,9 +149,10 @@ __global__ __launch_bounds__(1024) void full_log_softmax_onepass_kernel(FullArgs
   const float scale = a.scale;
   u32x4 v[CH];
 #pragma unroll
-  for (int q = 0; q < CH; ++q) {  // unconditional (clamped) loads; unit 0 exists (checked on the host)
+  for (int q = 0; q < CH; ++q) {  // unconditional (clamped) loads; a whole unit exists (checked on the host)
     const int u = tid + q * 1024;
-    v[q] = load_unit(src, (int64_t)(u < n_units ? u : 0) * 16);
+    if constexpr (WAVES == 8) v[q] = load_unit(src, (uint32_t)min(u, n_units - 1) * 16u);  // (64 registers without a spill)
+    else v[q] = load_unit(src, (int64_t)(u < n_units ? u : 0) * 16);
   }
   // the lane's running maximum (floored like every kernel of this path) and sum of 2^((x - maximum) * scale)
   float lm = kMaxFloor, ls = 0.f;
@@ -405,8 +411,13 @@ hipError_t full_log_softmax_onepass_launch(const void* in, void* out, int dtype,
     else hipLaunchKernelGGL((full_log_softmax_row_kernel<float, 17, 9, 3>), grid, block, 0, stream, a);
   } else if (V / 8 > (int64_t)kOnePassUnits * 1024) {
     hipLaunchKernelGGL((full_log_softmax_row_kernel<uint16_t, 17, 9, 3>), grid, block, 0, stream, a);
-  } else if (V / 8 <= 8 * 1024) hipLaunchKernelGGL((full_log_softmax_onepass_kernel<8>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((full_log_softmax_onepass_kernel<kOnePassUnits>), grid, block, 0, stream, a);
+  } else if (V / 8 > 8 * 1024) {
+    hipLaunchKernelGGL((full_log_softmax_onepass_kernel<kOnePassUnits, 4>), grid, block, 0, stream, a);
+  } else if (rows > 256) {
+    hipLaunchKernelGGL((full_log_softmax_onepass_kernel<8, 8>), grid, block, 0, stream, a);
+  } else {
+    hipLaunchKernelGGL((full_log_softmax_onepass_kernel<8, 4>), grid, block, 0, stream, a);
+  }
   return hipGetLastError();
 }
 
