@@ -71,8 +71,12 @@ __device__ __forceinline__ T log_softmax_one(T x, float inv_temp, float lse_t) {
 
 template <bool BF16, int UNROLL = kFullUnroll>
 __global__ __launch_bounds__(kFullWG) void full_log_softmax_kernel(FullArgs a) {
-  const int64_t r = blockIdx.x / a.chunks;
-  const int chunk = blockIdx.x % a.chunks;
+  int64_t r = blockIdx.x;  // (no division for short rows, as in the row kernel)
+  int chunk = 0;
+  if (a.chunks > 1) {
+    r = blockIdx.x / a.chunks;
+    chunk = blockIdx.x % a.chunks;
+  }
   float lse;
   if (a.splits > 1) {  // merge the row's partials (at most 64: one per lane of wave 0)
     __shared__ float lse_sh;
@@ -98,9 +102,12 @@ __global__ __launch_bounds__(kFullWG) void full_log_softmax_kernel(FullArgs a) {
   T* out_row = static_cast<T*>(a.out) + r * a.out_stride;
   const RowSpan<T> sp(out_row, a.V);
   const int64_t n_units = sp.n_units;
-  const int64_t per = (n_units + a.chunks - 1) / a.chunks;
-  const int64_t u0 = per * chunk;
-  const int64_t u1 = (u0 + per < n_units) ? u0 + per : n_units;
+  int64_t u0 = 0, u1 = n_units;
+  if (a.chunks > 1) {
+    const int per = ((int)n_units + a.chunks - 1) / a.chunks;
+    u0 = (int64_t)per * chunk;
+    u1 = u0 + per < n_units ? u0 + per : n_units;
+  }
   const float lse_t = BF16 ? bf16_rt(lse) : lse;
 
   const T* src = in_row + sp.head;

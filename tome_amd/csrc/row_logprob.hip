@@ -80,9 +80,15 @@ __global__ __launch_bounds__(WAVES * 64) void row_logprob_kernel(RowArgs a) {
   constexpr int kVec = Elem<T>::kVec;
   constexpr int kWG = WAVES * 64;
   __shared__ RowLdsT<WAVES> lds;
-  const int64_t r = blockIdx.x / a.splits;  // problem index
-  const int split = blockIdx.x % a.splits;
   const int tid = threadIdx.x;
+  // No division for rows that are not split, and a 32-bit one for those that are: batches of short rows are bound by what a
+  // workgroup does around its few loads (32768 x 300 fp32 60.8 -> 49.8 us, bf16 61.8 -> 51.2; 32768 x 2048 78.4 -> 61.9 and 69.7 -> 56.7).
+  int64_t r = blockIdx.x;  // problem index
+  int split = 0;
+  if (a.splits > 1) {
+    r = blockIdx.x / a.splits;
+    split = blockIdx.x % a.splits;
+  }
 
   if (!a.sel.valid(r)) {  // masked row: not read, outputs zeroed
     if (split == 0 && tid == 0) {
@@ -106,9 +112,12 @@ __global__ __launch_bounds__(WAVES * 64) void row_logprob_kernel(RowArgs a) {
 
   const T* row = static_cast<const T*>(a.logits) + src * a.row_stride;
   const RowSpan<T> sp(row, a.V);
-  const int64_t per_split = (sp.n_units + a.splits - 1) / a.splits;
-  const int64_t u0 = per_split * split;
-  const int64_t u1 = (u0 + per_split < sp.n_units) ? u0 + per_split : sp.n_units;
+  int64_t u0 = 0, u1 = sp.n_units;
+  if (a.splits > 1) {
+    const int per_split = ((int)sp.n_units + a.splits - 1) / a.splits;  // (a row has fewer than 2^29 units)
+    u0 = (int64_t)per_split * split;
+    u1 = u0 + per_split < sp.n_units ? u0 + per_split : sp.n_units;
+  }
 
   float x_t = 0.f;
   if (tid == 0 && a.splits == 1) x_t = load_target_logit<T>(a, row, r);
