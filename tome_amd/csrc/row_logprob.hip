@@ -7,7 +7,7 @@
 //
 // Grid: rows * splits workgroups of 4 wave64, or rows workgroups of 8 or 16 (row_waves_unsplit).  A workgroup owns a contiguous
 // range of 16-byte load units of one row (RowSpan: units start at the row's first 16-byte boundary), every lane keeps an online (max, sum 2^(y-m))
-// pair over the units it reads, lanes are merged by DPP and row swaps, the
+// pair over the units it reads, lanes are merged by DPP and LDS-crossbar exchanges, the
 // waves through LDS.  splits == 1 finishes in the same launch; otherwise per-split
 // partials go to the workspace and row_combine_kernel merges them (no float atomics, so
 // results do not depend on scheduling).
