@@ -150,3 +150,38 @@ def test_sample_step_draws_as_sample_tokens_does(dev):
     torch.cuda.synchronize()
     assert torch.equal(got, want.long()) and torch.equal(host[0], want.cpu())
     assert len(got.unique()) == 4
+
+
+@pytest.mark.parametrize("loop", ["rollout", "judge"])
+@pytest.mark.parametrize("temperature", [0.0, 0.8])
+def test_decode_loops_on_the_gpu_refuse_a_row_without_a_token(dev, loop, temperature):
+    """An active row whose logits are all -inf at the second step: RuntimeError names it, and its -1 has not been fed to the
+    model.  A finished row with such logits is not read."""
+    B, V_small, eos = 3, 40, 9
+    first = torch.zeros((B, V_small), device=dev)
+    first[:, 4] = 50.0
+    seen = []
+
+    def model_step(tokens, bad, at):
+        seen.append(tokens.tolist())
+        out = torch.zeros((B, V_small), device=dev)
+        out[:, 5] = 50.0
+        if len(seen) == 1:
+            out[2, eos] = 90.0                                         # row 2 ends at the first step
+        if len(seen) == at:
+            out[bad] = float("-inf")
+        return out
+
+    def run(bad, at):
+        seen.clear()
+        step = lambda tokens: model_step(tokens, bad, at)
+        if loop == "rollout":
+            return tome_amd.rollout_decode(step, first, 1, temperature, 5, eos)
+        return tome_amd.judge_decode(step, first, temperature, 5, eos)
+
+    with pytest.raises(RuntimeError, match=r"rows \[1\]"):
+        run(1, 2)
+    idle = eos if loop == "rollout" else 0
+    assert seen == [[4, 4, 4], [5, 5, idle]]
+    done = run(2, 2)                                                   # the row that has ended
+    assert [d["tokens"] for d in done] == [[4, 5, 5, 5, 5]] * 2 + ([[4, eos]] if loop == "rollout" else [[4]])

@@ -155,10 +155,11 @@ def test_sampler_buffers_overflow(dev, dtype, rows, V, kinds):
     np.testing.assert_allclose(got.lp.cpu().numpy(), p64[w, tok] / T + lse[w], atol=1e-4, rtol=0)
 
 
-@pytest.mark.parametrize("rows,V,dtype", [(2300, 65536, torch.float32), (1700, 32768, torch.bfloat16)])
+@pytest.mark.parametrize("rows,V,dtype", [(2300, 65536, torch.float32), (1700, 32768, torch.bfloat16), (4400, 31999, torch.bfloat16)])
 def test_sampler_streams_large_batches(dev, rows, V, dtype):
     """Batches beyond ~950 fp32 / ~340 bf16 rows of 151936 (counted in ranges of 8192 elements) take one streaming
-    workgroup per row; at that size the check runs on the GPU: the candidates' logits against torch.topk (values: ids
+    workgroup per row (bf16 rows of 32000 elements and more, as 1700 x 32768, still go through cells up to 2^28
+    elements a batch); at that size the check runs on the GPU: the candidates' logits against torch.topk (values: ids
     may differ among equal logits), the greedy id against torch.argmax wherever the maximum is unique, the log-prob of
     the drawn id against the row kernel."""
     k = 20
@@ -200,8 +201,8 @@ def test_sampler_ties_take_lower_ids_first(dev):
 
 @pytest.mark.parametrize("pattern", ["ascending", "descending", "sawtooth", "one_lane"])
 def test_sampler_adversarial_orderings(dev, pattern):
-    """Orderings that defeat the first bound (the k-th largest lane maximum): the candidate buffer overflows
-    and the kernel has to tighten the bound and rescan; the result must not change."""
+    """Orderings that defeat the first bound (the k-th largest lane maximum) in a decode batch: more cells than their buffer
+    holds, or all in one lane; the result must not change.  (test_sampler_buffers_overflow has the kernels of one workgroup a row.)"""
     V, k = 151936, 20
     base = np.arange(V, dtype=np.float32) * 1e-4
     if pattern == "ascending":
