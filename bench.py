@@ -239,6 +239,23 @@ def timing_fields(t):
     return d
 
 
+# What the printed line keeps of a leg behind the headline (--detail keeps all of it): the whole line had outgrown what keepers
+# of a run's output store.
+LEG_FIELDS = ("value", "unit", "ms_per_step", "sclk_mhz", "power_w", "frac", "achieved", "bound", "frac_of_sustained", "host_us_per_chunk",
+              "torch_mul_same_bytes_ms", "torch_log_softmax_ms")
+
+
+def short(obj, leg=False):
+    """An object of the bench line as it is printed: numbers to six digits; of a leg behind the headline LEG_FIELDS, its own
+    and those of what it holds (its shapes), in the same places."""
+    if isinstance(obj, float):
+        return float(f"{obj:.6g}")
+    if not isinstance(obj, dict):
+        return obj
+    kept = {k: short(v, leg) for k, v in obj.items() if not leg or k in LEG_FIELDS or isinstance(v, dict)}
+    return {k: v for k, v in kept.items() if v != {}}
+
+
 def hbm_roofline(nbytes, ms, traffic, kernel):
     gbs = nbytes / (ms * 1e-3) / 1e9
     return {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS,
@@ -560,8 +577,7 @@ def bench_lora(dev, steps, warmup):
 
 def bench_full_matrix(dev, steps, warmup, rows, dtype_name):
     """tome_full_log_softmax, the drop-in of fused_log_softmax (mlx-impl/model.py:77-89): the whole [rows, V] matrix
-    of log-probs in the input dtype.  Algorithmic bytes: 3 * V * sizeof(T) per row with two passes (one read for the row's
-    lse, one read and one write of the matrix), 2 * V * sizeof(T) where the one-pass kernel applies.  The small shape
+    of log-probs in the input dtype.  Algorithmic bytes: 2 * V * sizeof(T) per row (one read, one write).  The small shape
     rotates through 16 input / output pairs so that rows come from HBM, not from the last-level cache."""
     import torch
     import tome_amd
@@ -596,9 +612,9 @@ def bench_full_matrix(dev, steps, warmup, rows, dtype_name):
     tol = 1e-4 if dtype_name == "f32" else 0.25                              # bf16 output and subtraction: two ulps at |x| in [16, 32)
     assert (outs[0][sample].double() - want).abs().max().item() <= tol
     tm = time_steps(step, steps, warmup)
-    # bf16 rows of up to 155648 elements take the one-pass kernel (the row stays in a workgroup's registers): read once,
-    # written once.  Everything else is two passes: read for the row's lse, read again and written.
-    passes = 2 if (dtype_name == "bf16" and V >= 16384 and V // 8 <= 19 * 1024) else 3
+    # Both shapes are one launch whose rows stay on the chip: read once and written once (the fp32 kernel reads the third of a
+    # row that does not fit a second time, which is not counted).
+    passes = 2
     tm.update({"rows": rows, "bytes": passes * rows * V * esize, "passes_over_the_matrix": passes,
                "bytes_if_three_passes": 3 * rows * V * esize})
     if nbuf == 1:
@@ -836,6 +852,7 @@ def main():
     ap.add_argument("--row-variant", choices=["both", "mask", "list", "all"], default="both",
                     help="time config 2 with its padding mask, with the valid rows as a packed list, without the mask, "
                          "or all three (profiling runs pick one)")
+    ap.add_argument("--detail", default=None, help="also write the line with every field of every leg to this file")
     ap.add_argument("--calibrate-copy", action="store_true",
                     help="also run a plain 1 GiB device copy, so a counter run can scale FETCH_SIZE / WRITE_SIZE")
     args = ap.parse_args()
@@ -951,8 +968,7 @@ def main():
                                           "gbs_if_priced_on_three_passes": t["bytes_if_three_passes"] / (t["ms"] * 1e-3) / 1e9,
                                           "roofline": hbm_roofline(
                 t["bytes"], t["ms"], traffic_of(f"full_log_softmax_{rows}rows_{dn}"),
-                "full_log_softmax_onepass_kernel" if t["passes_over_the_matrix"] == 2 else
-                "row_logprob_kernel (lse partials) + full_log_softmax_kernel")}
+                "full_log_softmax_onepass_kernel" if dn == "bf16" else "full_log_softmax_row_kernel")}
             log(f"full matrix {rows} x {V} {dn}: {t['ms'] * 1e3:.1f} us, {shapes[f'{rows}x{V}_{dn}']['roofline']['frac']:.3f} of HBM peak")
             torch.cuda.empty_cache()
         big = shapes[f"4096x{V}_bf16"]
@@ -961,7 +977,7 @@ def main():
             **{k: big[k] for k in ("ms_per_step", "median_ms", "min_ms", "settle_launches")}, "dtype": "f32", "input_dtype": "bf16",
             "config": {"workload": "tome_full_log_softmax, the drop-in of fused_log_softmax (model.py:77-89): the whole log-prob matrix in the "
                                    "input dtype; [4096, 151936] bf16 (one pass: the row stays in a workgroup's registers, 2 V sizeof(T) bytes per row) "
-                                   "and [64, 151936] fp32 (the callers' dtype; two passes, 3 V sizeof(T) bytes per row; 16 rotating buffers)",
+                                   "and [64, 151936] fp32 (the callers' dtype; one launch, the row in registers and LDS; 16 rotating buffers)",
                        "shapes": shapes},
             "roofline": big["roofline"]}
         done("full_log_softmax")
@@ -1129,7 +1145,11 @@ def main():
             line[name] = obj
     if cpu is not None:
         line["cpu_baseline"] = cpu
-    print(json.dumps(line), flush=True)
+    if args.detail:
+        with open(args.detail, "w") as f:
+            json.dump(line, f, indent=1)
+    secondary = {name for name in legs if name != first}
+    print(json.dumps({k: short(v, k in secondary) for k, v in line.items()}), flush=True)
 
 
 if __name__ == "__main__":

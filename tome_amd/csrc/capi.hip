@@ -269,7 +269,7 @@ int tome_full_log_softmax(const void* logits, void* out, int dtype, int64_t rows
   const int esize = dtype == TOME_F32 ? 4 : 2;
   if (reinterpret_cast<uintptr_t>(logits) % esize != 0 || reinterpret_cast<uintptr_t>(out) % esize != 0) return TOME_E_ALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // bf16 rows that fit one workgroup's registers: read once, written once
+  // rows of 16384 to 524288 elements, but for small batches: one launch, the row kept in a workgroup's registers (and LDS)
   if (tome::full_log_softmax_one_pass(dtype, rows, V))
     return hip_result(tome::full_log_softmax_onepass_launch(logits, out, dtype, rows, V, in_row_stride, out_row_stride, temperature,
                                                             row_lse, s));
