@@ -23,9 +23,9 @@
 // and load unit is then paid per element, and the selection is done once a row instead of once a range (the form before:
 // every workgroup ranked the candidates of its range, a second launch merged splits * k keys).
 // Two launches either way; 64 x 151936 fp32 20.2 -> 15 us (6.5 streaming, 7 picking), 8 rows 14.6 -> 10, 64 x 50257 25 -> 11; bf16 64 x 151936
-// 20.4 -> 13, 256 rows 40 -> 23, 700 rows 67 -> 47, 1024 x 50257 172 -> 31.  These are rows
-// that the memory-side cache still holds; on rotating buffers the streaming launch takes 9.7 us (38.9 MB, 4.0 TB/s).  The other one is a chain of some 12000 cycles: kernel arguments and first loads 1500, cell maxima 1700,
-// the bound 1500, cells collected 1800, partial statistics 1200 (beside the elements' load), elements 1000, ranks 1100, draw 1000.
+// 20.4 -> 13, 256 rows 40 -> 23, 700 rows 67 -> 47, 1024 x 50257 172 -> 31.  (Rows that the memory-side cache still holds; on
+// rotating buffers the streaming launch takes 9.7 us, 38.9 MB at 4.0 TB/s.)  The other launch is a chain of some 12000 cycles: kernel
+// arguments and first loads 1500, cell maxima 1700, the bound 1500, cells collected 1800, partial statistics 1200 (beside the elements' load), elements 1000, ranks 1100, draw 1000.
 //
 // Large batches (row_sample_kernel, one workgroup a row, no workspace): per row,
 //   * the online (max, sum 2^(y-m)) for the full-vocabulary lse and every lane's own largest element;
