@@ -209,10 +209,10 @@ std::tuple<Tensor, Tensor, Tensor, MaybeTensor, MaybeTensor> sample_tokens(const
 }
 
 // One step of a decode loop: `active` int32 [rows] on the GPU (updated), `host` int32 [2, rows] in page-locked memory or on the GPU
-// (receives tokens and log-probs once the stream is synchronised); both dense: the kernel is given their addresses.  Returns the
-// next step's int64 input ids.
+// (receives tokens and log-probs once the stream is synchronised); both dense: the kernel is given their addresses.  `pinned`: the
+// caller has allocated `host` page-locked itself (asking the runtime costs 0.2 us a call).  Returns the next step's int64 input ids.
 Tensor sample_step(const Tensor& logits, double temperature, int64_t top_k, const MaybeTensor& uniforms, const Tensor& active,
-                   const Tensor& host, int64_t stop_token, int64_t idle_token, uintptr_t stream) {
+                   const Tensor& host, int64_t stop_token, int64_t idle_token, bool pinned, uintptr_t stream) {
   require_gpu(logits);
   const c10::Device dev = logits.device();
   const int dtype = dtype_code(logits);
@@ -227,7 +227,7 @@ Tensor sample_step(const Tensor& logits, double temperature, int64_t top_k, cons
   if (host.numel() != 2 * rows)
     throw py::value_error("host must hold two values per sequence (" + std::to_string(2 * rows) + "), got " + std::to_string(host.numel()));
   if (!active.is_contiguous() || !host.is_contiguous()) throw py::value_error("active and host must be contiguous");
-  if (rows > 0 && host.device() != dev && !(host.is_cpu() && host.is_pinned()))
+  if (rows > 0 && host.device() != dev && !(host.is_cpu() && (pinned || host.is_pinned())))
     throw py::value_error("host must be page-locked memory or on " + str(dev) + ": the GPU writes to it");
   Tensor u;
   if (uniforms) {

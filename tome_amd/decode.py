@@ -17,7 +17,8 @@ from typing import Callable, List, Optional
 import numpy as np
 import torch
 
-from .logprob import sample_step, sample_tokens
+from . import _lib
+from .logprob import _check_temperature, _stream, sample_tokens
 
 UniformSource = Callable[[int, int], torch.Tensor]
 
@@ -55,8 +56,8 @@ class _Loop:
         if temperature <= 0:
             uniforms = None
         if self.on_gpu:
-            self.next = sample_step(logits, temperature, top_k, uniforms, self.active, self.host,
-                                    self.stop if active is not None else -1, self.idle)
+            self.next = _lib.torch_ops().sample_step(logits, _check_temperature(temperature or 1.0), int(top_k), uniforms, self.active,
+                                                     self.host, self.stop if active is not None else -1, self.idle, True, _stream(logits))
             torch.cuda.current_stream(self.dev).synchronize()
             host = self.host_np
         else:

@@ -176,7 +176,7 @@ def sample_step(logits: torch.Tensor, temperature: float, top_k: int, uniforms, 
     ``temperature`` and ``uniforms`` as in ``sample_tokens``: 0 is greedy, uniforms are drawn when omitted."""
     temperature, uniforms = _draw(logits, temperature, uniforms, None)
     return _lib.torch_ops().sample_step(logits, temperature, int(top_k), _tensor(uniforms, logits), active, host, int(stop_token),
-                                        int(idle_token), _stream(logits))
+                                        int(idle_token), False, _stream(logits))
 
 
 class DecodeStepGraph:
