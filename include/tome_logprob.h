@@ -206,15 +206,15 @@ int tome_full_log_softmax(const void* logits, void* out, int dtype, int64_t rows
  *
  * Process-wide state of the library, all of it caches that do not change results and all of it kept per
  * device ordinal: the CU count (one workgroup per CU for batches of up to 128 tokens), a flag per large-LDS
- * kernel ("dynamic LDS limit raised", and "the 160 KB of the three-buffer sweep were refused": the two-buffer
+ * kernel ("dynamic LDS limit raised"), "the 160 KB of the three-buffer sweep were refused" (the two-buffer
  * sweep then serves), the device address of tome_row_logprob_noalloc's array; and the
  * two testing hooks (the selector below, tome_row_logprob_noalloc_limit).
  */
 /* Testing and tuning hook, no counterpart in the reference: kind 0 / 1 makes the fused entry points take
  * the generic / LDS-DMA sweep kernel wherever its shape rules allow, 3 the LDS-DMA kernel with every vocab
  * range cut at whole 256-row tiles (no 224-row tiles, no mixed tile heights), 4 / 5 the LDS-DMA kernel with its
- * 256-token tile on two / three W buffers whatever the shape, -1 (the default, also for any other value)
- * picks by shape.  Process-wide; set it while no call of this library is running; not for
+ * 256-token tile on two / three W buffers whatever the shape, 64 / 96 / 128 / 192 / 224 / 256 the LDS-DMA kernel with
+ * token tiles of that size, -1 (the default, also for any other value) picks by shape.  Process-wide; set it while no call of this library is running; not for
  * production callers. */
 void tome_select_fused_kernel(int kind);
 size_t tome_fused_lmhead_logprob_workspace(int64_t n_tokens, int64_t H, int64_t V);

@@ -433,3 +433,76 @@ def test_fused_matrices_of_4_gib_and_more(dev, which, kind, n):
     np.testing.assert_allclose(r.lse.cpu().numpy(), want["lse"], atol=TOL, rtol=0)
     assert r.argmax.cpu().numpy()[n - 1] == V - 3 == want["argmax"][n - 1]
     check_argmax(h, w, r.argmax.cpu().numpy(), want)
+
+
+TOKEN_TILES = [64, 96, 128, 192, 224, 256]
+
+
+@pytest.mark.parametrize("n,H,V,outputs", [
+    (1, 64, 700, "plain"), (65, 128, 256 * 5 + 33, "all"), (96, 64, 9000, "entropy"), (97, 192, 4481, "argmax"),
+    (192, 256, 30000, "plain"), (193, 64, 256 * 9 + 77, "all"), (224, 320, 20000, "argmax"), (225, 128, 223, "plain"),
+    (256, 1024, 20000, "entropy"), (449, 64, 33920, "all"), (577, 192, 12000, "plain"),
+])
+def test_fused_token_tiles_agree(dev, n, H, V, outputs):
+    """Every token tile size of the LDS-DMA kernel (64 .. 256, even and uneven pairs of token waves, batches that fill a tile,
+    that start a new one and that end inside either half of one) against the oracle, with and without a mask.  A logit's
+    products are summed in the same order whatever the tile, so all of them must name the same argmax; the row sums meet in
+    another order, which fp32 rounds within (number of partials + 16) * 2^-24 of a sum whose log is taken: under 1e-4."""
+    h, w, t = _inputs(dev, n, H, V, seed=n + V, w_scale=0.1)
+    edges = [v for v in (0, 15, 16, 127, 128, 223, 224, 255, 256, V - 33, V - 1) if 0 <= v < V][:n]
+    t[: len(edges)] = edges
+    ent, am = outputs in ("all", "entropy"), outputs in ("all", "argmax")
+    want = oracle.lmhead_stats(bf16_bits_of(h), bf16_bits_of(w), t, 0.9)
+    valid = np.ones(n, dtype=np.int32)
+    valid[np.random.default_rng(n).random(n) < 0.4] = 0
+    lib = tome_amd.load_library()
+    first = None
+    try:
+        for tile in TOKEN_TILES:
+            lib.tome_select_fused_kernel(tile)
+            for mask in (None, valid):
+                m = np.ones(n, bool) if mask is None else mask.astype(bool)
+                r = tome_amd.fused_lmhead_logprobs(h, w, torch.from_numpy(t).to(dev), 0.9, want_lse=True, want_entropy=ent, want_argmax=am,
+                                                   row_valid=None if mask is None else torch.from_numpy(mask).to(dev))
+                lp = r.lp.cpu().numpy()
+                np.testing.assert_allclose(lp[m], want["lp"][m], atol=TOL, rtol=0, err_msg=str(tile))
+                np.testing.assert_allclose(r.lse.cpu().numpy()[m], want["lse"][m], atol=TOL, rtol=0)
+                assert (lp[~m] == 0).all()
+                if ent:
+                    np.testing.assert_allclose(r.entropy.cpu().numpy()[m], want["entropy"][m], atol=TOL, rtol=0)
+                if am:
+                    check_argmax(h, w, r.argmax.cpu().numpy(), want, 0.9, rows=np.flatnonzero(m), min_clear=0.0)
+                if first is None:
+                    first = r
+                np.testing.assert_allclose(lp[m], first.lp.cpu().numpy()[m], atol=1e-4, rtol=0)
+                if am:
+                    np.testing.assert_array_equal(r.argmax.cpu().numpy()[m], first.argmax.cpu().numpy()[m])
+    finally:
+        lib.tome_select_fused_kernel(-1)
+
+
+@pytest.mark.parametrize("tile", TOKEN_TILES)
+def test_fused_token_tiles_stream_large_w(dev, tile):
+    """The non-temporal form, taken for a W beyond the memory-side cache and few token tiles: one ragged tile of every size."""
+    n, H, V = tile - 3, 1024, V_QWEN3
+    g = torch.Generator(device=dev)
+    g.manual_seed(tile)
+    h = torch.empty((n, H), device=dev, dtype=torch.bfloat16).normal_(0, 1, generator=g)
+    w = torch.empty((V, H), device=dev, dtype=torch.bfloat16).normal_(0, 0.02, generator=g)
+    t = torch.randint(0, V, (n,), device=dev, generator=g)
+    lib = tome_amd.load_library()
+    lib.tome_select_fused_kernel(tile)
+    try:
+        r = tome_amd.fused_lmhead_logprobs(h, w, t, 1.0, want_lse=True)
+    finally:
+        lib.tome_select_fused_kernel(-1)
+    lse = torch.full((n,), -float("inf"), device=dev)
+    hit = torch.zeros(n, device=dev)
+    for v0 in range(0, V, 16384):
+        x = h.float() @ w[v0:v0 + 16384].float().T
+        lse = torch.logaddexp(lse, torch.logsumexp(x, dim=-1))
+        rel = t - v0
+        inside = (rel >= 0) & (rel < x.shape[1])
+        hit = torch.where(inside, x.gather(1, rel.clamp(0, x.shape[1] - 1)[:, None])[:, 0], hit)
+    np.testing.assert_allclose(r.lse.cpu().numpy(), lse.cpu().numpy(), atol=TOL, rtol=0)
+    np.testing.assert_allclose(r.lp.cpu().numpy(), (hit - lse).cpu().numpy(), atol=TOL, rtol=0)

@@ -11,7 +11,8 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libtome_logprob.so")
 OPS_PATH = os.path.join(PKG_DIR, "_torch_ops.so")
-SOURCES = ["capi.hip", "row_logprob.hip", "row_sample.hip", "full_log_softmax.hip", "fused_lmhead.hip", "lora_merge.hip", "mfma_probe.hip"]
+SOURCES = [*(f"fused_dma_{k}{o}.hip" for o in ("entropy_argmax", "entropy", "argmax", "plain") for k in ("any_", "")),
+           "fused_lmhead.hip", "capi.hip", "row_logprob.hip", "row_sample.hip", "full_log_softmax.hip", "lora_merge.hip", "mfma_probe.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",

@@ -283,7 +283,8 @@ int tome_full_log_softmax(const void* logits, void* out, int dtype, int64_t rows
 }
 
 void tome_select_fused_kernel(int kind) {
-  tome::fused_force_kernel(kind == 0 || kind == 1 || (kind >= 3 && kind <= 5) ? kind : -1);
+  const bool tile = kind == 64 || kind == 96 || kind == 128 || kind == 192 || kind == 224 || kind == 256;
+  tome::fused_force_kernel(kind == 0 || kind == 1 || (kind >= 3 && kind <= 5) || tile ? kind : -1);
 }
 
 size_t tome_fused_lmhead_logprob_workspace(int64_t n_tokens, int64_t H, int64_t V) {

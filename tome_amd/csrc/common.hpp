@@ -70,6 +70,17 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_hw{lo, hi}, bf16x2_hw));
 }
 
+// Requests every cache line of a kernel's arguments at once.  Left to itself the compiler loads a field where it is first used, and
+// each first use of a line is a miss of its own, one after the other.
+template <typename A>
+__device__ __forceinline__ void touch_args(const A& a) {
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(&a);
+  constexpr int kWords = sizeof(A) / 4;
+  if constexpr (kWords > 48) asm volatile("" ::"s"(w[0]), "s"(w[16]), "s"(w[32]), "s"(w[48]), "s"(w[kWords - 1]));
+  else if constexpr (kWords > 32) asm volatile("" ::"s"(w[0]), "s"(w[16]), "s"(w[32]), "s"(w[kWords - 1]));
+  else asm volatile("" ::"s"(w[0]), "s"(w[16 < kWords ? 16 : 0]), "s"(w[kWords - 1]));
+}
+
 // ---- which rows count, and the id each is scored against -------------------------------------
 // Ids, masks and per-sequence lengths are read in the element types their owners keep them in (torch's int64 ids and bool
 // masks among them): converting them first is a launch of its own per array, 2-5 us each on the stream in front of

@@ -1,0 +1,340 @@
+// What the sweep kernels of the fused lm_head + log-softmax share: arguments, partial records, the work decomposition and
+// the fold of a 16x16 MFMA accumulator tile into the running row states.
+#pragma once
+#include "common.hpp"
+#include <atomic>
+#include <type_traits>
+
+namespace tome {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kBV = 256;                 // vocab rows per tile
+constexpr int kWaveV = 128;              // vocab rows per wave
+constexpr int kPartsPerSplit = kBV / kWaveV;
+constexpr int kDmaSlab = 64;             // K columns per step of the DMA kernel
+
+struct FusedPartial {  // 32 bytes per (token, part)
+  float mx, s, w, tx;
+  int bi;
+  int pad[3];
+};
+
+// Work decomposition: token tiles x vocab splits.  It depends on the number of valid tokens, which is
+// known on the host without a mask and only on the device with one, so it is computed by the host (and
+// passed by value) or by compact_rows_kernel (and read from the workspace header); both run the
+// same code.  Every kernel of a launch uses the same numbers.
+//
+// A workgroup owns one token tile and one contiguous range of vocab tiles.
+//   * Few token tiles (n_ttiles * 8 <= slots): as many splits as fill the chip in ONE round, rounded
+//     down - one workgroup too many would cost a whole extra round.
+//   * Many token tiles: several rounds.  The candidates 1..32 are priced as
+//         rounds * (longest vocab range + half a tile of prologue) * L2 penalty
+//     where the penalty prefers >= 8 splits: the workgroups resident on an XCD are then a block of
+//     ~4 token tiles x ~8 splits, which read 12 distinct slab streams through its L2 instead of 33
+//     (measured on MI355X: 65536 tokens, H = 4096: 1 split 1.09 PFLOP/s, 8-9 splits 1.4).
+struct FusedSchedule {
+  int n_ttiles, n_splits, n_wg;
+  int tile;              // index of FusedTile
+  int n_vunits, unit32;  // vocab units the splits share out, and 32-row blocks per unit
+};
+// A token tile and how the vocab axis is dealt to the splits with it: in whole tiles of 256 or 224 rows (unit32 = 8 / 7), or in
+// 32-row units, of which a workgroup makes tiles of up to 256 rows, all within one unit of each other.
+struct FusedTile {
+  int tokens, unit32;
+};
+constexpr int kFusedTiles = 9, kTileGeneric = 8;  // 0 .. 7: the DMA kernel's; 8: the generic kernel's
+__host__ __device__ constexpr FusedTile fused_tile(int i) {
+  return i == 0 ? FusedTile{256, 8} : i == 1 ? FusedTile{256, 7} : i == 2 ? FusedTile{224, 8} : i == 3 ? FusedTile{224, 7} :
+         i == 4 ? FusedTile{192, 1} : i == 5 ? FusedTile{128, 1} : i == 6 ? FusedTile{96, 1} : i == 7 ? FusedTile{64, 1} : FusedTile{128, 8};
+}
+// What the decomposition depends on beside the number of valid tokens.
+struct FusedShape {
+  int H, V;
+  int slots;       // workgroups that fit the chip at once
+  uint32_t tiles;  // bit i: FusedTile i may be taken
+  int vunits32, vunits224, vunits256;  // the vocab axis in 32-row units, 224-row and 256-row tiles
+  int whole;       // 1: vocab ranges in whole 256-row tiles whatever the token tile
+};
+inline FusedShape fused_shape(int64_t H, int64_t V, int slots, uint32_t tiles, bool whole) {
+  return FusedShape{(int)H, (int)V, slots, tiles, (int)((V + 31) / 32), (int)((V + 223) / 224), (int)((V + 255) / 256), whole ? 1 : 0};
+}
+__host__ __device__ inline bool fused_one_tile(const FusedShape& sh) { return (sh.tiles & (sh.tiles - 1)) == 0; }
+// The tiles below 256 tokens save padding where there are few of them; they are not taken beyond these numbers of valid tokens
+// (5074 tokens: 256 a tile 1148 us, 224 1207; the tiles up to 128 tokens are no better than 192 from two of those on).
+__host__ __device__ constexpr int fused_tile_most(int i) { return i >= 5 && i < kTileGeneric ? 256 : i >= 2 && i < 5 ? 2560 : 0x7fffffff; }
+__host__ __device__ inline bool fused_tile_allowed(const FusedShape& sh, int n_valid, int i) {
+  return ((sh.tiles >> i) & 1) && (n_valid <= fused_tile_most(i) || fused_one_tile(sh));
+}
+__host__ __device__ inline int fused_unit32(const FusedShape& sh, int i) { return sh.whole ? 8 : fused_tile(i).unit32; }
+__host__ __device__ inline int fused_vunits(const FusedShape& sh, int i) {
+  const int u = fused_unit32(sh, i);
+  return u == 1 ? sh.vunits32 : u == 7 ? sh.vunits224 : sh.vunits256;
+}
+__host__ __device__ inline int fused_ttiles(int n_valid, int bt) {
+  const int t = (n_valid + bt - 1) / bt;
+  return t < 1 ? 1 : t;
+}
+__host__ __device__ inline int fused_one_round_splits(int n_ttiles, int slots, int n_vtiles) {
+  int sp = slots / n_ttiles;
+  if (sp > n_vtiles) sp = n_vtiles;  // every split keeps at least one tile's worth of rows
+  return sp < 1 ? 1 : sp;
+}
+// What a batch costs on tile i where one round of workgroups holds it: the longest vocab range bounds the launch.  Fitted to 2300
+// timings (V = 32000 .. 151936, H = 768 .. 4096, 33 .. 4096 tokens, every tile): per K slab and vocab tile a constant, the tile's
+// MFMA work and the hidden rows' fill, and per vocab tile the fold.  Choosing by it is 0.1 % slower than choosing the measured
+// best in the mean, at most 6 % at any of the 290 shapes (32000 x 2560, 640 tokens: 192 a tile 102.5 us, 224 96.9).  Tiles of 224 and
+// 192 tokens are only taken for a gain of 3 %: below that the optional outputs and the sharing of W in L2 decide, which are not
+// priced (50257 x 2048, 1024 tokens, as five tiles of 224 instead of four of 256: 165 -> 174 us).
+// 224-row vocab tiles pay where they shorten the longest range: whole 256-row tiles deal V = 151936 as three tiles to 82
+// workgroups and two to the others, 224-row tiles as three to 167 and two to 89, an eighth less for the longest.
+// (In floats, quotients of whole numbers with half a unit to spare before the rounding: integer divisions by a lane's own divisor
+// are 40 instructions each, and behind a mask one wave prices the tiles between two launches.)
+__host__ __device__ inline float fused_tile_cost(const FusedShape& sh, int n_valid, int i) {
+  const float tokens = (float)fused_tile(i).tokens, unit32 = (float)fused_unit32(sh, i), units = (float)fused_vunits(sh, i);
+  const float vtiles = unit32 == 1.f ? (float)sh.vunits256 : units, nk = (float)(sh.H / kDmaSlab);
+  const float ttiles = floorf(((float)n_valid + tokens - 0.5f) / tokens);
+  float splits = floorf(((float)sh.slots + 0.5f) / (ttiles < 1.f ? 1.f : ttiles));
+  splits = splits > vtiles ? vtiles : splits < 1.f ? 1.f : splits;
+  const float longest = floorf((units + splits - 0.5f) / splits);
+  const float tiles = unit32 == 1.f ? floorf((longest + 7.f) * 0.125f) : longest, rows = longest * unit32 * 32.f;
+  const float cost = tiles * nk * (61.f * 65536.f + 39.f * 256.f * tokens) + rows * (nk * (100.f * tokens + 3.f * 256.f) + 143.f * tokens);
+  return i >= 2 && i < 5 ? cost * 1.03f : cost;
+}
+__host__ __device__ inline int64_t fused_split_cost(int n_ttiles, int n_splits, int slots, int n_vunits, int upt) {
+  const int rounds = (n_ttiles * n_splits + slots - 1) / slots;
+  const int longest = (n_vunits + n_splits - 1) / n_splits;  // in units
+  const int pen64 = 60 + 32 / (n_splits < 8 ? n_splits : 8);
+  return ((int64_t)rounds * (2 * longest + upt) * pen64) * 64 + n_splits;  // ties go to fewer splits
+}
+constexpr int kSplitCandidates = 32;
+// The schedule but for the number of splits where several rounds are needed; returns whether that is so.
+__host__ __device__ inline bool fused_schedule_begin(FusedSchedule& s, int n_valid, const FusedShape& sh, int tile) {
+  s.tile = tile;
+  s.unit32 = fused_unit32(sh, tile);
+  s.n_vunits = fused_vunits(sh, tile);
+  s.n_ttiles = fused_ttiles(n_valid, fused_tile(tile).tokens);
+  if (s.n_ttiles * 8 > sh.slots) return true;
+  s.n_splits = fused_one_round_splits(s.n_ttiles, sh.slots, s.unit32 == 1 ? (s.n_vunits + 7) / 8 : s.n_vunits);
+  s.n_wg = s.n_ttiles * s.n_splits;
+  return false;
+}
+inline FusedSchedule fused_schedule_on(int n_valid, const FusedShape& sh, int tile) {  // host
+  FusedSchedule s;
+  if (fused_schedule_begin(s, n_valid, sh, tile)) {
+    const int upt = s.unit32 == 1 ? 8 : 1, n_vtiles = (s.n_vunits + upt - 1) / upt;
+    int64_t best = INT64_MAX;
+    for (int c = 1; c <= kSplitCandidates && c <= n_vtiles; ++c) {
+      const int64_t cost = fused_split_cost(s.n_ttiles, c, sh.slots, s.n_vunits, upt);
+      if (cost < best) best = cost;
+    }
+    s.n_splits = (int)(best & 63);
+    s.n_wg = s.n_ttiles * s.n_splits;
+  }
+  return s;
+}
+inline FusedSchedule fused_schedule(int n_valid, const FusedShape& sh) {  // host
+  float best = INFINITY;
+  int tile = 0;
+  for (int i = 0; i < kFusedTiles; ++i) {
+    if (!fused_tile_allowed(sh, n_valid, i)) continue;
+    const float c = fused_tile_cost(sh, n_valid, i);
+    if (c < best) best = c, tile = i;
+  }
+  return fused_schedule_on(n_valid, sh, tile);
+}
+// The same on the device, by one whole wave: lane i prices tile i, lane c c + 1 splits.
+__device__ inline FusedSchedule fused_schedule_wave(int n_valid, const FusedShape& sh, int lane) {
+  int tile = __builtin_ctz(sh.tiles);
+  if (!fused_one_tile(sh)) {  // the DMA kernel's eight
+    const int i = lane & 7;
+    const float c = fused_tile_allowed(sh, n_valid, i) ? fused_tile_cost(sh, n_valid, i) : 3e38f;
+    // positive floats order like their bits; the last three carry the tile
+    unsigned key = (__float_as_uint(c) & ~7u) | (unsigned)i;
+    const unsigned a = (unsigned)wave_exchange<0>((int)key);
+    key = a < key ? a : key;
+    const unsigned b = (unsigned)wave_exchange<1>((int)key);
+    key = b < key ? b : key;
+    const unsigned d = (unsigned)wave_exchange<2>((int)key);
+    key = d < key ? d : key;
+    tile = __builtin_amdgcn_readfirstlane((int)(key & 7u));
+  }
+  FusedSchedule s;
+  if (fused_schedule_begin(s, n_valid, sh, tile)) {
+    const int upt = s.unit32 == 1 ? 8 : 1, n_vtiles = (s.n_vunits + upt - 1) / upt, c = lane + 1;
+    int64_t cost = c <= kSplitCandidates && c <= n_vtiles ? fused_split_cost(s.n_ttiles, c, sh.slots, s.n_vunits, upt) : INT64_MAX;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const int64_t o = __shfl_xor(cost, off, 64);
+      cost = o < cost ? o : cost;
+    }
+    s.n_splits = (int)(cost & 63);
+    s.n_wg = s.n_ttiles * s.n_splits;
+  }
+  return s;
+}
+
+// Workgroup id -> (token tile, vocab split).  The hardware deals consecutive workgroup ids round-robin
+// over the 8 XCDs, each with its own L2; XCD x is given the contiguous logical ids
+// [x * per, (x + 1) * per), and logical ids run over blocks of <= 8 splits, token tile by token tile,
+// so that the workgroups resident on an XCD at any time share token tiles AND vocab ranges.
+__device__ __forceinline__ bool fused_locate(const FusedSchedule& s, int bid, int& ttile, int& split) {
+  const int per = (s.n_wg + 7) >> 3;
+  const int li = bid >> 3;
+  int g = (bid & 7) * per + li;
+  if (li >= per || g >= s.n_wg) return false;  // the grid is sized for the worst case over n_valid
+  const int nb = (s.n_splits + 7) >> 3, base = s.n_splits / nb, rem = s.n_splits % nb;
+  int s0 = 0, w = base;
+  for (int sb = 0; sb < nb; ++sb) {
+    w = base + (sb < rem ? 1 : 0);
+    const int cnt = s.n_ttiles * w;
+    if (g < cnt) break;
+    g -= cnt;
+    s0 += w;
+  }
+  ttile = g / w;
+  split = s0 + g % w;
+  return true;
+}
+
+struct FusedArgs {
+  // What a workgroup needs to find its work comes first, in one cache line: a fresh launch misses on its arguments.
+  const int32_t* n_valid;    // device scalar, or nullptr = n_tokens
+  const FusedSchedule* sched_dev;  // written by compact_rows_kernel next to n_valid, or nullptr = `sched`
+  FusedSchedule sched;       // host-computed schedule (no mask)
+  int n_tokens;
+  int H;
+  int V;
+  float scale;               // log2(e) / temperature
+  const char* hidden;
+  const char* weight;
+  RowSel sel;                // its targets (the mask went into row_index)
+  const int32_t* row_index;  // compacted valid rows (position -> row of targets / outputs), or nullptr = identity
+  const int32_t* hidden_index;  // position -> row of `hidden`: row_index, the caller's row list, or nullptr when hidden is already compact
+  int n_rows;                   // rows of `hidden`; an entry of a caller's list outside them reads a row inside (and scores NaN)
+  FusedPartial* partials;
+  uint32_t hidden_stride_b;  // bytes
+  uint32_t weight_stride_b;
+  uint32_t hidden_bytes;     // extent of the hidden matrix (< 4 GiB, checked on the host)
+};
+
+// ---- 16x16x32 MFMA accumulator layout --------------------------------------------------------------
+// A 16x16 block lives in four registers: lane l holds token column l % 16 and vocab rows
+// 4*(l/16) + e, e = 0..3.  A lane therefore owns one token per 16-token block, and the four lane
+// groups l/16 share that token: they are merged once, at the end, over lane ^ 16 and lane ^ 32.
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+
+// Fold one wave tile (NBV x NBT blocks of 16x16) into the per-token running states.  Element e of
+// block i holds vocab row  vw0 + i*16 + 4*g + e  (g = lane / 16) for the token of block column j.
+// NBV of the NBV_ALLOC block rows the array holds are folded (a short tile uses the first few).
+template <bool ENT, bool AMAX, int NBV, int NBT, int NBV_ALLOC>
+__device__ __forceinline__ void fold_tile16(f32x4v (&acc)[NBV_ALLOC][NBT], RowStat (&st)[NBT], float (&tx)[NBT],
+                                            const int (&tgt)[NBT], int vw0, int g, bool partial_tile, int V,
+                                            float scale) {
+  if (partial_tile) {  // last vocab tile: rows past V do not exist
+#pragma unroll
+    for (int i = 0; i < NBV; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool dead = vw0 + i * 16 + 4 * g + e >= V;
+#pragma unroll
+        for (int j = 0; j < NBT; ++j) acc[i][j][e] = dead ? -INFINITY : acc[i][j][e];
+      }
+  }
+  const int vlane = vw0 + 4 * g;  // first vocab row this lane holds in block 0
+#pragma unroll
+  for (int j = 0; j < NBT; ++j) {
+    __builtin_amdgcn_sched_barrier(0);  // one scheduling region per token block (register pressure)
+    // Target capture: rare (one tile in V/256 per token), so behind a wave-uniform test.
+    const int rel = tgt[j] - vw0;
+    const bool mine = tgt[j] >= 0 && rel >= 0 && rel < NBV * 16 && ((rel >> 2) & 3) == g;
+    if (__any(mine)) {
+      const int want = mine ? ((rel >> 4) * 4 + (rel & 3)) : -1;
+#pragma unroll
+      for (int i = 0; i < NBV; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tx[j] = (want == i * 4 + e) ? acc[i][j][e] : tx[j];
+    }
+    float cm = st[j].mx;
+    int bi = st[j].bi;
+#pragma unroll
+    for (int i = 0; i < NBV; ++i) {
+      if constexpr (AMAX) {
+        // Seven more VALU operations per block, only when the argmax is asked for: the block maximum comes
+        // with the position of its first holder, and the running maximum carries the vocab row of the
+        // element that set it.  Only a strictly larger value replaces the holder and a lane meets its rows in
+        // ascending order, so the sweep itself names the first maximum of the fp32 logits it computed.
+        const float x0 = acc[i][j][0], x1 = acc[i][j][1], x2 = acc[i][j][2], x3 = acc[i][j][3];
+        const float m01 = raw_max(x0, x1), m23 = raw_max(x2, x3);
+        const int e01 = x1 > x0 ? 1 : 0, e23 = x3 > x2 ? 3 : 2;
+        const int e = m23 > m01 ? e23 : e01;
+        const float bm = raw_max(m01, m23);
+        bi = bm > cm ? vlane + i * 16 + e : bi;
+        cm = raw_max(cm, bm);
+      } else {
+        const float bm = raw_max3(acc[i][j][0], acc[i][j][1], raw_max(acc[i][j][2], acc[i][j][3]));
+        cm = raw_max(cm, bm);
+      }
+    }
+    const float dm = (st[j].mx - cm) * scale;
+    const float resc = fast_exp2(dm);
+    const float m = cm * scale;
+    // w: sum (y - m) 2^(y - m), relative to the running maximum (stat_merge has the rule for moving it)
+    float s0 = st[j].s * resc, s1 = 0.f, w0 = ENT ? fmaf(dm, st[j].s, st[j].w) * resc : 0.f, w1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < NBV; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        const float x0 = acc[i][j][e], x1 = acc[i][j][e + 1];
+        const float t0 = fmaf(x0, scale, -m), t1 = fmaf(x1, scale, -m);
+        const float e0 = fast_exp2(t0);
+        const float e1 = fast_exp2(t1);
+        s0 += e0;
+        s1 += e1;
+        if constexpr (ENT) {  // a masked row (-inf): floor * 0, not -inf * 0
+          w0 = fmaf(clamp_below(t0), e0, w0);
+          w1 = fmaf(clamp_below(t1), e1, w1);
+        }
+      }
+    st[j].mx = cm;
+    st[j].bi = bi;
+    st[j].s = s0 + s1;
+    if constexpr (ENT) st[j].w = w0 + w1;
+  }
+}
+
+// Merge the four lane groups that share a token and write one partial per (token, part).
+template <int NBT>
+__device__ __forceinline__ void write_partials16(RowStat (&st)[NBT], float (&tx)[NBT], FusedPartial* partials,
+                                                 int p0, int n_valid, int part, int n_parts, int l16, int g,
+                                                 float scale) {
+#pragma unroll
+  for (int j = 0; j < NBT; ++j) {
+    stat_wave_step<4>(st[j], scale);
+    stat_wave_step<5>(st[j], scale);
+    tx[j] = fmaxf(tx[j], wave_exchange<4>(tx[j]));
+    tx[j] = fmaxf(tx[j], wave_exchange<5>(tx[j]));
+    const int p = p0 + j * 16 + l16;
+    if (g == 0 && p < n_valid) {
+      FusedPartial out;
+      out.mx = st[j].mx;
+      out.s = st[j].s;
+      out.w = st[j].w;
+      out.tx = tx[j];
+      out.bi = st[j].bi;
+      out.pad[0] = out.pad[1] = out.pad[2] = 0;
+      partials[(int64_t)p * n_parts + part] = out;
+    }
+  }
+}
+
+// Opt in to more than 64 KB of dynamic LDS.
+template <typename K>
+static bool allow_big_lds(K kernel, int bytes) {
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess)
+    return true;
+  (void)hipGetLastError();  // the launch that follows reports its own error
+  return false;
+}
+
+}  // namespace tome

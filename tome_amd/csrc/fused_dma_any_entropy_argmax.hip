@@ -1,0 +1,6 @@
+// The DMA sweep on a token tile chosen on the device, with the entropy and the argmax.
+#include "fused_dma.hpp"
+
+namespace tome {
+template void launch_dma_any<true, true>(const FusedArgs&, bool, int, hipStream_t);
+}  // namespace tome

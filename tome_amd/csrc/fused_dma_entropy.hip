@@ -1,0 +1,6 @@
+// The DMA sweep on a token tile that the host knows, with the entropy.
+#include "fused_dma.hpp"
+
+namespace tome {
+template void launch_dma<true, false>(const FusedArgs&, int, bool, bool, int, hipStream_t);
+}  // namespace tome
