@@ -506,3 +506,28 @@ def test_fused_token_tiles_stream_large_w(dev, tile):
         hit = torch.where(inside, x.gather(1, rel.clamp(0, x.shape[1] - 1)[:, None])[:, 0], hit)
     np.testing.assert_allclose(r.lse.cpu().numpy(), lse.cpu().numpy(), atol=TOL, rtol=0)
     np.testing.assert_allclose(r.lp.cpu().numpy(), (hit - lse).cpu().numpy(), atol=TOL, rtol=0)
+
+
+@pytest.mark.parametrize("outputs", ["plain", "entropy", "argmax", "all"])
+@pytest.mark.parametrize("n,H,V", [(100, 128, 3000), (400, 512, 4500), (666, 128, 9000), (900, 64, 20000)])
+def test_fused_tile_chosen_on_device_every_logit(dev, n, H, V, outputs):
+    """Behind a mask the device picks the token tile; the last tile ends inside a 16-token block.  Every row's lp and lse against
+    an fp32 product (rounding of an H-long sum at these magnitudes: under 1e-4), so that a single wrong partial shows."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(n + V)
+    w = torch.empty((V, H), device=dev).normal_(0, 0.05, generator=g).to(torch.bfloat16)
+    for k in range(6):
+        h = torch.empty((n, H), device=dev).normal_(0, 1, generator=g).to(torch.bfloat16)
+        t = torch.randint(0, V, (n,), device=dev, generator=g)
+        valid = torch.rand(n, device=dev, generator=g) < 0.1 + 0.15 * k
+        r = tome_amd.fused_lmhead_logprobs(h, w, t, 1.0, row_valid=valid, want_lse=True, want_entropy=outputs in ("entropy", "all"),
+                                           want_argmax=outputs in ("argmax", "all"))
+        x = h.float() @ w.float().T
+        lse = torch.logsumexp(x, dim=-1)
+        m = valid.cpu().numpy()
+        np.testing.assert_allclose(r.lse.cpu().numpy()[m], lse.cpu().numpy()[m], atol=1e-4, rtol=0)
+        np.testing.assert_allclose(r.lp.cpu().numpy()[m], (x.gather(1, t[:, None])[:, 0] - lse).cpu().numpy()[m], atol=1e-4, rtol=0)
+        if r.entropy is not None:
+            p = torch.softmax(x.double(), dim=-1)
+            want = torch.logsumexp(x.double(), dim=-1) - (p * x.double()).sum(-1)
+            np.testing.assert_allclose(r.entropy.cpu().numpy()[m], want.cpu().numpy()[m], atol=2e-4, rtol=0)

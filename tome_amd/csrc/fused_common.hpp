@@ -303,6 +303,15 @@ __device__ __forceinline__ void fold_tile16(f32x4v (&acc)[NBV_ALLOC][NBT], RowSt
   }
 }
 
+// Target id of position p, -1 past the last token or outside [0, V).  Without a branch: registers spilled inside one that only
+// some lanes take are lost for the others (seen in a kernel at the limit of the register file: token positions stored under
+// the mask of the last block's tokens).
+__device__ __forceinline__ int token_target(const FusedArgs& a, int p, int n_valid) {
+  const int q = p < n_valid ? p : n_valid - 1;
+  const int t = a.sel.target(a.row_index ? a.row_index[q] : q);
+  return p < n_valid && t >= 0 && t < a.V ? t : -1;
+}
+
 // Merge the four lane groups that share a token and write one partial per (token, part).
 template <int NBT>
 __device__ __forceinline__ void write_partials16(RowStat (&st)[NBT], float (&tx)[NBT], FusedPartial* partials,

@@ -228,10 +228,7 @@ __device__ __forceinline__ void dma_sweep(const FusedArgs& a, const FusedSchedul
   for (int bt = 0; bt < k2NBT; ++bt) {
     st[bt] = stat_identity();
     tx[bt] = -INFINITY;
-    const int p = t0 + tok0 + bt * 16 + l16;
-    int t = -1;
-    if (p < n_valid) t = a.sel.target(a.row_index ? a.row_index[p] : p);
-    tgt[bt] = (t >= 0 && t < a.V) ? t : -1;
+    tgt[bt] = token_target(a, t0 + tok0 + bt * 16 + l16, n_valid);
   }
 
   // ---- fragment read offsets inside a slab (swizzled): lane group g reads chunk 4*ks + g ----------

@@ -199,10 +199,7 @@ __global__ __launch_bounds__(kFusedWG, 2) void fused_lmhead_kernel(FusedArgs a) 
   for (int bt = 0; bt < kNBT; ++bt) {
     st[bt] = stat_identity();
     tx[bt] = -INFINITY;
-    int p = t0 + wave_t * kWaveT + bt * 32 + l32;
-    int t = -1;
-    if (p < n_valid) t = a.sel.target(a.row_index ? a.row_index[p] : p);
-    tgt[bt] = (t >= 0 && t < a.V) ? t : -1;
+    tgt[bt] = token_target(a, t0 + wave_t * kWaveT + bt * 32 + l32, n_valid);
   }
 
   const int nk = (a.H + kBK - 1) / kBK;
@@ -322,10 +319,7 @@ __global__ __launch_bounds__(512) void fused_lmhead_small_kernel(FusedArgs a) {
   float tx[1] = {-INFINITY};
   int tgt[1] = {-1};
   if (wave < NBT) {
-    const int p = wave * 16 + l16;
-    int t = -1;
-    if (p < n_valid) t = a.sel.target(a.row_index ? a.row_index[p] : p);
-    tgt[0] = (t >= 0 && t < a.V) ? t : -1;
+    tgt[0] = token_target(a, wave * 16 + l16, n_valid);
   }
 
   // W loads are shaped for HBM, not for the MFMA: one instruction fetches 4 rows x 256 bytes (lane = row
