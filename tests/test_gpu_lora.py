@@ -199,6 +199,32 @@ def test_grpo_pair_matches_oracle(dev, with_norm, shared_w, n, H):
             np.testing.assert_array_equal(x.cpu().numpy(), y.cpu().numpy())
 
 
+@pytest.mark.parametrize("n,H,V,masked", [
+    (1, 256, 700, False), (8, 1024, 3000, True), (32, 512, 3000, False),    # one sweep over both matrices: streaming kernel
+    (33, 1024, 5000, False), (97, 128, 4481, True), (240, 64, 9000, True), (512, 192, 4481, False), (768, 128, 4481, True),
+    (513, 64, 4481, False), (769, 64, 4481, True), (100, 72, 1000, True),   # two sweeps: more tokens; the generic kernel
+])
+@pytest.mark.parametrize("with_norm", [False, True])
+def test_grpo_pair_shared_weight_joint_and_separate(dev, n, H, V, masked, with_norm):
+    """Small batches against one shared weight are one sweep over both hidden matrices.  Each matrix through the one-matrix
+    entry must give the same log-probs: the logits' sums are the same, the row sums meet in another order (fp32: under 1e-4)."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(n + V)
+    hp = torch.empty((n, H), device=dev).normal_(0, 1, generator=g).to(torch.bfloat16)
+    hr = hp + torch.empty((n, H), device=dev).normal_(0, 0.3, generator=g).to(torch.bfloat16)
+    w = torch.empty((V, H), device=dev).normal_(0, 0.05, generator=g).to(torch.bfloat16)
+    nw = (torch.rand(H, device=dev, generator=g) + 0.5).to(torch.bfloat16) if with_norm else None
+    t = torch.randint(0, V, (n,), device=dev, generator=g)
+    valid = (torch.rand(n, device=dev, generator=g) < 0.6).to(torch.int32) if masked else None
+    r = tome_amd.grpo_pair_logprobs(hp, hr, w, t, 0.9, row_valid=valid, norm_weight=nw)
+    pol = tome_amd.fused_lmhead_logprobs(hp, w, t, 0.9, row_valid=valid, want_entropy=True, norm_weight=nw)
+    ref = tome_amd.fused_lmhead_logprobs(hr, w, t, 0.9, row_valid=valid, norm_weight=nw)
+    for got, want in ((r.lp, pol.lp), (r.ref_lp, ref.lp), (r.entropy, pol.entropy)):
+        np.testing.assert_allclose(got.cpu().numpy(), want.cpu().numpy(), atol=1e-4, rtol=0)
+    np.testing.assert_allclose(r.k3.cpu().numpy(), oracle.k3(pol.lp.cpu().numpy().astype(np.float64), ref.lp.cpu().numpy().astype(np.float64)) *
+                               (1 if valid is None else valid.cpu().numpy()), atol=1e-3, rtol=1e-3)
+
+
 @pytest.mark.parametrize("name", ["m0", "m1", "m2", "m3"])
 def test_merge_matches_golden_vectors(dev, name):
     """The committed vectors (exact rational arithmetic, tests/golden/make_lora_golden.py); ranks 12 and 4 are

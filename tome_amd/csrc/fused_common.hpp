@@ -216,6 +216,9 @@ struct FusedArgs {
   uint32_t hidden_stride_b;  // bytes
   uint32_t weight_stride_b;
   uint32_t hidden_bytes;     // extent of the hidden matrix (< 4 GiB, checked on the host)
+  // Two hidden matrices in one sweep: tokens [0, n) are rows of `hidden`, [n, 2 n) the same rows of
+  // `hidden2`, n the number of valid tokens; n_tokens and the schedule count both.  nullptr: one matrix.
+  const char* hidden2;
 };
 
 // ---- 16x16x32 MFMA accumulator layout --------------------------------------------------------------
@@ -303,11 +306,22 @@ __device__ __forceinline__ void fold_tile16(f32x4v (&acc)[NBV_ALLOC][NBT], RowSt
   }
 }
 
+// Where position p of a sweep over n_valid tokens finds its hidden row and its target.
+struct TokenSource {
+  const char* hidden;
+  int q;  // position among the valid tokens
+};
+__device__ __forceinline__ TokenSource token_source(const FusedArgs& a, int p, int n_valid) {
+  const int n_one = a.hidden2 ? n_valid >> 1 : n_valid;
+  const bool second = p >= n_one;
+  return {second ? a.hidden2 : a.hidden, second ? p - n_one : p};
+}
+
 // Target id of position p, -1 past the last token or outside [0, V).  Without a branch: registers spilled inside one that only
 // some lanes take are lost for the others (seen in a kernel at the limit of the register file: token positions stored under
 // the mask of the last block's tokens).
 __device__ __forceinline__ int token_target(const FusedArgs& a, int p, int n_valid) {
-  const int q = p < n_valid ? p : n_valid - 1;
+  const int q = token_source(a, p < n_valid ? p : n_valid - 1, n_valid).q;
   const int t = a.sel.target(a.row_index ? a.row_index[q] : q);
   return p < n_valid && t >= 0 && t < a.V ? t : -1;
 }

@@ -216,8 +216,9 @@ __device__ __forceinline__ void dma_sweep(const FusedArgs& a, const FusedSchedul
   for (int j = 0; j < kBLoads; ++j) {
     int p = t0 + (j * 8 + wave) * 8 + dr;
     p = p < n_valid ? p : n_valid - 1;
-    const int tok = a.hidden_index ? min(max(a.hidden_index[p], 0), a.n_rows - 1) : p;
-    pb[j] = a.hidden + (int64_t)tok * a.hidden_stride_b + dc * 16;
+    const TokenSource src = token_source(a, p, n_valid);
+    const int tok = a.hidden_index ? min(max(a.hidden_index[src.q], 0), a.n_rows - 1) : src.q;
+    pb[j] = src.hidden + (int64_t)tok * a.hidden_stride_b + dc * 16;
   }
 
   // ---- per-lane token state: one token per 16-token block, shared by the four lane groups ---------
@@ -448,7 +449,7 @@ __global__ __launch_bounds__(k2WG) void fused_lmhead_dma_kernel(FusedArgs a) {
   int n_valid = a.n_tokens;
   FusedSchedule sch = a.sched;
   if (a.sched_dev) {  // behind a mask, next to the count
-    n_valid = *a.n_valid;
+    n_valid = *a.n_valid << (a.hidden2 ? 1 : 0);
     sch = *a.sched_dev;
   }
   int ttile, split;

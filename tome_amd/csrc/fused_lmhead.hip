@@ -292,7 +292,7 @@ __global__ __launch_bounds__(512) void fused_lmhead_small_kernel(FusedArgs a) {
   constexpr int kBuf = 16 / KSTEPS;                                 // tile buffers in flight (registers): 16 loads per lane
   constexpr int kRed = 2;                                           // reduction buffers (LDS)
   touch_args(a);
-  const int n_valid = a.n_valid ? *a.n_valid : a.n_tokens;
+  const int n_valid = a.n_valid ? *a.n_valid << (a.hidden2 ? 1 : 0) : a.n_tokens;
   if (n_valid <= 0) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -309,8 +309,9 @@ __global__ __launch_bounds__(512) void fused_lmhead_small_kernel(FusedArgs a) {
   for (int j = 0; j < NBT; ++j) {
     int p = j * 16 + l16;
     p = p < n_valid ? p : n_valid - 1;
-    const int tok = a.hidden_index ? min(max(a.hidden_index[p], 0), a.n_rows - 1) : p;
-    const char* hp = a.hidden + (int64_t)tok * a.hidden_stride_b + kb0;
+    const TokenSource src = token_source(a, p, n_valid);
+    const int tok = a.hidden_index ? min(max(a.hidden_index[src.q], 0), a.n_rows - 1) : src.q;
+    const char* hp = src.hidden + (int64_t)tok * a.hidden_stride_b + kb0;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) fb[ks][j] = *reinterpret_cast<const bf16x8*>(hp + ks * 64);
   }
@@ -415,6 +416,7 @@ struct CompactArgs {
   int32_t* out_argmax;
   int n;
   FusedShape shape;              // of the schedule, which this kernel derives from n_valid
+  int joint;                     // 1: every valid token is swept twice (two hidden matrices)
 };
 
 // Rows are taken in batches of up to 8192: each of the 16 waves owns a run of consecutive rows of a batch (a
@@ -454,7 +456,7 @@ __global__ __launch_bounds__(1024) void compact_rows_kernel(CompactArgs a) {
       else if (a.sel.valid_bytes == 1) load_mask_chunks(v, left, lane, [&](int r) { return (int)reinterpret_cast<const uint8_t*>(mask)[(unsigned)r]; });
       else load_mask_chunks(v, left, lane, [&](int r) { return *reinterpret_cast<const int32_t*>(mask + (unsigned)(r * a.sel.valid_bytes)); });
     }
-    if (wave == 15 && b0 == 0) sch = fused_schedule_wave(a.n, a.shape, lane);
+    if (wave == 15 && b0 == 0) sch = fused_schedule_wave(a.n << a.joint, a.shape, lane);
     int cnt = 0;
 #pragma unroll
     for (int c = 0; c < kChunks; ++c) {
@@ -492,7 +494,7 @@ __global__ __launch_bounds__(1024) void compact_rows_kernel(CompactArgs a) {
   }
   if (threadIdx.x == 0) *a.n_valid = done;
   if (wave == 15) {  // one wave also fixes the work decomposition, which depends on the total
-    if (done != a.n) sch = fused_schedule_wave(done, a.shape, lane);
+    if (done != a.n) sch = fused_schedule_wave(done << a.joint, a.shape, lane);
     if (lane == 0) *reinterpret_cast<FusedSchedule*>(a.n_valid + 4) = sch;
   }
 }
@@ -502,9 +504,9 @@ __global__ __launch_bounds__(1024) void compact_rows_kernel(CompactArgs a) {
 // mlx-impl/model.py:343 calls it on the last hidden states (model.py:536).  Only valid rows are
 // normalised, and they are written compactly: position p of the output is row row_index[p] of x.
 struct NormArgs {
-  const char* x;             // bf16 [n, H]
+  const char* x[2];          // bf16 [n, H]; the second for blockIdx.y = 1
   const uint16_t* w;         // bf16 [H]
-  char* y;                   // bf16 [n_valid, H], dense
+  char* y[2];                // bf16 [n_valid, H], dense
   const int32_t* row_index;  // or nullptr = identity; entries outside [0, n_rows) read a row inside
   const int32_t* n_valid;    // or nullptr = n
   uint32_t x_stride_b;
@@ -518,9 +520,9 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(NormArgs a) {
   const int n_valid = a.n_valid ? *a.n_valid : a.n;
   if (p >= n_valid) return;
   const int row = a.row_index ? min(max(a.row_index[p], 0), a.n_rows - 1) : p;
-  const u32x4* x = reinterpret_cast<const u32x4*>(a.x + (int64_t)row * a.x_stride_b);
+  const u32x4* x = reinterpret_cast<const u32x4*>(a.x[blockIdx.y] + (int64_t)row * a.x_stride_b);
   const u32x4* w = reinterpret_cast<const u32x4*>(a.w);
-  u32x4* y = reinterpret_cast<u32x4*>(a.y + (int64_t)p * a.H * 2);
+  u32x4* y = reinterpret_cast<u32x4*>(a.y[blockIdx.y] + (int64_t)p * a.H * 2);
   const int n_chunks = a.H / 8;
   float ss = 0.f;
   for (int c = lane; c < n_chunks; c += 64) {
@@ -553,7 +555,8 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(NormArgs a) {
 // ---- combine -----------------------------------------------------------------------------------
 struct CombineArgs {
   const FusedPartial* partials;      // policy (or the only) weight set
-  const FusedPartial* partials_ref;  // second weight set, or nullptr
+  const FusedPartial* partials_ref;  // second sweep, or nullptr
+  int joint;                         // 1: the second half of `partials` is the second matrix of a joint sweep
   const int32_t* row_index;
   const int32_t* n_valid;
   float* out_lp;
@@ -618,10 +621,11 @@ __global__ __launch_bounds__(256) void fused_combine_kernel(CombineArgs a) {
   // tx stays -inf only when the target id was outside [0, V).
   const float lp = tx == -INFINITY ? __builtin_nanf("") : (fmaf(tx, a.scale, -m) - log2s) * kLn2;
   float ref_lp = 0.f;
-  if (a.partials_ref) {
+  const FusedPartial* second = a.joint ? a.partials + (int64_t)n_valid * n_parts : a.partials_ref;
+  if (second) {
     RowStat sr;
     float txr;
-    combine_one(a.partials_ref + (int64_t)p * n_parts, n_parts, lane, a.scale, sr, txr);
+    combine_one(second + (int64_t)p * n_parts, n_parts, lane, a.scale, sr, txr);
     const float mr = sr.mx * a.scale;
     ref_lp = txr == -INFINITY ? __builtin_nanf("") : (fmaf(txr, a.scale, -mr) - fast_log2(sr.s)) * kLn2;
   }
@@ -825,11 +829,24 @@ static size_t partial_bytes(int64_t n_tokens, int64_t H, int64_t V) {
   return (a > b ? a : b) * sizeof(FusedPartial);
 }
 
+// Two hidden matrices against one weight are ONE sweep over both where that is a batch of up to this many tokens: W is streamed once
+// instead of twice and half-filled token tiles meet.  The sweep computes the entropy for the second matrix too, which at more tokens
+// costs what the sharing gives.  Two sweeps / one, us, V = 151936, H = 1024 | 2560: 16 tokens 104 / 56 | 239 / 124, 128: 126 / 90 |
+// 314 / 198, 512: 281 / 277 | 645 / 611, 768: 400 / 418 | 921 / 980; behind a mask that leaves 56 %, 128: 121 / 86 | 285 / 185, 512:
+// 170 / 140 | 380 / 301, 768: 236 / 222 | 538 / 471, 1024: 369 / 383 | 868 / 845.
+static bool joint_fits(int64_t n_tokens, int64_t H, bool masked) { return n_tokens <= (masked ? 768 : 512) && H % kDmaSlab == 0; }
+// All partials of a call of `n_sweeps` sweeps.
+static size_t partials_total(int64_t n_tokens, int64_t H, int64_t V, int n_sweeps) {
+  const size_t each = partial_bytes(n_tokens, H, V) * (size_t)n_sweeps;
+  const size_t joint = n_sweeps == 2 && joint_fits(n_tokens, H, true) ? partial_bytes(2 * n_tokens, H, V) : 0;
+  return each > joint ? each : joint;
+}
+
 // The generic kernel addresses both matrices through buffer descriptors with 32-bit byte offsets.
 bool fused_needs_32bit_extents(int64_t n_tokens, int64_t H, int64_t V) { return fused_plan(n_tokens, H, V, true, false, false).kind == kGeneric; }
 
 size_t fused_workspace_bytes(int64_t n_tokens, int64_t H, int64_t V, int n_weights, bool with_norm) {
-  return off_partials(n_tokens) + (size_t)n_weights * partial_bytes(n_tokens, H, V) + normed_bytes(n_tokens, H, with_norm);
+  return off_partials(n_tokens) + partials_total(n_tokens, H, V, n_weights) + normed_bytes(n_tokens, H, with_norm);
 }
 
 template <bool ENT, bool AMAX, int NBT, int KSTEPS>
@@ -890,14 +907,16 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
   if (!w1) w1 = w0;
   if (!hidden_ref) hidden_ref = hidden;
   char* ws = static_cast<char*>(workspace);
-  const FusedPlan plan = fused_plan(n_tokens, H, V, deep_lds_granted(), out_entropy != nullptr, sel.masked());
+  FusedPlan plan = fused_plan(n_tokens, H, V, deep_lds_granted(), out_entropy != nullptr, sel.masked());
+  const bool joint = second && w1 == w0 && hidden_ref != hidden && plan.kind != kGeneric && joint_fits(n_tokens, H, sel.masked());
+  if (joint) plan = fused_plan(2 * n_tokens, H, V, deep_lds_granted(), out_entropy != nullptr, sel.masked());
   int32_t* n_valid = nullptr;
   int32_t* row_index = nullptr;
   if (sel.masked()) {
     n_valid = reinterpret_cast<int32_t*>(ws);
     row_index = reinterpret_cast<int32_t*>(ws + off_index());
     CompactArgs c{sel, row_index, n_valid, out_lp, out_lse, out_entropy, out_ref_lp, out_k3, out_argmax,
-                  (int)n_tokens, plan.shape};
+                  (int)n_tokens, plan.shape, joint ? 1 : 0};
     hipLaunchKernelGGL(compact_rows_kernel, dim3(1), dim3(1024), 0, stream, c);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -914,29 +933,25 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
   a.hidden_bytes = (uint32_t)(((n_rows - 1) * hidden_stride + H) * 2);  // read by the generic kernel only (< 4 GiB there)
   const char* second_hidden = static_cast<const char*>(hidden_ref);
   if (norm_weight) {  // normalise the valid rows into a dense buffer and multiply that
-    char* normed = ws + off_partials(n_tokens) + (second ? 2 : 1) * partial_bytes(n_tokens, H, V);
-    NormArgs na{a.hidden, static_cast<const uint16_t*>(norm_weight), normed, a.hidden_index, n_valid,
+    char* normed = ws + off_partials(n_tokens) + partials_total(n_tokens, H, V, second ? 2 : 1);
+    char* normed_ref = hidden_ref != hidden ? normed + normed_bytes(n_tokens, H, true) : normed;
+    NormArgs na{{a.hidden, second_hidden}, static_cast<const uint16_t*>(norm_weight), {normed, normed_ref}, a.hidden_index, n_valid,
                 a.hidden_stride_b, (int)n_tokens, (int)n_rows, (int)H, norm_eps};
-    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((unsigned)((n_tokens + 3) / 4)), dim3(256), 0, stream, na);
-    if (hidden_ref != hidden) {
-      na.x = static_cast<const char*>(hidden_ref);
-      na.y = normed + normed_bytes(n_tokens, H, true);
-      hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((unsigned)((n_tokens + 3) / 4)), dim3(256), 0, stream, na);
-      second_hidden = na.y;
-    } else {
-      second_hidden = normed;
-    }
+    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((unsigned)((n_tokens + 3) / 4), hidden_ref != hidden ? 2 : 1), dim3(256), 0, stream, na);
+    second_hidden = normed_ref;
     a.hidden = normed;
     a.hidden_index = nullptr;
     a.hidden_stride_b = (uint32_t)(H * 2);
     a.hidden_bytes = (uint32_t)(n_tokens * H * 2);
   }
-  a.n_tokens = (int)n_tokens;
+  a.hidden2 = joint ? second_hidden : nullptr;
+  const int swept = (int)n_tokens << (joint ? 1 : 0);
+  a.n_tokens = swept;
   a.H = (int)H;
   a.V = (int)V;
-  // Workspace header: [0] n_valid, [16..32) the schedule derived from it on the device.
+  // Workspace header: [0] n_valid, [16..40) the schedule derived from it on the device.
   a.sched_dev = sel.masked() ? reinterpret_cast<const FusedSchedule*>(n_valid + 4) : nullptr;
-  a.sched = fused_schedule((int)n_tokens, plan.shape);
+  a.sched = fused_schedule(swept, plan.shape);
   a.scale = kLog2e / temperature;
   FusedPartial* p0 = reinterpret_cast<FusedPartial*>(ws + off_partials(n_tokens));
   FusedPartial* p1 = reinterpret_cast<FusedPartial*>(ws + off_partials(n_tokens) + partial_bytes(n_tokens, H, V));
@@ -950,7 +965,7 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
     a.sched_dev = nullptr;
   }
   const char* first_hidden = a.hidden;
-  if (second) {
+  if (second && !joint) {
     a.weight = static_cast<const char*>(w1);
     a.hidden = second_hidden;
     a.partials = p1;
@@ -962,7 +977,8 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
 
   CombineArgs c;
   c.partials = p0;
-  c.partials_ref = second ? p1 : nullptr;
+  c.partials_ref = second && !joint ? p1 : nullptr;
+  c.joint = joint ? 1 : 0;
   c.row_index = row_index;
   c.n_valid = n_valid;
   c.out_lp = out_lp;
