@@ -110,8 +110,14 @@ __device__ __forceinline__ void pair_reads() {
 // workgroups of an XCD that share a W tile want it kept (4096 x 1024: 936 -> 951), and so do three 128-token tiles
 // (384 x 1024: 130 -> 138).
 //
+// ROT (tiles of up to 128 tokens, W requested non-temporally): where one token tile streams W and its rows lie a multiple of 8 KB
+// apart, the workgroups start their K loops at different slabs (the sums just begin elsewhere).  In step, all of them would ask
+// the same few memory channels for the same columns of their rows: V = 50257 / 64001 / 100000 / 128256 / 151936 x H = 4096, 64 tokens
+// 96 -> 68, 120 -> 84, 144 -> 128, 161 -> 158, 194 -> 189 us, 128 tokens 100 -> 80, 123 -> 88, 157 -> 147, 172 -> 171, 213 -> 216.  Row
+// pitches of 2 and 5 KB gain nothing, nor does a W that the memory-side cache holds (32000 x 4096: 50.0 -> 50.5).
+__device__ __host__ inline bool dma_rotates(const FusedArgs& a) { return (a.weight_stride_b & 8191) == 0; }
 // NBT: this wave's token blocks; BT: the workgroup's token tile; tok0: this wave's first token in it.
-template <bool ENT, bool AMAX, int NBT, int BT, int HI, bool DEEP, bool WNT>
+template <bool ENT, bool AMAX, int NBT, int BT, int HI, bool DEEP, bool WNT, bool ROT>
 __device__ __forceinline__ void dma_sweep(const FusedArgs& a, const FusedSchedule& sch, int n_valid, int ttile, int split, int wave,
                                           int tok0) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];  // (handed down as a pointer it costs the sweep 2-4 %)
@@ -181,6 +187,8 @@ __device__ __forceinline__ void dma_sweep(const FusedArgs& a, const FusedSchedul
   // request and are rebased at vocab-tile changes, so a step carries no multiplies or divides.
   const int dr = lane >> 3;                                   // row inside the 8-row group
   const int dc = (lane & 7) ^ (4 * (wave & 1) + (dr >> 1));   // global chunk: position ^ ((row >> 1) & 7)
+  const int nk = a.H / k2BK;
+  const int k0 = ROT && sch.n_ttiles == 1 && dma_rotates(a) ? split % nk : 0;
   const char* pa[k2Loads];  // next W slab to request, per DMA instruction
   const char* pb[kBLoads];  // next hidden slab
   // Mixed heights: LDS row r of a W slab holds vocab row  base + (r / 128) * wr + min(r % 128, wr - 1)  of tile `tile`,
@@ -208,7 +216,7 @@ __device__ __forceinline__ void dma_sweep(const FusedArgs& a, const FusedSchedul
         v = base + ((HI == 4 || r < 2 * wr) ? r : r - 32);
       }
       v = v < a.V ? v : a.V - 1;
-      pa[j] = a.weight + v * a.weight_stride_b + dc * 16;
+      pa[j] = a.weight + v * a.weight_stride_b + dc * 16 + (ROT ? k0 * k2RowBytes : 0);
     }
   };
   point_a(0);
@@ -218,7 +226,7 @@ __device__ __forceinline__ void dma_sweep(const FusedArgs& a, const FusedSchedul
     p = p < n_valid ? p : n_valid - 1;
     const TokenSource src = token_source(a, p, n_valid);
     const int tok = a.hidden_index ? min(max(a.hidden_index[src.q], 0), a.n_rows - 1) : src.q;
-    pb[j] = src.hidden + (int64_t)tok * a.hidden_stride_b + dc * 16;
+    pb[j] = src.hidden + (int64_t)tok * a.hidden_stride_b + dc * 16 + (ROT ? k0 * k2RowBytes : 0);
   }
 
   // ---- per-lane token state: one token per 16-token block, shared by the four lane groups ---------
@@ -238,10 +246,10 @@ __device__ __forceinline__ void dma_sweep(const FusedArgs& a, const FusedSchedul
   const int rdA = (wave_v * (kMixed ? 128 : kMaxBlocks * 16) + l16) * k2RowBytes + swz;
   const int rdB = (tok0 + l16) * k2RowBytes + swz;
 
-  const int nk = a.H / k2BK;
   const int n_steps = n_tiles * nk;
   const int64_t slab_rewind = (int64_t)(nk - 1) * k2RowBytes;
   int i_kt = 0, i_tile = 0;  // slab the next request fetches
+  int i_col = k0;            // its place in the row (ROT)
   int issued = 0;            // slabs requested so far; request q lands in buffers q % kBufs
 
   // One of the DMA instructions of the next request (0-3: W rows; the others: hidden rows).  Past the last slab
@@ -255,6 +263,24 @@ __device__ __forceinline__ void dma_sweep(const FusedArgs& a, const FusedSchedul
   auto issue_done = [&]() {
     ++issued;
     if (issued >= n_steps) return;  // the stream stays on the last slab
+    if constexpr (ROT) {
+      int64_t on = k2RowBytes;
+      if (++i_col == nk) {
+        i_col = 0;
+        on = -slab_rewind;
+      }
+#pragma unroll
+      for (int j = 0; j < kBLoads; ++j) pb[j] += on;
+      if (++i_kt < nk) {
+#pragma unroll
+        for (int j = 0; j < k2Loads; ++j) pa[j] += on;
+      } else {
+        i_kt = 0;
+        ++i_tile;
+        if (i_tile < n_tiles) point_a(i_tile);
+      }
+      return;
+    }
     if (++i_kt < nk) {
 #pragma unroll
       for (int j = 0; j < k2Loads; ++j) pa[j] += k2RowBytes;
@@ -331,6 +357,9 @@ __device__ __forceinline__ void dma_sweep(const FusedArgs& a, const FusedSchedul
         acc[i0 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], decltype(fresh)::value ? zero : acc[i0 + i][j],
                                                                    0, 0, 0);
   };
+  // The two waves of a SIMD (w and w + 4) at different priorities: they fall out of step between barriers, one's fragment reads under
+  // the other's MFMAs (1 % at 96 .. 600 tokens, nothing where power decides: 200 x 2560 182.5 -> 180.7 us, 96 x 2560 142.6 -> 141.1).
+  if (wave >= 4) __builtin_amdgcn_s_setprio(1);
   int step = 0;
   // N times (one MFMA, then one DMA request).
   auto pair_dma = [](auto n) {
@@ -443,7 +472,7 @@ __device__ __forceinline__ void dma_sweep(const FusedArgs& a, const FusedSchedul
 // schedule names.  Behind a mask the number of tokens, and so the tile, is only known on the device.  The combined kernel
 // costs about 1 us a launch more and runs the 256-token tile 1-2 % slower than the kernels of one tile each.
 constexpr int kAnyTile = -1;
-template <bool ENT, bool AMAX, int TILE, bool DEEP, bool WNT>
+template <bool ENT, bool AMAX, int TILE, bool DEEP, bool WNT, bool ROT = false>
 __global__ __launch_bounds__(k2WG) void fused_lmhead_dma_kernel(FusedArgs a) {
   touch_args(a);
   int n_valid = a.n_tokens;
@@ -459,12 +488,13 @@ __global__ __launch_bounds__(k2WG) void fused_lmhead_dma_kernel(FusedArgs a) {
     constexpr FusedTile kTile = fused_tile(decltype(tile)::value);
     constexpr int BT = kTile.tokens, NA = (BT + 32) / 64, NB = BT / 32 - NA, HI = kTile.unit32 == 1 ? 0 : kTile.unit32 - 4;
     constexpr bool kDeep = DEEP && BT > 128;
+    constexpr bool kRot = BT <= 128 && (TILE == kAnyTile ? WNT : ROT);
     static_assert(BT == dma_tile_tokens(NA, NB), "two token waves of NA blocks, two of NB");
     const int wave_t = wave >> 1;
     if (NA == NB || wave_t < 2) {
-      dma_sweep<ENT, AMAX, NA, BT, HI, kDeep, WNT>(a, sch, n_valid, ttile, split, wave, wave_t * NA * 16);
+      dma_sweep<ENT, AMAX, NA, BT, HI, kDeep, WNT, kRot>(a, sch, n_valid, ttile, split, wave, wave_t * NA * 16);
     } else if constexpr (NA != NB) {  // the same steps, so the same barriers
-      dma_sweep<ENT, AMAX, NB, BT, HI, kDeep, WNT>(a, sch, n_valid, ttile, split, wave, 2 * NA * 16 + (wave_t - 2) * NB * 16);
+      dma_sweep<ENT, AMAX, NB, BT, HI, kDeep, WNT, kRot>(a, sch, n_valid, ttile, split, wave, 2 * NA * 16 + (wave_t - 2) * NB * 16);
     }
   };
   if constexpr (TILE != kAnyTile) {
@@ -483,12 +513,12 @@ __global__ __launch_bounds__(k2WG) void fused_lmhead_dma_kernel(FusedArgs a) {
   }
 }
 
-template <bool ENT, bool AMAX, int TILE, bool DEEP, bool WNT>
+template <bool ENT, bool AMAX, int TILE, bool DEEP, bool WNT, bool ROT = false>
 static void launch_dma_form(const FusedArgs& a, int grid, hipStream_t stream) {
   constexpr int kLds = dma_lds_bytes(TILE == kAnyTile ? 256 : fused_tile(TILE < 0 ? 0 : TILE).tokens, DEEP);
   static DeviceOnce attr_set;  // opt in to > 64 KB of dynamic LDS once per instantiation and device
-  if (attr_set.first_on_current_device()) allow_big_lds(&fused_lmhead_dma_kernel<ENT, AMAX, TILE, DEEP, WNT>, kLds);
-  hipLaunchKernelGGL((fused_lmhead_dma_kernel<ENT, AMAX, TILE, DEEP, WNT>), dim3((unsigned)grid), dim3(k2WG), kLds, stream, a);
+  if (attr_set.first_on_current_device()) allow_big_lds(&fused_lmhead_dma_kernel<ENT, AMAX, TILE, DEEP, WNT, ROT>, kLds);
+  hipLaunchKernelGGL((fused_lmhead_dma_kernel<ENT, AMAX, TILE, DEEP, WNT, ROT>), dim3((unsigned)grid), dim3(k2WG), kLds, stream, a);
 }
 // w_nt: non-temporal W requests (the kernel's WNT).
 template <bool ENT, bool AMAX>
@@ -501,6 +531,9 @@ void launch_dma(const FusedArgs& a, int tile, bool deep, bool w_nt, int grid, hi
   auto go = [&](auto t) {
     constexpr int TILE = decltype(t)::value;
     constexpr bool kBig = fused_tile(TILE).tokens > 128;
+    if constexpr (!kBig) {
+      if (w_nt && dma_rotates(a)) return launch_dma_form<ENT, AMAX, TILE, false, true, true>(a, grid, stream);
+    }
     if (w_nt && (deep || !kBig)) launch_dma_form<ENT, AMAX, TILE, kBig, true>(a, grid, stream);
     else if (deep || !kBig) launch_dma_form<ENT, AMAX, TILE, kBig, false>(a, grid, stream);
     else if constexpr (fused_tile(TILE).tokens == 256) launch_dma_form<ENT, AMAX, TILE, false, false>(a, grid, stream);

@@ -398,7 +398,12 @@ __global__ __launch_bounds__(512) void fused_lmhead_small_kernel(FusedArgs a) {
     }
   }
   // One partial per (token, workgroup): part index = workgroup id.
-  if (wave < NBT) write_partials16<1>(st, tx, a.partials, wave * 16, n_valid, (int)blockIdx.x, (int)gridDim.x, l16, g, a.scale);
+  // (the lane derived afresh: kept across the loop it is one register too many for two token blocks of 512 columns, and the loop's
+  // loads are then scheduled around a spill, 1-4 % at 17 .. 32 tokens x H = 4096)
+  int ln = (int)threadIdx.x;
+  asm volatile("" : "+v"(ln));
+  if (wave < NBT)
+    write_partials16<1>(st, tx, a.partials, wave * 16, n_valid, (int)blockIdx.x, (int)gridDim.x, ln & 15, (ln & 63) >> 4, a.scale);
 }
 
 // ---- compaction of valid rows ----------------------------------------------------------------
