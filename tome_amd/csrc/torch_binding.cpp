@@ -10,10 +10,6 @@
 #include <pybind11/pybind11.h>
 #include <torch/csrc/utils/pybind.h>
 
-#ifdef __SSE2__
-#include <emmintrin.h>
-#endif
-#include <algorithm>
 #include <cstring>
 #include <optional>
 #include <string>
@@ -395,29 +391,6 @@ std::pair<int64_t, int64_t> matrix_shape(int64_t n, std::vector<int64_t> shape) 
   return {shape[0], shape[1]};
 }
 
-// Bytes into memory that the GPU's copy engine reads next: stored past the caches, which would otherwise fetch every line of the
-// destination before it is overwritten (8 MB 280 -> 132 us on one thread).  A fence (stream_fence) before the copy is started.
-void stream_copy(void* dst, const void* src, size_t n) {
-#ifdef __SSE2__
-  char* d = static_cast<char*>(dst);
-  const char* s = static_cast<const char*>(src);
-  const size_t head = std::min(n, (size_t)(-reinterpret_cast<uintptr_t>(d) & 15));
-  std::memcpy(d, s, head);
-  size_t i = head;
-  for (; i + 64 <= n; i += 64)
-    for (int k = 0; k < 4; ++k)
-      _mm_stream_si128(reinterpret_cast<__m128i*>(d + i + 16 * k), _mm_loadu_si128(reinterpret_cast<const __m128i*>(s + i + 16 * k)));
-  std::memcpy(d + i, s + i, n - i);
-#else
-  std::memcpy(dst, src, n);
-#endif
-}
-void stream_fence() {
-#ifdef __SSE2__
-  _mm_sfence();
-#endif
-}
-
 struct Staged {  // one matrix: source, and its place (zero-padded to out_rows x out_cols) in the staging buffer
   const uint16_t* src;
   int64_t rows, cols, out_rows, out_cols, off;
@@ -425,7 +398,7 @@ struct Staged {  // one matrix: source, and its place (zero-padded to out_rows x
   void copy_to(uint16_t* stage) const {
     uint16_t* dst = stage + off;
     if (cols == out_cols) {
-      stream_copy(dst, src, (size_t)(rows * cols) * 2);
+      std::memcpy(dst, src, (size_t)(rows * cols) * 2);
       std::memset(dst + rows * cols, 0, (size_t)((out_rows - rows) * cols) * 2);
       return;
     }
@@ -440,9 +413,8 @@ struct Staged {  // one matrix: source, and its place (zero-padded to out_rows x
 // matrix on a 16-byte boundary, the rank zero-padded to a multiple of 8 (extra terms of the product are exact zeros).
 // Returns (lora_A [rank, in], lora_B [out, rank]) per entry, views of the buffer.  The bytes go through page-locked memory (torch's
 // pool, which holds a block until the copies that read it are done), a megabyte's copy under way while the next is filled.
-// (Four threads filled 7 MB with ordinary stores in 340 us where one took 310, but in 1000 to 4600 whenever the request's other
-// work had left the process's CPUs busy.  Merging the first layers while the later ones are filled was slower too: the copies that
-// then queue between kernels cost more than they hide, 855 us a request against 815, on a stream of their own 1030.)
+// (Four threads filled 7 MB in 340 us where this takes 310, but in 1000 to 4600 whenever the request's other work had left the
+// process's CPUs busy.)
 constexpr int64_t kStagePart = 1 << 19;  // elements
 std::vector<std::pair<Tensor, Tensor>> stage_adapters(const py::list& entries, const std::string& device) {
   const c10::Device dev(device);
@@ -481,7 +453,6 @@ std::vector<std::pair<Tensor, Tensor>> stage_adapters(const py::list& entries, c
       parts[i].copy_to(stage);
       const int64_t lo = parts[begin].off, hi = i + 1 < parts.size() ? parts[i + 1].off : total;
       if (hi - lo < kStagePart && i + 1 < parts.size()) continue;
-      stream_fence();
       if (dev.is_cuda()) buf.slice(0, lo, hi).copy_(host.slice(0, lo, hi), /*non_blocking=*/true);
       begin = i + 1;
     }
