@@ -352,6 +352,25 @@ def test_norm_lmhead_matches_oracle(dev, n, H, V, masked):
     assert np.abs(raw[m] - want["lp"][m]).max() > 0.1
 
 
+@pytest.mark.parametrize("n,H,masked", [(1, 8, False), (5, 504, False), (7, 520, True), (9, 4088, False), (6, 4096, True), (5, 4104, False),
+                                        (130, 6152, True), (3, 8192, False)])
+def test_norm_rows_held_in_registers_and_beyond(dev, n, H, masked):
+    """The norm kernel holds rows of up to 4096 elements in registers and reads what is longer a second time: less than one unit a
+    lane, remainders of a 512-element step, the last row held whole, one unit past it, twice its length."""
+    rng = np.random.default_rng(n * 7 + H)
+    h, w, t = _inputs(dev, n, H, 600, seed=n + H, h_scale=3.0, w_scale=1.0 / np.sqrt(H))
+    gamma = torch.from_numpy((1.0 + 0.2 * rng.standard_normal(H)).astype(np.float32)).to(dev).to(torch.bfloat16)
+    valid = np.arange(n) % 3 != 1 if masked else np.ones(n, bool)
+    r = tome_amd.fused_lmhead_logprobs(h, w, torch.from_numpy(t).to(dev), 1.0, want_lse=True, norm_weight=gamma, norm_eps=1e-6,
+                                       row_valid=torch.from_numpy(valid).to(dev) if masked else None)
+    normed = oracle.rms_norm_bf16(bf16_bits_of(h), bf16_bits_of(gamma), 1e-6)
+    want = oracle.lmhead_stats(normed, bf16_bits_of(w), t, 1.0)
+    # as above: 2e-3 of the fused path, and one-ulp flips (2^-8 of a value of up to ~4 times a weight of up to ~4 / sqrt(H))
+    atol = 2e-3 + 2.0 ** -8 * 16 / np.sqrt(H)
+    np.testing.assert_allclose(r.lp.cpu().numpy()[valid], want["lp"][valid], atol=atol, rtol=0)
+    np.testing.assert_allclose(r.lse.cpu().numpy()[valid], want["lse"][valid], atol=atol, rtol=0)
+
+
 @pytest.mark.parametrize("n,H,V,masked", [
     (1, 1024, 151936, False), (16, 1024, 40000, True), (17, 1024, 8191, False), (64, 1024, 151936, True),
     (33, 2048, 30001, False), (64, 2048, 12345, True), (9, 4096, 20000, False), (32, 4096, 33000, True),
