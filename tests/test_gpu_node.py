@@ -117,6 +117,44 @@ def test_entry_prenorm_mode_applies_the_final_norm_to_completion_rows(dev):
         tome_amd.RefLogprobServicer(model, device=dev, final_norm_weight=to_t(gamma))
 
 
+@pytest.mark.parametrize("H,layout,norm", [(128, "plain", False), (128, "plain", True), (72, "plain", False), (128, "odd", False),
+                                           (128, "odd", True), (128, "strided", False), (128, "strided", True)])
+def test_entry_hidden_mode_addresses_rows_in_place_or_gathers_them(dev, H, layout, norm):
+    """States the kernels can address (contiguous, on 16 bytes, H a multiple of 64) are read through the row list, others gathered:
+    the log-probs of the gathered rows through the public function, whatever the layout the model returns."""
+    g = torch.Generator(device=dev).manual_seed(H + norm)
+    emb = (torch.randn((V_STUB, H), device=dev, generator=g) * 0.3).to(torch.bfloat16)
+    gamma = (torch.rand(H, device=dev, generator=g) + 0.5).to(torch.bfloat16) if norm else None
+    seen = []
+
+    def model(full_ids, cache=None):
+        e = (emb[full_ids].float() * (1.0 + 0.1 * torch.arange(full_ids.shape[1], device=dev)[None, :, None])).to(torch.bfloat16)
+        if layout == "odd":        # rows that start 2 bytes off
+            buf = torch.empty(e.numel() + 1, device=dev, dtype=torch.bfloat16)
+            buf[1:] = e.flatten()
+            e = buf[1:].view(e.shape)
+        elif layout == "strided":  # a column slice of wider rows
+            wide = torch.zeros((*e.shape[:2], H + 8), device=dev, dtype=torch.bfloat16)
+            wide[..., :H] = e
+            e = wide[..., :H]
+        seen.append(e)
+        return e, None
+
+    prompts, results = make_batch(seed=9, n_prompts=2, G=2)
+    svc = tome_amd.RefLogprobServicer(model, device=dev, lm_head_weight=emb, final_norm_weight=gamma, norm_eps=1e-6)
+    svc.process_ref_logprobs_batched(prompts, results, 2, 0.9)
+    assert len(seen) == 1
+    seq = 0
+    for p, r in zip(prompts, results):
+        for c in r.completions:
+            first = len(p.tokens) - 1
+            rows = seen[0][seq, first:first + len(c.tokens)].clone()
+            want = tome_amd.fused_lmhead_logprobs(rows, emb, torch.tensor(c.tokens, device=dev, dtype=torch.int64), 0.9, norm_weight=gamma, norm_eps=1e-6).lp
+            # fp32 sums over a vocabulary split differently for another number of rows
+            np.testing.assert_allclose(c.ref_log_probs, want.cpu().numpy(), atol=2e-5, rtol=0)
+            seq += 1
+
+
 # ---- golden vectors through the C ABI ------------------------------------------------------------------
 @pytest.mark.parametrize("name", ["s0", "s1", "s2"])
 def test_golden_small(dev, name):

@@ -18,7 +18,7 @@ import numpy as np
 import torch
 
 from .wire import PackedRefChunk, iter_ref_work, scatter_ref_logprobs
-from .logprob import fused_lmhead_logprobs, token_logprobs_rows
+from .logprob import _lmhead_logprobs_rows, token_logprobs_rows
 
 logger = logging.getLogger(__name__)
 
@@ -114,9 +114,9 @@ class RefLogprobServicer:
         if self.lm_head_weight is None:
             lps = token_logprobs_rows(out, rows, tg, temp).lp             # only the listed rows are launched
         else:
-            picked = out.reshape(nb * max_len, out.shape[-1]).index_select(0, rows.long())   # completion rows only
-            lps = fused_lmhead_logprobs(picked, self.lm_head_weight, tg, temp,
-                                        norm_weight=self.final_norm_weight, norm_eps=self.norm_eps).lp
+            states = out.reshape(nb * max_len, out.shape[-1])
+            lps = _lmhead_logprobs_rows(states, self.lm_head_weight, rows, tg, temp,                 # completion rows only
+                                        self.final_norm_weight, self.norm_eps)
         slot.host_out[:n].copy_(lps, non_blocking=True)                   # node.py:456: the one copy back, of n floats
         slot.done.record(torch.cuda.current_stream(self.device))
         slot.chunk, slot.keep = chunk, (out, lps)                         # outputs stay alive until they have been read
