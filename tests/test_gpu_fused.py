@@ -184,6 +184,23 @@ def test_fused_argmax_spike_and_ties(dev):
     assert (masked.argmax.cpu().numpy() == -1).all()
 
 
+@pytest.mark.parametrize("n,masked,entropy", [(40, False, False), (90, False, True), (128, False, False), (100, True, False), (128, True, True)])
+def test_fused_argmax_ties_of_equal_rows_far_apart(dev, n, masked, entropy):
+    """Rows of W that are equal bit for bit have equal logits wherever they lie, so the lower id is the argmax.  Small batches on a W
+    that is streamed, rows 8 KB apart: the shape on which the plain sweep starts its K loops at different columns."""
+    H, V = 4096, 50257
+    g = torch.Generator(device=dev).manual_seed(n)
+    h = torch.empty((n, H), device=dev, dtype=torch.bfloat16).normal_(0, 1, generator=g)
+    w = torch.empty((V, H), device=dev, dtype=torch.bfloat16).normal_(0, 0.02, generator=g)
+    ids = torch.randperm(V, device=dev, generator=g)[: 2 * n].reshape(n, 2).sort(dim=1).values
+    w[ids[:, 0]] = w[ids[:, 1]] = (h.float() * 0.05).to(torch.bfloat16)   # token i's two rows: logit ~ 200, all others under 20
+    valid = torch.rand(n, device=dev, generator=g) < 0.8 if masked else torch.ones(n, dtype=torch.bool, device=dev)
+    r = tome_amd.fused_lmhead_logprobs(h, w, ids[:, 1], 1.0, want_argmax=True, want_entropy=entropy, row_valid=valid if masked else None)
+    m = valid.cpu().numpy()
+    np.testing.assert_array_equal(r.argmax.cpu().numpy()[m], ids[:, 0].cpu().numpy()[m])
+    np.testing.assert_allclose(r.lp.cpu().numpy()[m], -np.log(2.0), atol=TOL, rtol=0)
+
+
 @pytest.mark.parametrize("kind", ["generic", "dma", "dma_whole_tiles"])
 def test_fused_every_kernel_path(dev, kind, force_kernel):
     """The two GEMM kernels behind tome_fused_lmhead_logprob (generic / LDS-DMA) are picked
@@ -464,8 +481,8 @@ TOKEN_TILES = [64, 96, 128, 192, 224, 256]
 ])
 def test_fused_token_tiles_agree(dev, n, H, V, outputs):
     """Every token tile size of the LDS-DMA kernel (64 .. 256, even and uneven pairs of token waves, batches that fill a tile,
-    that start a new one and that end inside either half of one) against the oracle, with and without a mask.  A logit's
-    products are summed in the same order whatever the tile, so all of them must name the same argmax; the row sums meet in
+    that start a new one and that end inside either half of one) against the oracle, with and without a mask.  Where the
+    argmax is asked for a logit's products are summed in the same order whatever the tile, so all of them must name the same one; the row sums meet in
     another order, which fp32 rounds within (number of partials + 16) * 2^-24 of a sum whose log is taken: under 1e-4."""
     h, w, t = _inputs(dev, n, H, V, seed=n + V, w_scale=0.1)
     edges = [v for v in (0, 15, 16, 127, 128, 223, 224, 255, 256, V - 33, V - 1) if 0 <= v < V][:n]

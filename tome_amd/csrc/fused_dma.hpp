@@ -110,8 +110,9 @@ __device__ __forceinline__ void pair_reads() {
 // workgroups of an XCD that share a W tile want it kept (4096 x 1024: 936 -> 951), and so do three 128-token tiles
 // (384 x 1024: 130 -> 138).
 //
-// ROT (tiles of up to 128 tokens, W requested non-temporally): where one token tile streams W and its rows lie a multiple of 8 KB
-// apart, the workgroups start their K loops at different slabs (the sums just begin elsewhere).  In step, all of them would ask
+// ROT (tiles of up to 128 tokens, W requested non-temporally, no argmax): where one token tile streams W and its rows lie a multiple of
+// 8 KB apart, the workgroups start their K loops at different slabs (the sums just begin elsewhere).  Not with the argmax: rows of W
+// that are equal bit for bit must have equal logits wherever they lie, or the first of them is not the one that is named.  In step, all of them would ask
 // the same few memory channels for the same columns of their rows: V = 50257 / 64001 / 100000 / 128256 / 151936 x H = 4096, 64 tokens
 // 96 -> 68, 120 -> 84, 144 -> 128, 161 -> 158, 194 -> 189 us, 128 tokens 100 -> 80, 123 -> 88, 157 -> 147, 172 -> 171, 213 -> 216.  Row
 // pitches of 2 and 5 KB gain nothing, nor does a W that the memory-side cache holds (32000 x 4096: 50.0 -> 50.5).
@@ -488,7 +489,7 @@ __global__ __launch_bounds__(k2WG) void fused_lmhead_dma_kernel(FusedArgs a) {
     constexpr FusedTile kTile = fused_tile(decltype(tile)::value);
     constexpr int BT = kTile.tokens, NA = (BT + 32) / 64, NB = BT / 32 - NA, HI = kTile.unit32 == 1 ? 0 : kTile.unit32 - 4;
     constexpr bool kDeep = DEEP && BT > 128;
-    constexpr bool kRot = BT <= 128 && (TILE == kAnyTile ? WNT : ROT);
+    constexpr bool kRot = BT <= 128 && !AMAX && (TILE == kAnyTile ? WNT : ROT);
     static_assert(BT == dma_tile_tokens(NA, NB), "two token waves of NA blocks, two of NB");
     const int wave_t = wave >> 1;
     if (NA == NB || wave_t < 2) {
@@ -531,7 +532,7 @@ void launch_dma(const FusedArgs& a, int tile, bool deep, bool w_nt, int grid, hi
   auto go = [&](auto t) {
     constexpr int TILE = decltype(t)::value;
     constexpr bool kBig = fused_tile(TILE).tokens > 128;
-    if constexpr (!kBig) {
+    if constexpr (!kBig && !AMAX) {
       if (w_nt && dma_rotates(a)) return launch_dma_form<ENT, AMAX, TILE, false, true, true>(a, grid, stream);
     }
     if (w_nt && (deep || !kBig)) launch_dma_form<ENT, AMAX, TILE, kBig, true>(a, grid, stream);
