@@ -2,6 +2,7 @@
 // the fold of a 16x16 MFMA accumulator tile into the running row states.
 #pragma once
 #include "common.hpp"
+#include "fused_plan.hpp"
 #include <atomic>
 #include <type_traits>
 
@@ -9,140 +10,6 @@ namespace tome {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kBV = 256;                 // vocab rows per tile
-constexpr int kWaveV = 128;              // vocab rows per wave
-constexpr int kPartsPerSplit = kBV / kWaveV;
-constexpr int kDmaSlab = 64;             // K columns per step of the DMA kernel
-
-struct FusedPartial {  // 32 bytes per (token, part)
-  float mx, s, w, tx;
-  int bi;
-  int pad[3];
-};
-
-// Work decomposition: token tiles x vocab splits.  It depends on the number of valid tokens, which is
-// known on the host without a mask and only on the device with one, so it is computed by the host (and
-// passed by value) or by compact_rows_kernel (and read from the workspace header); both run the
-// same code.  Every kernel of a launch uses the same numbers.
-//
-// A workgroup owns one token tile and one contiguous range of vocab tiles.
-//   * Few token tiles (n_ttiles * 8 <= slots): as many splits as fill the chip in ONE round, rounded
-//     down - one workgroup too many would cost a whole extra round.
-//   * Many token tiles: several rounds.  The candidates 1..32 are priced as
-//         rounds * (longest vocab range + half a tile of prologue) * L2 penalty
-//     where the penalty prefers >= 8 splits: the workgroups resident on an XCD are then a block of
-//     ~4 token tiles x ~8 splits, which read 12 distinct slab streams through its L2 instead of 33
-//     (measured on MI355X: 65536 tokens, H = 4096: 1 split 1.09 PFLOP/s, 8-9 splits 1.4).
-struct FusedSchedule {
-  int n_ttiles, n_splits, n_wg;
-  int tile;              // index of FusedTile
-  int n_vunits, unit32;  // vocab units the splits share out, and 32-row blocks per unit
-};
-// A token tile and how the vocab axis is dealt to the splits with it: in whole tiles of 256 or 224 rows (unit32 = 8 / 7), or in
-// 32-row units, of which a workgroup makes tiles of up to 256 rows, all within one unit of each other.
-struct FusedTile {
-  int tokens, unit32;
-};
-constexpr int kFusedTiles = 9, kTileGeneric = 8;  // 0 .. 7: the DMA kernel's; 8: the generic kernel's
-__host__ __device__ constexpr FusedTile fused_tile(int i) {
-  return i == 0 ? FusedTile{256, 8} : i == 1 ? FusedTile{256, 7} : i == 2 ? FusedTile{224, 8} : i == 3 ? FusedTile{224, 7} :
-         i == 4 ? FusedTile{192, 1} : i == 5 ? FusedTile{128, 1} : i == 6 ? FusedTile{96, 1} : i == 7 ? FusedTile{64, 1} : FusedTile{128, 8};
-}
-// What the decomposition depends on beside the number of valid tokens.
-struct FusedShape {
-  int H, V;
-  int slots;       // workgroups that fit the chip at once
-  uint32_t tiles;  // bit i: FusedTile i may be taken
-  int vunits32, vunits224, vunits256;  // the vocab axis in 32-row units, 224-row and 256-row tiles
-  int whole;       // 1: vocab ranges in whole 256-row tiles whatever the token tile
-};
-inline FusedShape fused_shape(int64_t H, int64_t V, int slots, uint32_t tiles, bool whole) {
-  return FusedShape{(int)H, (int)V, slots, tiles, (int)((V + 31) / 32), (int)((V + 223) / 224), (int)((V + 255) / 256), whole ? 1 : 0};
-}
-__host__ __device__ inline bool fused_one_tile(const FusedShape& sh) { return (sh.tiles & (sh.tiles - 1)) == 0; }
-// The tiles below 256 tokens save padding where there are few of them; they are not taken beyond these numbers of valid tokens
-// (5074 tokens: 256 a tile 1148 us, 224 1207; the tiles up to 128 tokens are no better than 192 from two of those on).
-__host__ __device__ constexpr int fused_tile_most(int i) { return i >= 5 && i < kTileGeneric ? 256 : i >= 2 && i < 5 ? 2560 : 0x7fffffff; }
-__host__ __device__ inline bool fused_tile_allowed(const FusedShape& sh, int n_valid, int i) {
-  return ((sh.tiles >> i) & 1) && (n_valid <= fused_tile_most(i) || fused_one_tile(sh));
-}
-__host__ __device__ inline int fused_unit32(const FusedShape& sh, int i) { return sh.whole ? 8 : fused_tile(i).unit32; }
-__host__ __device__ inline int fused_vunits(const FusedShape& sh, int i) {
-  const int u = fused_unit32(sh, i);
-  return u == 1 ? sh.vunits32 : u == 7 ? sh.vunits224 : sh.vunits256;
-}
-__host__ __device__ inline int fused_ttiles(int n_valid, int bt) {
-  const int t = (n_valid + bt - 1) / bt;
-  return t < 1 ? 1 : t;
-}
-__host__ __device__ inline int fused_one_round_splits(int n_ttiles, int slots, int n_vtiles) {
-  int sp = slots / n_ttiles;
-  if (sp > n_vtiles) sp = n_vtiles;  // every split keeps at least one tile's worth of rows
-  return sp < 1 ? 1 : sp;
-}
-// What a batch costs on tile i where one round of workgroups holds it: the longest vocab range bounds the launch.  Fitted to 2300
-// timings (V = 32000 .. 151936, H = 768 .. 4096, 33 .. 4096 tokens, every tile): per K slab and vocab tile a constant, the tile's
-// MFMA work and the hidden rows' fill, and per vocab tile the fold.  Choosing by it is 0.1 % slower than choosing the measured
-// best in the mean, at most 6 % at any of the 290 shapes (32000 x 2560, 640 tokens: 192 a tile 102.5 us, 224 96.9).  Tiles of 224 and
-// 192 tokens are only taken for a gain of 3 %: below that the optional outputs and the sharing of W in L2 decide, which are not
-// priced (50257 x 2048, 1024 tokens, as five tiles of 224 instead of four of 256: 165 -> 174 us).
-// 224-row vocab tiles pay where they shorten the longest range: whole 256-row tiles deal V = 151936 as three tiles to 82
-// workgroups and two to the others, 224-row tiles as three to 167 and two to 89, an eighth less for the longest.
-// (In floats, quotients of whole numbers with half a unit to spare before the rounding: integer divisions by a lane's own divisor
-// are 40 instructions each, and behind a mask one wave prices the tiles between two launches.)
-__host__ __device__ inline float fused_tile_cost(const FusedShape& sh, int n_valid, int i) {
-  const float tokens = (float)fused_tile(i).tokens, unit32 = (float)fused_unit32(sh, i), units = (float)fused_vunits(sh, i);
-  const float vtiles = unit32 == 1.f ? (float)sh.vunits256 : units, nk = (float)(sh.H / kDmaSlab);
-  const float ttiles = floorf(((float)n_valid + tokens - 0.5f) / tokens);
-  float splits = floorf(((float)sh.slots + 0.5f) / (ttiles < 1.f ? 1.f : ttiles));
-  splits = splits > vtiles ? vtiles : splits < 1.f ? 1.f : splits;
-  const float longest = floorf((units + splits - 0.5f) / splits);
-  const float tiles = unit32 == 1.f ? floorf((longest + 7.f) * 0.125f) : longest, rows = longest * unit32 * 32.f;
-  const float cost = tiles * nk * (61.f * 65536.f + 39.f * 256.f * tokens) + rows * (nk * (100.f * tokens + 3.f * 256.f) + 143.f * tokens);
-  return i >= 2 && i < 5 ? cost * 1.03f : cost;
-}
-__host__ __device__ inline int64_t fused_split_cost(int n_ttiles, int n_splits, int slots, int n_vunits, int upt) {
-  const int rounds = (n_ttiles * n_splits + slots - 1) / slots;
-  const int longest = (n_vunits + n_splits - 1) / n_splits;  // in units
-  const int pen64 = 60 + 32 / (n_splits < 8 ? n_splits : 8);
-  return ((int64_t)rounds * (2 * longest + upt) * pen64) * 64 + n_splits;  // ties go to fewer splits
-}
-constexpr int kSplitCandidates = 32;
-// The schedule but for the number of splits where several rounds are needed; returns whether that is so.
-__host__ __device__ inline bool fused_schedule_begin(FusedSchedule& s, int n_valid, const FusedShape& sh, int tile) {
-  s.tile = tile;
-  s.unit32 = fused_unit32(sh, tile);
-  s.n_vunits = fused_vunits(sh, tile);
-  s.n_ttiles = fused_ttiles(n_valid, fused_tile(tile).tokens);
-  if (s.n_ttiles * 8 > sh.slots) return true;
-  s.n_splits = fused_one_round_splits(s.n_ttiles, sh.slots, s.unit32 == 1 ? (s.n_vunits + 7) / 8 : s.n_vunits);
-  s.n_wg = s.n_ttiles * s.n_splits;
-  return false;
-}
-inline FusedSchedule fused_schedule_on(int n_valid, const FusedShape& sh, int tile) {  // host
-  FusedSchedule s;
-  if (fused_schedule_begin(s, n_valid, sh, tile)) {
-    const int upt = s.unit32 == 1 ? 8 : 1, n_vtiles = (s.n_vunits + upt - 1) / upt;
-    int64_t best = INT64_MAX;
-    for (int c = 1; c <= kSplitCandidates && c <= n_vtiles; ++c) {
-      const int64_t cost = fused_split_cost(s.n_ttiles, c, sh.slots, s.n_vunits, upt);
-      if (cost < best) best = cost;
-    }
-    s.n_splits = (int)(best & 63);
-    s.n_wg = s.n_ttiles * s.n_splits;
-  }
-  return s;
-}
-inline FusedSchedule fused_schedule(int n_valid, const FusedShape& sh) {  // host
-  float best = INFINITY;
-  int tile = 0;
-  for (int i = 0; i < kFusedTiles; ++i) {
-    if (!fused_tile_allowed(sh, n_valid, i)) continue;
-    const float c = fused_tile_cost(sh, n_valid, i);
-    if (c < best) best = c, tile = i;
-  }
-  return fused_schedule_on(n_valid, sh, tile);
-}
 // The same on the device, by one whole wave: lane i prices tile i, lane c c + 1 splits.
 __device__ inline FusedSchedule fused_schedule_wave(int n_valid, const FusedShape& sh, int lane) {
   int tile = __builtin_ctz(sh.tiles);

@@ -678,26 +678,10 @@ __global__ __launch_bounds__(256) void fused_combine_kernel(CombineArgs a) {
 // The DMA kernel needs whole 64-wide K slabs (ragged H goes to the generic kernel); its token tile shrinks
 // with the batch.  Decode-sized batches whose hidden states fit the waves' registers take the streaming kernel.
 
-enum FusedKind { kGeneric = 0, kDma = 1, kSmall = 2 };
-constexpr int kForceDmaWholeTiles = 3;  // selector value: the DMA kernel with vocab ranges cut at whole 256-row tiles
-constexpr int kForceDmaTwoWBuffers = 4, kForceDmaThreeWBuffers = 5;  // the DMA kernel, its 256-token tile with two / three W buffers
-constexpr int kForceDmaTile = 64;       // 64, 96 .. 256: the DMA kernel with token tiles of that size
-
 // Kernel selector for tests and tuning runs: -1 (the default) picks by shape, kGeneric / kDma force that
 // sweep kernel wherever its shape rules allow.  Process-wide; set it while no call is in flight.
 static std::atomic<int> g_forced_kind{-1};
 void fused_force_kernel(int kind) { g_forced_kind.store(kind, std::memory_order_relaxed); }
-
-struct FusedPlan {
-  FusedKind kind;
-  bool deep, deep_lp;                        // kDma only: three W buffers, for the first sweep / one without optional outputs
-  bool w_nt;                                 // kDma only: W requested non-temporally (few token tiles: see the kernel's WNT)
-  int small_nbt, small_ksteps, small_waves;  // kSmall only
-  FusedShape shape;
-  bool any_tile;       // kDma: behind a mask the device picks the token tile
-  int grid;            // workgroups to launch: the most any number of valid tokens can ask for
-  size_t max_records;  // partial records any number of valid tokens can produce
-};
 
 // The DMA kernels' launches (fused_dma.hpp), instantiated in the fused_dma_*.hip files: one token tile, or the tile of the schedule
 // on the device; the 160 KB of LDS their largest form asks for.
@@ -743,134 +727,13 @@ static int small_wg_count() {
   return n;
 }
 
-// Shape rules of the small-batch kernel: <= 64 tokens, K split over 2..8 waves in slices of 256 or 512
-// (slices of 128 on twice the waves measured 2 us slower at H = 1024).  At H = 1024 it keeps up to 16 tokens only: since
-// the tiled kernel requests W non-temporally where it streams through once, its 64- and 128-token tiles are faster there
-// from 17 tokens on (17..64 tokens: 53.3-54.8 against 54.7-59 us; 65..128, which this kernel served with eight token blocks
-// on K slices of 128: 61-64 against 67-72 us); at 1280, 1536 and 1792 the two are within 3 % of each other either way, at
-// 2048 and above this kernel wins (64 x 2048: 108 against 125 us).
-static bool small_shape(int64_t n_tokens, int64_t H, int64_t V, int& nbt, int& ksteps, int& waves) {
-  if (n_tokens > 64 || V < 64) return false;
-  if (H == 1024 && n_tokens > 16) return false;
-  nbt = n_tokens <= 16 ? 1 : (n_tokens <= 32 ? 2 : 4);
-  if (H % 256 == 0 && H / 256 <= 8 && H / 256 >= 2) {
-    ksteps = 8;
-    waves = (int)(H / 256);
-  } else if (H % 512 == 0 && H / 512 <= 8 && H / 512 >= 2 && nbt <= 2) {
-    ksteps = 16;
-    waves = (int)(H / 512);
-  } else {
-    return false;
-  }
-  if (ksteps == 8 && nbt == 2) nbt = 4;  // instantiated token-block counts: 1 and 4 (K 256), 1 and 2 (K 512)
-  return waves >= nbt;
-}
-
-// Behind a mask of up to this many tokens the device picks the token tile from the valid ones (60 % valid of 200 / 384 / 600 tokens, V =
-// 151936, H = 2560: 185 -> 170, 246 -> 197, 331 -> 269 us); the tiles that more tokens fill evenly enough are run by a
-// kernel of their own (2100 tokens: 0.975 .. 1.08 with the choice).
-constexpr int64_t kAnyTileTokens = 2048;
-
-static FusedPlan fused_plan(int64_t n_tokens, int64_t H, int64_t V, bool deep_lds, bool entropy, bool masked) {
-  FusedPlan p;
-  p.kind = H % kDmaSlab == 0 ? kDma : kGeneric;
-  p.small_nbt = p.small_ksteps = p.small_waves = 0;
-  const int forced = g_forced_kind.load(std::memory_order_relaxed);
-  // The streaming kernel runs one workgroup per CU: without a CU count (no device) the tiled kernels serve.
-  if (small_shape(n_tokens, H, V, p.small_nbt, p.small_ksteps, p.small_waves) && small_wg_count() >= 2) p.kind = kSmall;
-  if (forced == kGeneric) p.kind = kGeneric;
-  if ((forced == kDma || forced >= kForceDmaWholeTiles) && H % kDmaSlab == 0) p.kind = kDma;
-  // The third W buffer (see the kernel), measured against the two-buffer form in the same runs.  One or two token tiles:
-  // 6-13 % faster with any outputs (256 x 1024: 96 -> 87 us, 256 x 4096: 338 -> 297, 512 x 4096: 534 -> 503).  More token
-  // tiles, log-probs only: 4096 x 1024 -2.3 %, 8192 x 1024 -1.5 %, 1024 x 4096 -5 %, 4096 x 4096 -1.7 %, 16384 x 2560 -2.6 %,
-  // 8192 x 4096 -1.6..+0.2 % over boxes, but 32768 x 4096 +0.7 %, 65536 x 4096 +0.5..2 %.  With the argmax alone it follows
-  // (1024 x 4096 -4 %, 4096 x 1024 equal, 8192 x 4096 -1 %); with the entropy the fold of the deeper form spills 29-37
-  // registers around every tile change: 1024 x 4096 -3 %, but 4096 x 1024 +2.6 % and 8192 x 4096 +2.3 %.
-  p.deep_lp = deep_lds && (H < 4096 || n_tokens <= 8192);
-  p.deep = deep_lds && n_tokens <= 1024;
-  if (forced == kForceDmaTwoWBuffers) p.deep = p.deep_lp = false;
-  if (forced == kForceDmaThreeWBuffers) p.deep = p.deep_lp = deep_lds;
-  // Token tiles.  The two-buffer form has 256 tokens only, and a call of two sweeps one schedule for both.
-  const bool any = masked && n_tokens <= kAnyTileTokens && n_tokens > 64;
-  const bool all_deep = p.deep_lp && (p.deep || !entropy || any);
-  p.shape = fused_shape(H, V, 256, all_deep ? 0xffu : 3u, forced == kForceDmaWholeTiles);
-  if (forced == kForceDmaTwoWBuffers || forced == kForceDmaThreeWBuffers) p.shape.tiles = 3;
-  if (forced >= kForceDmaTile && all_deep) {
-    uint32_t only = 0;
-    for (int i = 0; i < kTileGeneric; ++i) only |= (uint32_t)(fused_tile(i).tokens == forced) << i;
-    p.shape.tiles = only ? only : p.shape.tiles;
-  }
-  if (p.shape.whole) p.shape.tiles &= ~((1u << 1) | (1u << 3));  // no vocab tiles of 224 rows
-  if (p.kind != kDma) {
-    p.shape.tiles = 1u << kTileGeneric;
-    p.shape.slots = 512;  // resident workgroups on 256 CUs: 2 per CU, or 1 for the DMA path's LDS (two 64-token workgroups
-                          // of 80 KB per CU measured slower than one: 288 against 277 us at 64 x 4096)
-  }
-  // A mask of up to 64 tokens leaves the smallest tile; beyond kAnyTileTokens the 256-token tile serves.
-  if (masked && p.kind == kDma && n_tokens > kAnyTileTokens) p.shape.tiles &= 3u;
-  if (masked && p.kind == kDma && (n_tokens <= 64 || n_tokens > kAnyTileTokens || !all_deep)) p.shape.tiles = 1u << fused_schedule((int)n_tokens, p.shape).tile;
-  p.any_tile = masked && p.kind == kDma && !fused_one_tile(p.shape);
-  p.w_nt = false;
-  p.grid = 0;
-  p.max_records = 0;
-  if (p.kind == kSmall) {
-    // One partial per (token, workgroup); one workgroup per CU, at most 512.  The schedule is ignored.
-    p.max_records = (size_t)64 * 512;
-    return p;
-  }
-  // Non-temporal W (the kernel's WNT): few token tiles, and a W larger than the 256 MB memory-side cache - a smaller one is
-  // found there again by the next call as long as it is requested normally (repeated calls, 64 tokens: V = 32000, H = 4096,
-  // 262 MB: 48 us against 71 non-temporally; V = 50257, H = 768, 77 MB: 21.0 against 23.3).  Five token tiles already want
-  // it kept (50257 x 4096, 1024 tokens as five tiles of 224: 396 us non-temporally, 354 normally).
-  const FusedSchedule full = fused_schedule((int)n_tokens, p.shape);
-  p.w_nt = full.n_ttiles <= (fused_tile(full.tile).tokens > 128 ? 4 : 1) && V * H * 2 >= (int64_t)288 << 20;
-  for (int i = 0; i < kFusedTiles; ++i) {  // whatever number of valid tokens and tile the device may end up with
-    if (!((p.shape.tiles >> i) & 1)) continue;
-    const int bt = fused_tile(i).tokens;
-    const int64_t most = n_tokens < fused_tile_most(i) || fused_one_tile(p.shape) ? n_tokens : fused_tile_most(i);
-    for (int64_t tt = 1; tt <= (most + bt - 1) / bt; ++tt) {
-      const FusedSchedule s = fused_schedule_on((int)(tt * bt), p.shape, i);
-      const int padded = 8 * ((s.n_wg + 7) / 8);  // fused_locate deals whole rows of 8 workgroup ids
-      if (padded > p.grid) p.grid = padded;
-      const size_t rec = (size_t)tt * bt * s.n_splits * kPartsPerSplit;
-      if (rec > p.max_records) p.max_records = rec;
-    }
-  }
-  return p;
-}
-
-// Layout: [n_valid + schedule: 256 B][row_index: n_tokens int32, 256-aligned][partials per weight set]
-// [normalised hidden rows, only with a norm weight].
-static size_t off_index() { return 256; }
-static size_t off_partials(int64_t n_tokens) { return 256 + (((size_t)n_tokens * 4 + 255) & ~(size_t)255); }
-static size_t normed_bytes(int64_t n_tokens, int64_t H, bool with_norm) {
-  return with_norm ? (((size_t)n_tokens * H * 2 + 255) & ~(size_t)255) : 0;
-}
-// The same on every device and for every output, whichever plan that makes.
-static size_t partial_bytes(int64_t n_tokens, int64_t H, int64_t V) {
-  const size_t a = fused_plan(n_tokens, H, V, true, false, false).max_records;
-  const size_t b = fused_plan(n_tokens, H, V, false, false, false).max_records;
-  return (a > b ? a : b) * sizeof(FusedPartial);
-}
-
-// Two hidden matrices against one weight are ONE sweep over both where that is a batch of up to this many tokens: W is streamed once
-// instead of twice and half-filled token tiles meet.  The sweep computes the entropy for the second matrix too, which at more tokens
-// costs what the sharing gives.  Two sweeps / one, us, V = 151936, H = 1024 | 2560: 16 tokens 104 / 56 | 239 / 124, 128: 126 / 90 |
-// 314 / 198, 512: 281 / 277 | 645 / 611, 768: 400 / 418 | 921 / 980; behind a mask that leaves 56 %, 128: 121 / 86 | 285 / 185, 512:
-// 170 / 140 | 380 / 301, 768: 236 / 222 | 538 / 471, 1024: 369 / 383 | 868 / 845.
-static bool joint_fits(int64_t n_tokens, int64_t H, bool masked) { return n_tokens <= (masked ? 768 : 512) && H % kDmaSlab == 0; }
-// All partials of a call of `n_sweeps` sweeps.
-static size_t partials_total(int64_t n_tokens, int64_t H, int64_t V, int n_sweeps) {
-  const size_t each = partial_bytes(n_tokens, H, V) * (size_t)n_sweeps;
-  const size_t joint = n_sweeps == 2 && joint_fits(n_tokens, H, true) ? partial_bytes(2 * n_tokens, H, V) : 0;
-  return each > joint ? each : joint;
-}
+static FusedEnv fused_env() { return FusedEnv{g_forced_kind.load(std::memory_order_relaxed), small_wg_count()}; }
 
 // The generic kernel addresses both matrices through buffer descriptors with 32-bit byte offsets.
-bool fused_needs_32bit_extents(int64_t n_tokens, int64_t H, int64_t V) { return fused_plan(n_tokens, H, V, true, false, false).kind == kGeneric; }
+bool fused_needs_32bit_extents(int64_t n_tokens, int64_t H, int64_t V) { return fused_plan(fused_env(), n_tokens, H, V, true, false, false).kind == kGeneric; }
 
 size_t fused_workspace_bytes(int64_t n_tokens, int64_t H, int64_t V, int n_weights, bool with_norm) {
-  return off_partials(n_tokens) + partials_total(n_tokens, H, V, n_weights) + normed_bytes(n_tokens, H, with_norm);
+  return off_partials(n_tokens) + partials_total(fused_env(), n_tokens, H, V, n_weights) + normed_bytes(n_tokens, H, with_norm);
 }
 
 template <bool ENT, bool AMAX, int NBT, int KSTEPS>
@@ -931,9 +794,10 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
   if (!w1) w1 = w0;
   if (!hidden_ref) hidden_ref = hidden;
   char* ws = static_cast<char*>(workspace);
-  FusedPlan plan = fused_plan(n_tokens, H, V, deep_lds_granted(), out_entropy != nullptr, sel.masked());
+  const FusedEnv env = fused_env();
+  FusedPlan plan = fused_plan(env, n_tokens, H, V, deep_lds_granted(), out_entropy != nullptr, sel.masked());
   const bool joint = second && w1 == w0 && hidden_ref != hidden && plan.kind != kGeneric && joint_fits(n_tokens, H, sel.masked());
-  if (joint) plan = fused_plan(2 * n_tokens, H, V, deep_lds_granted(), out_entropy != nullptr, sel.masked());
+  if (joint) plan = fused_plan(env, 2 * n_tokens, H, V, deep_lds_granted(), out_entropy != nullptr, sel.masked());
   int32_t* n_valid = nullptr;
   int32_t* row_index = nullptr;
   if (sel.masked()) {
@@ -957,7 +821,7 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
   a.hidden_bytes = (uint32_t)(((n_rows - 1) * hidden_stride + H) * 2);  // read by the generic kernel only (< 4 GiB there)
   const char* second_hidden = static_cast<const char*>(hidden_ref);
   if (norm_weight) {  // normalise the valid rows into a dense buffer and multiply that
-    char* normed = ws + off_partials(n_tokens) + partials_total(n_tokens, H, V, second ? 2 : 1);
+    char* normed = ws + off_partials(n_tokens) + partials_total(env, n_tokens, H, V, second ? 2 : 1);
     char* normed_ref = hidden_ref != hidden ? normed + normed_bytes(n_tokens, H, true) : normed;
     NormArgs na{{a.hidden, second_hidden}, static_cast<const uint16_t*>(norm_weight), {normed, normed_ref}, a.hidden_index, n_valid,
                 a.hidden_stride_b, (int)n_tokens, (int)n_rows, (int)H, norm_eps};
@@ -978,7 +842,7 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
   a.sched = fused_schedule(swept, plan.shape);
   a.scale = kLog2e / temperature;
   FusedPartial* p0 = reinterpret_cast<FusedPartial*>(ws + off_partials(n_tokens));
-  FusedPartial* p1 = reinterpret_cast<FusedPartial*>(ws + off_partials(n_tokens) + partial_bytes(n_tokens, H, V));
+  FusedPartial* p1 = reinterpret_cast<FusedPartial*>(ws + off_partials(n_tokens) + partial_bytes(env, n_tokens, H, V));
 
   a.weight = static_cast<const char*>(w0);
   a.partials = p0;
