@@ -567,3 +567,32 @@ def test_fused_tile_chosen_on_device_every_logit(dev, n, H, V, outputs):
             p = torch.softmax(x.double(), dim=-1)
             want = torch.logsumexp(x.double(), dim=-1) - (p * x.double()).sum(-1)
             np.testing.assert_allclose(r.entropy.cpu().numpy()[m], want.cpu().numpy()[m], atol=2e-4, rtol=0)
+
+
+@pytest.mark.parametrize("n,entropy", [(1100, True), (2049, True), (2600, False), (7300, False)])
+def test_fused_named_token_tiles_at_many_tokens(dev, n, entropy):
+    """A named token tile holds for any number of tokens: with the entropy behind a mask, past the sizes it would be picked for, in several
+    rounds of workgroups.  Every row against an fp32 product (rounding of an H-long sum at these magnitudes: under 1e-4)."""
+    H, V = 128, 1068
+    g = torch.Generator(device=dev).manual_seed(n)
+    h = torch.empty((n, H), device=dev).normal_(0, 1, generator=g).to(torch.bfloat16)
+    w = torch.empty((V, H), device=dev).normal_(0, 0.05, generator=g).to(torch.bfloat16)
+    t = torch.randint(0, V, (n,), device=dev, generator=g)
+    x = h.float() @ w.float().T
+    lse = torch.logsumexp(x, dim=-1)
+    lp = x.gather(1, t[:, None])[:, 0] - lse
+    some = torch.rand(n, device=dev, generator=g) < 0.7
+    lib = tome_amd.load_library()
+    try:
+        for tile in TOKEN_TILES:
+            lib.tome_select_fused_kernel(tile)
+            for valid in (None, some):
+                r = tome_amd.fused_lmhead_logprobs(h, w, t, 1.0, row_valid=valid, want_lse=True, want_entropy=entropy)
+                m = slice(None) if valid is None else valid
+                np.testing.assert_allclose(r.lse[m].cpu().numpy(), lse[m].cpu().numpy(), atol=1e-4, rtol=0, err_msg=str(tile))
+                np.testing.assert_allclose(r.lp[m].cpu().numpy(), lp[m].cpu().numpy(), atol=1e-4, rtol=0, err_msg=str(tile))
+                if entropy:
+                    want = lse[m].double() - (torch.softmax(x[m].double(), dim=-1) * x[m].double()).sum(-1)
+                    np.testing.assert_allclose(r.entropy[m].cpu().numpy(), want.cpu().numpy(), atol=2e-4, rtol=0, err_msg=str(tile))
+    finally:
+        lib.tome_select_fused_kernel(-1)

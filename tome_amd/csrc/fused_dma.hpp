@@ -527,8 +527,10 @@ void launch_dma_any(const FusedArgs& a, bool w_nt, int grid, hipStream_t stream)
   if (w_nt) launch_dma_form<ENT, AMAX, kAnyTile, true, true>(a, grid, stream);
   else launch_dma_form<ENT, AMAX, kAnyTile, true, false>(a, grid, stream);
 }
+// False, and nothing launched, for a tile without the form asked for.
 template <bool ENT, bool AMAX>
-void launch_dma(const FusedArgs& a, int tile, bool deep, bool w_nt, int grid, hipStream_t stream) {
+bool launch_dma(const FusedArgs& a, int tile, bool deep, bool w_nt, int grid, hipStream_t stream) {
+  if (tile < 0 || tile >= kTileGeneric || !dma_has_form(tile, deep)) return false;
   auto go = [&](auto t) {
     constexpr int TILE = decltype(t)::value;
     constexpr bool kBig = fused_tile(TILE).tokens > 128;
@@ -537,7 +539,7 @@ void launch_dma(const FusedArgs& a, int tile, bool deep, bool w_nt, int grid, hi
     }
     if (w_nt && (deep || !kBig)) launch_dma_form<ENT, AMAX, TILE, kBig, true>(a, grid, stream);
     else if (deep || !kBig) launch_dma_form<ENT, AMAX, TILE, kBig, false>(a, grid, stream);
-    else if constexpr (fused_tile(TILE).tokens == 256) launch_dma_form<ENT, AMAX, TILE, false, false>(a, grid, stream);
+    else if constexpr (dma_has_form(TILE, false)) launch_dma_form<ENT, AMAX, TILE, false, false>(a, grid, stream);
   };
   switch (tile) {
     case 0: go(std::integral_constant<int, 0>{}); break;
@@ -549,6 +551,7 @@ void launch_dma(const FusedArgs& a, int tile, bool deep, bool w_nt, int grid, hi
     case 6: go(std::integral_constant<int, 6>{}); break;
     default: go(std::integral_constant<int, 7>{}); break;
   }
+  return true;
 }
 
 }  // namespace tome

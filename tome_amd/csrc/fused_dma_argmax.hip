@@ -2,5 +2,5 @@
 #include "fused_dma.hpp"
 
 namespace tome {
-template void launch_dma<false, true>(const FusedArgs&, int, bool, bool, int, hipStream_t);
+template bool launch_dma<false, true>(const FusedArgs&, int, bool, bool, int, hipStream_t);
 }  // namespace tome

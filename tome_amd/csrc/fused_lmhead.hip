@@ -686,7 +686,7 @@ void fused_force_kernel(int kind) { g_forced_kind.store(kind, std::memory_order_
 // The DMA kernels' launches (fused_dma.hpp), instantiated in the fused_dma_*.hip files: one token tile, or the tile of the schedule
 // on the device; the 160 KB of LDS their largest form asks for.
 template <bool ENT, bool AMAX>
-void launch_dma(const FusedArgs& a, int tile, bool deep, bool w_nt, int grid, hipStream_t stream);
+bool launch_dma(const FusedArgs& a, int tile, bool deep, bool w_nt, int grid, hipStream_t stream);
 template <bool ENT, bool AMAX>
 void launch_dma_any(const FusedArgs& a, bool w_nt, int grid, hipStream_t stream);
 bool dma_allow_deep_lds();
@@ -752,7 +752,7 @@ static int launch_small(const FusedArgs& a, int waves, hipStream_t stream) {
 }
 
 // Launches the sweep kernel of `plan`.  Returns the number of partials per token it leaves (0 = the
-// schedule's own count).
+// schedule's own count, -1 = no kernel for the plan, nothing launched).
 template <bool ENT>
 static int launch_main(const FusedArgs& a, const FusedPlan& plan, bool want_argmax, hipStream_t stream) {
   if (plan.kind == kSmall) {
@@ -772,8 +772,10 @@ static int launch_main(const FusedArgs& a, const FusedPlan& plan, bool want_argm
     if (a.sched_dev && plan.any_tile) {
       if (want_argmax) launch_dma_any<ENT, true>(a, plan.w_nt, plan.grid, stream);
       else launch_dma_any<ENT, false>(a, plan.w_nt, plan.grid, stream);
-    } else if (want_argmax) launch_dma<ENT, true>(a, a.sched.tile, deep, plan.w_nt, plan.grid, stream);
-    else launch_dma<ENT, false>(a, a.sched.tile, deep, plan.w_nt, plan.grid, stream);
+    } else if (!(want_argmax ? launch_dma<ENT, true>(a, a.sched.tile, deep, plan.w_nt, plan.grid, stream)
+                             : launch_dma<ENT, false>(a, a.sched.tile, deep, plan.w_nt, plan.grid, stream))) {
+      return -1;
+    }
   } else {
     if (want_argmax) hipLaunchKernelGGL((fused_lmhead_kernel<ENT, true>), dim3((unsigned)plan.grid), dim3(kFusedWG), 0, stream, a);
     else hipLaunchKernelGGL((fused_lmhead_kernel<ENT, false>), dim3((unsigned)plan.grid), dim3(kFusedWG), 0, stream, a);
@@ -848,6 +850,7 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
   a.partials = p0;
   int n_parts = out_entropy ? launch_main<true>(a, plan, out_argmax != nullptr, stream)
                             : launch_main<false>(a, plan, out_argmax != nullptr, stream);
+  if (n_parts < 0) return hipErrorInvalidConfiguration;
   if (n_parts > 0) {  // small-batch kernel: one part per workgroup, whatever the mask
     a.sched = FusedSchedule{1, n_parts / kPartsPerSplit, n_parts, kTileGeneric, 0, 0};
     a.sched_dev = nullptr;
@@ -857,7 +860,7 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
     a.weight = static_cast<const char*>(w1);
     a.hidden = second_hidden;
     a.partials = p1;
-    launch_main<false>(a, plan, false, stream);
+    if (launch_main<false>(a, plan, false, stream) < 0) return hipErrorInvalidConfiguration;
     a.hidden = first_hidden;
   }
   hipError_t e = hipGetLastError();

@@ -54,17 +54,20 @@ struct FusedShape {
   uint32_t tiles;  // bit i: FusedTile i may be taken
   int vunits32, vunits224, vunits256;  // the vocab axis in 32-row units, 224-row and 256-row tiles
   int whole;       // 1: vocab ranges in whole 256-row tiles whatever the token tile
+  int named;       // 1: the selector names the token tile, which is then taken for any number of tokens
 };
-inline FusedShape fused_shape(int64_t H, int64_t V, int slots, uint32_t tiles, bool whole) {
-  return FusedShape{(int)H, (int)V, slots, tiles, (int)((V + 31) / 32), (int)((V + 223) / 224), (int)((V + 255) / 256), whole ? 1 : 0};
+inline FusedShape fused_shape(int64_t H, int64_t V, int slots, uint32_t tiles, bool whole, bool named) {
+  return FusedShape{(int)H, (int)V, slots, tiles, (int)((V + 31) / 32), (int)((V + 223) / 224), (int)((V + 255) / 256), whole ? 1 : 0, named ? 1 : 0};
 }
 __host__ __device__ inline bool fused_one_tile(const FusedShape& sh) { return (sh.tiles & (sh.tiles - 1)) == 0; }
 // The tiles below 256 tokens save padding where there are few of them; they are not taken beyond these numbers of valid tokens
 // (5074 tokens: 256 a tile 1148 us, 224 1207; the tiles up to 128 tokens are no better than 192 from two of those on).
 __host__ __device__ constexpr int fused_tile_most(int i) { return i >= 5 && i < kTileGeneric ? 256 : i >= 2 && i < 5 ? 2560 : 0x7fffffff; }
 __host__ __device__ inline bool fused_tile_allowed(const FusedShape& sh, int n_valid, int i) {
-  return ((sh.tiles >> i) & 1) && (n_valid <= fused_tile_most(i) || fused_one_tile(sh));
+  return ((sh.tiles >> i) & 1) && (n_valid <= fused_tile_most(i) || sh.named);
 }
+// The forms the DMA kernel is built in: two W buffers for 256 tokens, three for 192 .. 256, and the tiles of up to 128 tokens.
+__host__ __device__ constexpr bool dma_has_form(int i, bool deep) { return fused_tile(i).tokens <= 128 || deep || fused_tile(i).tokens == 256; }
 __host__ __device__ inline int fused_unit32(const FusedShape& sh, int i) { return sh.whole ? 8 : fused_tile(i).unit32; }
 __host__ __device__ inline int fused_vunits(const FusedShape& sh, int i) {
   const int u = fused_unit32(sh, i);
@@ -134,7 +137,7 @@ inline FusedSchedule fused_schedule_on(int n_valid, const FusedShape& sh, int ti
 }
 inline FusedSchedule fused_schedule(int n_valid, const FusedShape& sh) {  // host
   float best = INFINITY;
-  int tile = 0;
+  int tile = __builtin_ctz(sh.tiles);
   for (int i = 0; i < kFusedTiles; ++i) {
     if (!fused_tile_allowed(sh, n_valid, i)) continue;
     const float c = fused_tile_cost(sh, n_valid, i);
@@ -212,15 +215,13 @@ inline FusedPlan fused_plan(const FusedEnv& env, int64_t n_tokens, int64_t H, in
   if (forced == kForceDmaTwoWBuffers) p.deep = p.deep_lp = false;
   if (forced == kForceDmaThreeWBuffers) p.deep = p.deep_lp = deep_lds;
   // Token tiles.  The two-buffer form has 256 tokens only, and a call of two sweeps one schedule for both.
+  uint32_t named = 0;
+  for (int i = 0; i < kTileGeneric; ++i) named |= (uint32_t)(forced >= kForceDmaTile && fused_tile(i).tokens == forced && dma_has_form(i, deep_lds)) << i;
+  if (named && !dma_has_form(__builtin_ctz(named), false)) p.deep = p.deep_lp = true;
   const bool any = masked && n_tokens <= kAnyTileTokens && n_tokens > 64;
   const bool all_deep = p.deep_lp && (p.deep || !entropy || any);
-  p.shape = fused_shape(H, V, 256, all_deep ? 0xffu : 3u, forced == kForceDmaWholeTiles);
+  p.shape = fused_shape(H, V, 256, named ? named : all_deep ? 0xffu : 3u, forced == kForceDmaWholeTiles, named != 0);
   if (forced == kForceDmaTwoWBuffers || forced == kForceDmaThreeWBuffers) p.shape.tiles = 3;
-  if (forced >= kForceDmaTile && all_deep) {
-    uint32_t only = 0;
-    for (int i = 0; i < kTileGeneric; ++i) only |= (uint32_t)(fused_tile(i).tokens == forced) << i;
-    p.shape.tiles = only ? only : p.shape.tiles;
-  }
   if (p.shape.whole) p.shape.tiles &= ~((1u << 1) | (1u << 3));  // no vocab tiles of 224 rows
   if (p.kind != kDma) {
     p.shape.tiles = 1u << kTileGeneric;
@@ -228,7 +229,7 @@ inline FusedPlan fused_plan(const FusedEnv& env, int64_t n_tokens, int64_t H, in
                           // of 80 KB per CU measured slower than one: 288 against 277 us at 64 x 4096)
   }
   // A mask of up to 64 tokens leaves the smallest tile; beyond kAnyTileTokens the 256-token tile serves.
-  if (masked && p.kind == kDma && n_tokens > kAnyTileTokens) p.shape.tiles &= 3u;
+  if (masked && p.kind == kDma && n_tokens > kAnyTileTokens && !named) p.shape.tiles &= 3u;
   if (masked && p.kind == kDma && (n_tokens <= 64 || n_tokens > kAnyTileTokens || !all_deep)) p.shape.tiles = 1u << fused_schedule((int)n_tokens, p.shape).tile;
   p.any_tile = masked && p.kind == kDma && !fused_one_tile(p.shape);
   p.w_nt = false;
@@ -248,7 +249,7 @@ inline FusedPlan fused_plan(const FusedEnv& env, int64_t n_tokens, int64_t H, in
   for (int i = 0; i < kFusedTiles; ++i) {  // whatever number of valid tokens and tile the device may end up with
     if (!((p.shape.tiles >> i) & 1)) continue;
     const int bt = fused_tile(i).tokens;
-    const int64_t most = n_tokens < fused_tile_most(i) || fused_one_tile(p.shape) ? n_tokens : fused_tile_most(i);
+    const int64_t most = n_tokens < fused_tile_most(i) || named ? n_tokens : fused_tile_most(i);
     for (int64_t tt = 1; tt <= (most + bt - 1) / bt; ++tt) {
       const FusedSchedule s = fused_schedule_on((int)(tt * bt), p.shape, i);
       const int padded = 8 * ((s.n_wg + 7) / 8);  // fused_locate deals whole rows of 8 workgroup ids
