@@ -1,10 +1,13 @@
 // Checks the planning of fused lm_head calls (tome_amd/csrc/fused_plan.hpp) over random calls, without a GPU: whatever tile and number
 // of valid tokens a call may end up with, a kernel form exists for it, the grid holds its workgroups, the workspace its partials, and
-// every vocab range is one that the kernels can cut into tiles.  Prints the first faults and their number.
+// every vocab range is one that the kernels can cut into tiles.  Prints the first faults and their number; `time N ...`: what one
+// call of N tokens plans on the host, in us.
 #include "fused_plan.hpp"
 #include <algorithm>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <random>
 
 using namespace tome;
@@ -25,7 +28,8 @@ static void check_call(const FusedEnv& env, int64_t n, int64_t H, int64_t V, boo
     return;
   }
   if (p.kind == kDma && H % kDmaSlab != 0) FAULT("ragged H on the DMA kernel", n, -1);
-  const int host_tile = fused_schedule((int)n, p.shape).tile;
+  const int host_tile = p.full.tile;
+  if (fused_schedule((int)n, p.shape).tile != host_tile) FAULT("the plan's schedule", n, host_tile);
   const bool tile_holds = env.forced <= 128 || env.forced == 256 || deep;  // 192 and 224 need the third W buffer
   if (p.kind == kDma && env.forced >= 64 && tile_holds && fused_tile(host_tile).tokens != env.forced) FAULT("selected token tile not taken", n, host_tile);
   auto on_tile = [&](int64_t n_valid, int tile) {
@@ -60,7 +64,29 @@ static void check_call(const FusedEnv& env, int64_t n, int64_t H, int64_t V, boo
   }
 }
 
+// The workspace's size (the caller's, and the check's), the choice of the kernel, the plan.
+static size_t plan_one_call(const FusedEnv& env, int64_t n, int64_t H, int64_t V) {
+  size_t sum = fused_layout(env, n, H, V, 1, 0).total;
+  sum += fused_kernel(env, n, H, V).kind + fused_layout(env, n, H, V, 1, 0).normed;
+  const FusedPlan p = fused_plan(env, n, H, V, true, false, false);
+  return sum + p.grid + p.full.n_wg;
+}
+
 int main(int argc, char** argv) {
+  if (argc > 1 && !std::strcmp(argv[1], "time")) {  // one call's planning, best of several runs, us
+    for (int i = 2; i < argc; ++i) {
+      const int64_t n = std::atoll(argv[i]);
+      double best = 1e9;
+      size_t sink = 0;
+      for (int r = 0; r < 200; ++r) {
+        const auto t0 = std::chrono::steady_clock::now();
+        for (int k = 0; k < 4; ++k) sink += plan_one_call(FusedEnv{-1, 256}, n, 1024, 151936 + (int)(sink & 1));
+        best = std::min(best, std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count() / 4);
+      }
+      std::printf("%lld %.3f\n", (long long)n, sink ? best : 0.0);
+    }
+    return 0;
+  }
   std::mt19937_64 rng(argc > 1 ? std::strtoull(argv[1], nullptr, 10) : 1);
   auto spread = [&](double lo, double hi) { return std::exp(std::uniform_real_distribution<double>(std::log(lo), std::log(hi))(rng)); };
   const int selectors[] = {-1, -1, -1, -1, 0, 1, 3, 4, 5, 64, 96, 128, 192, 224, 256};

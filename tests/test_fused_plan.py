@@ -23,3 +23,12 @@ def test_every_plan_can_be_launched_and_fits(checker, seed):
     vocab ranges that cover the vocabulary, and the token tile that the selector names."""
     run = subprocess.run([checker, str(seed)], capture_output=True, text=True)
     assert run.returncode == 0, run.stdout
+
+
+def test_planning_stays_off_the_clock(checker):
+    """A call's planning on the host (best of 200 runs, so a busy machine does not count): 0.2 - 0.3 us up to 8192 tokens and 3 beyond,
+    where walking every number of token tiles took 1.8, 3.5, 117 and 797."""
+    out = subprocess.run([checker, "time", "200", "4096", "16384", "65536"], capture_output=True, text=True, check=True).stdout
+    took = {int(n): float(us) for n, us in (line.split() for line in out.splitlines())}
+    for n, most in ((200, 1.2), (4096, 1.2), (16384, 30.0), (65536, 60.0)):
+        assert took[n] < most, took

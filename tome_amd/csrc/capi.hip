@@ -6,6 +6,7 @@
 
 #include "../../include/tome_logprob.h"
 #include "common.hpp"
+#include "fused_plan.hpp"
 
 namespace tome {
 hipError_t row_logprob_launch(const void* logits, int dtype, int64_t rows, int64_t V, int64_t row_stride,
@@ -34,18 +35,18 @@ hipError_t row_sample_launch(const void* logits, int dtype, int64_t rows, int64_
                              hipStream_t stream);
 size_t row_sample_workspace_bytes(int64_t rows, int64_t V, int dtype_vec, int top_k);
 bool row_sample_needs_workspace(int64_t rows, int64_t V, int vec);
-size_t fused_workspace_bytes(int64_t n_tokens, int64_t H, int64_t V, int n_weights, bool with_norm);
+FusedLayout fused_call_layout(int64_t n_tokens, int64_t H, int64_t V, int n_sweeps, int n_normed);
 bool fused_needs_32bit_extents(int64_t n_tokens, int64_t H, int64_t V);
 void fused_force_kernel(int kind);
 hipError_t fused_lmhead_launch(const void* hidden, const int32_t* hidden_rows, int64_t n_rows, const void* norm_weight, float norm_eps,
                                const void* w0, const void* w1, int64_t n_tokens, int64_t H, int64_t V, int64_t hidden_stride,
                                int64_t weight_stride, const RowSel& sel, float temperature, float* out_lp, float* out_lse,
                                float* out_entropy, int32_t* out_argmax, float* out_ref_lp, float* out_k3,
-                               void* workspace, hipStream_t stream);
+                               const FusedLayout& layout, void* workspace, hipStream_t stream);
 hipError_t fused_pair_launch(const void* hidden, const void* hidden_ref, const void* norm_weight, float norm_eps,
                              const void* w0, const void* w1, int64_t n_tokens, int64_t H, int64_t V,
                              int64_t hidden_stride, int64_t weight_stride, const RowSel& sel, float temperature, float* out_lp,
-                             float* out_entropy, float* out_ref_lp, float* out_k3, void* workspace, hipStream_t stream);
+                             float* out_entropy, float* out_ref_lp, float* out_k3, const FusedLayout& layout, void* workspace, hipStream_t stream);
 hipError_t mfma_probe_launch(const void* operands, int n_workgroups, int steps, int flags, float* sink, hipStream_t stream);
 struct LoraJobHost;
 hipError_t lora_merge_launch(const LoraJobHost* jobs, int n_jobs, void* workspace, hipStream_t stream);
@@ -289,7 +290,7 @@ void tome_select_fused_kernel(int kind) {
 
 size_t tome_fused_lmhead_logprob_workspace(int64_t n_tokens, int64_t H, int64_t V) {
   if (n_tokens <= 0 || H <= 0 || V <= 0) return 0;
-  return align256(tome::fused_workspace_bytes(n_tokens, H, V, 1, false));
+  return tome::fused_call_layout(n_tokens, H, V, 1, 0).total;
 }
 
 int tome_fused_lmhead_logprob(const void* hidden, const void* weight, int64_t n_tokens, int64_t H, int64_t V,
@@ -317,7 +318,7 @@ int tome_lmhead_logprob_sel(const void* hidden, const int32_t* hidden_rows, int6
 
 size_t tome_norm_lmhead_logprob_workspace(int64_t n_tokens, int64_t H, int64_t V) {
   if (n_tokens <= 0 || H <= 0 || V <= 0) return 0;
-  return align256(tome::fused_workspace_bytes(n_tokens, H, V, 1, true));
+  return tome::fused_call_layout(n_tokens, H, V, 1, 1).total;
 }
 
 int tome_norm_lmhead_logprob(const void* hidden, const void* norm_weight, float norm_eps, const void* weight,
@@ -333,7 +334,7 @@ int tome_norm_lmhead_logprob(const void* hidden, const void* norm_weight, float 
 
 size_t tome_grpo_dual_workspace(int64_t n_tokens, int64_t H, int64_t V) {
   if (n_tokens <= 0 || H <= 0 || V <= 0) return 0;
-  return align256(tome::fused_workspace_bytes(n_tokens, H, V, 2, false));
+  return tome::fused_call_layout(n_tokens, H, V, 2, 0).total;
 }
 
 int tome_grpo_dual(const void* hidden, const void* w_policy, const void* w_ref, int64_t n_tokens, int64_t H,
@@ -344,19 +345,18 @@ int tome_grpo_dual(const void* hidden, const void* w_policy, const void* w_ref, 
   if (rc != TOME_OK || n_tokens == 0) return rc;
   if (!w_ref || !out_lp || !out_ref_lp) return TOME_E_NULL;
   if (reinterpret_cast<uintptr_t>(w_ref) % 16 != 0) return TOME_E_ALIGN;
-  const size_t need = tome_grpo_dual_workspace(n_tokens, H, V);
-  if (!workspace || workspace_bytes < need) return TOME_E_WORKSPACE;
+  const tome::FusedLayout layout = tome::fused_call_layout(n_tokens, H, V, 2, 0);
+  if (!workspace || workspace_bytes < layout.total) return TOME_E_WORKSPACE;
   return hip_result(tome::fused_lmhead_launch(hidden, nullptr, n_tokens, nullptr, 0.f, w_policy, w_ref, n_tokens, H, V,
                                               hidden_stride, weight_stride, plain_sel(targets, row_valid), temperature, out_lp, nullptr, out_entropy,
-                                              nullptr, out_ref_lp, out_k3, workspace,
+                                              nullptr, out_ref_lp, out_k3, layout, workspace,
                                               static_cast<hipStream_t>(stream)));
 }
 
 size_t tome_grpo_pair_workspace(int64_t n_tokens, int64_t H, int64_t V, int with_norm) {
   if (n_tokens <= 0 || H <= 0 || V <= 0) return 0;
   // two partial sets; with a norm weight, one normalised copy per hidden-state matrix
-  return align256(tome::fused_workspace_bytes(n_tokens, H, V, 2, with_norm != 0) +
-                  (with_norm ? align256((size_t)n_tokens * H * 2) : 0));
+  return tome::fused_call_layout(n_tokens, H, V, 2, with_norm ? 2 : 0).total;
 }
 
 int tome_grpo_pair(const void* hidden_policy, const void* hidden_ref, const void* norm_weight, float norm_eps,
@@ -480,11 +480,11 @@ int fused_checked(const void* hidden, const int32_t* hidden_rows, int64_t n_rows
   if (!out_lp) return TOME_E_NULL;
   if (reinterpret_cast<uintptr_t>(norm_weight) % 16 != 0) return TOME_E_ALIGN;
   if (norm_weight && (!(norm_eps >= 0.f) || !isfinite(norm_eps))) return TOME_E_SHAPE;
-  const size_t need = align256(tome::fused_workspace_bytes(n_tokens, H, V, 1, norm_weight != nullptr));
-  if (!workspace || workspace_bytes < need) return TOME_E_WORKSPACE;
+  const tome::FusedLayout layout = tome::fused_call_layout(n_tokens, H, V, 1, norm_weight ? 1 : 0);
+  if (!workspace || workspace_bytes < layout.total) return TOME_E_WORKSPACE;
   return hip_result(tome::fused_lmhead_launch(hidden, hidden_rows, n_rows, norm_weight, norm_eps, weight, nullptr, n_tokens, H, V,
                                               hidden_stride, weight_stride, sel, temperature, out_lp, out_lse, out_entropy,
-                                              out_argmax, nullptr, nullptr, workspace, static_cast<hipStream_t>(stream)));
+                                              out_argmax, nullptr, nullptr, layout, workspace, static_cast<hipStream_t>(stream)));
 }
 
 int pair_checked(const void* hidden_policy, const void* hidden_ref, const void* norm_weight, float norm_eps,
@@ -498,11 +498,11 @@ int pair_checked(const void* hidden_policy, const void* hidden_ref, const void* 
       reinterpret_cast<uintptr_t>(norm_weight) % 16 != 0)
     return TOME_E_ALIGN;
   if (norm_weight && (!(norm_eps >= 0.f) || !isfinite(norm_eps))) return TOME_E_SHAPE;
-  const size_t need = tome_grpo_pair_workspace(n_tokens, H, V, norm_weight != nullptr);
-  if (!workspace || workspace_bytes < need) return TOME_E_WORKSPACE;
+  const tome::FusedLayout layout = tome::fused_call_layout(n_tokens, H, V, 2, norm_weight ? 2 : 0);
+  if (!workspace || workspace_bytes < layout.total) return TOME_E_WORKSPACE;
   return hip_result(tome::fused_pair_launch(hidden_policy, hidden_ref, norm_weight, norm_eps, w_policy, w_ref, n_tokens,
                                             H, V, hidden_stride, weight_stride, sel, temperature,
-                                            out_lp, out_entropy, out_ref_lp, out_k3, workspace,
+                                            out_lp, out_entropy, out_ref_lp, out_k3, layout, workspace,
                                             static_cast<hipStream_t>(stream)));
 }
 }  // namespace

@@ -730,10 +730,10 @@ static int small_wg_count() {
 static FusedEnv fused_env() { return FusedEnv{g_forced_kind.load(std::memory_order_relaxed), small_wg_count()}; }
 
 // The generic kernel addresses both matrices through buffer descriptors with 32-bit byte offsets.
-bool fused_needs_32bit_extents(int64_t n_tokens, int64_t H, int64_t V) { return fused_plan(fused_env(), n_tokens, H, V, true, false, false).kind == kGeneric; }
+bool fused_needs_32bit_extents(int64_t n_tokens, int64_t H, int64_t V) { return fused_kernel(fused_env(), n_tokens, H, V).kind == kGeneric; }
 
-size_t fused_workspace_bytes(int64_t n_tokens, int64_t H, int64_t V, int n_weights, bool with_norm) {
-  return off_partials(n_tokens) + partials_total(fused_env(), n_tokens, H, V, n_weights) + normed_bytes(n_tokens, H, with_norm);
+FusedLayout fused_call_layout(int64_t n_tokens, int64_t H, int64_t V, int n_sweeps, int n_normed) {
+  return fused_layout(fused_env(), n_tokens, H, V, n_sweeps, n_normed);
 }
 
 template <bool ENT, bool AMAX, int NBT, int KSTEPS>
@@ -791,20 +791,20 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
                                     int64_t V, int64_t hidden_stride, int64_t weight_stride, const RowSel& sel,
                                     float temperature, float* out_lp, float* out_lse,
                                     float* out_entropy, int32_t* out_argmax, float* out_ref_lp, float* out_k3,
-                                    void* workspace, hipStream_t stream) {
+                                    const FusedLayout& layout, void* workspace, hipStream_t stream) {
   const bool second = w1 != nullptr || hidden_ref != nullptr;
   if (!w1) w1 = w0;
   if (!hidden_ref) hidden_ref = hidden;
   char* ws = static_cast<char*>(workspace);
   const FusedEnv env = fused_env();
-  FusedPlan plan = fused_plan(env, n_tokens, H, V, deep_lds_granted(), out_entropy != nullptr, sel.masked());
-  const bool joint = second && w1 == w0 && hidden_ref != hidden && plan.kind != kGeneric && joint_fits(n_tokens, H, sel.masked());
-  if (joint) plan = fused_plan(env, 2 * n_tokens, H, V, deep_lds_granted(), out_entropy != nullptr, sel.masked());
+  const bool joint = second && w1 == w0 && hidden_ref != hidden && joint_fits(n_tokens, H, sel.masked()) && env.forced != kGeneric;
+  const int swept = (int)n_tokens << (joint ? 1 : 0);
+  const FusedPlan plan = fused_plan(env, swept, H, V, deep_lds_granted(), out_entropy != nullptr, sel.masked());
   int32_t* n_valid = nullptr;
   int32_t* row_index = nullptr;
   if (sel.masked()) {
     n_valid = reinterpret_cast<int32_t*>(ws);
-    row_index = reinterpret_cast<int32_t*>(ws + off_index());
+    row_index = reinterpret_cast<int32_t*>(ws + kFusedIndexOffset);
     CompactArgs c{sel, row_index, n_valid, out_lp, out_lse, out_entropy, out_ref_lp, out_k3, out_argmax,
                   (int)n_tokens, plan.shape, joint ? 1 : 0};
     hipLaunchKernelGGL(compact_rows_kernel, dim3(1), dim3(1024), 0, stream, c);
@@ -823,8 +823,8 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
   a.hidden_bytes = (uint32_t)(((n_rows - 1) * hidden_stride + H) * 2);  // read by the generic kernel only (< 4 GiB there)
   const char* second_hidden = static_cast<const char*>(hidden_ref);
   if (norm_weight) {  // normalise the valid rows into a dense buffer and multiply that
-    char* normed = ws + off_partials(n_tokens) + partials_total(env, n_tokens, H, V, second ? 2 : 1);
-    char* normed_ref = hidden_ref != hidden ? normed + normed_bytes(n_tokens, H, true) : normed;
+    char* normed = ws + layout.normed;
+    char* normed_ref = hidden_ref != hidden ? ws + layout.normed_second : normed;
     NormArgs na{{a.hidden, second_hidden}, static_cast<const uint16_t*>(norm_weight), {normed, normed_ref}, a.hidden_index, n_valid,
                 a.hidden_stride_b, (int)n_tokens, (int)n_rows, (int)H, norm_eps};
     hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((unsigned)((n_tokens + 3) / 4), hidden_ref != hidden ? 2 : 1), dim3(256), 0, stream, na);
@@ -835,16 +835,15 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
     a.hidden_bytes = (uint32_t)(n_tokens * H * 2);
   }
   a.hidden2 = joint ? second_hidden : nullptr;
-  const int swept = (int)n_tokens << (joint ? 1 : 0);
   a.n_tokens = swept;
   a.H = (int)H;
   a.V = (int)V;
   // Workspace header: [0] n_valid, [16..40) the schedule derived from it on the device.
   a.sched_dev = sel.masked() ? reinterpret_cast<const FusedSchedule*>(n_valid + 4) : nullptr;
-  a.sched = fused_schedule(swept, plan.shape);
+  a.sched = plan.full;
   a.scale = kLog2e / temperature;
-  FusedPartial* p0 = reinterpret_cast<FusedPartial*>(ws + off_partials(n_tokens));
-  FusedPartial* p1 = reinterpret_cast<FusedPartial*>(ws + off_partials(n_tokens) + partial_bytes(env, n_tokens, H, V));
+  FusedPartial* p0 = reinterpret_cast<FusedPartial*>(ws + layout.partials);
+  FusedPartial* p1 = reinterpret_cast<FusedPartial*>(ws + layout.partials_second);
 
   a.weight = static_cast<const char*>(w0);
   a.partials = p0;
@@ -892,19 +891,19 @@ hipError_t fused_lmhead_launch(const void* hidden, const int32_t* hidden_rows, i
                                const void* w1, int64_t n_tokens, int64_t H, int64_t V, int64_t hidden_stride,
                                int64_t weight_stride, const RowSel& sel, float temperature, float* out_lp, float* out_lse,
                                float* out_entropy, int32_t* out_argmax, float* out_ref_lp, float* out_k3,
-                               void* workspace, hipStream_t stream) {
+                               const FusedLayout& layout, void* workspace, hipStream_t stream) {
   return fused_launch_impl(hidden, hidden_rows, n_rows, nullptr, norm_weight, norm_eps, w0, w1, n_tokens, H, V, hidden_stride, weight_stride,
                            sel, temperature, out_lp, out_lse, out_entropy, out_argmax, out_ref_lp, out_k3,
-                           workspace, stream);
+                           layout, workspace, stream);
 }
 
 hipError_t fused_pair_launch(const void* hidden, const void* hidden_ref, const void* norm_weight, float norm_eps,
                              const void* w0, const void* w1, int64_t n_tokens, int64_t H, int64_t V,
                              int64_t hidden_stride, int64_t weight_stride, const RowSel& sel, float temperature, float* out_lp, float* out_entropy,
-                             float* out_ref_lp, float* out_k3, void* workspace, hipStream_t stream) {
+                             float* out_ref_lp, float* out_k3, const FusedLayout& layout, void* workspace, hipStream_t stream) {
   return fused_launch_impl(hidden, nullptr, n_tokens, hidden_ref, norm_weight, norm_eps, w0, w1, n_tokens, H, V, hidden_stride,
                            weight_stride, sel, temperature, out_lp, nullptr, out_entropy, nullptr,
-                           out_ref_lp, out_k3, workspace, stream);
+                           out_ref_lp, out_k3, layout, workspace, stream);
 }
 
 }  // namespace tome

@@ -103,11 +103,14 @@ __host__ __device__ inline float fused_tile_cost(const FusedShape& sh, int n_val
   const float cost = tiles * nk * (61.f * 65536.f + 39.f * 256.f * tokens) + rows * (nk * (100.f * tokens + 3.f * 256.f) + 143.f * tokens);
   return i >= 2 && i < 5 ? cost * 1.03f : cost;
 }
-__host__ __device__ inline int64_t fused_split_cost(int n_ttiles, int n_splits, int slots, int n_vunits, int upt) {
-  const int rounds = (n_ttiles * n_splits + slots - 1) / slots;
+__host__ __device__ inline int fused_split_round_cost(int n_splits, int n_vunits, int upt) {
   const int longest = (n_vunits + n_splits - 1) / n_splits;  // in units
   const int pen64 = 60 + 32 / (n_splits < 8 ? n_splits : 8);
-  return ((int64_t)rounds * (2 * longest + upt) * pen64) * 64 + n_splits;  // ties go to fewer splits
+  return (2 * longest + upt) * pen64;
+}
+__host__ __device__ inline int64_t fused_split_cost(int n_ttiles, int n_splits, int slots, int n_vunits, int upt) {
+  const int rounds = (n_ttiles * n_splits + slots - 1) / slots;
+  return (int64_t)rounds * fused_split_round_cost(n_splits, n_vunits, upt) * 64 + n_splits;  // ties go to fewer splits
 }
 constexpr int kSplitCandidates = 32;
 // The schedule but for the number of splits where several rounds are needed; returns whether that is so.
@@ -134,6 +137,28 @@ inline FusedSchedule fused_schedule_on(int n_valid, const FusedShape& sh, int ti
     s.n_wg = s.n_ttiles * s.n_splits;
   }
   return s;
+}
+// The most workgroups that any number of valid tokens up to `most` can ask for on one tile.  One round holds at most `slots` of them;
+// where several are needed the splits do not follow the number of token tiles in order, and every number is looked at.
+inline int fused_most_workgroups(const FusedShape& sh, int tile, int64_t most) {  // host
+  const int upt = fused_unit32(sh, tile) == 1 ? 8 : 1, n_vunits = fused_vunits(sh, tile), n_vtiles = (n_vunits + upt - 1) / upt;
+  const int64_t ttiles = fused_ttiles((int)most, fused_tile(tile).tokens), one_round = sh.slots / 8;
+  const int64_t splits = (ttiles < one_round ? ttiles : one_round) * n_vtiles;
+  int best = (int)(splits < sh.slots ? splits : sh.slots);
+  if (ttiles <= one_round) return best;
+  const int candidates = n_vtiles < kSplitCandidates ? n_vtiles : kSplitCandidates, shift = __builtin_ctz((unsigned)sh.slots);  // slots: a power of two
+  int64_t round_cost[kSplitCandidates];
+  for (int c = 1; c <= candidates; ++c) round_cost[c - 1] = (int64_t)fused_split_round_cost(c, n_vunits, upt) * 64;
+  for (int64_t tt = ttiles; tt > one_round && tt * candidates > best; --tt) {
+    int64_t cheapest = INT64_MAX;
+    for (int c = 1; c <= candidates; ++c) {
+      const int64_t cost = ((tt * c + sh.slots - 1) >> shift) * round_cost[c - 1] + c;
+      cheapest = cost < cheapest ? cost : cheapest;
+    }
+    const int n_wg = (int)(tt * (cheapest & 63));
+    best = n_wg > best ? n_wg : best;
+  }
+  return best;
 }
 inline FusedSchedule fused_schedule(int n_valid, const FusedShape& sh) {  // host
   float best = INFINITY;
@@ -162,9 +187,9 @@ struct FusedPlan {
   bool w_nt;                                 // kDma only: W requested non-temporally (few token tiles: see the kernel's WNT)
   int small_nbt, small_ksteps, small_waves;  // kSmall only
   FusedShape shape;
+  FusedSchedule full;  // of all tokens
   bool any_tile;       // kDma: behind a mask the device picks the token tile
-  int grid;            // workgroups to launch: the most any number of valid tokens can ask for
-  size_t max_records;  // partial records any number of valid tokens can produce
+  int grid;            // workgroups to launch: behind a mask the most that any number of valid tokens can ask for
 };
 
 // Shape rules of the small-batch kernel: <= 64 tokens, K split over 2..8 waves in slices of 256 or 512
@@ -195,15 +220,44 @@ inline bool small_shape(int64_t n_tokens, int64_t H, int64_t V, int& nbt, int& k
 // kernel of their own (2100 tokens: 0.975 .. 1.08 with the choice).
 constexpr int64_t kAnyTileTokens = 2048;
 
+struct FusedKernel {
+  FusedKind kind;
+  int nbt, ksteps, waves;  // of the streaming kernel; nbt = 0 for shapes that it does not take
+};
+inline FusedKernel fused_kernel(const FusedEnv& env, int64_t n_tokens, int64_t H, int64_t V) {
+  FusedKernel k{H % kDmaSlab == 0 ? kDma : kGeneric, 0, 0, 0};
+  // The streaming kernel runs one workgroup per CU: without a CU count (no device) the tiled kernels serve.
+  if (!small_shape(n_tokens, H, V, k.nbt, k.ksteps, k.waves)) k.nbt = 0;
+  else if (env.small_wgs >= 2) k.kind = kSmall;
+  if (env.forced == kGeneric) k.kind = kGeneric;
+  if ((env.forced == kDma || env.forced >= kForceDmaWholeTiles) && H % kDmaSlab == 0) k.kind = kDma;
+  return k;
+}
+// Token tiles that the selector names; 192 and 224 exist with three W buffers only.
+inline uint32_t fused_named_tiles(const FusedEnv& env, bool deep_lds) {
+  uint32_t named = 0;
+  if (env.forced >= kForceDmaTile)
+    for (int i = 0; i < kTileGeneric; ++i) named |= (uint32_t)(fused_tile(i).tokens == env.forced && dma_has_form(i, deep_lds)) << i;
+  return named;
+}
+// resident workgroups on 256 CUs: 2 per CU, or 1 for the DMA path's LDS (two 64-token workgroups of 80 KB per CU measured
+// slower than one: 288 against 277 us at 64 x 4096)
+inline FusedShape fused_shape_on(const FusedEnv& env, FusedKind kind, int64_t H, int64_t V, uint32_t tiles, bool named) {
+  if (kind != kDma) return fused_shape(H, V, 512, 1u << kTileGeneric, env.forced == kForceDmaWholeTiles, false);
+  return fused_shape(H, V, 256, tiles, env.forced == kForceDmaWholeTiles, named);
+}
+
+// One plan a call.  The host's planning of a whole call, the workspace's size asked for twice (by the caller and in the check), us: 200
+// tokens 1.8 -> 0.3, 4096 3.5 -> 0.2, 16384 117 -> 2.6, 65536 797 -> 2.9, against walking every number of token tiles of every tile, seven
+// times a call.
 inline FusedPlan fused_plan(const FusedEnv& env, int64_t n_tokens, int64_t H, int64_t V, bool deep_lds, bool entropy, bool masked) {
   FusedPlan p;
-  p.kind = H % kDmaSlab == 0 ? kDma : kGeneric;
-  p.small_nbt = p.small_ksteps = p.small_waves = 0;
   const int forced = env.forced;
-  // The streaming kernel runs one workgroup per CU: without a CU count (no device) the tiled kernels serve.
-  if (small_shape(n_tokens, H, V, p.small_nbt, p.small_ksteps, p.small_waves) && env.small_wgs >= 2) p.kind = kSmall;
-  if (forced == kGeneric) p.kind = kGeneric;
-  if ((forced == kDma || forced >= kForceDmaWholeTiles) && H % kDmaSlab == 0) p.kind = kDma;
+  const FusedKernel kernel = fused_kernel(env, n_tokens, H, V);
+  p.kind = kernel.kind;
+  p.small_nbt = kernel.nbt;
+  p.small_ksteps = kernel.ksteps;
+  p.small_waves = kernel.waves;
   // The third W buffer (see the kernel), measured against the two-buffer form in the same runs.  One or two token tiles:
   // 6-13 % faster with any outputs (256 x 1024: 96 -> 87 us, 256 x 4096: 338 -> 297, 512 x 4096: 534 -> 503).  More token
   // tiles, log-probs only: 4096 x 1024 -2.3 %, 8192 x 1024 -1.5 %, 1024 x 4096 -5 %, 4096 x 4096 -1.7 %, 16384 x 2560 -2.6 %,
@@ -215,64 +269,56 @@ inline FusedPlan fused_plan(const FusedEnv& env, int64_t n_tokens, int64_t H, in
   if (forced == kForceDmaTwoWBuffers) p.deep = p.deep_lp = false;
   if (forced == kForceDmaThreeWBuffers) p.deep = p.deep_lp = deep_lds;
   // Token tiles.  The two-buffer form has 256 tokens only, and a call of two sweeps one schedule for both.
-  uint32_t named = 0;
-  for (int i = 0; i < kTileGeneric; ++i) named |= (uint32_t)(forced >= kForceDmaTile && fused_tile(i).tokens == forced && dma_has_form(i, deep_lds)) << i;
+  const uint32_t named = fused_named_tiles(env, deep_lds);
   if (named && !dma_has_form(__builtin_ctz(named), false)) p.deep = p.deep_lp = true;
   const bool any = masked && n_tokens <= kAnyTileTokens && n_tokens > 64;
   const bool all_deep = p.deep_lp && (p.deep || !entropy || any);
-  p.shape = fused_shape(H, V, 256, named ? named : all_deep ? 0xffu : 3u, forced == kForceDmaWholeTiles, named != 0);
-  if (forced == kForceDmaTwoWBuffers || forced == kForceDmaThreeWBuffers) p.shape.tiles = 3;
-  if (p.shape.whole) p.shape.tiles &= ~((1u << 1) | (1u << 3));  // no vocab tiles of 224 rows
-  if (p.kind != kDma) {
-    p.shape.tiles = 1u << kTileGeneric;
-    p.shape.slots = 512;  // resident workgroups on 256 CUs: 2 per CU, or 1 for the DMA path's LDS (two 64-token workgroups
-                          // of 80 KB per CU measured slower than one: 288 against 277 us at 64 x 4096)
+  p.shape = fused_shape_on(env, p.kind, H, V, named ? named : all_deep ? 0xffu : 3u, named != 0);
+  if (p.kind == kDma) {
+    if (forced == kForceDmaTwoWBuffers || forced == kForceDmaThreeWBuffers) p.shape.tiles = 3;
+    if (p.shape.whole) p.shape.tiles &= ~((1u << 1) | (1u << 3));  // no vocab tiles of 224 rows
+    if (masked && n_tokens > kAnyTileTokens && !named) p.shape.tiles &= 3u;
   }
+  p.full = fused_schedule((int)n_tokens, p.shape);
   // A mask of up to 64 tokens leaves the smallest tile; beyond kAnyTileTokens the 256-token tile serves.
-  if (masked && p.kind == kDma && n_tokens > kAnyTileTokens && !named) p.shape.tiles &= 3u;
-  if (masked && p.kind == kDma && (n_tokens <= 64 || n_tokens > kAnyTileTokens || !all_deep)) p.shape.tiles = 1u << fused_schedule((int)n_tokens, p.shape).tile;
-  p.any_tile = masked && p.kind == kDma && !fused_one_tile(p.shape);
+  if (masked && (n_tokens <= 64 || n_tokens > kAnyTileTokens || !all_deep)) p.shape.tiles = 1u << p.full.tile;
+  p.any_tile = masked && !fused_one_tile(p.shape);
   p.w_nt = false;
   p.grid = 0;
-  p.max_records = 0;
-  if (p.kind == kSmall) {
-    // One partial per (token, workgroup); one workgroup per CU, at most 512.  The schedule is ignored.
-    p.max_records = (size_t)64 * 512;
-    return p;
-  }
+  if (p.kind == kSmall) return p;  // a grid of its own; the schedule is ignored
   // Non-temporal W (the kernel's WNT): few token tiles, and a W larger than the 256 MB memory-side cache - a smaller one is
   // found there again by the next call as long as it is requested normally (repeated calls, 64 tokens: V = 32000, H = 4096,
   // 262 MB: 48 us against 71 non-temporally; V = 50257, H = 768, 77 MB: 21.0 against 23.3).  Five token tiles already want
   // it kept (50257 x 4096, 1024 tokens as five tiles of 224: 396 us non-temporally, 354 normally).
-  const FusedSchedule full = fused_schedule((int)n_tokens, p.shape);
-  p.w_nt = full.n_ttiles <= (fused_tile(full.tile).tokens > 128 ? 4 : 1) && V * H * 2 >= (int64_t)288 << 20;
-  for (int i = 0; i < kFusedTiles; ++i) {  // whatever number of valid tokens and tile the device may end up with
-    if (!((p.shape.tiles >> i) & 1)) continue;
-    const int bt = fused_tile(i).tokens;
-    const int64_t most = n_tokens < fused_tile_most(i) || named ? n_tokens : fused_tile_most(i);
-    for (int64_t tt = 1; tt <= (most + bt - 1) / bt; ++tt) {
-      const FusedSchedule s = fused_schedule_on((int)(tt * bt), p.shape, i);
-      const int padded = 8 * ((s.n_wg + 7) / 8);  // fused_locate deals whole rows of 8 workgroup ids
-      if (padded > p.grid) p.grid = padded;
-      const size_t rec = (size_t)tt * bt * s.n_splits * kPartsPerSplit;
-      if (rec > p.max_records) p.max_records = rec;
+  p.w_nt = p.full.n_ttiles <= (fused_tile(p.full.tile).tokens > 128 ? 4 : 1) && V * H * 2 >= (int64_t)288 << 20;
+  p.grid = p.full.n_wg;
+  if (masked) {  // whatever number of valid tokens and tile the device may end up with
+    for (int i = 0; i < kFusedTiles; ++i) {
+      if (!((p.shape.tiles >> i) & 1)) continue;
+      const int n_wg = fused_most_workgroups(p.shape, i, n_tokens < fused_tile_most(i) || named ? n_tokens : fused_tile_most(i));
+      p.grid = n_wg > p.grid ? n_wg : p.grid;
     }
   }
+  p.grid = 8 * ((p.grid + 7) / 8);  // fused_locate deals whole rows of 8 workgroup ids
   return p;
 }
 
-// Layout: [n_valid + schedule: 256 B][row_index: n_tokens int32, 256-aligned][partials per weight set]
-// [normalised hidden rows, only with a norm weight].
-inline size_t off_index() { return 256; }
-inline size_t off_partials(int64_t n_tokens) { return 256 + (((size_t)n_tokens * 4 + 255) & ~(size_t)255); }
-inline size_t normed_bytes(int64_t n_tokens, int64_t H, bool with_norm) {
-  return with_norm ? (((size_t)n_tokens * H * 2 + 255) & ~(size_t)255) : 0;
-}
-// The same on every device and for every output, whichever plan that makes.
+// Partials that a sweep over up to n_tokens can leave: the same on every device, with and without a mask and for every output, whichever
+// plan that makes.
 inline size_t partial_bytes(const FusedEnv& env, int64_t n_tokens, int64_t H, int64_t V) {
-  const size_t a = fused_plan(env, n_tokens, H, V, true, false, false).max_records;
-  const size_t b = fused_plan(env, n_tokens, H, V, false, false, false).max_records;
-  return (a > b ? a : b) * sizeof(FusedPartial);
+  const FusedKernel kernel = fused_kernel(env, n_tokens, H, V);
+  size_t most = kernel.nbt ? (size_t)64 * 512 : 0;  // the streaming kernel: one partial per (token, workgroup), at most 512
+  if (kernel.kind != kSmall) {
+    const uint32_t named = fused_named_tiles(env, true);
+    const FusedShape shape = fused_shape_on(env, kernel.kind, H, V, named | 3u | (named ? 0u : 0xffu), named != 0);
+    for (int i = 0; i < kFusedTiles; ++i) {
+      if (!((shape.tiles >> i) & 1)) continue;
+      const int64_t tokens = named || n_tokens < fused_tile_most(i) ? n_tokens : fused_tile_most(i);
+      const size_t records = (size_t)fused_most_workgroups(shape, i, tokens) * fused_tile(i).tokens * kPartsPerSplit;
+      most = records > most ? records : most;
+    }
+  }
+  return most * sizeof(FusedPartial);
 }
 
 // Two hidden matrices against one weight are ONE sweep over both where that is a batch of up to this many tokens: W is streamed once
@@ -281,11 +327,24 @@ inline size_t partial_bytes(const FusedEnv& env, int64_t n_tokens, int64_t H, in
 // 314 / 198, 512: 281 / 277 | 645 / 611, 768: 400 / 418 | 921 / 980; behind a mask that leaves 56 %, 128: 121 / 86 | 285 / 185, 512:
 // 170 / 140 | 380 / 301, 768: 236 / 222 | 538 / 471, 1024: 369 / 383 | 868 / 845.
 inline bool joint_fits(int64_t n_tokens, int64_t H, bool masked) { return n_tokens <= (masked ? 768 : 512) && H % kDmaSlab == 0; }
-// All partials of a call of `n_sweeps` sweeps.
-inline size_t partials_total(const FusedEnv& env, int64_t n_tokens, int64_t H, int64_t V, int n_sweeps) {
-  const size_t each = partial_bytes(env, n_tokens, H, V) * (size_t)n_sweeps;
+// Layout of the workspace: [n_valid + schedule: 256 B][row_index: n_tokens int32, 256-aligned][partials of the first sweep, of the
+// second][normalised hidden rows, per matrix, only with a norm weight].  Offsets in bytes.
+constexpr size_t kFusedIndexOffset = 256;
+struct FusedLayout {
+  size_t partials, partials_second, normed, normed_second, total;
+};
+inline size_t fused_align(size_t n) { return (n + 255) & ~(size_t)255; }
+inline FusedLayout fused_layout(const FusedEnv& env, int64_t n_tokens, int64_t H, int64_t V, int n_sweeps, int n_normed) {
+  FusedLayout l;
+  const size_t each = partial_bytes(env, n_tokens, H, V);
   const size_t joint = n_sweeps == 2 && joint_fits(n_tokens, H, true) ? partial_bytes(env, 2 * n_tokens, H, V) : 0;
-  return each > joint ? each : joint;
+  const size_t normed = fused_align((size_t)n_tokens * H * 2);
+  l.partials = kFusedIndexOffset + fused_align((size_t)n_tokens * 4);
+  l.partials_second = l.partials + each;
+  l.normed = l.partials + (each * n_sweeps > joint ? each * n_sweeps : joint);
+  l.normed_second = l.normed + normed;
+  l.total = fused_align(l.normed + normed * n_normed);
+  return l;
 }
 
 }  // namespace tome
