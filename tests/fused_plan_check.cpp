@@ -19,8 +19,8 @@ static void fault(const char* what, const FusedEnv& env, int64_t n, int64_t H, i
                 (long long)n, (long long)H, (long long)V, ent, masked, deep, (long long)n_valid, tile);
 }
 
-static void check_call(const FusedEnv& env, int64_t n, int64_t H, int64_t V, bool ent, bool masked, bool deep) {
-  const FusedPlan p = fused_plan(env, n, H, V, deep, ent, masked);
+static void check_call(const FusedEnv& env, int64_t n, int64_t H, int64_t V, bool ent, bool amax, bool masked, bool deep) {
+  const FusedPlan p = fused_plan(env, n, H, V, deep, ent, amax, masked);
   const size_t records = partial_bytes(env, n, H, V) / sizeof(FusedPartial);
 #define FAULT(what, n_valid, tile) fault(what, env, n, H, V, ent, masked, deep, n_valid, tile)
   if (p.kind == kSmall) {
@@ -37,6 +37,7 @@ static void check_call(const FusedEnv& env, int64_t n, int64_t H, int64_t V, boo
     if (p.kind == kDma && !p.any_tile) {  // launched by tile; a second sweep is one without the entropy
       if (!dma_has_form(tile, ent ? p.deep : p.deep_lp) || !dma_has_form(tile, p.deep_lp)) FAULT("no kernel form", n_valid, tile);
     }
+    if (p.any_tile && ent && !p.any_deep && p.w_nt) FAULT("non-temporal W without the third W buffer", n_valid, tile);
     if (p.any_tile && !deep) FAULT("device-chosen tile without the third W buffer", n_valid, tile);
     const FusedSchedule s = fused_schedule_on((int)n_valid, p.shape, tile);
     if (s.tile != tile || s.n_wg != s.n_ttiles * s.n_splits || s.n_splits < 1 || (int64_t)s.n_ttiles * fused_tile(tile).tokens < n_valid) FAULT("schedule", n_valid, tile);
@@ -68,7 +69,7 @@ static void check_call(const FusedEnv& env, int64_t n, int64_t H, int64_t V, boo
 static size_t plan_one_call(const FusedEnv& env, int64_t n, int64_t H, int64_t V) {
   size_t sum = fused_layout(env, n, H, V, 1, 0).total;
   sum += fused_kernel(env, n, H, V).kind + fused_layout(env, n, H, V, 1, 0).normed;
-  const FusedPlan p = fused_plan(env, n, H, V, true, false, false);
+  const FusedPlan p = fused_plan(env, n, H, V, true, false, false, false);
   return sum + p.grid + p.full.n_wg;
 }
 
@@ -95,12 +96,13 @@ int main(int argc, char** argv) {
     const FusedEnv env{selectors[rng() % 15], rng() % 8 ? 256 : 0};
     const int64_t n = (int64_t)spread(1, rng() % 4 ? 4000 : 70000), H = rng() % 8 ? 64 * (1 + (int64_t)(spread(1, 100))) : 8 * (1 + rng() % 500);
     const int64_t V = (int64_t)spread(16, 260000);
-    check_call(env, n, H, V, rng() & 1, rng() & 1, rng() % 8 != 0);
+    check_call(env, n, H, V, rng() & 1, rng() & 1, rng() & 1, rng() % 8 != 0);
   }
   for (const int selector : selectors)  // sizes at the rules' own lines
     for (const int64_t n : {1, 64, 65, 256, 257, 1024, 1025, 1452, 2048, 2049, 2560, 2561, 8192, 8193, 15580})
       for (const int64_t V : {223, 1068, 32000, 151936})
-        for (int bits = 0; bits < 8; ++bits, ++calls) check_call(FusedEnv{selector, 256}, n, bits & 4 ? 4864 : 1024, V, bits & 1, bits & 2, true);
+        for (int bits = 0; bits < 24; ++bits, ++calls)
+          check_call(FusedEnv{selector, 256}, n, bits >= 16 ? 4864 : bits >= 8 ? 1024 : 512, V, bits & 1, bits & 2, bits & 4, true);
   std::printf("%d calls, %d faults\n", calls, faults);
   return faults != 0;
 }

@@ -545,10 +545,12 @@ def test_fused_token_tiles_stream_large_w(dev, tile):
 
 
 @pytest.mark.parametrize("outputs", ["plain", "entropy", "argmax", "all"])
-@pytest.mark.parametrize("n,H,V", [(100, 128, 3000), (400, 512, 4500), (666, 128, 9000), (900, 64, 20000)])
+@pytest.mark.parametrize("n,H,V", [(100, 128, 3000), (400, 512, 4500), (666, 128, 9000), (900, 64, 20000), (1100, 512, 4500), (1100, 2048, 3000),
+                                   (1500, 1536, 2100), (2048, 64, 9000), (2048, 1024, 4481)])
 def test_fused_tile_chosen_on_device_every_logit(dev, n, H, V, outputs):
     """Behind a mask the device picks the token tile; the last tile ends inside a 16-token block.  Every row's lp and lse against
-    an fp32 product (rounding of an H-long sum at these magnitudes: under 1e-4), so that a single wrong partial shows."""
+    an fp32 product (rounding of an H-long sum at these magnitudes: under 1e-4), so that a single wrong partial shows.  The argmax'
+    logit is the product's largest up to both sums' rounding, and the id the product's wherever the second is further off."""
     g = torch.Generator(device=dev)
     g.manual_seed(n + V)
     w = torch.empty((V, H), device=dev).normal_(0, 0.05, generator=g).to(torch.bfloat16)
@@ -563,6 +565,14 @@ def test_fused_tile_chosen_on_device_every_logit(dev, n, H, V, outputs):
         m = valid.cpu().numpy()
         np.testing.assert_allclose(r.lse.cpu().numpy()[m], lse.cpu().numpy()[m], atol=1e-4, rtol=0)
         np.testing.assert_allclose(r.lp.cpu().numpy()[m], (x.gather(1, t[:, None])[:, 0] - lse).cpu().numpy()[m], atol=1e-4, rtol=0)
+        if r.argmax is not None:
+            top = x.topk(2, dim=-1)
+            bound = 4 * H * 2.0 ** -24 * h.float().abs().amax(dim=-1) * w.float().abs().max()  # twice conftest's: the product rounds as well
+            got = r.argmax.long()
+            assert (got[~valid] == -1).all()
+            assert (top.values[:, 0] - x.gather(1, got.clamp(min=0)[:, None])[:, 0] <= bound)[valid].all()
+            clear = valid & (top.values[:, 0] - top.values[:, 1] > bound)
+            assert clear.sum() >= 0.9 * valid.sum() and (got == top.indices[:, 0])[clear].all()
         if r.entropy is not None:
             p = torch.softmax(x.double(), dim=-1)
             want = torch.logsumexp(x.double(), dim=-1) - (p * x.double()).sum(-1)

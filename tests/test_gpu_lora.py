@@ -203,6 +203,7 @@ def test_grpo_pair_matches_oracle(dev, with_norm, shared_w, n, H):
     (1, 256, 700, False), (8, 1024, 3000, True), (32, 512, 3000, False),    # one sweep over both matrices: streaming kernel
     (33, 1024, 5000, False), (97, 128, 4481, True), (240, 64, 9000, True), (512, 192, 4481, False), (768, 128, 4481, True),
     (513, 64, 4481, False), (769, 64, 4481, True), (100, 72, 1000, True),   # two sweeps: more tokens; the generic kernel
+    (700, 2560, 1500, True), (768, 512, 4481, True),                        # one sweep past 1024 tokens: three and two W buffers
 ])
 @pytest.mark.parametrize("with_norm", [False, True])
 def test_grpo_pair_shared_weight_joint_and_separate(dev, n, H, V, masked, with_norm):

@@ -488,7 +488,7 @@ __global__ __launch_bounds__(k2WG) void fused_lmhead_dma_kernel(FusedArgs a) {
   auto sweep = [&](auto tile) {
     constexpr FusedTile kTile = fused_tile(decltype(tile)::value);
     constexpr int BT = kTile.tokens, NA = (BT + 32) / 64, NB = BT / 32 - NA, HI = kTile.unit32 == 1 ? 0 : kTile.unit32 - 4;
-    constexpr bool kDeep = DEEP && BT > 128;
+    constexpr bool kDeep = BT > 128 && (DEEP || BT < 256);
     constexpr bool kRot = BT <= 128 && !AMAX && (TILE == kAnyTile ? WNT : ROT);
     static_assert(BT == dma_tile_tokens(NA, NB), "two token waves of NA blocks, two of NB");
     const int wave_t = wave >> 1;
@@ -516,16 +516,22 @@ __global__ __launch_bounds__(k2WG) void fused_lmhead_dma_kernel(FusedArgs a) {
 
 template <bool ENT, bool AMAX, int TILE, bool DEEP, bool WNT, bool ROT = false>
 static void launch_dma_form(const FusedArgs& a, int grid, hipStream_t stream) {
-  constexpr int kLds = dma_lds_bytes(TILE == kAnyTile ? 256 : fused_tile(TILE < 0 ? 0 : TILE).tokens, DEEP);
+  constexpr int kTokens = fused_tile(TILE < 0 ? 0 : TILE).tokens;
+  constexpr int kLds = TILE != kAnyTile ? dma_lds_bytes(kTokens, DEEP) : DEEP ? dma_lds_bytes(256, true) : dma_lds_bytes(224, true);
+  static_assert(dma_lds_bytes(224, true) >= dma_lds_bytes(256), "the largest body of the combined kernel");
   static DeviceOnce attr_set;  // opt in to > 64 KB of dynamic LDS once per instantiation and device
   if (attr_set.first_on_current_device()) allow_big_lds(&fused_lmhead_dma_kernel<ENT, AMAX, TILE, DEEP, WNT, ROT>, kLds);
   hipLaunchKernelGGL((fused_lmhead_dma_kernel<ENT, AMAX, TILE, DEEP, WNT, ROT>), dim3((unsigned)grid), dim3(k2WG), kLds, stream, a);
 }
-// w_nt: non-temporal W requests (the kernel's WNT).
+// deep: three W buffers for the 256-token tile too (FusedPlan::any_deep); w_nt: non-temporal W requests (the kernel's WNT), which up to four
+// token tiles take and so never without `deep`.
 template <bool ENT, bool AMAX>
-void launch_dma_any(const FusedArgs& a, bool w_nt, int grid, hipStream_t stream) {
-  if (w_nt) launch_dma_form<ENT, AMAX, kAnyTile, true, true>(a, grid, stream);
-  else launch_dma_form<ENT, AMAX, kAnyTile, true, false>(a, grid, stream);
+void launch_dma_any(const FusedArgs& a, bool deep, bool w_nt, int grid, hipStream_t stream) {
+  if (w_nt) return launch_dma_form<ENT, AMAX, kAnyTile, true, true>(a, grid, stream);
+  if constexpr (ENT) {
+    if (!deep) return launch_dma_form<ENT, AMAX, kAnyTile, false, false>(a, grid, stream);
+  }
+  launch_dma_form<ENT, AMAX, kAnyTile, true, false>(a, grid, stream);
 }
 // False, and nothing launched, for a tile without the form asked for.
 template <bool ENT, bool AMAX>

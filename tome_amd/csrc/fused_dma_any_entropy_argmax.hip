@@ -2,5 +2,5 @@
 #include "fused_dma.hpp"
 
 namespace tome {
-template void launch_dma_any<true, true>(const FusedArgs&, bool, int, hipStream_t);
+template void launch_dma_any<true, true>(const FusedArgs&, bool, bool, int, hipStream_t);
 }  // namespace tome

@@ -688,7 +688,7 @@ void fused_force_kernel(int kind) { g_forced_kind.store(kind, std::memory_order_
 template <bool ENT, bool AMAX>
 bool launch_dma(const FusedArgs& a, int tile, bool deep, bool w_nt, int grid, hipStream_t stream);
 template <bool ENT, bool AMAX>
-void launch_dma_any(const FusedArgs& a, bool w_nt, int grid, hipStream_t stream);
+void launch_dma_any(const FusedArgs& a, bool deep, bool w_nt, int grid, hipStream_t stream);
 bool dma_allow_deep_lds();
 
 // Does the current device grant the 160 KB of dynamic LDS that the third W buffer asks for - all of a CU's LDS, which a
@@ -770,8 +770,8 @@ static int launch_main(const FusedArgs& a, const FusedPlan& plan, bool want_argm
   if (plan.kind == kDma) {
     const bool deep = ENT ? plan.deep : plan.deep_lp;
     if (a.sched_dev && plan.any_tile) {
-      if (want_argmax) launch_dma_any<ENT, true>(a, plan.w_nt, plan.grid, stream);
-      else launch_dma_any<ENT, false>(a, plan.w_nt, plan.grid, stream);
+      if (want_argmax) launch_dma_any<ENT, true>(a, plan.any_deep, plan.w_nt, plan.grid, stream);
+      else launch_dma_any<ENT, false>(a, plan.any_deep, plan.w_nt, plan.grid, stream);
     } else if (!(want_argmax ? launch_dma<ENT, true>(a, a.sched.tile, deep, plan.w_nt, plan.grid, stream)
                              : launch_dma<ENT, false>(a, a.sched.tile, deep, plan.w_nt, plan.grid, stream))) {
       return -1;
@@ -799,7 +799,7 @@ static hipError_t fused_launch_impl(const void* hidden, const int32_t* hidden_ro
   const FusedEnv env = fused_env();
   const bool joint = second && w1 == w0 && hidden_ref != hidden && joint_fits(n_tokens, H, sel.masked()) && env.forced != kGeneric;
   const int swept = (int)n_tokens << (joint ? 1 : 0);
-  const FusedPlan plan = fused_plan(env, swept, H, V, deep_lds_granted(), out_entropy != nullptr, sel.masked());
+  const FusedPlan plan = fused_plan(env, swept, H, V, deep_lds_granted(), out_entropy != nullptr, out_argmax != nullptr, sel.masked());
   int32_t* n_valid = nullptr;
   int32_t* row_index = nullptr;
   if (sel.masked()) {

@@ -189,6 +189,7 @@ struct FusedPlan {
   FusedShape shape;
   FusedSchedule full;  // of all tokens
   bool any_tile;       // kDma: behind a mask the device picks the token tile
+  bool any_deep;       // ... with three W buffers for 256 tokens too (sweeps with the entropy; the others always)
   int grid;            // workgroups to launch: behind a mask the most that any number of valid tokens can ask for
 };
 
@@ -250,7 +251,7 @@ inline FusedShape fused_shape_on(const FusedEnv& env, FusedKind kind, int64_t H,
 // One plan a call.  The host's planning of a whole call, the workspace's size asked for twice (by the caller and in the check), us: 200
 // tokens 1.8 -> 0.3, 4096 3.5 -> 0.2, 16384 117 -> 2.6, 65536 797 -> 2.9, against walking every number of token tiles of every tile, seven
 // times a call.
-inline FusedPlan fused_plan(const FusedEnv& env, int64_t n_tokens, int64_t H, int64_t V, bool deep_lds, bool entropy, bool masked) {
+inline FusedPlan fused_plan(const FusedEnv& env, int64_t n_tokens, int64_t H, int64_t V, bool deep_lds, bool entropy, bool argmax, bool masked) {
   FusedPlan p;
   const int forced = env.forced;
   const FusedKernel kernel = fused_kernel(env, n_tokens, H, V);
@@ -278,11 +279,21 @@ inline FusedPlan fused_plan(const FusedEnv& env, int64_t n_tokens, int64_t H, in
     if (forced == kForceDmaTwoWBuffers || forced == kForceDmaThreeWBuffers) p.shape.tiles = 3;
     if (p.shape.whole) p.shape.tiles &= ~((1u << 1) | (1u << 3));  // no vocab tiles of 224 rows
     if (masked && n_tokens > kAnyTileTokens && !named) p.shape.tiles &= 3u;
+    // 224 tokens and both optional outputs: the fold's spills outweigh the padding saved (660 of 1100 x 512 1.06 -> 0.98, 1.0 = 256 tokens)
+    if (any && n_tokens > 1024 && entropy && argmax && H < 1024 && !named) p.shape.tiles &= ~((1u << 2) | (1u << 3));
   }
   p.full = fused_schedule((int)n_tokens, p.shape);
+  const bool w_streams = V * H * 2 >= (int64_t)288 << 20;  // larger than the 256 MB memory-side cache
   // A mask of up to 64 tokens leaves the smallest tile; beyond kAnyTileTokens the 256-token tile serves.
   if (masked && (n_tokens <= 64 || n_tokens > kAnyTileTokens || !all_deep)) p.shape.tiles = 1u << p.full.tile;
   p.any_tile = masked && !fused_one_tile(p.shape);
+  // The combined kernel's 256-token body on three W buffers spills 67 registers around every fold with the entropy, 87 with the argmax too.
+  // Up to 1024 tokens, where few token tiles wait for the W stream, it wins all the same; beyond, where W does not stay in the caches and a
+  // tile has the K steps to pay for its fold.  To the 256-token kernel without a choice, three | two W buffers, 1280 .. 2048 tokens of which
+  // 25 .. 100 % count.  Entropy: H = 256 1.10 .. 1.14 | 1.00, 512 1.10 .. 1.18 | 1.01, 1024 1.01 .. 1.04 | 1.01, 1536 0.95 .. 1.03 | 1.01,
+  // 2048 0.93 .. 1.02 | 0.99.  Both: 512 1.19 .. 1.25 | 1.00, 1024 1.04 .. 1.10 | 1.00, 1536 0.97 .. 1.05 | 1.00, 2048 0.94 .. 1.02 | 1.00.  A W of
+  // 164 MB, H = 2560: up to 1536 tokens 0.57 .. 1.02 | 0.58 .. 1.01 (pairs 0.80 | 0.84), 1800 and 2048 1.00 .. 1.06 | 0.99 .. 1.01.
+  p.any_deep = n_tokens <= 1024 || (H >= (argmax ? 2048 : 1536) && (w_streams || (!argmax && n_tokens <= 1536)));
   p.w_nt = false;
   p.grid = 0;
   if (p.kind == kSmall) return p;  // a grid of its own; the schedule is ignored
@@ -290,7 +301,7 @@ inline FusedPlan fused_plan(const FusedEnv& env, int64_t n_tokens, int64_t H, in
   // found there again by the next call as long as it is requested normally (repeated calls, 64 tokens: V = 32000, H = 4096,
   // 262 MB: 48 us against 71 non-temporally; V = 50257, H = 768, 77 MB: 21.0 against 23.3).  Five token tiles already want
   // it kept (50257 x 4096, 1024 tokens as five tiles of 224: 396 us non-temporally, 354 normally).
-  p.w_nt = p.full.n_ttiles <= (fused_tile(p.full.tile).tokens > 128 ? 4 : 1) && V * H * 2 >= (int64_t)288 << 20;
+  p.w_nt = w_streams && p.full.n_ttiles <= (fused_tile(p.full.tile).tokens > 128 ? 4 : 1);
   p.grid = p.full.n_wg;
   if (masked) {  // whatever number of valid tokens and tile the device may end up with
     for (int i = 0; i < kFusedTiles; ++i) {
@@ -325,8 +336,11 @@ inline size_t partial_bytes(const FusedEnv& env, int64_t n_tokens, int64_t H, in
 // instead of twice and half-filled token tiles meet.  The sweep computes the entropy for the second matrix too, which at more tokens
 // costs what the sharing gives.  Two sweeps / one, us, V = 151936, H = 1024 | 2560: 16 tokens 104 / 56 | 239 / 124, 128: 126 / 90 |
 // 314 / 198, 512: 281 / 277 | 645 / 611, 768: 400 / 418 | 921 / 980; behind a mask that leaves 56 %, 128: 121 / 86 | 285 / 185, 512:
-// 170 / 140 | 380 / 301, 768: 236 / 222 | 538 / 471, 1024: 369 / 383 | 868 / 845.
+// 170 / 140 | 380 / 301, 768: 236 / 222 | 538 / 471, 1024: 369 / 383 | 868 / 845.  All tokens valid behind a mask, 640: 406 / 358 | 956 / 772,
+// 704 .. 768: 412 / 416 | 946 / 940 (H = 512: 221 / 219, 2048: 754 / 767), on the combined kernel's two W buffers (FusedPlan::any_deep; on three
+// 6 % more than two sweeps at H = 512, 4 at 1024).
 inline bool joint_fits(int64_t n_tokens, int64_t H, bool masked) { return n_tokens <= (masked ? 768 : 512) && H % kDmaSlab == 0; }
+
 // Layout of the workspace: [n_valid + schedule: 256 B][row_index: n_tokens int32, 256-aligned][partials of the first sweep, of the
 // second][normalised hidden rows, per matrix, only with a norm weight].  Offsets in bytes.
 constexpr size_t kFusedIndexOffset = 256;
