@@ -471,6 +471,76 @@ def test_fused_matrices_of_4_gib_and_more(dev, which, kind, n):
     check_argmax(h, w, r.argmax.cpu().numpy(), want)
 
 
+def _check_every_row(h, w, t, temperature, r, rows):
+    """lp, lse and, where returned, entropy and argmax of `rows` (bool, on the device) against the fp32 product, by vocabulary slices.
+    An H-long fp32 sum in another order: under 1e-4 at the magnitudes used here (logits of order 1), the row sums as much again."""
+    V = w.shape[0]
+    n = h.shape[0]
+    lse = torch.full((n,), -float("inf"), device=h.device, dtype=torch.float64)
+    hit, best = torch.zeros(n, device=h.device), torch.full((n,), -float("inf"), device=h.device)
+    mean = torch.zeros(n, device=h.device, dtype=torch.float64)     # sum of x * exp(x); logits are small
+    got = None if r.argmax is None else r.argmax.long().clamp(min=0)
+    at_got = torch.zeros(n, device=h.device)
+    hf = h.float()
+    for v0 in range(0, V, 16384):
+        x = hf @ w[v0:v0 + 16384].float().T / temperature
+        lse = torch.logaddexp(lse, torch.logsumexp(x.double(), dim=-1))
+        mean += (x.double() * x.double().exp()).sum(-1)
+        best = torch.maximum(best, x.amax(dim=-1))
+        for ids, into in ((t.long(), hit),) + (((got, at_got),) if got is not None else ()):
+            inside = (ids >= v0) & (ids < v0 + x.shape[1])
+            into[inside] = x.gather(1, (ids - v0).clamp(0, x.shape[1] - 1)[:, None])[inside, 0]
+    np.testing.assert_allclose(r.lse[rows].cpu().numpy(), lse[rows].cpu().numpy(), atol=2e-4, rtol=0)
+    np.testing.assert_allclose(r.lp[rows].cpu().numpy(), (hit - lse)[rows].cpu().numpy(), atol=2e-4, rtol=0)
+    if r.entropy is not None:
+        np.testing.assert_allclose(r.entropy[rows].cpu().numpy(), (lse - mean / lse.exp())[rows].cpu().numpy(), atol=4e-4, rtol=0)
+    if got is not None:
+        bound = 4 * h.shape[1] * 2.0 ** -24 * hf.abs().amax(dim=-1) * w.float().abs().max() / temperature
+        assert (r.argmax[rows] >= 0).all() and (best - at_got <= bound)[rows].all()
+        assert (r.argmax[~rows] == -1).all()
+
+
+OUTPUTS = {"plain": {}, "entropy": dict(want_entropy=True), "argmax": dict(want_argmax=True), "all": dict(want_entropy=True, want_argmax=True)}
+
+
+@pytest.mark.parametrize("outputs", list(OUTPUTS))
+@pytest.mark.parametrize("n,H,V,pitch,valid", [
+    (40, 4096, 50257, 4096, None), (90, 4096, 50257, 4096, None), (128, 4096, 50257, 4096, None),   # a tile of 64, 96, 128 tokens
+    (33, 4096, 36900, 4096, None), (70, 4096, 131072 + 9, 4096, None),                            # one tile a workgroup, and several
+    (100, 3968, 40000, 4096, None), (50, 8192, 20000, 8192, None),                                # a padded pitch; rows 16 KB apart
+    (60, 4096, 50257, 4096, 0.7), (128, 4096, 50257, 4096, 0.5), (300, 4096, 37000, 4096, 0.25),  # behind a mask
+])
+def test_fused_k_loops_start_apart(dev, n, H, V, pitch, valid, outputs):
+    """W is streamed, its rows lie a multiple of 8 KB apart and one tile of up to 128 tokens holds the batch: without the argmax the
+    workgroups start their K loops at different columns, with it they do not."""
+    g = torch.Generator(device=dev).manual_seed(n + V)
+    h = torch.empty((n, H), device=dev, dtype=torch.bfloat16).normal_(0, 1, generator=g)
+    w = torch.empty((V, pitch), device=dev, dtype=torch.bfloat16).normal_(0, 0.02, generator=g)[:, :H]
+    t = torch.randint(0, V, (n,), device=dev, generator=g)
+    t[:2] = torch.tensor([0, V - 1], device=dev)
+    rows = torch.rand(n, device=dev, generator=g) < (valid or 2.0)
+    r = tome_amd.fused_lmhead_logprobs(h, w, t, 0.9, row_valid=None if valid is None else rows, want_lse=True, **OUTPUTS[outputs])
+    _check_every_row(h, w, t, 0.9, r, rows)
+    assert (r.lp[~rows] == 0).all()
+
+
+@pytest.mark.parametrize("outputs", list(OUTPUTS))
+@pytest.mark.parametrize("n,H", [(100, 1024), (300, 1024), (700, 1024), (1024, 1024), (1100, 1024), (2048, 1024), (200, 2560), (1300, 2560)])
+def test_fused_tile_chosen_on_device_over_streamed_w(dev, n, H, outputs):
+    """Behind a mask, on a vocabulary whose W no cache holds: the kernel that chooses its tile on the device, non-temporally up to four tiles
+    and normally beyond, with shares of valid tokens that lead to different tiles."""
+    V = V_QWEN3
+    g = torch.Generator(device=dev).manual_seed(n + H)
+    h = torch.empty((n, H), device=dev, dtype=torch.bfloat16).normal_(0, 1, generator=g)
+    w = torch.empty((V, H), device=dev, dtype=torch.bfloat16).normal_(0, 0.02, generator=g)
+    t = torch.randint(0, V, (n,), device=dev, generator=g)
+    for share in (0.08, 0.3, 0.55, 0.8, 1.0):
+        rows = torch.rand(n, device=dev, generator=g) < share
+        r = tome_amd.fused_lmhead_logprobs(h, w, t, 1.0, row_valid=rows, want_lse=True, **OUTPUTS[outputs])
+        _check_every_row(h, w, t, 1.0, r, rows)
+        assert (r.lp[~rows] == 0).all()
+
+
 TOKEN_TILES = [64, 96, 128, 192, 224, 256]
 
 
@@ -519,7 +589,7 @@ def test_fused_token_tiles_agree(dev, n, H, V, outputs):
 
 @pytest.mark.parametrize("tile", TOKEN_TILES)
 def test_fused_token_tiles_stream_large_w(dev, tile):
-    """The non-temporal form, taken for a W beyond the memory-side cache and few token tiles: one ragged tile of every size."""
+    """The non-temporal form without a mask, taken for a W beyond the memory-side cache and few token tiles: one ragged tile of every size."""
     n, H, V = tile - 3, 1024, V_QWEN3
     g = torch.Generator(device=dev)
     g.manual_seed(tile)

@@ -204,6 +204,8 @@ def test_grpo_pair_matches_oracle(dev, with_norm, shared_w, n, H):
     (33, 1024, 5000, False), (97, 128, 4481, True), (240, 64, 9000, True), (512, 192, 4481, False), (768, 128, 4481, True),
     (513, 64, 4481, False), (769, 64, 4481, True), (100, 72, 1000, True),   # two sweeps: more tokens; the generic kernel
     (700, 2560, 1500, True), (768, 512, 4481, True),                        # one sweep past 1024 tokens: three and two W buffers
+    (24, 1024, 151936, True), (130, 1024, 151936, True), (300, 1024, 151936, True), (200, 2560, 151936, False),  # one sweep over a streamed W
+    (40, 4096, 50257, True),                                                 # ... its rows 8 KB apart
 ])
 @pytest.mark.parametrize("with_norm", [False, True])
 def test_grpo_pair_shared_weight_joint_and_separate(dev, n, H, V, masked, with_norm):

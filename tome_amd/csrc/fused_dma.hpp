@@ -114,8 +114,9 @@ __device__ __forceinline__ void pair_reads() {
 // 8 KB apart, the workgroups start their K loops at different slabs (the sums just begin elsewhere).  Not with the argmax: rows of W
 // that are equal bit for bit must have equal logits wherever they lie, or the first of them is not the one that is named.  In step, all of them would ask
 // the same few memory channels for the same columns of their rows: V = 50257 / 64001 / 100000 / 128256 / 151936 x H = 4096, 64 tokens
-// 96 -> 68, 120 -> 84, 144 -> 128, 161 -> 158, 194 -> 189 us, 128 tokens 100 -> 80, 123 -> 88, 157 -> 147, 172 -> 171, 213 -> 216.  Row
-// pitches of 2 and 5 KB gain nothing, nor does a W that the memory-side cache holds (32000 x 4096: 50.0 -> 50.5).
+// 94 -> 68, 119 -> 86, 143 -> 130, 197 -> 165, 201 -> 190 us, 96 tokens 96 -> 75, 121 -> 87, 152 -> 135, 198 -> 162, 221 -> 197, 128 tokens
+// 98 -> 81, 122 -> 91, 155 -> 151, 204 -> 174, 222 -> 218 (to the kernels before it; 42 shapes up to H = 8192 0.72 .. 0.98).  Row pitches
+// of 2 and 5 KB gain nothing, nor does a W that the memory-side cache holds (32000 x 4096: 50.0 -> 50.5).
 __device__ __host__ inline bool dma_rotates(const FusedArgs& a) { return (a.weight_stride_b & 8191) == 0; }
 // NBT: this wave's token blocks; BT: the workgroup's token tile; tok0: this wave's first token in it.
 template <bool ENT, bool AMAX, int NBT, int BT, int HI, bool DEEP, bool WNT, bool ROT>
