@@ -44,7 +44,7 @@ namespace tome {
 // all four SIMDs alike; the two widths are two bodies of one kernel that meet at the same barriers.  A tile costs its full
 // MFMA work and fill however few of its tokens exist, and at up to ~1500 tokens that padding was what most shapes were
 // furthest from their floor by (V = 151936, us before -> now, H = 1024 / 2560: 130 tokens 82 -> 70 / 183 -> 163, 200:
-// 83 -> 77 / 192 -> 187, 300: 131 -> 109 / 330 -> 262, 384: 132 -> 109 / 338 -> 256, 600: 193 -> 178 / 454 -> 425, 1300: 376 -> 351 /
+// 83 -> 77 / 189 -> 181, 300: 131 -> 109 / 330 -> 262, 384: 132 -> 109 / 338 -> 256, 600: 193 -> 178 / 454 -> 425, 1300: 376 -> 351 /
 // 883 -> 817).  160 = (3, 2) was built too: equal to 192 where it could be used.  fused_tile_cost holds the choice.
 constexpr int k2BV = 256, k2WG = 512;
 constexpr int k2BK = kDmaSlab;
@@ -101,8 +101,8 @@ __device__ __forceinline__ void pair_reads() {
 // barrier - and the hidden half, which comes from L2, one step ahead, after the step's own barrier; before a barrier
 // the four W instructions of the newest request stay in flight.  Faster wherever a step waits for its fill: 10-15 %
 // where every workgroup streams W rows of its own (one token tile), 2-3 % at 4096 x 1024 tokens x hidden, nothing from
-// 8192 x 4096 on; with the entropy or the argmax its fold spills and it only pays at one or two token tiles
-// (fused_plan holds the rule and the figures).
+// 8192 x 4096 on; with the entropy its fold spills and it only pays up to 1024 tokens, behind a mask also beyond where a tile has the
+// K steps for it (fused_plan, FusedPlan::any_deep: rules and figures).
 //
 // WNT: W is requested non-temporally.  Where W streams through once or a few times (up to four token tiles) its rows have
 // no business in the caches that the hidden rows and the partials live in: 64 x 4096 tokens x hidden 221 -> 205 us,

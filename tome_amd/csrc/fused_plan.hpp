@@ -287,7 +287,7 @@ inline FusedPlan fused_plan(const FusedEnv& env, int64_t n_tokens, int64_t H, in
   // A mask of up to 64 tokens leaves the smallest tile; beyond kAnyTileTokens the 256-token tile serves.
   if (masked && (n_tokens <= 64 || n_tokens > kAnyTileTokens || !all_deep)) p.shape.tiles = 1u << p.full.tile;
   p.any_tile = masked && !fused_one_tile(p.shape);
-  // The combined kernel's 256-token body on three W buffers spills 67 registers around every fold with the entropy, 87 with the argmax too.
+  // The combined kernel's 256-token body on three W buffers spills 67 registers with the entropy, 87 with the argmax too, most of them around every fold.
   // Up to 1024 tokens, where few token tiles wait for the W stream, it wins all the same; beyond, where W does not stay in the caches and a
   // tile has the K steps to pay for its fold.  To the 256-token kernel without a choice, three | two W buffers, 1280 .. 2048 tokens of which
   // 25 .. 100 % count.  Entropy: H = 256 1.10 .. 1.14 | 1.00, 512 1.10 .. 1.18 | 1.01, 1024 1.01 .. 1.04 | 1.01, 1536 0.95 .. 1.03 | 1.01,

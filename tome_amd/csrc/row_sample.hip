@@ -595,7 +595,7 @@ __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 // head and tail) are left to the second launch.
 template <typename T>
 __global__ __launch_bounds__(kRowWG) __attribute__((amdgpu_waves_per_eu(6, 8))) void row_sample_cells_kernel(SampleArgs a) {
-  touch_args(a);  // 64 x 151936 fp32, both launches, 13.46 -> 13.39 us; in the pick launch, which loads cells first, it costs 0.1
+  touch_args(a);  // 64 x 151936 fp32 in a captured graph, both launches, 13.23 -> 13.16 us (whole calls: equal); in the pick launch, which loads cells first, it costs 0.1
   constexpr int kVec = Elem<T>::kVec;
   const int64_t r = blockIdx.x / a.splits;
   const int split = blockIdx.x % a.splits;
