@@ -38,6 +38,7 @@ static void check_call(const FusedEnv& env, int64_t n, int64_t H, int64_t V, boo
       if (!dma_has_form(tile, ent ? p.deep : p.deep_lp) || !dma_has_form(tile, p.deep_lp)) FAULT("no kernel form", n_valid, tile);
     }
     if (p.any_tile && ent && !p.any_deep && p.w_nt) FAULT("non-temporal W without the third W buffer", n_valid, tile);
+    if (p.any_tile && env.forced == kForceDmaThreeWBuffers && !p.any_deep) FAULT("selected third W buffer not taken", n_valid, tile);
     if (p.any_tile && !deep) FAULT("device-chosen tile without the third W buffer", n_valid, tile);
     const FusedSchedule s = fused_schedule_on((int)n_valid, p.shape, tile);
     if (s.tile != tile || s.n_wg != s.n_ttiles * s.n_splits || s.n_splits < 1 || (int64_t)s.n_ttiles * fused_tile(tile).tokens < n_valid) FAULT("schedule", n_valid, tile);

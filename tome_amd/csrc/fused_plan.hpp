@@ -293,7 +293,7 @@ inline FusedPlan fused_plan(const FusedEnv& env, int64_t n_tokens, int64_t H, in
   // 25 .. 100 % count.  Entropy: H = 256 1.10 .. 1.14 | 1.00, 512 1.10 .. 1.18 | 1.01, 1024 1.01 .. 1.04 | 1.01, 1536 0.95 .. 1.03 | 1.01,
   // 2048 0.93 .. 1.02 | 0.99.  Both: 512 1.19 .. 1.25 | 1.00, 1024 1.04 .. 1.10 | 1.00, 1536 0.97 .. 1.05 | 1.00, 2048 0.94 .. 1.02 | 1.00.  A W of
   // 164 MB, H = 2560: up to 1536 tokens 0.57 .. 1.02 | 0.58 .. 1.01 (pairs 0.80 | 0.84), 1800 and 2048 1.00 .. 1.06 | 0.99 .. 1.01.
-  p.any_deep = n_tokens <= 1024 || (H >= (argmax ? 2048 : 1536) && (w_streams || (!argmax && n_tokens <= 1536)));
+  p.any_deep = n_tokens <= 1024 || forced == kForceDmaThreeWBuffers || (H >= (argmax ? 2048 : 1536) && (w_streams || (!argmax && n_tokens <= 1536)));
   p.w_nt = false;
   p.grid = 0;
   if (p.kind == kSmall) return p;  // a grid of its own; the schedule is ignored
